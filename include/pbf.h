@@ -208,8 +208,10 @@ int pbf_density(pbf_ctx* ctx, const float* d_x, const int* d_index, const int* d
 
 /* DensityPBD::constrain (DensityPBD.cu:271-302) over a caller NeighborList
  * (d_index: n row starts, d_elems: nelems ids; any list, symmetric or not):
- * `iterations` Jacobi rounds of density, lambda and pairwise displacement
- * (float atomics, as the reference), then v += (x - x_old)/dt. x and v are
+ * `iterations` Jacobi rounds of density, lambda and pairwise displacement,
+ * then v += (x - x_old)/dt. A list that lists every pair both ways (checked on
+ * the device) runs without atomics and gives the same bits every time; any
+ * other one sums the displacements with float atomics, as the reference. x and v are
  * updated in place; d_rho (may be NULL) receives the last iteration's
  * density. */
 int pbf_pbd_constrain(pbf_ctx* ctx, float* d_x, float* d_v, const int* d_index,
@@ -226,10 +228,10 @@ int pbf_pbd_constrain_mass(pbf_ctx* ctx, float* d_x, float* d_v, const int* d_in
  * for callers that cannot allocate device memory (code under HIP graph
  * capture, tight serving loops, harnesses that forbid hipMalloc). Same
  * arguments, semantics and results (to float-atomic summation order) as
- * pbf_pbd_constrain, but its scratch (iterate positions and displacement
- * sums) is a fixed array in the library, one copy per device, instead of the
+ * pbf_pbd_constrain, but its scratch (two buffers of iterate
+ * positions) is a fixed array in the library, one copy per device, instead of the
  * context's reservation: at most PBF_NOALLOC_MAX_PARTICLES particles
- * (PBF_ERR_UNSUPPORTED beyond). The array holds 28 MiB on every device the
+ * (PBF_ERR_UNSUPPORTED beyond). The array holds 32 MiB on every device the
  * library runs on until the process ends. Every call on one device shares
  * that device's array: calls that overlap on one device (several streams,
  * threads or contexts) race and must be serialized by the caller. The

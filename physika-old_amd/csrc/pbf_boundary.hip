@@ -8,6 +8,7 @@
 //    a sampled signed distance field of the box (DistanceField3D.cu:90-129,
 //    194-201,283-291) and K_ConstrainSDF (BoundaryConstraint.cu:30-67), run on
 //    the particles before each fluid step.
+#include "pbf_csr.h"
 #include "pbf_nbr.h"
 
 namespace pbf {
@@ -348,22 +349,29 @@ __global__ __launch_bounds__(kBlock) void k_csr_viscosity(const float4* __restri
                                                           const float4* __restrict__ v_in,
                                                           float4* __restrict__ v_next, float* __restrict__ v_out,
                                                           VisConst vc) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= nb.n) return;
+  const CsrRow row = csr_row(nb);
+  if (row.i >= nb.n) return;
+  const int i = row.i;
   const float4 xi = xa[i];
   float tw = 0.0f, dx = 0.0f, dy = 0.0f, dz = 0.0f;
-  for (int e = nb.begin(i), end = nb.end(i); e < end; ++e) {
-    const int j = nb.elems[e];
-    const PairGeom g = pair_geom(xi, xa[j], vc.inv_h);
-    if (g.r > vc.eps) {
-      const float w = vc.cw * g.t;
-      const float4 vj = v_in[j];
-      tw += w;
-      dx += w * vj.x;
-      dy += w * vj.y;
-      dz += w * vj.z;
-    }
-  }
+  csr_each(
+      nb, row, [&](int j) { return VisPair{xa[j], v_in[j]}; },
+      [&](int, int, const VisPair& q, bool on) {
+        const PairGeom g = pair_geom(xi, q.x, vc.inv_h);
+        if (on && g.r > vc.eps) {
+          const float w = vc.cw * g.t;
+          tw += w;
+          dx += w * q.v.x;
+          dy += w * q.v.y;
+          dz += w * q.v.z;
+        }
+      },
+      [] {});
+  tw = row_sum(tw);
+  dx = row_sum(dx);
+  dy = row_sum(dy);
+  dz = row_sum(dz);
+  if (row.lane != 0) return;
   const float b = tw < vc.eps ? 0.0f : vc.b;
   tw = tw < vc.eps ? 1.0f : tw;
   const float ob = 1.0f + b;
@@ -382,7 +390,7 @@ __global__ __launch_bounds__(kBlock) void k_csr_viscosity(const float4* __restri
 
 void launch_csr_viscosity(const float4* xa, const Csr& nb, const float4* v_old, const float4* v_in, float4* v_next,
                           float* v_out, const VisConst& vc, hipStream_t st) {
-  k_csr_viscosity<<<(nb.n + kBlock - 1) / kBlock, kBlock, 0, st>>>(xa, nb, v_old, v_in, v_next, v_out, vc);
+  k_csr_viscosity<<<csr_blocks(nb.n), kBlock, 0, st>>>(xa, nb, v_old, v_in, v_next, v_out, vc);
 }
 
 }  // namespace pbf

@@ -18,13 +18,13 @@
 
 using namespace pbf;
 
-// Scratch of pbf_pbd_constrain_noalloc: the iterate positions (float4) and the
-// displacement sums (3 floats) of up to PBF_NOALLOC_MAX_PARTICLES particles,
-// 28 MiB on every device the library runs on, held until the process ends.
+// Scratch of pbf_pbd_constrain_noalloc: two buffers of iterate positions
+// (float4) of up to PBF_NOALLOC_MAX_PARTICLES particles and the list's pairing
+// sums, 32 MiB on every device the library runs on, held until the process ends.
 // In host code the name is no device address: each device's copy is looked
 // up once (scratch_address) and only that pointer reaches kernels.
 static __device__ __align__(256) unsigned char
-    scratch[(size_t)PBF_NOALLOC_MAX_PARTICLES * (sizeof(float4) + 3 * sizeof(float))];
+    scratch[2 * (size_t)PBF_NOALLOC_MAX_PARTICLES * sizeof(float4) + kPairingSlots * sizeof(unsigned long long)];
 
 struct pbf_ctx {
   pbf_params p{};
@@ -55,7 +55,7 @@ struct pbf_ctx {
   int *nbr_cnt = nullptr, *cnt_orig = nullptr;
   float4 *xn = nullptr, *x0 = nullptr, *xa = nullptr, *xb = nullptr, *vs = nullptr, *vv = nullptr;
   float* xc = nullptr;  // sorted x^n as three coordinate planes of cap + kXnPad floats
-  float* dpos = nullptr;
+  unsigned long long* pairing = nullptr;  // kPairingSlots: pairing sums of a caller's list
   // neighbor pass output: per-wave metadata, bit masks (scratch), lists
   long long* mask_base = nullptr;
   long long* list_base = nullptr;
@@ -539,7 +539,7 @@ int ensure_particles(pbf_ctx* c, int n, int nscenes) {
   dfree(c->sid); dfree(c->ssid); dfree(c->bpart); dfree(c->nbr_cnt); dfree(c->cnt_orig);
   dfree(c->tid); dfree(c->pid);
   dfree(c->xn); dfree(c->x0); dfree(c->xa); dfree(c->xb); dfree(c->vs); dfree(c->vv); dfree(c->xc);
-  dfree(c->dpos); dfree(c->mask_base); dfree(c->list_base); dfree(c->list_jbase); dfree(c->list_mode);
+  dfree(c->mask_base); dfree(c->list_base); dfree(c->list_jbase); dfree(c->list_mode);
   dfree(c->stage); dfree(c->cnt_a); dfree(c->wave_stat); dfree(c->oog_rcnt); dfree(c->oog_rev);
   dfree(c->oog_flag); dfree(c->oog_pre);
   c->cap_n = 0;
@@ -563,8 +563,6 @@ int ensure_particles(pbf_ctx* c, int n, int nscenes) {
   PBF_HIP(c, hipMalloc(&c->xb, nf4));
   PBF_HIP(c, hipMalloc(&c->vs, nf4));
   PBF_HIP(c, hipMalloc(&c->vv, nf4));
-  PBF_HIP(c, hipMalloc(&c->dpos, 3 * sizeof(float) * (size_t)cap));
-  PBF_HIP(c, hipMemset(c->dpos, 0, 3 * sizeof(float) * (size_t)cap));
   const size_t nwv = (size_t)(cap / 64 + 4);
   PBF_HIP(c, hipMalloc(&c->mask_base, sizeof(long long) * nwv));
   PBF_HIP(c, hipMalloc(&c->list_base, sizeof(long long) * nwv));
@@ -802,7 +800,9 @@ int record_counters(pbf_ctx* c, hipStream_t st) {
 }
 
 // CSR of the last search in original ids, in the reference's NeighborList
-// layout: d_index[0..n-1] exclusive row starts, *total elements.
+// layout: d_index[0..n-1] exclusive row starts, *total elements. The row starts
+// are counted and the total read back once per search: a caller asks for the
+// size first, then for the lists.
 int export_csr(pbf_ctx* c, int n, int* d_index, int* d_elems, long long cap, long long* total, hipStream_t st) {
   if (n == 0) {
     *total = 0;
@@ -861,20 +861,6 @@ hipError_t scratch_address(int device, void** out) {
   }
   *out = g_scratch_ptr[device];
   return hipSuccess;
-}
-
-// DensityPBD::takeOneIteration x K over a caller list (DensityPBD.cu:306-365),
-// then DP_UpdateVelocity (:368-388): xa holds the caller's x on entry, dpos
-// zeros; minv selects the massInv variant.
-void pbd_csr_rounds(const pbf_ctx* c, float4* xa, float* dpos, const Csr& nb, float* d_x, float* d_v,
-                    float* d_rho, int n, const float* minv, hipStream_t st) {
-  for (int it = 0; it < c->p.iterations; ++it) {
-    const bool last = it + 1 == c->p.iterations;
-    launch_csr_lambda(xa, nb, last ? d_rho : nullptr, c->pc, st, minv);
-    launch_csr_dx_atomic(xa, nb, dpos, c->pc, st, minv);
-    launch_csr_apply(xa, dpos, n, st);
-  }
-  launch_csr_finish(xa, d_x, d_v, n, c->pc.dt, st);
 }
 
 // Samples of the box field (K_DistanceFieldToBox, computed on the device once
@@ -1294,7 +1280,8 @@ int pbf_create(const pbf_params* p, pbf_ctx** out) {
       hipEventCreateWithFlags(&c->counters_ev, hipEventDisableTiming) != hipSuccess ||
       hipStreamCreateWithFlags(&c->cap_stream, hipStreamNonBlocking) != hipSuccess ||
       hipMalloc(&c->off1, sizeof(int) * 2) != hipSuccess || hipMalloc(&c->total_cells, sizeof(int)) != hipSuccess ||
-      hipMalloc(&c->scan_part, sizeof(int) * (kScanDevBlocks + 1)) != hipSuccess) {
+      hipMalloc(&c->scan_part, sizeof(int) * (kScanDevBlocks + 1)) != hipSuccess ||
+      hipMalloc(&c->pairing, sizeof(unsigned long long) * kPairingSlots) != hipSuccess) {
     pbf_destroy(c);
     return PBF_ERR_HIP;
   }
@@ -1318,12 +1305,13 @@ int pbf_destroy(pbf_ctx* c) {
   if (!c) return PBF_ERR_INVALID;
   (void)hipDeviceSynchronize();
   dfree(c->off1); dfree(c->scene_minmax); dfree(c->win); dfree(c->total_cells); dfree(c->scan_part);
+  dfree(c->pairing);
   dfree(c->cell_cnt); dfree(c->cell_start);
   dfree(c->key); dfree(c->slot); dfree(c->tmp); dfree(c->perm); dfree(c->inv);
   dfree(c->sid); dfree(c->ssid); dfree(c->bpart); dfree(c->nbr_cnt); dfree(c->cnt_orig);
   dfree(c->tid); dfree(c->pid);
   dfree(c->xn); dfree(c->x0); dfree(c->xa); dfree(c->xb); dfree(c->vs); dfree(c->vv); dfree(c->xc);
-  dfree(c->dpos); dfree(c->mask_base); dfree(c->list_base); dfree(c->list_jbase); dfree(c->list_mode);
+  dfree(c->mask_base); dfree(c->list_base); dfree(c->list_jbase); dfree(c->list_mode);
   dfree(c->stage); dfree(c->cnt_a); dfree(c->wave_stat); dfree(c->oog_rcnt); dfree(c->oog_rev);
   dfree(c->oog_flag); dfree(c->oog_pre);
   dfree(c->mask); dfree(c->list); dfree(c->scan_scratch); dfree(c->bf.d);
@@ -1449,8 +1437,7 @@ int pbf_pbd_constrain(pbf_ctx* c, float* d_x, float* d_v, const int* d_index, co
   s = ensure_particles(c, n, 1);
   if (s) return s;
   hipStream_t st = (hipStream_t)stream;
-  launch_aos_to_f4(d_x, c->xa, n, st);
-  pbd_csr_rounds(c, c->xa, c->dpos, nb, d_x, d_v, d_rho, n, nullptr, st);
+  launch_csr_constrain(c->xa, c->xb, c->pairing, nb, d_x, d_v, d_rho, c->pc, c->p.iterations, nullptr, st);
   PBF_LAUNCHED(c);
   return PBF_OK;
 }
@@ -1470,9 +1457,9 @@ int pbf_pbd_constrain_noalloc(pbf_ctx* c, float* d_x, float* d_v, const int* d_i
   if (s) return s;
   hipStream_t st = (hipStream_t)stream;
   float4* xa = static_cast<float4*>(c->noalloc_scratch);
-  float* dpos = reinterpret_cast<float*>(xa + PBF_NOALLOC_MAX_PARTICLES);
-  launch_aos_to_f4_clear(d_x, xa, dpos, n, st);
-  pbd_csr_rounds(c, xa, dpos, nb, d_x, d_v, d_rho, n, nullptr, st);
+  float4* xb = xa + PBF_NOALLOC_MAX_PARTICLES;
+  auto* pairing = reinterpret_cast<unsigned long long*>(xb + PBF_NOALLOC_MAX_PARTICLES);
+  launch_csr_constrain(xa, xb, pairing, nb, d_x, d_v, d_rho, c->pc, c->p.iterations, nullptr, st);
   PBF_LAUNCHED(c);
   return PBF_OK;
 }
@@ -1802,8 +1789,7 @@ int pbf_pbd_constrain_mass(pbf_ctx* c, float* d_x, float* d_v, const int* d_inde
   s = ensure_particles(c, n, 1);
   if (s) return s;
   hipStream_t st = (hipStream_t)stream;
-  launch_aos_to_f4(d_x, c->xa, n, st);
-  pbd_csr_rounds(c, c->xa, c->dpos, nb, d_x, d_v, d_rho, n, d_mass_inv, st);
+  launch_csr_constrain(c->xa, c->xb, c->pairing, nb, d_x, d_v, d_rho, c->pc, c->p.iterations, d_mass_inv, st);
   PBF_LAUNCHED(c);
   return PBF_OK;
 }

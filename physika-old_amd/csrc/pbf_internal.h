@@ -321,18 +321,16 @@ void launch_csr_viscosity(const float4* xa, const Csr& nb, const float4* v_old, 
 void launch_integrate(float* x, float* v, const float* f, int n, const PhysConst& pc, hipStream_t st);
 void launch_csr_density(const float* x, const Csr& nb, float* rho, const PhysConst& pc, hipStream_t st);
 void launch_aos_to_f4(const float* x, float4* xa, int n, hipStream_t st);
-// as launch_aos_to_f4, and dpos[0 .. 3n) := 0
-void launch_aos_to_f4_clear(const float* x, float4* xa, float* dpos, int n, hipStream_t st);
-void launch_csr_lambda(float4* xa, const Csr& nb, float* rho, const PhysConst& pc, hipStream_t st,
-                       const float* minv = nullptr);
-void launch_csr_dx_atomic(const float4* xa, const Csr& nb, float* dpos, const PhysConst& pc, hipStream_t st,
-                          const float* minv = nullptr);
+// DensityPBD::constrain, K rounds, over a caller list of any form: xa and xb
+// hold n float4 each, pairing kPairingSlots words (nothing of them is read
+// before it is written).
+constexpr int kPairingSlots = 16;
+void launch_csr_constrain(float4* xa, float4* xb, unsigned long long* pairing, const Csr& nb, float* x, float* v,
+                          float* rho, const PhysConst& pc, int K, const float* minv, hipStream_t st);
 // Fixed-capacity rows (the `limit` nearest of each neighbor set, by distance
 // then id) in original ids; limit <= kFixedMax.
 constexpr int kFixedMax = 32;
 void launch_nbr_fixed(const NbrView& nv, const int* perm, int limit, int* counts, int* elems, hipStream_t st);
-void launch_csr_apply(float4* xa, float* dpos, int n, hipStream_t st);
-void launch_csr_finish(const float4* xa, float* x, float* v, int n, float dt, hipStream_t st);
 
 // Records msg as the context's last error and returns status (host code of
 // the library's other translation units).
