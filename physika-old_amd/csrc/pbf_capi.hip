@@ -173,6 +173,7 @@ struct pbf_ctx {
   bool counters_pending = false;
 
   int last_n = -1;  // particle count of the last neighbor search (-1: none)
+  long long csr_total = -1;  // its list elements once cnt_orig holds their row starts (-1: not yet)
 
   int pass_block = kBlock;  // threads per workgroup of the PBD passes (pbf_tuning)
   bool pass_persistent = false;  // persistent launches of the PBD passes (pbf_tuning)
@@ -781,6 +782,7 @@ int search(pbf_ctx* c, const SortIn& in, int n, const int* scene_off, int nscene
   c->stats_waves = (n + 63) / 64;
   PBF_LAUNCHED(c);
   c->last_n = n;
+  c->csr_total = -1;
   return PBF_OK;
 }
 
@@ -808,20 +810,26 @@ int export_csr(pbf_ctx* c, int n, int* d_index, int* d_elems, long long cap, lon
     *total = 0;
     return PBF_OK;
   }
-  launch_invert(c->perm, c->inv, n, st);
-  launch_csr_count(c->nbr_cnt, c->inv, n, c->cnt_orig, st);
-  // cnt_orig holds cap_n > n entries: the scan writes n + 1 in place
-  scan_exclusive(c->cnt_orig, c->cnt_orig, n, c->scan_scratch, st);
-  PBF_LAUNCHED(c);
+  const bool counted = c->csr_total >= 0;
+  if (!counted) {
+    launch_invert(c->perm, c->inv, n, st);
+    launch_csr_count(c->nbr_cnt, c->inv, n, c->cnt_orig, st);
+    // cnt_orig holds cap_n > n entries: the scan writes n + 1 in place
+    scan_exclusive(c->cnt_orig, c->cnt_orig, n, c->scan_scratch, st);
+    PBF_LAUNCHED(c);
+  }
   PBF_HIP(c, hipMemcpyAsync(d_index, c->cnt_orig, sizeof(int) * (size_t)n, hipMemcpyDeviceToDevice, st));
-  int tot = 0;
-  PBF_HIP(c, hipMemcpyAsync(&tot, c->cnt_orig + n, sizeof(int), hipMemcpyDeviceToHost, st));
-  PBF_HIP(c, hipStreamSynchronize(st));
-  *total = tot;
+  if (!counted) {
+    int tot = 0;
+    PBF_HIP(c, hipMemcpyAsync(&tot, c->cnt_orig + n, sizeof(int), hipMemcpyDeviceToHost, st));
+    PBF_HIP(c, hipStreamSynchronize(st));
+    c->csr_total = tot;
+  }
+  *total = c->csr_total;
   if (d_elems == nullptr) return PBF_OK;
-  if (cap < (long long)tot)
+  if (cap < c->csr_total)
     return fail(c, PBF_ERR_CAPACITY, "neighbor element buffer holds " + std::to_string(cap) + ", need " +
-                                         std::to_string(tot));
+                                         std::to_string(c->csr_total));
   launch_csr_fill(view_of(c, n), c->perm, c->cnt_orig, d_elems, cap, st);
   PBF_LAUNCHED(c);
   return PBF_OK;

@@ -109,6 +109,22 @@ __device__ __forceinline__ int wave_max_full(int v) {
              max(__builtin_amdgcn_readlane(v, 47), __builtin_amdgcn_readlane(v, 63)));
 }
 
+// Exchanges a and b when c holds (per lane: selects on values in registers; a
+// select between whole structs becomes one between their addresses, which puts
+// them in memory).
+__device__ __forceinline__ void swap_if(bool c, float& a, float& b) {
+  const float x = c ? b : a, y = c ? a : b;
+  a = x;
+  b = y;
+}
+
+// Between LDS writes and reads of one wave (its LDS operations complete in
+// order): keeps the compiler from moving any across.
+__device__ __forceinline__ void wave_lds_fence() {
+  asm volatile("" ::: "memory");
+  __builtin_amdgcn_wave_barrier();
+}
+
 __device__ __forceinline__ int wave_inclusive_scan(int v) {
   const int lane = threadIdx.x & 63;
 #pragma unroll

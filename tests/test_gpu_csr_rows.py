@@ -6,7 +6,7 @@ without atomics, every other one as the reference's pairwise scatter. Each form
 is held against a literal scatter in double (dp_ij to i, -dp_ij to j for every
 listed pair, K_ComputeDisplacement, DensityPBD.cu:135-179) with the bars of the
 step parity: 1e-6 m, 1e-3 m/s and 1e-5 of the density, or twice what the same
-scatter in single precision is from it.
+scatter in single precision is from it. The limited rows and the list export are whole numbers: exact.
 Every call goes through the C ABI."""
 import numpy as np
 import pytest
@@ -151,3 +151,44 @@ def test_density_and_viscosity_row_lengths(fluid, scene):
         if w.sum() > 0:
             mean = (w[:, None] * v[row]).sum(0) / w.sum()
             assert np.abs(vd[i].cpu().numpy() - (v[i] + mean * b) / (1 + b)).max() <= 1e-5
+
+
+@pytest.mark.parametrize("storage, spacing", [("list", 0.0061), ("list", 0.0028), ("staged", 0.0061),
+                                              ("staged", 0.0028), ("masks", 0.0061), ("masks", 0.0028),
+                                              ("index32", 0.005)])
+def test_limited_rows_and_export(fluid, scene, storage, spacing):
+    """Limited rows of 1, 20 and 32 and the exported list, over rows of up to 45
+    (spacing 0.0061), 81 (0.005; a slab whose cell planes hold 41k particles, so
+    that waves keep 32-bit lists) and over 300 neighbors (0.0028, several
+    rounds), against a search over all particles."""
+    if storage == "index32":
+        x = scene.jittered_lattice((128, 128, 8), (0.18, 0.18, 0.4), spacing, 0.1, seed=6)
+    else:
+        x = scene.jittered_lattice((14, 13, 11), (0.3, 0.5, 0.3), spacing, 0.1, seed=33)
+        x = np.ascontiguousarray(x[np.random.default_rng(11).permutation(len(x))])
+    n = len(x)
+    opts = {"staged": dict(stage_min_particles=1), "masks": dict(list_slots=4)}.get(storage, {})
+    ctx = fluid.Context("cuda:0", **opts)
+    xd = dev(x)
+    for _ in range(2):  # the second search has lists as long as it needs
+        nl = ctx.neighbor_query(xd)
+        torch.cuda.synchronize()
+    got = nl.rows()
+    limits = (1, 20, 32)
+    fixed = [(r.elements.cpu().numpy(), r.index.cpu().numpy())
+             for r in (ctx.neighbor_query_fixed(xd, k) for k in limits)]
+    f = np.float32
+    longest = 0
+    for i in range(0, n, max(1, n // 400)):
+        d = (x[i] - x).astype(f)
+        r = np.sqrt((d[:, 0] * d[:, 0] + d[:, 1] * d[:, 1]) + d[:, 2] * d[:, 2])
+        near = np.flatnonzero(r < f(0.0125))
+        longest = max(longest, len(near))
+        np.testing.assert_array_equal(np.sort(got[i]), near)
+        order = near[np.lexsort((near, r[near]))]
+        for k, (el, counts) in zip(limits, fixed):
+            assert counts[i] == min(k, len(near))
+            np.testing.assert_array_equal(el[k * i:k * i + counts[i]], order[:k])
+            assert (el[k * i + counts[i]:k * (i + 1)] == -1).all()
+    say(f"limited rows and export, {storage}, spacing {spacing}: {n} particles, rows of up to {longest}")
+    assert longest > (128 if spacing < 0.005 else 32)
