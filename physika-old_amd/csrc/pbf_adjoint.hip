@@ -27,8 +27,8 @@
 // p_bar_0 - c. c can exceed the rest by orders of magnitude, so the iterates
 // are carried as e = p_bar - c (e_K = x_bar', e_k = e_{k+1} + J_k^T (e_{k+1}
 // + c), x*_bar = e_0) and f = e + c enters only the pair terms.
-// Arithmetic is not contracted, so every neighbor-storage path of the list
-// traversal gives the same bits.
+// Fused multiply-adds are written out and nothing else is contracted, so every
+// neighbor-storage path of the list traversal gives the same bits.
 #include "pbf_nbr.h"
 
 namespace pbf {
@@ -66,7 +66,7 @@ __device__ __forceinline__ void adj_lambda_term(float& acc, float4 ps, float4 as
 #pragma clang fp contract(off)
   const PairGeom g = pair_geom(ps, q.a, pc.inv_h);
   const float u = g.r > pc.pair_eps ? g.t * g.t * g.rinv : 0.0f;
-  acc += u * ((as.x - q.b.x) * g.dx + (as.y - q.b.y) * g.dy + (as.z - q.b.z) * g.dz);
+  acc = fmaf(u, fmaf(as.z - q.b.z, g.dz, fmaf(as.y - q.b.y, g.dy, (as.x - q.b.x) * g.dx)), acc);
 }
 
 __device__ __forceinline__ void adj_lambda_finish(int s, float4 ps, float4 as, float acc,
@@ -79,7 +79,9 @@ __device__ __forceinline__ void adj_lambda_finish(int s, float4 ps, float4 as, f
   const float rho_bar = active ? -lam_bar * ax.w : 0.0f;
   const float s_bar = active ? -lam_bar * ps.w * ax.w : 0.0f;
   q1[s] = make_float4(as.x, as.y, as.z, rho_bar);
-  q2[s] = make_float4(s_bar * pc.cG * ax.x, s_bar * pc.cG * ax.y, s_bar * pc.cG * ax.z, s_bar);
+  // 2 S_bar G and 2 S_bar, as adj_pos_term uses them
+  const float s2 = 2.0f * s_bar;
+  q2[s] = make_float4(s2 * pc.cG * ax.x, s2 * pc.cG * ax.y, s2 * pc.cG * ax.z, s2);
 }
 
 // Sums of the adjoint passes run as one partial sum per entry parity in the
@@ -94,14 +96,10 @@ __global__ __launch_bounds__(kBlock) void k_adj_lambda(NbrView nv, const float4*
   if (s >= nv.n) return;
   const float4 ps = P[s], as = f[s];
   float acc[2] = {0.0f, 0.0f};
-  for_each_neighbor_p(
-      nv, s, wave_list(nv, __builtin_amdgcn_readfirstlane(s >> 6)), [&](int j) { return F4x2{P[j], f[j]}; },
+  for_each_neighbor_p<false, 16>(
+      nv, s, wave_list(nv, __builtin_amdgcn_readfirstlane(s >> 6)), [&](int o) { return F4x2{record_at(P, o), record_at(f, o)}; },
       [&](int, const F4x2& q, auto par) { adj_lambda_term(acc[decltype(par)::value], ps, as, q, pc); },
-      [&](bool odd) {
-        const float x = odd ? acc[1] : acc[0], y = odd ? acc[0] : acc[1];
-        acc[0] = x;
-        acc[1] = y;
-      });
+      [&](bool odd) { swap_if(odd, acc[0], acc[1]); });
   adj_lambda_finish(s, ps, as, acc[0] + acc[1], aux, q1, q2, pc);
 }
 
@@ -116,9 +114,9 @@ __global__ __launch_bounds__(kBlock) void k_adj_lambda2(NbrView nv, const float4
   const int s = g >> 1, h = g & 1;
   if (s >= nv.n) return;  // both lanes of the pair
   const float4 ps = P[s], as = f[s];
-  auto gather = [&](int j) { return F4x2{P[j], f[j]}; };
+  auto gather = [&](int o) { return F4x2{record_at(P, o), record_at(f, o)}; };
   float acc = 0.0f;
-  if (for_each_neighbor_half_idx(nv, s, h, gather,
+  if (for_each_record_half<16>(nv, s, h, gather,
                                  [&](int, const F4x2& q) { adj_lambda_term(acc, ps, as, q, pc); })) {
     const float odd = __shfl_xor(acc, 1);
     if (h == 0) adj_lambda_finish(s, ps, as, acc + odd, aux, q1, q2, pc);
@@ -126,14 +124,10 @@ __global__ __launch_bounds__(kBlock) void k_adj_lambda2(NbrView nv, const float4
   }
   if (h != 0) return;
   float a2[2] = {0.0f, 0.0f};
-  for_each_neighbor_p(
+  for_each_neighbor_p<false, 16>(
       nv, s, wave_list(nv, __builtin_amdgcn_readfirstlane(s >> 6)), gather,
       [&](int, const F4x2& q, auto par) { adj_lambda_term(a2[decltype(par)::value], ps, as, q, pc); },
-      [&](bool odd) {
-        const float x = odd ? a2[1] : a2[0], y = odd ? a2[0] : a2[1];
-        a2[0] = x;
-        a2[1] = y;
-      });
+      [&](bool odd) { swap_if(odd, a2[0], a2[1]); });
   adj_lambda_finish(s, ps, as, a2[0] + a2[1], aux, q1, q2, pc);
 }
 
@@ -141,33 +135,34 @@ struct AdjSums {
   float x = 0.0f, y = 0.0f, z = 0.0f;
 };
 
-// p_bar's pair sum for neighbor (P_j, q1_j, q2_j).
-__device__ __forceinline__ void adj_pos_term(AdjSums& b, float4 ps, float4 q1s, float4 q2s, float Gx, float Gy,
-                                             float Gz, const F4x3& q, const PhysConst& pc) {
+// p_bar's pair sum for neighbor (P_j, q1_j, q2_j), q1 = (f, rho_bar), q2 = 2 S_bar
+// (G, 1). With d the pair's distance vector and g = cG u d:
+//   w = C (lam_i + lam_j)(f_i - f_j) + 2 (S_bar_i + S_bar_j) g + 2 (S_bar_i G_i - S_bar_j G_j)
+//   J w + psi = cG u w + [(rho_bar_i + rho_bar_j) cpsi t^2/r - cG (2 t/h + u)(d.w)/r^2] d,
+// so the terms along d are one factor: 46 operations, as fused multiply-adds
+// (each written as one, so that all traversals round alike), where evaluating
+// every term by itself took about 95.
+__device__ __forceinline__ void adj_pos_term(AdjSums& b, float4 ps, float4 q1s, float4 q2s, const F4x3& q,
+                                             const PhysConst& pc) {
 #pragma clang fp contract(off)
   const float C = 2.0f * pc.corr;
   const float cpsi = -3.0f * pc.cW * pc.inv_h;
   const PairGeom g = pair_geom(ps, q.a, pc.inv_h);
-  const float t2 = g.t * g.t;
-  // density term, every listed pair (zero for the self pair: d = 0)
-  const float cr = (q1s.w + q.b.w) * cpsi * t2 * g.rinv;
-  b.x += cr * g.dx;
-  b.y += cr * g.dy;
-  b.z += cr * g.dz;
-  if (g.r > pc.pair_eps) {
-    const float u = t2 * g.rinv;
-    const float cg = pc.cG * u;
-    const float gx = cg * g.dx, gy = cg * g.dy, gz = cg * g.dz;
-    const float cl = C * (ps.w + q.a.w);
-    const float wx = cl * (q1s.x - q.b.x) + 2.0f * q2s.w * (gx + Gx) + 2.0f * (q.c.w * gx - q.c.x);
-    const float wy = cl * (q1s.y - q.b.y) + 2.0f * q2s.w * (gy + Gy) + 2.0f * (q.c.w * gy - q.c.y);
-    const float wz = cl * (q1s.z - q.b.z) + 2.0f * q2s.w * (gz + Gz) + 2.0f * (q.c.w * gz - q.c.z);
-    const float dw = g.dx * wx + g.dy * wy + g.dz * wz;
-    const float k2 = (2.0f * g.t * pc.inv_h + u) * g.rinv * g.rinv * dw;
-    b.x += pc.cG * (u * wx - k2 * g.dx);
-    b.y += pc.cG * (u * wy - k2 * g.dy);
-    b.z += pc.cG * (u * wz - k2 * g.dz);
-  }
+  const bool far = g.r > pc.pair_eps;  // closer pairs (and the self pair) have the density term only
+  const float v = g.t * g.t * g.rinv;
+  const float u = far ? v : 0.0f;
+  const float cg = pc.cG * u;
+  const float cl = C * (ps.w + q.a.w), sg = (q2s.w + q.c.w) * cg;
+  const float wx = fmaf(cl, q1s.x - q.b.x, fmaf(sg, g.dx, q2s.x - q.c.x));
+  const float wy = fmaf(cl, q1s.y - q.b.y, fmaf(sg, g.dy, q2s.y - q.c.y));
+  const float wz = fmaf(cl, q1s.z - q.b.z, fmaf(sg, g.dz, q2s.z - q.c.z));
+  const float dw = fmaf(g.dz, wz, fmaf(g.dy, wy, g.dx * wx));
+  const float k = fmaf(g.t, 2.0f * pc.inv_h, u) * (g.rinv * g.rinv) * dw;
+  const float k2 = far ? k : 0.0f;
+  const float cd = fmaf(-pc.cG, k2, (q1s.w + q.b.w) * cpsi * v);
+  b.x = fmaf(cg, wx, fmaf(cd, g.dx, b.x));
+  b.y = fmaf(cg, wy, fmaf(cd, g.dy, b.y));
+  b.z = fmaf(cg, wz, fmaf(cd, g.dz, b.z));
 }
 
 __device__ __forceinline__ void adj_pos_finish(int s, const AdjSums& b, const float4* __restrict__ e_in,
@@ -189,45 +184,43 @@ __device__ __forceinline__ AdjSums add_parities(const AdjSums& e, const AdjSums&
 }
 
 __device__ __forceinline__ void swap_if(bool c, AdjSums& a, AdjSums& b) {
-  const AdjSums x = c ? b : a, y = c ? a : b;
-  a = x;
-  b = y;
+  swap_if(c, a.x, b.x);
+  swap_if(c, a.y, b.y);
+  swap_if(c, a.z, b.z);
 }
 
 __global__ __launch_bounds__(kBlock) void k_adj_pos(NbrView nv, const float4* __restrict__ P,
-                                                    const float4* __restrict__ aux, const float4* __restrict__ q1,
-                                                    const float4* __restrict__ q2, const float4* __restrict__ e_in,
-                                                    const float4* __restrict__ c, float4* __restrict__ e_out,
-                                                    float4* __restrict__ f_out, PhysConst pc) {
+                                                    const float4* __restrict__ q1, const float4* __restrict__ q2,
+                                                    const float4* __restrict__ e_in, const float4* __restrict__ c,
+                                                    float4* __restrict__ e_out, float4* __restrict__ f_out,
+                                                    PhysConst pc) {
 #pragma clang fp contract(off)
   const int s = xcd_block(blockIdx.x, gridDim.x) * blockDim.x + threadIdx.x;
   if (s >= nv.n) return;
-  const float4 ps = P[s], q1s = q1[s], q2s = q2[s], ax = aux[s];
-  const float Gx = pc.cG * ax.x, Gy = pc.cG * ax.y, Gz = pc.cG * ax.z;
+  const float4 ps = P[s], q1s = q1[s], q2s = q2[s];
   AdjSums b[2];
-  for_each_neighbor_p(
+  for_each_neighbor_p<false, 16>(
       nv, s, wave_list(nv, __builtin_amdgcn_readfirstlane(s >> 6)),
-      [&](int j) { return F4x3{P[j], q1[j], q2[j]}; },
-      [&](int, const F4x3& q, auto par) { adj_pos_term(b[decltype(par)::value], ps, q1s, q2s, Gx, Gy, Gz, q, pc); },
+      [&](int o) { return F4x3{record_at(P, o), record_at(q1, o), record_at(q2, o)}; },
+      [&](int, const F4x3& q, auto par) { adj_pos_term(b[decltype(par)::value], ps, q1s, q2s, q, pc); },
       [&](bool odd) { swap_if(odd, b[0], b[1]); });
   adj_pos_finish(s, add_parities(b[0], b[1]), e_in, c, e_out, f_out);
 }
 
 __global__ __launch_bounds__(kBlock) void k_adj_pos2(NbrView nv, const float4* __restrict__ P,
-                                                     const float4* __restrict__ aux, const float4* __restrict__ q1,
-                                                     const float4* __restrict__ q2, const float4* __restrict__ e_in,
-                                                     const float4* __restrict__ c, float4* __restrict__ e_out,
-                                                     float4* __restrict__ f_out, PhysConst pc) {
+                                                     const float4* __restrict__ q1, const float4* __restrict__ q2,
+                                                     const float4* __restrict__ e_in, const float4* __restrict__ c,
+                                                     float4* __restrict__ e_out, float4* __restrict__ f_out,
+                                                     PhysConst pc) {
 #pragma clang fp contract(off)
   const int g = xcd_block(blockIdx.x, gridDim.x) * blockDim.x + threadIdx.x;
   const int s = g >> 1, h = g & 1;
   if (s >= nv.n) return;  // both lanes of the pair
-  const float4 ps = P[s], q1s = q1[s], q2s = q2[s], ax = aux[s];
-  const float Gx = pc.cG * ax.x, Gy = pc.cG * ax.y, Gz = pc.cG * ax.z;
-  auto gather = [&](int j) { return F4x3{P[j], q1[j], q2[j]}; };
+  const float4 ps = P[s], q1s = q1[s], q2s = q2[s];
+  auto gather = [&](int o) { return F4x3{record_at(P, o), record_at(q1, o), record_at(q2, o)}; };
   AdjSums b;
-  if (for_each_neighbor_half_idx(nv, s, h, gather, [&](int, const F4x3& q) {
-        adj_pos_term(b, ps, q1s, q2s, Gx, Gy, Gz, q, pc);
+  if (for_each_record_half<16>(nv, s, h, gather, [&](int, const F4x3& q) {
+        adj_pos_term(b, ps, q1s, q2s, q, pc);
       })) {
     AdjSums o;
     o.x = __shfl_xor(b.x, 1);
@@ -238,9 +231,9 @@ __global__ __launch_bounds__(kBlock) void k_adj_pos2(NbrView nv, const float4* _
   }
   if (h != 0) return;
   AdjSums b2[2];
-  for_each_neighbor_p(
+  for_each_neighbor_p<false, 16>(
       nv, s, wave_list(nv, __builtin_amdgcn_readfirstlane(s >> 6)), gather,
-      [&](int, const F4x3& q, auto par) { adj_pos_term(b2[decltype(par)::value], ps, q1s, q2s, Gx, Gy, Gz, q, pc); },
+      [&](int, const F4x3& q, auto par) { adj_pos_term(b2[decltype(par)::value], ps, q1s, q2s, q, pc); },
       [&](bool odd) { swap_if(odd, b2[0], b2[1]); });
   adj_pos_finish(s, add_parities(b2[0], b2[1]), e_in, c, e_out, f_out);
 }
@@ -273,10 +266,10 @@ void launch_adjoint_step(const NbrView& nv, float4* const* P, float4* const* aux
   for (int k = K - 1; k >= 0; --k) {
     if (lanes == 2) {
       k_adj_lambda2<<<nb2, kBlock, 0, st>>>(nv, P[k], aux[k], ab.f, ab.q1, ab.q2, pc);
-      k_adj_pos2<<<nb2, kBlock, 0, st>>>(nv, P[k], aux[k], ab.q1, ab.q2, e, ab.c, e2, ab.f, pc);
+      k_adj_pos2<<<nb2, kBlock, 0, st>>>(nv, P[k], ab.q1, ab.q2, e, ab.c, e2, ab.f, pc);
     } else {
       k_adj_lambda<<<nb, kBlock, 0, st>>>(nv, P[k], aux[k], ab.f, ab.q1, ab.q2, pc);
-      k_adj_pos<<<nb, kBlock, 0, st>>>(nv, P[k], aux[k], ab.q1, ab.q2, e, ab.c, e2, ab.f, pc);
+      k_adj_pos<<<nb, kBlock, 0, st>>>(nv, P[k], ab.q1, ab.q2, e, ab.c, e2, ab.f, pc);
     }
     float4* t = e;
     e = e2;

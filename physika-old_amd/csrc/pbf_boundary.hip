@@ -291,6 +291,13 @@ __device__ __forceinline__ VisSums add_parities(const VisSums& e, const VisSums&
   return t;
 }
 
+__device__ __forceinline__ void swap_if(bool c, VisSums& a, VisSums& b) {
+  swap_if(c, a.tw, b.tw);
+  swap_if(c, a.dx, b.dx);
+  swap_if(c, a.dy, b.dy);
+  swap_if(c, a.dz, b.dz);
+}
+
 // One Jacobi iteration (K_ApplyViscosity, ImplicitViscosity.cu:20-62) in
 // sorted order over the step's lists, the sums kept as one partial sum per
 // entry parity in the neighbor order (as the PBD passes). kPair: thread g
@@ -307,9 +314,9 @@ __global__ __launch_bounds__(kBlock) void k_viscosity(NbrView nv, const float4* 
   const int s = kPair ? g >> 1 : g, h = kPair ? g & 1 : 0;
   if (s >= nv.n) return;
   const float4 xi = xs[s];
-  auto gather = [&](int j) { return VisPair{xs[j], v_in[j]}; };
+  auto gather = [&](int o) { return VisPair{record_at(xs, o), record_at(v_in, o)}; };
   VisSums t;
-  if (kPair && for_each_neighbor_half_idx(nv, s, h, gather, [&](int, const VisPair& q) { vis_term(t, xi, q, vc); })) {
+  if (kPair && for_each_record_half<16>(nv, s, h, gather, [&](int, const VisPair& q) { vis_term(t, xi, q, vc); })) {
     VisSums o;
     o.tw = __shfl_xor(t.tw, 1);
     o.dx = __shfl_xor(t.dx, 1);
@@ -320,14 +327,10 @@ __global__ __launch_bounds__(kBlock) void k_viscosity(NbrView nv, const float4* 
   }
   if (h != 0) return;
   VisSums a[2];
-  for_each_neighbor_p(
+  for_each_neighbor_p<false, 16>(
       nv, s, wave_list(nv, __builtin_amdgcn_readfirstlane(s >> 6)), gather,
       [&](int, const VisPair& q, auto par) { vis_term(a[decltype(par)::value], xi, q, vc); },
-      [&](bool odd) {
-        const VisSums x = odd ? a[1] : a[0], y = odd ? a[0] : a[1];
-        a[0] = x;
-        a[1] = y;
-      });
+      [&](bool odd) { swap_if(odd, a[0], a[1]); });
   vis_finish(s, xi, add_parities(a[0], a[1]), v_old, v_next, vc, perm, x_out, v_out);
 }
 

@@ -274,7 +274,7 @@ struct AdjBufs {
   float4* f;    // e + c, gathered by the pair terms
   float4* c;    // v_bar' / dt
   float4* q1;   // (f, rho_bar)
-  float4* q2;   // (S_bar * G, S_bar)
+  float4* q2;   // 2 S_bar (G, 1)
   float4* vsb;  // adjoint of the integrated velocities
   int* flag;    // set when a taped step had out-of-grid particles
 };

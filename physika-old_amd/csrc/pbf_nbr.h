@@ -172,16 +172,38 @@ struct Group4 {
   int j[4];
 };
 
-// Indices of group b (entries 4b..4b+3). kFull: the group is complete;
-// otherwise entries past cnt become `past`.
-template <bool kFull>
-__device__ __forceinline__ Group4 decode16(uint2 e, int jb, int b, int cnt, int past) {
+// A neighbor is handed on as j * kRec: its sorted index (kRec 1) or the byte
+// offset of its record in an array of kRec bytes per particle, which a load
+// takes as it is (scalar base + 32-bit vector offset; fewer than kMaxParticles
+// records of at most 32 bytes). An index would cost a shift and, sign-extended,
+// 64-bit address arithmetic per record. The entry in the low (kHigh false) or
+// high half of w with base = jbase * kRec (wave-uniform) decodes in one
+// v_mad_u32_u16 (op_sel selects the half of the first operand).
+template <int kRec, bool kHigh>
+__device__ __forceinline__ int entry_at(uint32_t w, uint32_t base) {
+  static_assert(kRec == 1 || kRec == 16 || kRec == 32, "an index or records of 16 or 32 bytes");
+  if constexpr (kRec == 1) {
+    return (int)(base + (kHigh ? w >> 16 : w & 0xffffu));
+  } else {
+    uint32_t r;
+    if (kHigh)
+      asm("v_mad_u32_u16 %0, %1, %3, %2 op_sel:[1,0,0,0]" : "=v"(r) : "v"(w), "s"(base), "n"(kRec));
+    else
+      asm("v_mad_u32_u16 %0, %1, %3, %2" : "=v"(r) : "v"(w), "s"(base), "n"(kRec));
+    return (int)r;
+  }
+}
+
+// Group b (entries 4b..4b+3) of a 16-bit list. kFull: the group is complete;
+// otherwise entries past cnt become `past` (in the units of kRec).
+template <bool kFull, int kRec>
+__device__ __forceinline__ Group4 decode16(uint2 e, uint32_t base, int b, int cnt, int past) {
   const int k = b << 2;
   Group4 g;
-  g.j[0] = jb + (int)(e.x & 0xffffu);
-  g.j[1] = jb + (int)(e.x >> 16);
-  g.j[2] = jb + (int)(e.y & 0xffffu);
-  g.j[3] = jb + (int)(e.y >> 16);
+  g.j[0] = entry_at<kRec, false>(e.x, base);
+  g.j[1] = entry_at<kRec, true>(e.x, base);
+  g.j[2] = entry_at<kRec, false>(e.y, base);
+  g.j[3] = entry_at<kRec, true>(e.y, base);
   if (!kFull) {
 #pragma unroll
     for (int u = 0; u < 4; ++u) g.j[u] = k + u < cnt ? g.j[u] : past;
@@ -208,45 +230,15 @@ struct StageMap {
   }
 };
 
-// Byte offset e * 16 + base of the 16-bit list entry e held in the low
-// (kHigh false) or high half of w, in one v_mad_u32_u16 (op_sel selects the
-// half of the first operand); base is wave-uniform.
-template <bool kHigh>
-__device__ __forceinline__ int entry_bytes(uint32_t w, uint32_t base) {
-  uint32_t r;
-  if (kHigh)
-    asm("v_mad_u32_u16 %0, %1, 16, %2 op_sel:[1,0,0,0]" : "=v"(r) : "v"(w), "s"(base));
-  else
-    asm("v_mad_u32_u16 %0, %1, 16, %2" : "=v"(r) : "v"(w), "s"(base));
-  return (int)r;
-}
-
-// decode16 into byte offsets: entry e becomes e * 16 + base, entries past cnt
-// become past (a byte offset too).
-template <bool kFull>
-__device__ __forceinline__ Group4 decode16_bytes(uint2 e, uint32_t base, int b, int cnt, int past) {
-  const int k = b << 2;
-  Group4 g;
-  g.j[0] = entry_bytes<false>(e.x, base);
-  g.j[1] = entry_bytes<true>(e.x, base);
-  g.j[2] = entry_bytes<false>(e.y, base);
-  g.j[3] = entry_bytes<true>(e.y, base);
-  if (!kFull) {
-#pragma unroll
-    for (int u = 0; u < 4; ++u) g.j[u] = k + u < cnt ? g.j[u] : past;
-  }
-  return g;
-}
-
-// decode16 of stage slots into sorted indices.
-template <bool kFull>
+// decode16 of stage slots.
+template <bool kFull, int kRec>
 __device__ __forceinline__ Group4 decode16_staged(uint2 e, const StageMap& m, int b, int cnt, int past) {
   const int k = b << 2;
   Group4 g;
-  g.j[0] = m.index_of((int)(e.x & 0xffffu));
-  g.j[1] = m.index_of((int)(e.x >> 16));
-  g.j[2] = m.index_of((int)(e.y & 0xffffu));
-  g.j[3] = m.index_of((int)(e.y >> 16));
+  g.j[0] = m.index_of((int)(e.x & 0xffffu)) * kRec;
+  g.j[1] = m.index_of((int)(e.x >> 16)) * kRec;
+  g.j[2] = m.index_of((int)(e.y & 0xffffu)) * kRec;
+  g.j[3] = m.index_of((int)(e.y >> 16)) * kRec;
   if (!kFull) {
 #pragma unroll
     for (int u = 0; u < 4; ++u) g.j[u] = k + u < cnt ? g.j[u] : past;
@@ -254,14 +246,14 @@ __device__ __forceinline__ Group4 decode16_staged(uint2 e, const StageMap& m, in
   return g;
 }
 
-template <bool kFull>
+template <bool kFull, int kRec>
 __device__ __forceinline__ Group4 decode32(int4 e, int b, int cnt, int past) {
   const int k = b << 2;
   Group4 g;
-  g.j[0] = e.x;
-  g.j[1] = e.y;
-  g.j[2] = e.z;
-  g.j[3] = e.w;
+  g.j[0] = e.x * kRec;
+  g.j[1] = e.y * kRec;
+  g.j[2] = e.z * kRec;
+  g.j[3] = e.w * kRec;
   if (!kFull) {
 #pragma unroll
     for (int u = 0; u < 4; ++u) g.j[u] = k + u < cnt ? g.j[u] : past;
@@ -406,29 +398,30 @@ __device__ __forceinline__ WaveList wave_list(const NbrView& nv, int wave) {
 
 // Calls body(j, gather(j), parity) for every neighbor j of sorted particle s,
 // in the canonical order (parity: EvenEntry or OddEntry, the entry's index mod
-// 2, with flip as described at EvenEntry). The list is used when the wave has
-// one; otherwise (reservation exhausted) the words come from the masks, or are
-// recomputed from xn. kPadded (list path only): the body also runs on up to
-// three entries of the padding particle nv.pad, whose position lies far outside
-// every stencil; a body whose terms vanish with the kernel's t = 0 (and are
-// finite) adds exact zeros for them. wl: the words of s's wave (wave_list).
-template <bool kPadded = false, class GatherFn, class Body, class Flip>
+// 2, with flip as described at EvenEntry); j in the units of kRec (entry_at).
+// The list is used when the wave has one; otherwise (reservation exhausted) the
+// words come from the masks, or are recomputed from xn. kPadded (list path
+// only): the body also runs on up to three entries of the padding particle
+// nv.pad, whose position lies far outside every stencil; a body whose terms
+// vanish with the kernel's t = 0 (and are finite) adds exact zeros for them.
+// wl: the words of s's wave (wave_list).
+template <bool kPadded, int kRec, class GatherFn, class Body, class Flip>
 __device__ __forceinline__ void for_each_neighbor_p(const NbrView& nv, int s, const WaveList& wl, GatherFn&& gather,
                                                     Body&& body, Flip&& flip) {
   const int wave = __builtin_amdgcn_readfirstlane(s >> 6), lane = s & 63;
   const long long lb = wl.lb;
   const int cnt = nv.nbr_cnt[s];  // issued with the wave's words (unused on the mask path)
   if (lb >= 0) {
-    const int past = kPadded ? nv.pad : s;
+    const int past = (kPadded ? nv.pad : s) * kRec;
     const int lm = wl.lm;
     const int nfull = lm >> 2;
+    const uint32_t base = (uint32_t)wl.jb * kRec;
     if ((lm & 3) == kListDelta16) {
       const uint4* L = reinterpret_cast<const uint4*>(nv.list + lb) + lane;
-      const int jb = wl.jb;
       list_loop_pairs<kPadded>(
           cnt, nfull, L,
-          [&](uint2 e, int b, auto full) { return decode16<decltype(full)::value>(e, jb, b, cnt, past); }, gather,
-          body);
+          [&](uint2 e, int b, auto full) { return decode16<decltype(full)::value, kRec>(e, base, b, cnt, past); },
+          gather, body);
     } else if ((lm & 3) == kListStaged) {
       // stage slots of the first three runs (then pads up to kA), then offsets
       const uint4* L = reinterpret_cast<const uint4*>(nv.list + lb) + lane;
@@ -437,19 +430,20 @@ __device__ __forceinline__ void for_each_neighbor_p(const NbrView& nv, int s, co
       m.load(st);
       const int ka = st[7], ca = nv.cnt_a[s], cb = cnt - ca;
       list_loop_pairs<kPadded>(
-          ca, 0, L, [&](uint2 e, int b, auto) { return decode16_staged<false>(e, m, b, ca, past); }, gather, body);
-      const int jb = wl.jb;
+          ca, 0, L, [&](uint2 e, int b, auto) { return decode16_staged<false, kRec>(e, m, b, ca, past); }, gather,
+          body);
       flip((ca & 1) != 0);  // the offsets part starts at index ca
       list_loop_pairs<kPadded>(
           cb, nfull, L + ((long long)(ka >> 3) << 6),
-          [&](uint2 e, int b, auto full) { return decode16<decltype(full)::value>(e, jb, b, cb, past); }, gather,
-          body);
+          [&](uint2 e, int b, auto full) { return decode16<decltype(full)::value, kRec>(e, base, b, cb, past); },
+          gather, body);
       flip((ca & 1) != 0);
     } else {
       const int4* L = reinterpret_cast<const int4*>(nv.list + lb) + lane;
       list_loop<kPadded, int4>(
           cnt, nfull, [&](int b) { return L[(long long)b << 6]; },
-          [&](int4 e, int b, auto full) { return decode32<decltype(full)::value>(e, b, cnt, past); }, gather, body);
+          [&](int4 e, int b, auto full) { return decode32<decltype(full)::value, kRec>(e, b, cnt, past); }, gather,
+          body);
     }
     return;
   }
@@ -470,7 +464,7 @@ __device__ __forceinline__ void for_each_neighbor_p(const NbrView& nv, int s, co
       uint32_t bits = mb >= 0 ? nv.mask[mb + ((long long)(wofs + w) << 6) + lane]
                               : test_word(nv.xn + jb, xni, min(32, rl - (w << 5)), nv.thr2);
       while (bits) {
-        const int j = jb + pop_first(bits);
+        const int j = (jb + pop_first(bits)) * kRec;
         if (k & 1)
           body(j, gather(j), OddEntry{});
         else
@@ -486,7 +480,7 @@ __device__ __forceinline__ void for_each_neighbor_p(const NbrView& nv, int s, co
 // the canonical order.
 template <bool kPadded = false, class GatherFn, class Body>
 __device__ __forceinline__ void for_each_neighbor(const NbrView& nv, int s, GatherFn&& gather, Body&& body) {
-  for_each_neighbor_p<kPadded>(
+  for_each_neighbor_p<kPadded, 1>(
       nv, s, wave_list(nv, __builtin_amdgcn_readfirstlane(s >> 6)), gather,
       [&](int j, const auto& a, auto) { body(j, a); }, [](bool) {});
 }
@@ -500,17 +494,16 @@ __device__ __forceinline__ void for_each_neighbor_x(const NbrView& nv, int s, co
 
 // A lane of a lane pair takes every other entry of a 16-bit list: halfword
 // hh of each 32-bit word of a 16-byte chunk, i.e. entries 8c + 2u + hh (u =
-// 0..3) of chunk c, decoded into byte addresses (entry * 16 + base; sh =
-// 16 hh). Entry k = 4c + u of the lane at or past cnt (the lane's count)
-// becomes past.
-template <bool kFull>
-__device__ __forceinline__ Group4 decode_half_bytes(uint4 e, uint32_t sh, uint32_t base, int c, int cnt, int past) {
+// 0..3) of chunk c (sh = 16 hh), in the units of kRec. Entry k = 4c + u of the
+// lane at or past cnt (the lane's count) becomes past.
+template <bool kFull, int kRec>
+__device__ __forceinline__ Group4 decode_half(uint4 e, uint32_t sh, uint32_t base, int c, int cnt, int past) {
   const int k = c << 2;
   Group4 g;
-  g.j[0] = entry_bytes<false>(e.x >> sh, base);
-  g.j[1] = entry_bytes<false>(e.y >> sh, base);
-  g.j[2] = entry_bytes<false>(e.z >> sh, base);
-  g.j[3] = entry_bytes<false>(e.w >> sh, base);
+  g.j[0] = entry_at<kRec, false>(e.x >> sh, base);
+  g.j[1] = entry_at<kRec, false>(e.y >> sh, base);
+  g.j[2] = entry_at<kRec, false>(e.z >> sh, base);
+  g.j[3] = entry_at<kRec, false>(e.w >> sh, base);
   if (!kFull) {
 #pragma unroll
     for (int u = 0; u < 4; ++u) g.j[u] = k + u < cnt ? g.j[u] : past;
@@ -554,7 +547,7 @@ __device__ __forceinline__ void for_each_neighbor_staged(const NbrView& nv, int 
   const long long lb = wl.lb;
   const int lm = wl.lm;
   if (lb < 0 || (lm & 3) != kListStaged) {
-    for_each_neighbor_p<true>(nv, s, wl, [&](int j) { return load_pos<kW>(xs, j); }, body, flip);
+    for_each_neighbor_p<true, 16>(nv, s, wl, [&](int o) { return load_pos_bytes<kW>(xs, (uint32_t)o); }, body, flip);
     return;
   }
   const int* st = nv.stage + kStageInts * wave;
@@ -574,14 +567,14 @@ __device__ __forceinline__ void for_each_neighbor_staged(const NbrView& nv, int 
   // stage part: ka entries on every lane (pads read the padding particle)
   const uint32_t lds = __builtin_amdgcn_readfirstlane(lds_address(buf));
   list_loop_pairs<true>(
-      ka, ka >> 2, L, [&](uint2 e, int b, auto) { return decode16_bytes<true>(e, lds, b, ka, 0); },
+      ka, ka >> 2, L, [&](uint2 e, int b, auto) { return decode16<true, 16>(e, lds, b, ka, 0); },
       [&](int a) { return lds_load_pos<kW>((uint32_t)a); }, body);
   const uint32_t jb16 = (uint32_t)wl.jb << 4;
   const int past = (int)((uint32_t)nv.pad << 4);
   flip((ca & 1) != 0);  // the offsets part starts at index ca
   list_loop_pairs<true>(
       cb, lm >> 2, L + ((long long)(ka >> 3) << 6),
-      [&](uint2 e, int b, auto full) { return decode16_bytes<decltype(full)::value>(e, jb16, b, cb, past); },
+      [&](uint2 e, int b, auto full) { return decode16<decltype(full)::value, 16>(e, jb16, b, cb, past); },
       [&](int o) { return load_pos_bytes<kW>(xs, (uint32_t)o); }, body);
   flip((ca & 1) != 0);
 }
@@ -616,7 +609,7 @@ __device__ __forceinline__ bool for_each_neighbor_half(const NbrView& nv, int s,
     list_loop<true, uint4>(
         ch, nfull, [&](int c) { return L[(long long)c << 6]; },
         [&](uint4 e, int c, auto full) {
-          return decode_half_bytes<decltype(full)::value>(e, sh, jb16, c, ch, past);
+          return decode_half<decltype(full)::value, 16>(e, sh, jb16, c, ch, past);
         },
         gather, each);
     return true;
@@ -641,7 +634,7 @@ __device__ __forceinline__ bool for_each_neighbor_half(const NbrView& nv, int s,
   const uint32_t sh1 = (uint32_t)h << 4;
   list_loop<true, uint4>(
       ka >> 1, ka >> 3, [&](int c) { return L[(long long)c << 6]; },
-      [&](uint4 e, int c, auto) { return decode_half_bytes<true>(e, sh1, lds, c, ka >> 1, 0); },
+      [&](uint4 e, int c, auto) { return decode_half<true, 16>(e, sh1, lds, c, ka >> 1, 0); },
       [&](int a) { return lds_load_pos<kW>((uint32_t)a); }, each);
   // offsets part: its entry p has index ca + p, so the lane takes p of parity
   // h ^ (ca & 1)
@@ -652,65 +645,53 @@ __device__ __forceinline__ bool for_each_neighbor_half(const NbrView& nv, int s,
   list_loop<true, uint4>(
       ch, nfull, [&](int c) { return L2[(long long)c << 6]; },
       [&](uint4 e, int c, auto full) {
-        return decode_half_bytes<decltype(full)::value>(e, sh2, jb16, c, ch, past);
+        return decode_half<decltype(full)::value, 16>(e, sh2, jb16, c, ch, past);
       },
       gather, each);
   return true;
 }
 
-// The lane-pair decode by index: halfword hh of each word of a 16-byte chunk
-// (entries 8c + 2u + hh), as sorted indices jb + entry (16-bit offsets) or
-// through the stage map (stage slots); entry k = 4c + u of the lane at or past
-// cnt becomes past.
-template <bool kFull>
-__device__ __forceinline__ Group4 decode_half_idx(uint4 e, uint32_t sh, int jb, int c, int cnt, int past) {
-  const int k = c << 2;
-  Group4 g;
-  g.j[0] = jb + (int)((e.x >> sh) & 0xffffu);
-  g.j[1] = jb + (int)((e.y >> sh) & 0xffffu);
-  g.j[2] = jb + (int)((e.z >> sh) & 0xffffu);
-  g.j[3] = jb + (int)((e.w >> sh) & 0xffffu);
-  if (!kFull) {
-#pragma unroll
-    for (int u = 0; u < 4; ++u) g.j[u] = k + u < cnt ? g.j[u] : past;
-  }
-  return g;
-}
+// decode_half of stage slots, through the stage map.
+template <int kRec>
 __device__ __forceinline__ Group4 decode_half_staged(uint4 e, uint32_t sh, const StageMap& m, int c, int cnt,
                                                      int past) {
   const int k = c << 2;
   Group4 g;
-  g.j[0] = m.index_of((int)((e.x >> sh) & 0xffffu));
-  g.j[1] = m.index_of((int)((e.y >> sh) & 0xffffu));
-  g.j[2] = m.index_of((int)((e.z >> sh) & 0xffffu));
-  g.j[3] = m.index_of((int)((e.w >> sh) & 0xffffu));
+  g.j[0] = m.index_of((int)((e.x >> sh) & 0xffffu)) * kRec;
+  g.j[1] = m.index_of((int)((e.y >> sh) & 0xffffu)) * kRec;
+  g.j[2] = m.index_of((int)((e.z >> sh) & 0xffffu)) * kRec;
+  g.j[3] = m.index_of((int)((e.w >> sh) & 0xffffu)) * kRec;
 #pragma unroll
   for (int u = 0; u < 4; ++u) g.j[u] = k + u < cnt ? g.j[u] : past;
   return g;
 }
 
-// for_each_neighbor for a lane pair, by index: lane h (0 or 1) of the pair
-// that holds particle s calls body(j, gather(j)) for the entries of s's list
-// whose index in the canonical order has parity h, in that order (entries past
-// the lane's count and the stage pads are not visited). Returns false, with
-// nothing run, when s's wave has no 16-bit or staged list.
-template <class GatherFn, class Body>
-__device__ __forceinline__ bool for_each_neighbor_half_idx(const NbrView& nv, int s, int h, GatherFn&& gather,
-                                                           Body&& body) {
+// for_each_neighbor for a lane pair and records of kRec bytes: lane h (0 or 1)
+// of the pair that holds particle s calls body(o, gather(o)) for the entries of
+// s's list whose index in the canonical order has parity h, in that order
+// (entries past the lane's count and the stage pads are not visited), o the
+// record's byte offset. Returns false, with nothing run, when s's wave has no
+// 16-bit or staged list.
+template <int kRec, class GatherFn, class Body>
+__device__ __forceinline__ bool for_each_record_half(const NbrView& nv, int s, int h, GatherFn&& gather,
+                                                     Body&& body) {
   const int wave = __builtin_amdgcn_readfirstlane(s >> 6), lane = s & 63;
   const WaveList wl = wave_list(nv, wave);
   const int mode = wl.lm & 3;
   if (wl.lb < 0 || (mode != kListDelta16 && mode != kListStaged)) return false;
   const uint4* L = reinterpret_cast<const uint4*>(nv.list + wl.lb) + lane;
-  const int cnt = nv.nbr_cnt[s];
+  const int cnt = nv.nbr_cnt[s], past = s * kRec;
+  const uint32_t base = (uint32_t)wl.jb * kRec;
   const int nfull = (wl.lm >> 2) >> 1;  // as in for_each_neighbor_half
-  auto each = [&](int j, const auto& a, auto) { body(j, a); };
+  auto each = [&](int o, const auto& a, auto) { body(o, a); };
   if (mode == kListDelta16) {
     const int ch = (cnt - h + 1) >> 1;
     const uint32_t sh = (uint32_t)h << 4;
     list_loop<false, uint4>(
         ch, nfull, [&](int c) { return L[(long long)c << 6]; },
-        [&](uint4 e, int c, auto full) { return decode_half_idx<decltype(full)::value>(e, sh, wl.jb, c, ch, s); },
+        [&](uint4 e, int c, auto full) {
+          return decode_half<decltype(full)::value, kRec>(e, sh, base, c, ch, past);
+        },
         gather, each);
     return true;
   }
@@ -724,16 +705,24 @@ __device__ __forceinline__ bool for_each_neighbor_half_idx(const NbrView& nv, in
   const uint32_t sh1 = (uint32_t)h << 4;
   list_loop<false, uint4>(
       c1, 0, [&](int c) { return L[(long long)c << 6]; },
-      [&](uint4 e, int c, auto) { return decode_half_staged(e, sh1, m, c, c1, s); }, gather, each);
+      [&](uint4 e, int c, auto) { return decode_half_staged<kRec>(e, sh1, m, c, c1, past); }, gather, each);
   const int hh = h ^ (ca & 1);
   const int ch = (cb - hh + 1) >> 1;
   const uint32_t sh2 = (uint32_t)hh << 4;
   const uint4* L2 = L + ((long long)(ka >> 3) << 6);
   list_loop<false, uint4>(
       ch, nfull, [&](int c) { return L2[(long long)c << 6]; },
-      [&](uint4 e, int c, auto full) { return decode_half_idx<decltype(full)::value>(e, sh2, wl.jb, c, ch, s); },
+      [&](uint4 e, int c, auto full) {
+        return decode_half<decltype(full)::value, kRec>(e, sh2, base, c, ch, past);
+      },
       gather, each);
   return true;
+}
+
+// The record at byte offset o of an array (see entry_at).
+template <class T>
+__device__ __forceinline__ T record_at(const T* __restrict__ a, int o) {
+  return *reinterpret_cast<const T*>(reinterpret_cast<const char*>(a) + (uint32_t)o);
 }
 
 }  // namespace pbf

@@ -558,8 +558,8 @@ __device__ __forceinline__ void density_lambda_at2(const NbrView& nv, int s, int
   if (h != 0) return;
   // neither a 16-bit nor a staged list: the even lane takes the whole list
   const DensitySums t = density_one_lane(xi, pc, [&](auto&& body, auto&& flip) {
-    for_each_neighbor_p<true>(nv, s, wave_list(nv, __builtin_amdgcn_readfirstlane(s >> 6)),
-                              [&](int j) { return load_pos<false>(xs, j); }, body, flip);
+    for_each_neighbor_p<true, 16>(nv, s, wave_list(nv, __builtin_amdgcn_readfirstlane(s >> 6)),
+                                  [&](int o) { return load_pos_bytes<false>(xs, (uint32_t)o); }, body, flip);
   });
   density_lambda_finish(s, xs, pc, rho_out, perm, aux, t);
 }
@@ -830,8 +830,8 @@ __device__ __forceinline__ void displacement_at2(const NbrView& nv, int s, int h
   if (h != 0) return;
   // neither a 16-bit nor a staged list: the even lane takes the whole list
   const DispSums t = disp_one_lane(xi, pc, [&](auto&& body, auto&& flip) {
-    for_each_neighbor_p<true>(nv, s, wave_list(nv, __builtin_amdgcn_readfirstlane(s >> 6)),
-                              [&](int j) { return load_pos<true>(xs, j); }, body, flip);
+    for_each_neighbor_p<true, 16>(nv, s, wave_list(nv, __builtin_amdgcn_readfirstlane(s >> 6)),
+                                  [&](int o) { return load_pos_bytes<true>(xs, (uint32_t)o); }, body, flip);
   });
   displacement_finish(nv, s, xs, xd, pc, last, x0, vs, perm, x_out, v_out, v_sorted, id_out, xi, t);
 }

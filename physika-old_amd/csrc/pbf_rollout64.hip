@@ -35,10 +35,17 @@ __device__ __forceinline__ PairGeom64 pair_geom64(const double4& a, const double
   p.dx = a.x - b.x;
   p.dy = a.y - b.y;
   p.dz = a.z - b.z;
-  const double r2 = (p.dx * p.dx + p.dy * p.dy) + p.dz * p.dz;
-  p.r = sqrt(r2);
-  p.rinv = r2 > 0.0 ? 1.0 / p.r : 0.0;
-  p.t = fmax(1.0 - p.r * inv_h, 0.0);
+  // r2 >= 1e-60 keeps the reciprocal finite (a particle paired with itself)
+  const double r2 = fma(p.dz, p.dz, fma(p.dy, p.dy, fma(p.dx, p.dx, 1e-60)));
+  // 1/sqrt(r2) from the hardware's estimate (relative error below 2^-23) by one
+  // step of y (1 + e/2 + 3 e^2/8), e = 1 - r2 y^2, whose error is 5 e^3/16:
+  // below an ulp, in 6 operations where a square root and a division take
+  // about 45
+  const double y = __builtin_amdgcn_rsq(r2);
+  const double e = fma(-(r2 * y), y, 1.0);
+  p.rinv = fma(y * e, fma(e, 0.375, 0.5), y);
+  p.r = r2 * p.rinv;
+  p.t = fmax(fma(-p.r, inv_h, 1.0), 0.0);
   return p;
 }
 
@@ -101,7 +108,7 @@ struct SumsD {
 template <int N, class Gather, class Term>
 __device__ __forceinline__ SumsD<N> sums64_one_lane(const NbrView& nv, int s, Gather&& gather, Term&& term) {
   SumsD<N> a[2];
-  for_each_neighbor_p(
+  for_each_neighbor_p<false, 32>(
       nv, s, wave_list(nv, __builtin_amdgcn_readfirstlane(s >> 6)), gather,
       [&](int, const auto& q, auto par) { term(a[decltype(par)::value], q); },
       [&](bool odd) {
@@ -125,7 +132,7 @@ template <int N, class Gather, class Term>
 __device__ __forceinline__ bool sums64_lane_pair(const NbrView& nv, int s, int h, Gather&& gather, Term&& term,
                                                  SumsD<N>& t) {
   SumsD<N> a;
-  if (!for_each_neighbor_half_idx(nv, s, h, gather, [&](int, const auto& q) { term(a, q); })) return false;
+  if (!for_each_record_half<32>(nv, s, h, gather, [&](int, const auto& q) { term(a, q); })) return false;
 #pragma unroll
   for (int i = 0; i < N; ++i) {
     const double o = __shfl_xor(a.v[i], 1);
@@ -154,23 +161,23 @@ __global__ __launch_bounds__(kBlock) void k64_density_lambda(NbrView nv, double4
                                                              double4* __restrict__ aux, double* __restrict__ rho_out,
                                                              const int* __restrict__ perm) {
 #pragma clang fp contract(off)
-  const int g = blockIdx.x * blockDim.x + threadIdx.x;
+  const int g = xcd_block(blockIdx.x, gridDim.x) * blockDim.x + threadIdx.x;
   const int s = kPair ? g >> 1 : g, h = kPair ? g & 1 : 0;
   if (s >= nv.n) return;
   const double4 ps = P[s];
   SumsD<5> t;  // rho, G, |g|^2
   if (!sums64_of<kPair, 5>(
-          nv, s, h, [&](int j) { return P[j]; },
+          nv, s, h, [&](int o) { return record_at(P, o); },
           [&](auto& a, const double4& pj) {
             const PairGeom64 q = pair_geom64(ps, pj, pc.inv_h);
             const double t2 = q.t * q.t;
-            a.v[0] += t2 * q.t;
+            a.v[0] = fma(t2, q.t, a.v[0]);
             const double tg = q.r > pc.pair_eps ? t2 : 0.0;
             const double u = tg * q.rinv;
-            a.v[1] += u * q.dx;
-            a.v[2] += u * q.dy;
-            a.v[3] += u * q.dz;
-            a.v[4] += tg * tg;
+            a.v[1] = fma(u, q.dx, a.v[1]);
+            a.v[2] = fma(u, q.dy, a.v[2]);
+            a.v[3] = fma(u, q.dz, a.v[3]);
+            a.v[4] = fma(tg, tg, a.v[4]);
           },
           t))
     return;
@@ -194,19 +201,19 @@ __global__ __launch_bounds__(kBlock) void k64_displacement(NbrView nv, const dou
                                                            const int* __restrict__ perm, double* __restrict__ x_out,
                                                            double* __restrict__ v_out) {
 #pragma clang fp contract(off)
-  const int g = blockIdx.x * blockDim.x + threadIdx.x;
+  const int g = xcd_block(blockIdx.x, gridDim.x) * blockDim.x + threadIdx.x;
   const int s = kPair ? g >> 1 : g, h = kPair ? g & 1 : 0;
   if (s >= nv.n) return;
   const double4 ps = P[s];
   SumsD<3> t;
   if (!sums64_of<kPair, 3>(
-          nv, s, h, [&](int j) { return P[j]; },
+          nv, s, h, [&](int o) { return record_at(P, o); },
           [&](auto& a, const double4& pj) {
             const PairGeom64 q = pair_geom64(ps, pj, pc.inv_h);
             const double c = q.r > pc.pair_eps ? (ps.w + pj.w) * (q.t * q.t) * q.rinv : 0.0;
-            a.v[0] += c * q.dx;
-            a.v[1] += c * q.dy;
-            a.v[2] += c * q.dz;
+            a.v[0] = fma(c, q.dx, a.v[0]);
+            a.v[1] = fma(c, q.dy, a.v[1]);
+            a.v[2] = fma(c, q.dz, a.v[2]);
           },
           t))
     return;
@@ -262,17 +269,17 @@ __global__ __launch_bounds__(kBlock) void k64_adj_lambda(NbrView nv, const doubl
                                                          const double4* __restrict__ f, double4* __restrict__ q1,
                                                          double4* __restrict__ q2, PhysConst64 pc) {
 #pragma clang fp contract(off)
-  const int g = blockIdx.x * blockDim.x + threadIdx.x;
+  const int g = xcd_block(blockIdx.x, gridDim.x) * blockDim.x + threadIdx.x;
   const int s = kPair ? g >> 1 : g, h = kPair ? g & 1 : 0;
   if (s >= nv.n) return;
   const double4 ps = P[s], as = f[s];
   SumsD<1> t;
   if (!sums64_of<kPair, 1>(
-          nv, s, h, [&](int j) { return D4x2{P[j], f[j]}; },
+          nv, s, h, [&](int o) { return D4x2{record_at(P, o), record_at(f, o)}; },
           [&](auto& a, const D4x2& q) {
             const PairGeom64 r = pair_geom64(ps, q.a, pc.inv_h);
             const double u = r.r > pc.pair_eps ? r.t * r.t * r.rinv : 0.0;
-            a.v[0] += u * ((as.x - q.b.x) * r.dx + (as.y - q.b.y) * r.dy + (as.z - q.b.z) * r.dz);
+            a.v[0] = fma(u, fma(as.z - q.b.z, r.dz, fma(as.y - q.b.y, r.dy, (as.x - q.b.x) * r.dx)), a.v[0]);
           },
           t))
     return;
@@ -282,50 +289,46 @@ __global__ __launch_bounds__(kBlock) void k64_adj_lambda(NbrView nv, const doubl
   const double rho_bar = active ? -lam_bar * ax.w : 0.0;
   const double s_bar = active ? -lam_bar * ps.w * ax.w : 0.0;
   q1[s] = make_double4(as.x, as.y, as.z, rho_bar);
-  q2[s] = make_double4(s_bar * pc.cG * ax.x, s_bar * pc.cG * ax.y, s_bar * pc.cG * ax.z, s_bar);
+  // 2 S_bar G and 2 S_bar, as the position pass uses them
+  const double s2 = 2.0 * s_bar;
+  q2[s] = make_double4(s2 * pc.cG * ax.x, s2 * pc.cG * ax.y, s2 * pc.cG * ax.z, s2);
 }
 
 // e_k = e_{k+1} + sum_j [J(d) w + (rho_bar_i + rho_bar_j) psi(d)], f = e + c.
 template <bool kPair>
 __global__ __launch_bounds__(kBlock) void k64_adj_pos(NbrView nv, const double4* __restrict__ P,
-                                                      const double4* __restrict__ aux,
                                                       const double4* __restrict__ q1,
                                                       const double4* __restrict__ q2,
                                                       const double4* __restrict__ e_in,
                                                       const double4* __restrict__ c, double4* __restrict__ e_out,
                                                       double4* __restrict__ f_out, PhysConst64 pc) {
 #pragma clang fp contract(off)
-  const int g = blockIdx.x * blockDim.x + threadIdx.x;
+  const int g = xcd_block(blockIdx.x, gridDim.x) * blockDim.x + threadIdx.x;
   const int s = kPair ? g >> 1 : g, h = kPair ? g & 1 : 0;
   if (s >= nv.n) return;
-  const double4 ps = P[s], q1s = q1[s], q2s = q2[s], ax = aux[s];
-  const double Gx = pc.cG * ax.x, Gy = pc.cG * ax.y, Gz = pc.cG * ax.z;
+  const double4 ps = P[s], q1s = q1[s], q2s = q2[s];
   const double C = 2.0 * pc.corr;
   const double cpsi = -3.0 * pc.cW * pc.inv_h;
   SumsD<3> t;
   if (!sums64_of<kPair, 3>(
-          nv, s, h, [&](int j) { return D4x3{P[j], q1[j], q2[j]}; },
+          nv, s, h, [&](int o) { return D4x3{record_at(P, o), record_at(q1, o), record_at(q2, o)}; },
           [&](auto& a, const D4x3& q) {
+            // the terms of adj_pos_term (pbf_adjoint.hip)
             const PairGeom64 r = pair_geom64(ps, q.a, pc.inv_h);
-            const double t2 = r.t * r.t;
-            const double cr = (q1s.w + q.b.w) * cpsi * t2 * r.rinv;
-            a.v[0] += cr * r.dx;
-            a.v[1] += cr * r.dy;
-            a.v[2] += cr * r.dz;
-            if (r.r > pc.pair_eps) {
-              const double u = t2 * r.rinv;
-              const double cg = pc.cG * u;
-              const double gx = cg * r.dx, gy = cg * r.dy, gz = cg * r.dz;
-              const double cl = C * (ps.w + q.a.w);
-              const double wx = cl * (q1s.x - q.b.x) + 2.0 * q2s.w * (gx + Gx) + 2.0 * (q.c.w * gx - q.c.x);
-              const double wy = cl * (q1s.y - q.b.y) + 2.0 * q2s.w * (gy + Gy) + 2.0 * (q.c.w * gy - q.c.y);
-              const double wz = cl * (q1s.z - q.b.z) + 2.0 * q2s.w * (gz + Gz) + 2.0 * (q.c.w * gz - q.c.z);
-              const double dw = r.dx * wx + r.dy * wy + r.dz * wz;
-              const double k2 = (2.0 * r.t * pc.inv_h + u) * r.rinv * r.rinv * dw;
-              a.v[0] += pc.cG * (u * wx - k2 * r.dx);
-              a.v[1] += pc.cG * (u * wy - k2 * r.dy);
-              a.v[2] += pc.cG * (u * wz - k2 * r.dz);
-            }
+            const bool far = r.r > pc.pair_eps;
+            const double v = r.t * r.t * r.rinv;
+            const double u = far ? v : 0.0;
+            const double cg = pc.cG * u;
+            const double cl = C * (ps.w + q.a.w), sg = (q2s.w + q.c.w) * cg;
+            const double wx = fma(cl, q1s.x - q.b.x, fma(sg, r.dx, q2s.x - q.c.x));
+            const double wy = fma(cl, q1s.y - q.b.y, fma(sg, r.dy, q2s.y - q.c.y));
+            const double wz = fma(cl, q1s.z - q.b.z, fma(sg, r.dz, q2s.z - q.c.z));
+            const double dw = fma(r.dz, wz, fma(r.dy, wy, r.dx * wx));
+            const double k = fma(r.t, 2.0 * pc.inv_h, u) * (r.rinv * r.rinv) * dw;
+            const double cd = fma(-pc.cG, far ? k : 0.0, (q1s.w + q.b.w) * cpsi * v);
+            a.v[0] = fma(cg, wx, fma(cd, r.dx, a.v[0]));
+            a.v[1] = fma(cg, wy, fma(cd, r.dy, a.v[1]));
+            a.v[2] = fma(cg, wz, fma(cd, r.dz, a.v[2]));
           },
           t))
     return;
@@ -391,10 +394,10 @@ void launch64_adjoint_step(const NbrView& nv, double4* const* P, double4* const*
   for (int k = K - 1; k >= 0; --k) {
     if (lanes == 2) {
       k64_adj_lambda<true><<<nbp, kBlock, 0, st>>>(nv, P[k], aux[k], ab.f, ab.q1, ab.q2, pc);
-      k64_adj_pos<true><<<nbp, kBlock, 0, st>>>(nv, P[k], aux[k], ab.q1, ab.q2, e, ab.c, e2, ab.f, pc);
+      k64_adj_pos<true><<<nbp, kBlock, 0, st>>>(nv, P[k], ab.q1, ab.q2, e, ab.c, e2, ab.f, pc);
     } else {
       k64_adj_lambda<false><<<nb, kBlock, 0, st>>>(nv, P[k], aux[k], ab.f, ab.q1, ab.q2, pc);
-      k64_adj_pos<false><<<nb, kBlock, 0, st>>>(nv, P[k], aux[k], ab.q1, ab.q2, e, ab.c, e2, ab.f, pc);
+      k64_adj_pos<false><<<nb, kBlock, 0, st>>>(nv, P[k], ab.q1, ab.q2, e, ab.c, e2, ab.f, pc);
     }
     double4* t = e;
     e = e2;
