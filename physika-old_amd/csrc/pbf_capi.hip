@@ -633,6 +633,14 @@ NbrView view_of(const pbf_ctx* c, int n) {
   return nv;
 }
 
+// Largest unstaged search whose neighbor pass runs eight lanes per particle. A
+// run of candidates fills their rounds at 2.5 spacings in h (39 candidates a
+// run; 65,536 particles 35 -> 30 us, 100,003 particles 38 -> 45 us) but not at 1.2
+// spacings (4 a run; 32,768 particles 13.4 -> 11.9 us, 65,536 14.3 -> 19.8 us).
+int small_search_max(const pbf_ctx* c) {
+  return c->p.smoothing_length >= 2.25f * c->p.sampling_distance ? 65536 : 32768;
+}
+
 NbrOut out_of(pbf_ctx* c) {
   NbrOut o;
   o.mask = c->mask;
@@ -645,6 +653,7 @@ NbrOut out_of(pbf_ctx* c) {
   o.list_mode = c->list_mode;
   o.stage = c->stage;
   o.stage_lists = 0;
+  o.small_max = small_search_max(c);
   o.oog_rcnt = c->oog_rcnt;
   o.oog_rev = c->oog_rev;
   o.cnt_a = c->cnt_a;

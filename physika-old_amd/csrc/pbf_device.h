@@ -109,6 +109,16 @@ __device__ __forceinline__ int wave_max_full(int v) {
              max(__builtin_amdgcn_readlane(v, 47), __builtin_amdgcn_readlane(v, 63)));
 }
 
+// Wave-wide sum with every lane active (DPP row shifts, then lane reads).
+__device__ __forceinline__ int wave_sum_full(int v) {
+  v += dpp_row_shr<0x111>(0, v);
+  v += dpp_row_shr<0x112>(0, v);
+  v += dpp_row_shr<0x114>(0, v);
+  v += dpp_row_shr<0x118>(0, v);
+  return __builtin_amdgcn_readlane(v, 15) + __builtin_amdgcn_readlane(v, 31) + __builtin_amdgcn_readlane(v, 47) +
+         __builtin_amdgcn_readlane(v, 63);
+}
+
 // Exchanges a and b when c holds (per lane: selects on values in registers; a
 // select between whole structs becomes one between their addresses, which puts
 // them in memory).

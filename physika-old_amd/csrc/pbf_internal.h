@@ -170,6 +170,7 @@ struct NbrOut {
   int* list_mode;
   int* stage;
   int stage_lists;      // 1: waves that allow it write kListStaged lists
+  int small_max;        // unstaged searches of at most this many particles run several lanes per particle
   int* nbr_cnt;
   uint16_t* cnt_a;
   int* oog_rcnt;        // zeroed by the sort; out-of-grid lanes count themselves into their neighbors'
@@ -220,8 +221,8 @@ constexpr int kBlock = 256;
 // (16 bytes per particle, plus the padding entries).
 constexpr int kMaxParticles = 1 << 27;
 // Entries allocated past the end of the sorted position array xn, so that a
-// candidate group of 8 may read past a run's end.
-constexpr int kXnPad = 32;
+// group of candidates may read past a run's end.
+constexpr int kXnPad = 64;
 // Blocks of the device-length scan.
 constexpr int kScanDevBlocks = 128;
 

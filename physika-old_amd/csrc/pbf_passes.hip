@@ -173,7 +173,6 @@ __device__ __forceinline__ void write_list_runs(uint16_t* list, long long lb, in
 // whose three intervals hold at most kStageCap particles together (and contain
 // every lane's runs, checked) writes those neighbors as stage slots, so that
 // the PBD passes read them from LDS.
-template <int kG>
 __global__ __launch_bounds__(64) void k_neighbors(NbrView nv, NbrOut out, unsigned long long* __restrict__ counters) {
   __shared__ uint2 lword[kNbLdsWords * 64];
   const int wave = xcd_block(blockIdx.x, gridDim.x);
@@ -260,7 +259,7 @@ __global__ __launch_bounds__(64) void k_neighbors(NbrView nv, NbrOut out, unsign
     const int nw = (rl[q] + 31) >> 5;
     for (int w = 0; w < nw; ++w) {
       const int jb = ra[q] + (w << 5);
-      const uint32_t bits = test_word_planes<kG>(nv.cx, nv.cy, nv.cz, jb, xi, min(32, rl[q] - (w << 5)), nv.thr2);
+      const uint32_t bits = test_word_planes(nv.cx, nv.cy, nv.cz, jb, xi, min(32, rl[q] - (w << 5)), nv.thr2);
       if (in_lds) {
         const uint32_t base = mode == kListIndex32
                                   ? (uint32_t)jb
@@ -290,7 +289,7 @@ __global__ __launch_bounds__(64) void k_neighbors(NbrView nv, NbrOut out, unsign
         const int jb = ra[q] + (w << 5);
         uint32_t bits = (!in_lds && mb >= 0)
                             ? gcol[(long long)(wo + w) << 6]
-                            : test_word_planes<kG>(nv.cx, nv.cy, nv.cz, jb, xi, min(32, rl[q] - (w << 5)), nv.thr2);
+                            : test_word_planes(nv.cx, nv.cy, nv.cz, jb, xi, min(32, rl[q] - (w << 5)), nv.thr2);
         while (bits) {
           const int j = jb + pop_first(bits);
           const int slot = atomicAdd(&out.oog_rcnt[j], 1);
@@ -355,7 +354,7 @@ __global__ __launch_bounds__(64) void k_neighbors(NbrView nv, NbrOut out, unsign
         write_list_lds<0>(out.list, lb, lane, lcol, cnt, n_sl, pad_to);
     } else if (in_lds) {  // this lane's words did not fit: test its candidates again
       auto retest = [&](int q, int w, int) {
-        return test_word_planes<kG>(nv.cx, nv.cy, nv.cz, ra[q] + (w << 5), xi, min(32, rl[q] - (w << 5)), nv.thr2);
+        return test_word_planes(nv.cx, nv.cy, nv.cz, ra[q] + (w << 5), xi, min(32, rl[q] - (w << 5)), nv.thr2);
       };
       if (mode == kListIndex32)
         write_list_runs<1>(out.list, lb, lane, ra, rl, retest, jbase, sdel, 0, 0);
@@ -371,29 +370,240 @@ __global__ __launch_bounds__(64) void k_neighbors(NbrView nv, NbrOut out, unsign
   }
 }
 
-// A search of at most kWideGroupMaxParticles particles runs one wave or fewer
-// per SIMD, and each wave waits on its own candidate loads: it tests sixteen
-// candidates per load round trip. Larger searches keep groups of eight (issue
-// slots bound them, and a run's partly empty last group costs more in groups
-// of sixteen). Both give the same bits.
-constexpr int kWideGroupMaxParticles = 65536;
+// The neighbor pass of a small search: kCoLanes lanes per particle, one
+// workgroup per list wave. A search of few waves waits on its own loads and on
+// the serial walk of 64 lists: one lane per particle took 28 us at 1,728
+// particles and at 32,768 alike. Here a particle's lanes test consecutive
+// candidates of a run with one coalesced load, the ballot of the hits gives
+// every hit its place in the list (the same order: runs in visit order,
+// ascending index), and the list is put together in LDS and written out in
+// 16-byte pieces. Same results as k_neighbors without staged lists, bit for
+// bit. Measured (us, one lane per particle -> this): 31 -> 12 at 2,000
+// particles of a lattice with 2.5 spacings in h, 33 -> 17 at 32,768, 35 -> 30 at
+// 65,536, but 38 -> 45 at 100,003, where issue slots count: 1,230 vector
+// instructions per wave of eight particles against 6,700 per wave of 64.
+// small_search_max (pbf_capi.hip) draws the line. Sixteen lanes per particle
+// took 17, 33 and 59 us. Rows of 700 neighbors: 1,045 -> 197 at 32,768.
+constexpr int kCoLanes = 8, kCoBlock = 64 * kCoLanes, kCoWaves = kCoBlock / 64;
+constexpr int kCoRounds = 5;   // rounds of kCoLanes candidates in flight: a run of a lattice in one go
+constexpr int kCoList = 128;   // list entries per particle in LDS
+constexpr int kCoStride = kCoList + 8;
+static_assert(kXnPad >= kCoLanes * kCoRounds, "a group of rounds may start at a run's last candidate");
 
-template <int kG>
-void launch_neighbors_g(const NbrView& nv, const NbrOut& out, unsigned long long* counters, hipStream_t st,
-                        const KernelEvents* ev) {
-  if (ev)
-    hipExtLaunchKernelGGL(k_neighbors<kG>, dim3((nv.n + 63) / 64), dim3(64), 0, st, ev->start, ev->stop, 0, nv, out,
-                          counters);
-  else
-    k_neighbors<kG><<<(nv.n + 63) / 64, 64, 0, st>>>(nv, out, counters);
+__global__ __launch_bounds__(kCoBlock) void k_neighbors_small(NbrView nv, NbrOut out,
+                                                              unsigned long long* __restrict__ counters) {
+  __shared__ __attribute__((aligned(16))) uint16_t entry[64 * kCoStride];
+  __shared__ int red[kCoWaves][4];
+  __shared__ long long mask_at;
+  const int wave = xcd_block(blockIdx.x, gridDim.x);
+  const int l = threadIdx.x / kCoLanes, h = threadIdx.x % kCoLanes;  // particle of the list wave, lane of it
+  const int hw = threadIdx.x >> 6, lane = threadIdx.x & 63, sh = lane & ~(kCoLanes - 1);
+  const int s = (wave << 6) + l;
+  const bool active = s < nv.n;
+  // lane h looks up run h, every lane the last run
+  float4 xi = make_float4(0.f, 0.f, 0.f, 0.f);
+  int a_h = 0, l_h = 0, a_8 = 0, l_8 = 0;
+  bool oog = false;
+  if (active) {
+    const SceneWin win = nv.win[nv.ssid[s]];
+    xi = nv.xn[s];
+    int ci, cj, ck, xlo, xhi;
+    float frac;
+    cell_of(nv.g, xi.x, xi.y, xi.z, ci, cj, ck, frac);
+    stencil_x(nv.g, ci, frac, xlo, xhi);
+    run_range(nv.cell_start, win, ci, cj, ck, xlo, xhi, h, a_h, l_h);
+    run_range(nv.cell_start, win, ci, cj, ck, xlo, xhi, 8, a_8, l_8);
+    oog = !in_window(win, ci, cj, ck);
+  }
+  int ra[9], rl[9];
+#pragma unroll
+  for (int q = 0; q < 8; ++q) {
+    ra[q] = __shfl(a_h, sh + q);
+    rl[q] = __shfl(l_h, sh + q);
+  }
+  ra[8] = a_8;
+  rl[8] = l_8;
+  // reductions over the list wave: each hardware wave's part, then all of them
+  auto reduce = [&](int a, int b, int c, int d) {
+    if (lane == 0) {
+      red[hw][0] = a;
+      red[hw][1] = b;
+      red[hw][2] = c;
+      red[hw][3] = d;
+    }
+    __syncthreads();
+    int4 r = make_int4(red[0][0], red[0][1], red[0][2], red[0][3]);
+#pragma unroll
+    for (int w = 1; w < kCoWaves; ++w)
+      r = make_int4(min(r.x, red[w][0]), max(r.y, red[w][1]), max(r.z, red[w][2]), r.w + red[w][3]);
+    __syncthreads();
+    return r;
+  };
+  const int jlo = min(l_h > 0 ? a_h : INT_MAX, l_8 > 0 ? a_8 : INT_MAX);
+  const int jhi = max(l_h > 0 ? a_h + l_h - 1 : -1, l_8 > 0 ? a_8 + l_8 - 1 : -1);
+  const int4 r1 = reduce(wave_min_full(jlo), wave_max_full(jhi), wave_max_full(max(l_h, l_8)),
+                         wave_sum_full(l_h + (h == 0 ? l_8 : 0)));
+  const int wjlo = r1.x, tcand = r1.w;
+  const bool wide = r1.y >= wjlo && r1.y - wjlo > 65535;
+  const int jbase = wide ? 0 : wjlo;
+  const int per = out.list_per;
+  const long long lb0 = (long long)wave * 64 * per;
+  // places of a lane's list inside the wave's region (whole groups)
+  const int cap = wide ? (per >> 1) & ~3 : per & ~7;
+  char* const list = reinterpret_cast<char*>(out.list + lb0) + 16 * l;
+  uint16_t* const mine = entry + kCoStride * l;
+  const uint32_t below = (1u << h) - 1u, bits_at = sh & 31;
+  const bool upper = lane >= 32;
+
+  // the hits of one round of candidates as bits of the particle's lanes
+  auto round_hits = [&](float cx, float cy, float cz, bool on, bool& hit) {
+    hit = on && sq_dist(xi, make_float4(cx, cy, cz, 0.0f)) < nv.thr2;
+    const unsigned long long b = __ballot(hit);
+    const uint32_t w = upper ? (uint32_t)(b >> 32) : (uint32_t)b;
+    return __builtin_amdgcn_ubfe(w, bits_at, kCoLanes);
+  };
+  struct Round {
+    float x[kCoRounds], y[kCoRounds], z[kCoRounds];
+  };
+  auto load = [&](int a, Round& c) {  // candidates a + kCoLanes u + h (past the run's end: unused)
+    const char* base = reinterpret_cast<const char*>(nv.xn) + ((uint32_t)(a + h) << 4);
+#pragma unroll
+    for (int u = 0; u < kCoRounds; ++u) {
+      const float* p = reinterpret_cast<const float*>(base + 16 * kCoLanes * u);
+      c.x[u] = p[0];
+      c.y[u] = p[1];
+      c.z[u] = p[2];
+    }
+  };
+  // every hit of the nine runs, in order: hit(pos, j) on its lane; returns their count
+  auto walk = [&](auto&& on_hit) {
+    int cnt = 0;
+    auto test = [&](int a, int left, const Round& c) {  // left: candidates from this lane's first one on
+#pragma unroll
+      for (int u = 0; u < kCoRounds; ++u) {
+        const bool on = left > kCoLanes * u;
+        if (u > 0 && !__any(on)) break;  // the wave's longest run ends here
+        bool hit;
+        const uint32_t m = round_hits(c.x[u], c.y[u], c.z[u], on, hit);
+        if (hit) on_hit(cnt + __popc(m & below), a + kCoLanes * u);
+        cnt += __popc(m);
+      }
+    };
+    // two buffers: the next run's first candidates are on their way while this
+    // run's are tested
+    Round c0, c1;
+    load(ra[0], c0);
+#pragma unroll
+    for (int q = 0; q < 9; ++q) {
+      Round& cur = q & 1 ? c1 : c0;
+      Round& next = q & 1 ? c0 : c1;
+      if (q < 8) load(ra[q + 1], next);
+      asm volatile("" ::: "memory");  // keep these loads ahead of the tests
+      test(ra[q] + h, rl[q] - h, cur);
+      for (int k0 = kCoLanes * kCoRounds; k0 < rl[q]; k0 += kCoLanes * kCoRounds) {
+        load(ra[q] + k0, cur);
+        test(ra[q] + k0 + h, rl[q] - k0 - h, cur);
+      }
+    }
+    return cnt;
+  };
+  // a wave whose lists fit LDS puts them together there; others (32-bit entries,
+  // long lists, found out by their candidates or by the count) write entry by entry
+  int cnt = 0;
+  bool direct = wide || r1.z > kCoList;
+  if (!direct) {
+    cnt = walk([&](int pos, int j) {
+      if (pos < kCoList) mine[pos] = (uint16_t)(j - jbase);
+    });
+    direct = __any(cnt > kCoList);
+    wave_lds_fence();
+    if (!direct) {
+      const int end = min(cnt, cap);
+      for (int c = h; 8 * c < end; c += kCoLanes)
+        *reinterpret_cast<uint4*>(list + (c << 10)) = *reinterpret_cast<const uint4*>(mine + 8 * c);
+    }
+  }
+  if (direct) {
+    cnt = walk([&](int pos, int j) {
+      if (pos >= cap) return;
+      if (wide)
+        *reinterpret_cast<int*>(list + ((pos >> 2) << 10) + ((pos & 3) << 2)) = j;
+      else
+        *reinterpret_cast<uint16_t*>(list + ((pos >> 3) << 10) + ((pos & 7) << 1)) = (uint16_t)(j - jbase);
+    });
+  }
+  // an out-of-grid particle registers itself with each one it lists (k_neighbors)
+  if (__any(oog)) {
+    walk([&](int, int j) {
+      if (!oog) return;
+      const int slot = atomicAdd(&out.oog_rcnt[j], 1);
+      if (slot < kOogRev) out.oog_rev[(size_t)j * kOogRev + slot] = s;
+    });
+  }
+  int words = 0;
+#pragma unroll
+  for (int q = 0; q < 9; ++q) words += (rl[q] + 31) >> 5;
+  const int4 r2 = reduce(wave_min_full(active ? cnt : INT_MAX), wave_max_full(cnt), wave_max_full(words),
+                         wave_sum_full(h == 0 ? cnt : 0));
+  const int cmax = r2.y, wmax = r2.z, tot = r2.w;
+  const int need = wide ? ((cmax + 3) & ~3) << 1 : (cmax + 7) & ~7;  // 16-bit slots per lane
+  const bool listed = need <= per;
+  long long mb = -1;
+  if (!listed && wmax > kNbMaxWords) {
+    // no room for the list: a wave of many candidate words keeps them as bit masks
+    if (threadIdx.x == 0) {
+      const unsigned long long want = 64ull * (unsigned long long)wmax;
+      const unsigned long long at = atomicAdd(&counters[C_MASK_WORDS], want);
+      const bool fits = (long long)(at + want) <= out.mask_cap;
+      if (!fits) atomicAdd(&counters[C_FALLBACK], 1ull);
+      mask_at = fits ? (long long)at : -1;
+    }
+    __syncthreads();
+    mb = mask_at;
+    if (mb >= 0) {
+      int wofs = 0;
+#pragma unroll
+      for (int q = 0; q < 9; ++q) {
+        for (int k0 = 0; k0 < rl[q]; k0 += 32) {
+          uint32_t word = 0;
+#pragma unroll
+          for (int u = 0; u < 32 / kCoLanes; ++u) {
+            const int k = k0 + kCoLanes * u + h;
+            const float4 c = nv.xn[ra[q] + k];
+            bool hit;
+            word |= round_hits(c.x, c.y, c.z, k < rl[q], hit) << (kCoLanes * u);
+          }
+          if (h == 0) out.mask[mb + ((long long)wofs << 6) + l] = __brev(word);
+          ++wofs;
+        }
+      }
+    }
+  }
+  if (active && h == 0) out.nbr_cnt[s] = cnt;
+  if (threadIdx.x == 0) {
+    out.mask_base[wave] = mb;
+    out.list_base[wave] = listed ? lb0 : -1;
+    out.list_jbase[wave] = wjlo;
+    out.list_mode[wave] = (wide ? kListIndex32 : kListDelta16) | ((r2.x >> 2) << 2);
+    out.wave_stat[wave] = make_int4(tot, tcand, need, 0);
+  }
 }
 
 void launch_neighbors(const NbrView& nv, const NbrOut& out, unsigned long long* counters, hipStream_t st,
                       const KernelEvents* ev) {
-  if (nv.n <= kWideGroupMaxParticles)
-    launch_neighbors_g<16>(nv, out, counters, st, ev);
-  else
-    launch_neighbors_g<8>(nv, out, counters, st, ev);
+  const int waves = (nv.n + 63) / 64;
+  const bool small = nv.n <= out.small_max && !out.stage_lists;
+  if (ev) {
+    if (small)
+      hipExtLaunchKernelGGL(k_neighbors_small, dim3(waves), dim3(kCoBlock), 0, st, ev->start, ev->stop, 0, nv, out,
+                            counters);
+    else
+      hipExtLaunchKernelGGL(k_neighbors, dim3(waves), dim3(64), 0, st, ev->start, ev->stop, 0, nv, out, counters);
+  } else if (small) {
+    k_neighbors_small<<<waves, kCoBlock, 0, st>>>(nv, out, counters);
+  } else {
+    k_neighbors<<<waves, 64, 0, st>>>(nv, out, counters);
+  }
 }
 
 // One block: sums and maxima over the per-wave statistics.

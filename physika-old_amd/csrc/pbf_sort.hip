@@ -234,16 +234,6 @@ constexpr int kBoundsBlock = 256, kBoundsPer = 4, kBoundsSpan = kBoundsBlock * k
 
 size_t bounds_part_ints(long long n) { return 8 * (size_t)((n + kBoundsSpan - 1) / kBoundsSpan + 1); }
 
-// Wave-wide sum with every lane active (DPP row shifts, then lane reads).
-__device__ __forceinline__ int wave_sum_full(int v) {
-  v += dpp_row_shr<0x111>(0, v);
-  v += dpp_row_shr<0x112>(0, v);
-  v += dpp_row_shr<0x114>(0, v);
-  v += dpp_row_shr<0x118>(0, v);
-  return __builtin_amdgcn_readlane(v, 15) + __builtin_amdgcn_readlane(v, 31) + __builtin_amdgcn_readlane(v, 47) +
-         __builtin_amdgcn_readlane(v, 63);
-}
-
 template <bool kCellOrder>
 __global__ __launch_bounds__(kBoundsBlock) void k_scene_bounds(SortIn in, int n, GridDev g,
                                                                const int* __restrict__ off, int nscenes,
