@@ -171,7 +171,8 @@ __device__ __forceinline__ float box_jitter(int id) {
 }
 
 // K_ConstrainSDF (BoundaryConstraint.cu:30-67) on (x_in, v_in) -> (x_out,
-// v_out); the particle id is its index inside its scene.
+// v_out); the particle id is its index inside its scene (scene_off null: one
+// scene).
 __global__ __launch_bounds__(kBlock) void k_box_constrain(BoxField f, const float* __restrict__ x_in,
                                                           const float* __restrict__ v_in, float* __restrict__ x_out,
                                                           float* __restrict__ v_out, int n,
@@ -195,7 +196,7 @@ __global__ __launch_bounds__(kBlock) void k_box_constrain(BoxField f, const floa
         hi = mid;
     }
     const float olddist = -dist;
-    dist = box_jitter(i - scene_off[lo]);
+    dist = box_jitter(i - (scene_off ? scene_off[lo] : 0));
     const float s = olddist + dist;
     px = px - s * nr.x;
     py = py - s * nr.y;

@@ -36,7 +36,6 @@ struct pbf_ctx {
 
   // scenes
   int scene_cap = 0;
-  int* off1 = nullptr;          // offsets {0, n} of a one-scene call
   int* scene_minmax = nullptr;  // 6 per scene
   SceneWin* win = nullptr;
   int* total_cells = nullptr;
@@ -168,7 +167,8 @@ struct pbf_ctx {
   long long graph_replays = 0, graph_captures = 0;
 
   unsigned long long* counters = nullptr;     // device, C_COUNT
-  unsigned long long* h_counters = nullptr;   // pinned host copy
+  unsigned long long* h_counters = nullptr;   // pinned, mapped host copy, written by k_wave_stats
+  unsigned long long* h_counters_dev = nullptr;  // its device address
   hipEvent_t counters_ev = nullptr;
   bool counters_pending = false;
 
@@ -522,7 +522,7 @@ int ensure_list(pbf_ctx* c, long long slots) {
   c->gen++;
   dfree(c->list);
   c->list_cap = 0;
-  PBF_HIP(c, hipMalloc(&c->list, sizeof(uint16_t) * (size_t)slots));
+  PBF_HIP(c, hipMalloc(&c->list, sizeof(uint16_t) * ((size_t)slots + kListPad)));
   c->list_cap = slots;
   return PBF_OK;
 }
@@ -628,6 +628,7 @@ NbrView view_of(const pbf_ctx* c, int n) {
   nv.mask = c->mask;
   nv.counters = c->counters;
   nv.thr2 = c->pc.thr2;
+  nv.list_per = list_per_of(c);
   nv.n = n;
   nv.pad = n;
   return nv;
@@ -801,10 +802,9 @@ int search(pbf_ctx* c, const float* x, const float* v, int n, const int* scene_o
 }
 
 int record_counters(pbf_ctx* c, hipStream_t st) {
-  launch_wave_stats(c->wave_stat, c->stats_waves, c->counters, st);
+  launch_wave_stats(c->wave_stat, c->stats_waves, c->counters, c->h_counters_dev, st);
   c->stats_waves = 0;
-  PBF_HIP(c, hipMemcpyAsync(c->h_counters, c->counters, sizeof(unsigned long long) * C_COUNT,
-                            hipMemcpyDeviceToHost, st));
+  PBF_LAUNCHED(c);
   PBF_HIP(c, hipEventRecord(c->counters_ev, st));
   c->counters_pending = true;
   return PBF_OK;
@@ -1107,7 +1107,7 @@ int ensure_tape(pbf_ctx* c, int m) {
     PBF_HIP(c, hipMalloc(&t.list_mode, sizeof(int) * nwv));
     PBF_HIP(c, hipMalloc(&t.stage, sizeof(int) * kStageInts * nwv));
     PBF_HIP(c, hipMalloc(&t.cnt_a, sizeof(uint16_t) * cap));
-    PBF_HIP(c, hipMalloc(&t.list, sizeof(uint16_t) * std::max<size_t>(c->slot_list, 1)));
+    PBF_HIP(c, hipMalloc(&t.list, sizeof(uint16_t) * (c->slot_list + kListPad)));
     PBF_HIP(c, hipMalloc(&t.mask, sizeof(uint32_t) * std::max<size_t>(c->slot_mask, 1)));
     PBF_HIP(c, hipMalloc(&t.cell_start, sizeof(int) * ((size_t)c->cell_cap + 2)));
     PBF_HIP(c, hipMalloc(&t.win, sizeof(SceneWin) * (size_t)std::max(c->scene_cap, 1)));
@@ -1293,10 +1293,11 @@ int pbf_create(const pbf_params* p, pbf_ctx** out) {
   }
   if (hipGetDevice(&c->device) != hipSuccess ||
       hipMalloc(&c->counters, sizeof(unsigned long long) * C_COUNT) != hipSuccess ||
-      hipHostMalloc(&c->h_counters, sizeof(unsigned long long) * C_COUNT) != hipSuccess ||
+      hipHostMalloc(&c->h_counters, sizeof(unsigned long long) * C_COUNT, hipHostMallocMapped) != hipSuccess ||
+      hipHostGetDevicePointer((void**)&c->h_counters_dev, c->h_counters, 0) != hipSuccess ||
       hipEventCreateWithFlags(&c->counters_ev, hipEventDisableTiming) != hipSuccess ||
       hipStreamCreateWithFlags(&c->cap_stream, hipStreamNonBlocking) != hipSuccess ||
-      hipMalloc(&c->off1, sizeof(int) * 2) != hipSuccess || hipMalloc(&c->total_cells, sizeof(int)) != hipSuccess ||
+      hipMalloc(&c->total_cells, sizeof(int)) != hipSuccess ||
       hipMalloc(&c->scan_part, sizeof(int) * (kScanDevBlocks + 1)) != hipSuccess ||
       hipMalloc(&c->pairing, sizeof(unsigned long long) * kPairingSlots) != hipSuccess) {
     pbf_destroy(c);
@@ -1321,7 +1322,7 @@ int pbf_create(const pbf_params* p, pbf_ctx** out) {
 int pbf_destroy(pbf_ctx* c) {
   if (!c) return PBF_ERR_INVALID;
   (void)hipDeviceSynchronize();
-  dfree(c->off1); dfree(c->scene_minmax); dfree(c->win); dfree(c->total_cells); dfree(c->scan_part);
+  dfree(c->scene_minmax); dfree(c->win); dfree(c->total_cells); dfree(c->scan_part);
   dfree(c->pairing);
   dfree(c->cell_cnt); dfree(c->cell_start);
   dfree(c->key); dfree(c->slot); dfree(c->tmp); dfree(c->perm); dfree(c->inv);
@@ -1404,8 +1405,7 @@ int pbf_neighbor_query(pbf_ctx* c, const float* d_x, int n, int* d_index, int* d
   }
   s = adapt_reservations(c);
   if (s) return s;
-  launch_set_offsets(c->off1, n, st);
-  s = search(c, d_x, nullptr, n, c->off1, 1, false, st);
+  s = search(c, d_x, nullptr, n, nullptr, 1, false, st);
   if (s) return s;
   s = record_counters(c, st);
   if (s) return s;
@@ -1491,8 +1491,7 @@ int pbf_step(pbf_ctx* c, float* d_x, float* d_v, float* d_rho, int n, int nsteps
   if (s) return s;
   s = adapt_reservations(c);
   if (s) return s;
-  launch_set_offsets(c->off1, n, st);
-  return run_steps(c, d_x, d_v, d_rho, n, c->off1, 1, nsteps, st);
+  return run_steps(c, d_x, d_v, d_rho, n, nullptr, 1, nsteps, st);
 }
 
 int pbf_batch_step(pbf_ctx* c, float* d_x, float* d_v, float* d_rho, const int* d_scene_offsets, int nscenes, int n,
@@ -1786,8 +1785,7 @@ int pbf_neighbor_query_fixed(pbf_ctx* c, const float* d_x, int n, int limit, int
   if (s) return s;
   s = adapt_reservations(c);
   if (s) return s;
-  launch_set_offsets(c->off1, n, st);
-  s = search(c, d_x, nullptr, n, c->off1, 1, false, st);
+  s = search(c, d_x, nullptr, n, nullptr, 1, false, st);
   if (s) return s;
   launch_nbr_fixed(view_of(c, n), c->perm, limit, d_counts, d_elems, st);
   PBF_LAUNCHED(c);
@@ -1843,8 +1841,7 @@ int pbf_box_constrain(pbf_ctx* c, float* d_x, float* d_v, int n, void* stream) {
   int s = ensure_particles(c, n, 1);
   if (s) return s;
   if ((s = ensure_box(c, st))) return s;
-  launch_set_offsets(c->off1, n, st);
-  launch_box_constrain(c->bf, d_x, d_v, d_x, d_v, n, c->off1, 1, c->keep_normal, c->damp, st);
+  launch_box_constrain(c->bf, d_x, d_v, d_x, d_v, n, nullptr, 1, c->keep_normal, c->damp, st);
   PBF_LAUNCHED(c);
   return PBF_OK;
 }

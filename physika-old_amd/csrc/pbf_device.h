@@ -51,6 +51,15 @@ __device__ __forceinline__ bool in_grid(const GridDev& g, int fi, int cj, int ck
   return fi >= 0 && fi < 2 * g.nx && cj >= 0 && cj < g.ny && ck >= 0 && ck < g.nz;
 }
 
+__device__ __forceinline__ bool in_window(const SceneWin& w, int ci, int cj, int ck) {
+  return ci >= w.lo[0] && ci < w.lo[0] + w.dim[0] && cj >= w.lo[1] && cj < w.lo[1] + w.dim[1] && ck >= w.lo[2] &&
+         ck < w.lo[2] + w.dim[2];
+}
+
+__device__ __forceinline__ int window_cell(const SceneWin& w, int ci, int cj, int ck) {
+  return w.cell_base + (ci - w.lo[0]) + w.dim[0] * ((cj - w.lo[1]) + w.dim[1] * (ck - w.lo[2]));
+}
+
 // |x_i - x_j| < h exactly as NeighborQuery.cu:266-267 evaluates it: the squared
 // norm in glm's order ((dx*dx + dy*dy) + dz*dz, no fused multiply-add) against
 // thr2, the least float whose correctly rounded square root reaches h (the

@@ -149,6 +149,7 @@ struct NbrView {
   const int* oog_rev;          // their sorted indices, kOogRev slots per particle (in no order)
   const unsigned long long* counters;
   float thr2;
+  int list_per;       // 16-bit slots per particle of a wave's list region (wave w's list, if any, starts at 64 w list_per)
   int n;
   int pad;            // padding particle of the position buffers (index n)
 };
@@ -180,7 +181,7 @@ struct NbrOut {
 
 // Sorting state of a step (device arrays).
 struct SortBufs {
-  const int* scene_off;   // nscenes + 1 particle offsets
+  const int* scene_off;   // nscenes + 1 particle offsets; null: one scene of all particles
   int nscenes;
   int* sid;               // scene of each input particle (in the input's order)
   int* ssid;              // scene of each sorted particle
@@ -223,6 +224,9 @@ constexpr int kMaxParticles = 1 << 27;
 // Entries allocated past the end of the sorted position array xn, so that a
 // group of candidates may read past a run's end.
 constexpr int kXnPad = 64;
+// 16-bit slots allocated past the lists: two 16-byte chunks of a wave's 64 lanes,
+// which the lane-pair passes read before they know whether the wave has a list.
+constexpr int kListPad = 2 * 64 * 8;
 // Blocks of the device-length scan.
 constexpr int kScanDevBlocks = 128;
 
@@ -241,8 +245,10 @@ void launch_set_offsets(int* off, int n, hipStream_t st);
 void launch_copy_cells(const int* src, int* dst, const int* total_cells, long long cap, hipStream_t st);
 void launch_neighbors(const NbrView& nv, const NbrOut& out, unsigned long long* counters, hipStream_t st, const KernelEvents* ev = nullptr);
 // Sums the per-wave statistics of the last neighbor pass (nwaves waves) into
-// counters[C_PAIRS], [C_CANDIDATES], [C_LIST_SLOTS] and [C_LIST_NEED].
-void launch_wave_stats(const int4* wave_stat, int nwaves, unsigned long long* counters, hipStream_t st);
+// counters[C_PAIRS], [C_CANDIDATES], [C_LIST_SLOTS] and [C_LIST_NEED], and copies
+// all counters to host (mapped host memory).
+void launch_wave_stats(const int4* wave_stat, int nwaves, unsigned long long* counters, unsigned long long* host,
+                       hipStream_t st);
 // block: threads per workgroup, 64, 128, 256 or 512; persistent: as many
 // blocks as stay resident, each wave walking 64-particle tiles; lanes: 1, or 2
 // for a lane pair per particle (not persistent). The results depend on none of

@@ -52,15 +52,6 @@ __device__ __forceinline__ void run_range(const int* __restrict__ cell_start, co
   len = ok ? a1 - a0 : 0;
 }
 
-__device__ __forceinline__ bool in_window(const SceneWin& w, int ci, int cj, int ck) {
-  return ci >= w.lo[0] && ci < w.lo[0] + w.dim[0] && cj >= w.lo[1] && cj < w.lo[1] + w.dim[1] && ck >= w.lo[2] &&
-         ck < w.lo[2] + w.dim[2];
-}
-
-__device__ __forceinline__ int window_cell(const SceneWin& w, int ci, int cj, int ck) {
-  return w.cell_base + (ci - w.lo[0]) + w.dim[0] * ((cj - w.lo[1]) + w.dim[1] * (ck - w.lo[2]));
-}
-
 // bits * 2 + (s < thr2): the squared distance of one candidate shifted into a
 // word (v_cmp into VCC, then an add with carry-in; NaN compares false as in the
 // reference's test). thr2 is uniform and read from a scalar register.
@@ -290,20 +281,21 @@ __device__ __forceinline__ void group_bodies(int b, Full, int cnt, const Group4&
 // entry against the count. kPadded: entries past the count were decoded to a
 // padding particle whose terms are exactly zero, and the body runs on them
 // unguarded. decode(e, b, full) returns the indices of group b.
+// first, second: groups 0 and 1 (second unused in a list of one group).
 template <bool kPadded, class GroupT, class LoadFn, class DecodeFn, class GatherFn, class Body>
-__device__ __forceinline__ void list_loop(int cnt, int nfull, LoadFn&& load_group, DecodeFn&& decode,
-                                          GatherFn&& gather, Body&& body) {
+__device__ __forceinline__ void list_loop_from(int cnt, int nfull, GroupT first, GroupT second, LoadFn&& load_group,
+                                               DecodeFn&& decode, GatherFn&& gather, Body&& body) {
   using T = decltype(gather(0));
   const int ng = (cnt + 3) >> 2;
   if (ng == 0) return;
   // two group buffers that trade roles every step (no register copies)
   Group4 g0, g1;
   T a0[4], a1[4];
-  GroupT e = load_group(0);
+  GroupT e = first;
   g0 = nfull > 0 ? decode(e, 0, std::true_type{}) : decode(e, 0, std::false_type{});
 #pragma unroll
   for (int u = 0; u < 4; ++u) a0[u] = gather(g0.j[u]);
-  e = load_group(min(1, ng - 1));
+  e = second;
   // runs the bodies of group b (gc, ac) while group b+1 is gathered into
   // (gx, ax) and the indices of group b+2 are loaded
   auto step = [&](int b, auto full, const Group4& gc, const T(&ac)[4], Group4& gx, T(&ax)[4]) {
@@ -327,6 +319,14 @@ __device__ __forceinline__ void list_loop(int cnt, int nfull, LoadFn&& load_grou
     if (b + 1 >= ng) break;
     step(b + 1, std::false_type{}, g1, a1, g0, a0);
   }
+}
+
+template <bool kPadded, class GroupT, class LoadFn, class DecodeFn, class GatherFn, class Body>
+__device__ __forceinline__ void list_loop(int cnt, int nfull, LoadFn&& load_group, DecodeFn&& decode,
+                                          GatherFn&& gather, Body&& body) {
+  if (cnt <= 0) return;
+  list_loop_from<kPadded, GroupT>(cnt, nfull, load_group(0), load_group(min(1, ((cnt + 3) >> 2) - 1)), load_group,
+                                  decode, gather, body);
 }
 
 // list_loop for 16-bit lists: one 16-byte load brings two groups. An even
@@ -391,6 +391,26 @@ struct WaveList {
 __device__ __forceinline__ WaveList wave_list(const NbrView& nv, int wave) {
   return WaveList{nv.list_base[wave], nv.list_mode[wave], nv.list_jbase[wave]};
 }
+
+// What a lane pair's traversal reads first, all at once: the particle's count,
+// the first two chunks of its list (where the wave's list lies if it has one: at
+// the start of the wave's region; the allocation is padded by two chunks of a
+// wave) and the wave's words. Were the words read first, a search of few waves
+// would wait once more on memory.
+struct ListHead {
+  WaveList wl;
+  const uint4* L;  // the wave's region at this particle's lane
+  int cnt;
+  uint4 c0, c1;    // chunks 0 and 1
+  __device__ __forceinline__ void load(const NbrView& nv, int wave, int s) {
+    L = reinterpret_cast<const uint4*>(nv.list + (long long)wave * 64 * nv.list_per) + (s & 63);
+    cnt = nv.nbr_cnt[s];
+    c0 = L[0];
+    c1 = L[64];
+    wl = wave_list(nv, wave);
+    asm volatile("" ::: "memory");  // issue the loads here
+  }
+};
 
 // Calls body(j, gather(j), parity) for every neighbor j of sorted particle s,
 // in the canonical order (parity: EvenEntry or OddEntry, the entry's index mod
@@ -586,12 +606,14 @@ __device__ __forceinline__ void for_each_neighbor_staged(const NbrView& nv, int 
 template <bool kW, class Body>
 __device__ __forceinline__ bool for_each_neighbor_half(const NbrView& nv, int s, int h, const float4* __restrict__ xs,
                                                        float4* buf, Body&& body) {
-  const int wave = __builtin_amdgcn_readfirstlane(s >> 6), lane = s & 63;
-  const WaveList wl = wave_list(nv, wave);
+  const int wave = __builtin_amdgcn_readfirstlane(s >> 6);
+  ListHead head;
+  head.load(nv, wave, s);
+  const WaveList& wl = head.wl;
   const int mode = wl.lm & 3;
   if (wl.lb < 0 || (mode != kListDelta16 && mode != kListStaged)) return false;
-  const uint4* L = reinterpret_cast<const uint4*>(nv.list + wl.lb) + lane;
-  const int cnt = nv.nbr_cnt[s];
+  const uint4* L = head.L;
+  const int cnt = head.cnt;
   const uint32_t jb16 = (uint32_t)wl.jb << 4;
   const int past = (int)((uint32_t)nv.pad << 4);
   auto each = [&](int, const float4& xj, auto) { body(xj); };
@@ -602,8 +624,9 @@ __device__ __forceinline__ bool for_each_neighbor_half(const NbrView& nv, int s,
   if (mode == kListDelta16) {
     const int ch = (cnt - h + 1) >> 1;
     const uint32_t sh = (uint32_t)h << 4;
-    list_loop<true, uint4>(
-        ch, nfull, [&](int c) { return L[(long long)c << 6]; },
+    if (ch > 0)
+      list_loop_from<true, uint4>(
+        ch, nfull, head.c0, head.c1, [&](int c) { return L[(long long)c << 6]; },
         [&](uint4 e, int c, auto full) {
           return decode_half<decltype(full)::value, 16>(e, sh, jb16, c, ch, past);
         },
@@ -671,20 +694,23 @@ __device__ __forceinline__ Group4 decode_half_staged(uint4 e, uint32_t sh, const
 template <int kRec, class GatherFn, class Body>
 __device__ __forceinline__ bool for_each_record_half(const NbrView& nv, int s, int h, GatherFn&& gather,
                                                      Body&& body) {
-  const int wave = __builtin_amdgcn_readfirstlane(s >> 6), lane = s & 63;
-  const WaveList wl = wave_list(nv, wave);
+  const int wave = __builtin_amdgcn_readfirstlane(s >> 6);
+  ListHead head;
+  head.load(nv, wave, s);
+  const WaveList& wl = head.wl;
   const int mode = wl.lm & 3;
   if (wl.lb < 0 || (mode != kListDelta16 && mode != kListStaged)) return false;
-  const uint4* L = reinterpret_cast<const uint4*>(nv.list + wl.lb) + lane;
-  const int cnt = nv.nbr_cnt[s], past = s * kRec;
+  const uint4* L = head.L;
+  const int cnt = head.cnt, past = s * kRec;
   const uint32_t base = (uint32_t)wl.jb * kRec;
   const int nfull = (wl.lm >> 2) >> 1;  // as in for_each_neighbor_half
   auto each = [&](int o, const auto& a, auto) { body(o, a); };
   if (mode == kListDelta16) {
     const int ch = (cnt - h + 1) >> 1;
     const uint32_t sh = (uint32_t)h << 4;
-    list_loop<false, uint4>(
-        ch, nfull, [&](int c) { return L[(long long)c << 6]; },
+    if (ch > 0)
+      list_loop_from<false, uint4>(
+        ch, nfull, head.c0, head.c1, [&](int c) { return L[(long long)c << 6]; },
         [&](uint4 e, int c, auto full) {
           return decode_half<decltype(full)::value, kRec>(e, sh, base, c, ch, past);
         },

@@ -606,9 +606,11 @@ void launch_neighbors(const NbrView& nv, const NbrOut& out, unsigned long long* 
   }
 }
 
-// One block: sums and maxima over the per-wave statistics.
+// One block: sums and maxima over the per-wave statistics; then all counters
+// go to the host's copy (mapped memory: no copy command of its own).
 __global__ __launch_bounds__(1024) void k_wave_stats(const int4* __restrict__ ws, int nwaves,
-                                                     unsigned long long* __restrict__ counters) {
+                                                     unsigned long long* __restrict__ counters,
+                                                     unsigned long long* __restrict__ host) {
   __shared__ unsigned long long sp[16], sc[16];
   __shared__ int sn[16], ss[16];
   unsigned long long pairs = 0, cand = 0;
@@ -647,11 +649,15 @@ __global__ __launch_bounds__(1024) void k_wave_stats(const int4* __restrict__ ws
     counters[C_LIST_NEED] = (unsigned long long)need;
     counters[C_STAGED] = (unsigned long long)staged;
     counters[C_LIST_SLOTS] = 64ull * (unsigned long long)nwaves * (unsigned long long)need;
+#pragma unroll
+    for (int k = 0; k < C_COUNT; ++k) host[k] = counters[k];
+    __threadfence_system();
   }
 }
 
-void launch_wave_stats(const int4* wave_stat, int nwaves, unsigned long long* counters, hipStream_t st) {
-  if (nwaves > 0) k_wave_stats<<<1, 1024, 0, st>>>(wave_stat, nwaves, counters);
+void launch_wave_stats(const int4* wave_stat, int nwaves, unsigned long long* counters, unsigned long long* host,
+                       hipStream_t st) {
+  k_wave_stats<<<1, 1024, 0, st>>>(wave_stat, nwaves, counters, host);
 }
 
 // ---------------------------------------------------------------------------
@@ -933,12 +939,13 @@ __device__ __forceinline__ void displacement_finish(const NbrView& nv, int s, co
                                                     const float4* __restrict__ x0, const float4* __restrict__ vs,
                                                     const int* __restrict__ perm, float* __restrict__ x_out,
                                                     float* __restrict__ v_out, float4* __restrict__ v_sorted,
-                                                    int* __restrict__ id_out, float4 xi, const DispSums& a) {
+                                                    int* __restrict__ id_out, float4 xi, const DispSums& a,
+                                                    bool any_oog) {
   // nothing contracted, so every kernel that inlines this rounds it alike
 #pragma clang fp contract(off)
   float fa = 2.0f;
   DispSums b;  // pairs of out-of-grid particles that list s
-  if (nv.counters[C_OOG] != 0) {  // some scene has out-of-grid particles
+  if (any_oog) {  // some scene has out-of-grid particles
     const SceneWin win = nv.win[nv.ssid[s]];
     const int ob = win.cell_base + win.ncell;  // the scene's out-of-grid bucket
     const int o0 = nv.cell_start[ob], o1 = nv.cell_start[ob + 1];
@@ -1012,11 +1019,12 @@ __device__ __forceinline__ void displacement_at(const NbrView& nv, int s, const 
   if (s == 0 && (!last || v_sorted)) xd[nv.pad] = make_float4(kPadCoord, kPadCoord, kPadCoord, 0.0f);
   if (s >= nv.n) return;
   const float4 xi = xs[s];
+  const bool any_oog = nv.counters[C_OOG] != 0;  // read here: after the list it would wait on memory again
   // sum over the listed j of (lambda_i + lambda_j) t^2 / r (x_i - x_j)
   const DispSums a = disp_one_lane(xi, pc, [&](auto&& body, auto&& flip) {
     for_each_neighbor_staged<true>(nv, s, xs, stage, body, flip);
   });
-  displacement_finish(nv, s, xs, xd, pc, last, x0, vs, perm, x_out, v_out, v_sorted, id_out, xi, a);
+  displacement_finish(nv, s, xs, xd, pc, last, x0, vs, perm, x_out, v_out, v_sorted, id_out, xi, a, any_oog);
 }
 
 // Pass B with a lane pair per particle, as density_lambda_at2.
@@ -1029,12 +1037,13 @@ __device__ __forceinline__ void displacement_at2(const NbrView& nv, int s, int h
   if (s == 0 && h == 0 && (!last || v_sorted)) xd[nv.pad] = make_float4(kPadCoord, kPadCoord, kPadCoord, 0.0f);
   if (s >= nv.n) return;  // both lanes of the pair
   const float4 xi = xs[s];
+  const bool any_oog = nv.counters[C_OOG] != 0;
   DispSums a;
   if (for_each_neighbor_half<true>(nv, s, h, xs, stage, [&](float4 xj) { disp_term(a, xi, xj, pc); })) {
     const DispSums o = partner_sums(a);
     if (h == 0)
       displacement_finish(nv, s, xs, xd, pc, last, x0, vs, perm, x_out, v_out, v_sorted, id_out, xi,
-                          add_parities(a, o));
+                          add_parities(a, o), any_oog);
     return;
   }
   if (h != 0) return;
@@ -1043,7 +1052,7 @@ __device__ __forceinline__ void displacement_at2(const NbrView& nv, int s, int h
     for_each_neighbor_p<true, 16>(nv, s, wave_list(nv, __builtin_amdgcn_readfirstlane(s >> 6)),
                                   [&](int o) { return load_pos_bytes<true>(xs, (uint32_t)o); }, body, flip);
   });
-  displacement_finish(nv, s, xs, xd, pc, last, x0, vs, perm, x_out, v_out, v_sorted, id_out, xi, t);
+  displacement_finish(nv, s, xs, xd, pc, last, x0, vs, perm, x_out, v_out, v_sorted, id_out, xi, t, any_oog);
 }
 
 template <int B>

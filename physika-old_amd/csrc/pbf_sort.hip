@@ -111,13 +111,13 @@ __device__ __forceinline__ void dev_chunk(int n, int& lo, int& hi) {
   hi = min(n, lo + per * kScanPerBlock);
 }
 
-// Length min(*n_ptr, n_max); gate (may be null): the scan runs only when
+// Length min(*n_ptr, n_max), n_max without n_ptr; gate (may be null): the scan runs only when
 // *gate != 0.
 __global__ __launch_bounds__(1024) void k_scan_dev_reduce(const int* in, const int* n_ptr, int n_max, int* part,
                                                           const unsigned long long* gate) {
   __shared__ int wsum[16];
   if (gate && *gate == 0) return;
-  const int n = min(*n_ptr, n_max);
+  const int n = n_ptr ? min(*n_ptr, n_max) : n_max;
   int lo, hi;
   dev_chunk(n, lo, hi);
   int acc = 0;
@@ -139,7 +139,7 @@ __global__ __launch_bounds__(1024) void k_scan_dev_reduce(const int* in, const i
 __global__ __launch_bounds__(1024) void k_scan_dev_down(int* in, int* out, const int* n_ptr, int n_max,
                                                         const int* part, const unsigned long long* gate) {
   if (gate && *gate == 0) return;
-  const int n = min(*n_ptr, n_max);
+  const int n = n_ptr ? min(*n_ptr, n_max) : n_max;
   int lo, hi;
   dev_chunk(n, lo, hi);
   int before;
@@ -184,6 +184,10 @@ __global__ void k_scene_reset(int* minmax, int nscenes) {
 void launch_scene_reset(int* minmax, int nscenes, hipStream_t st) {
   if (nscenes > 0) k_scene_reset<<<(6 * nscenes + kBlock - 1) / kBlock, kBlock, 0, st>>>(minmax, nscenes);
 }
+
+// Particle range of scene s (off null: the one scene of a call, all n).
+__device__ __forceinline__ int scene_begin(const int* __restrict__ off, int s) { return off ? off[s] : 0; }
+__device__ __forceinline__ int scene_end(const int* __restrict__ off, int s, int n) { return off ? min(off[s + 1], n) : n; }
 
 __device__ __forceinline__ int scene_of(const int* __restrict__ off, int nscenes, int i) {
   int lo = 0, hi = nscenes;  // off[lo] <= i < off[hi]
@@ -489,7 +493,7 @@ __global__ __launch_bounds__(kBlock) void k_bin(SortIn in, int n, GridDev g,
   if (blockIdx.x == 0 && counters[C_OOG] != 0) {
     for (int s = threadIdx.x; s < nscenes; s += blockDim.x) {
       const SceneWin w = win[s];
-      cell_cnt[w.cell_base + w.ncell] = oog_pre[min(scene_off[s + 1], n)] - oog_pre[min(scene_off[s], n)];
+      cell_cnt[w.cell_base + w.ncell] = oog_pre[scene_end(scene_off, s, n)] - oog_pre[min(scene_begin(scene_off, s), n)];
     }
   }
   if (i >= n) return;
@@ -522,7 +526,7 @@ __global__ __launch_bounds__(kBlock) void k_bin(SortIn in, int n, GridDev g,
   } else if (inside) {
     sl = atomicAdd(&cell_cnt[k], 1);
   }
-  if (!inside) sl = oog_pre[kCellOrder ? in.id[i] : i] - oog_pre[min(scene_off[sid[i]], n)];
+  if (!inside) sl = oog_pre[kCellOrder ? in.id[i] : i] - oog_pre[min(scene_begin(scene_off, sid[i]), n)];
   slot[i] = sl;
 }
 
@@ -602,6 +606,215 @@ __global__ __launch_bounds__(kBlock) void k_reorder(const int* __restrict__ key,
   }
 }
 
+// ---------------------------------------------------------------------------
+// The whole sort of a one-scene search of at most kSortOneMax particles in one
+// workgroup: nine launches of 1.5 to 5 us each, most of it launch and memory
+// latency, become one (and one that returns at once unless the window is
+// large). The particles go to LDS buckets of consecutive cells, and a
+// particle's place is its bucket's start plus the number of its bucket's
+// particles before it by (cell, original index): the order of the sort above,
+// for cells and out-of-grid buckets of any size. The starts of the window's
+// cells are found in the sorted keys.
+constexpr int kSortOneMax = 4096, kSortOneBlock = 1024, kSortOnePer = kSortOneMax / kSortOneBlock;
+constexpr int kSortBuckets = 8192, kBucketsPer = kSortBuckets / kSortOneBlock;
+
+// First position of keys[0..n) whose key is at least c.
+__device__ __forceinline__ int lower_key(const int* keys, int n, int c) {
+  int lo = 0, hi = n;
+  while (lo < hi) {
+    const int mid = (lo + hi) >> 1;
+    if (keys[mid] < c)
+      lo = mid + 1;
+    else
+      hi = mid;
+  }
+  return lo;
+}
+
+template <bool kCellOrder>
+__global__ __launch_bounds__(kSortOneBlock) void k_sort_one(SortIn in, int n, GridDev g, SceneWin* __restrict__ win,
+                                                            int* __restrict__ total_cells,
+                                                            unsigned long long* __restrict__ counters,
+                                                            int* __restrict__ cell_start, int* __restrict__ keys,
+                                                            int* __restrict__ perm, int* __restrict__ ssid,
+                                                            float4* __restrict__ xn, float4* __restrict__ x0,
+                                                            float4* __restrict__ vs, PhysConst pc, int integrate,
+                                                            float* __restrict__ xc, int xc_stride,
+                                                            int* __restrict__ oog_rcnt) {
+#pragma clang fp contract(off)
+  __shared__ int start[kSortBuckets + 1];
+  __shared__ int skey[kSortOneMax], sid[kSortOneMax], src[kSortOneMax];
+  __shared__ int red[kSortOneBlock / 64][8];
+  __shared__ SceneWin sw;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  for (int b = tid; b <= kSortBuckets; b += kSortOneBlock) start[b] = 0;
+  // cells and their box
+  int c[kSortOnePer][3];
+  bool inside[kSortOnePer];
+  int lo[3] = {INT_MAX, INT_MAX, INT_MAX}, hi[3] = {INT_MIN, INT_MIN, INT_MIN};
+  int counts = 0;  // out-of-grid | non-finite << 16
+#pragma unroll
+  for (int q = 0; q < kSortOnePer; ++q) {
+    const int i = tid + q * kSortOneBlock;
+    bool nonfinite = false;
+    inside[q] = false;
+    if (i < n) {
+      inside[q] = grid_cell(g, in_pos<kCellOrder>(in, i), c[q][0], c[q][1], c[q][2], nonfinite);
+      counts += (inside[q] ? 0 : 1) + (nonfinite ? 1 << 16 : 0);
+    }
+    if (inside[q]) {
+#pragma unroll
+      for (int a = 0; a < 3; ++a) {
+        lo[a] = min(lo[a], c[q][a]);
+        hi[a] = max(hi[a], c[q][a]);
+      }
+    }
+  }
+#pragma unroll
+  for (int a = 0; a < 3; ++a) {
+    lo[a] = wave_min_full(lo[a]);
+    hi[a] = wave_max_full(hi[a]);
+  }
+  counts = wave_sum_full(counts);
+  if (lane == 0) {
+#pragma unroll
+    for (int a = 0; a < 3; ++a) {
+      red[wave][a] = lo[a];
+      red[wave][3 + a] = hi[a];
+    }
+    red[wave][6] = counts & 0xffff;
+    red[wave][7] = counts >> 16;
+  }
+  __syncthreads();
+  if (wave == 0) {
+    int r[8];
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+      const int id = k < 3 ? INT_MAX : (k < 6 ? INT_MIN : 0);
+      const int v = lane < kSortOneBlock / 64 ? red[lane][k] : id;
+      r[k] = k < 3 ? wave_min_full(v) : (k < 6 ? wave_max_full(v) : wave_sum_full(v));
+    }
+    if (lane == 0) {
+      SceneWin w{};
+      const bool any = r[3] >= r[0];
+#pragma unroll
+      for (int a = 0; a < 3; ++a) {
+        w.lo[a] = any ? r[a] : 0;
+        w.dim[a] = any ? r[3 + a] - r[a] + 1 : 0;
+      }
+      w.cell_base = 0;
+      w.ncell = w.dim[0] * w.dim[1] * w.dim[2];
+      sw = w;
+      win[0] = w;
+      *total_cells = w.ncell + 1;
+      counters[C_CELLS] = (unsigned long long)w.ncell + 1;
+      counters[C_OOG] = (unsigned long long)r[6];
+      counters[C_NONFINITE] = (unsigned long long)r[7];
+      counters[C_MASK_WORDS] = 0;
+      counters[C_FALLBACK] = 0;
+    }
+  }
+  __syncthreads();
+  const SceneWin w = sw;
+  // buckets of 2^shift consecutive cells (the out-of-grid bucket is cell ncell)
+  const int shift = max(0, 32 - __clz(w.ncell) - 13);
+  int key[kSortOnePer], slot[kSortOnePer];
+#pragma unroll
+  for (int q = 0; q < kSortOnePer; ++q) {
+    key[q] = inside[q] ? window_cell(w, c[q][0], c[q][1], c[q][2]) : w.ncell;
+    slot[q] = tid + q * kSortOneBlock < n ? atomicAdd(&start[key[q] >> shift], 1) : 0;
+  }
+  __syncthreads();
+  {  // exclusive scan of the bucket counts, kBucketsPer per thread
+    int v[kBucketsPer], sum = 0;
+#pragma unroll
+    for (int k = 0; k < kBucketsPer; ++k) {
+      v[k] = start[tid * kBucketsPer + k];
+      sum += v[k];
+    }
+    int total;
+    int e = block_scan4(sum, 0, 0, 0, total);
+#pragma unroll
+    for (int k = 0; k < kBucketsPer; ++k) {
+      start[tid * kBucketsPer + k] = e;
+      e += v[k];
+    }
+    if (tid == 0) start[kSortBuckets] = n;
+  }
+  __syncthreads();
+#pragma unroll
+  for (int q = 0; q < kSortOnePer; ++q) {
+    const int i = tid + q * kSortOneBlock;
+    if (i < n) {
+      const int p = start[key[q] >> shift] + slot[q];
+      skey[p] = key[q];
+      sid[p] = kCellOrder ? in.id[i] : i;
+      src[p] = i;
+    }
+  }
+  __syncthreads();
+  // the place of each entry, then its arrays
+#pragma unroll
+  for (int q = 0; q < kSortOnePer; ++q) {
+    const int t = tid + q * kSortOneBlock;
+    if (t >= n) continue;
+    const int k = skey[t], id = sid[t], b = k >> shift;
+    const int a = start[b], e = start[b + 1];
+    int rank = 0;
+    for (int u = a; u < e; ++u) {
+      const int ku = skey[u];
+      rank += ku < k || (ku == k && sid[u] < id);
+    }
+    const int s = a + rank;
+    const int i = src[t];
+    perm[s] = id;
+    ssid[s] = 0;
+    oog_rcnt[s] = 0;
+    keys[s] = k;
+    const float3 p = in_pos<kCellOrder>(in, i);
+    xn[s] = make_float4(p.x, p.y, p.z, 0.0f);
+    xc[s] = p.x;
+    xc[xc_stride + s] = p.y;
+    xc[2 * (size_t)xc_stride + s] = p.z;
+    if (integrate) {
+      const float3 v = in_vel<kCellOrder>(in, i);
+      const float vx = v.x + pc.gdt[0];
+      const float vy = v.y + pc.gdt[1];
+      const float vz = v.z + pc.gdt[2];
+      x0[s] = make_float4(p.x + vx * pc.dt, p.y + vy * pc.dt, p.z + vz * pc.dt, 0.0f);
+      vs[s] = make_float4(vx, vy, vz, 0.0f);
+    } else {
+      x0[s] = make_float4(p.x, p.y, p.z, 0.0f);
+    }
+  }
+  if (tid == 0) x0[n] = make_float4(kPadCoord, kPadCoord, kPadCoord, 0.0f);  // the padding particle
+  if (w.ncell >= kSortBuckets) return;  // k_cell_starts
+  // a bucket is one cell: its start is the cell's
+  for (int b = tid; b <= w.ncell + 1; b += kSortOneBlock) cell_start[b] = b <= w.ncell ? start[b] : n;
+}
+
+// Starts of the cells of a window too large for k_sort_one's buckets, from the
+// sorted keys.
+__global__ __launch_bounds__(kBlock) void k_cell_starts(const SceneWin* __restrict__ win, const int* __restrict__ keys,
+                                                        int n, int* __restrict__ cell_start) {
+  const int ncell = win[0].ncell;
+  if (ncell < kSortBuckets) return;
+  const int stride = gridDim.x * blockDim.x;
+  for (int c = blockIdx.x * blockDim.x + threadIdx.x; c <= ncell + 1; c += stride)
+    cell_start[c] = c <= ncell ? lower_key(keys, n, c) : n;
+}
+
+template <bool kCellOrder>
+void sort_one(const SortBufs& sb, const GridDev& g, const SortIn& in, int n, float4* xn, float4* x0, float4* vs,
+              const PhysConst* integrate, unsigned long long* counters, hipStream_t st) {
+  PhysConst pc{};
+  if (integrate) pc = *integrate;
+  k_sort_one<kCellOrder><<<1, kSortOneBlock, 0, st>>>(in, n, g, sb.win, sb.total_cells, counters, sb.cell_start,
+                                                      sb.key, sb.perm, sb.ssid, xn, x0, vs, pc, integrate ? 1 : 0,
+                                                      sb.xc, sb.xc_stride, sb.oog_rcnt);
+  k_cell_starts<<<128, kBlock, 0, st>>>(sb.win, sb.key, n, sb.cell_start);
+}
+
 template <bool kCellOrder>
 void sort_in(const SortBufs& sb, const GridDev& g, const SortIn& in, int n, float4* xn, float4* x0, float4* vs,
              const PhysConst* integrate, unsigned long long* counters, hipStream_t st) {
@@ -616,7 +829,7 @@ void sort_in(const SortBufs& sb, const GridDev& g, const SortIn& in, int n, floa
   // out-of-grid ranks by original index (only when the bounds pass found any;
   // the last scene offset is n)
   const unsigned long long* any_oog = counters + C_OOG;
-  const int* n_dev = sb.scene_off + sb.nscenes;
+  const int* n_dev = sb.scene_off ? sb.scene_off + sb.nscenes : nullptr;
   k_scan_dev_reduce<<<kScanDevBlocks, 1024, 0, st>>>(sb.oog_flag, n_dev, n, sb.scan_part, any_oog);
   k_scan_dev_down<<<kScanDevBlocks, 1024, 0, st>>>(sb.oog_flag, sb.oog_pre, n_dev, n, sb.scan_part, any_oog);
   k_bin<kCellOrder><<<nb, kBlock, 0, st>>>(in, n, g, sb.sid, sb.win, sb.key, sb.slot, sb.cell_cnt, sb.scene_off,
@@ -634,7 +847,12 @@ void sort_in(const SortBufs& sb, const GridDev& g, const SortIn& in, int n, floa
 
 void launch_sort(const SortBufs& sb, const GridDev& g, const SortIn& in, int n, float4* xn, float4* x0, float4* vs,
                  const PhysConst* integrate, unsigned long long* counters, hipStream_t st) {
-  if (in.x4)
+  if (sb.nscenes == 1 && n <= kSortOneMax) {
+    if (in.x4)
+      sort_one<true>(sb, g, in, n, xn, x0, vs, integrate, counters, st);
+    else
+      sort_one<false>(sb, g, in, n, xn, x0, vs, integrate, counters, st);
+  } else if (in.x4)
     sort_in<true>(sb, g, in, n, xn, x0, vs, integrate, counters, st);
   else
     sort_in<false>(sb, g, in, n, xn, x0, vs, integrate, counters, st);
