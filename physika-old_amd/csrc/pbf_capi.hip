@@ -36,10 +36,11 @@ struct pbf_ctx {
 
   // scenes
   int scene_cap = 0;
-  int* scene_minmax = nullptr;  // 6 per scene
+  int* scene_minmax = nullptr;  // kBoxInts per scene
   SceneWin* win = nullptr;
   int* total_cells = nullptr;
-  int* scan_part = nullptr;     // kScanDevBlocks + 1
+  int* scan_part = nullptr;     // 2 kScanDevBlocks
+  int* ticket = nullptr;        // of the bounds pass, zero between launches
 
   // compact cell arrays
   long long cell_cap = 0;
@@ -451,7 +452,7 @@ int ensure_scenes(pbf_ctx* c, int nscenes) {
     dfree(c->scene_minmax);
     dfree(c->win);
     c->scene_cap = 0;
-    PBF_HIP(c, hipMalloc(&c->scene_minmax, sizeof(int) * 6 * (size_t)nscenes));
+    PBF_HIP(c, hipMalloc(&c->scene_minmax, sizeof(int) * kBoxInts * (size_t)nscenes));
     PBF_HIP(c, hipMalloc(&c->win, sizeof(SceneWin) * (size_t)nscenes));
     launch_scene_reset(c->scene_minmax, nscenes, nullptr);  // the sort keeps them empty between calls
     PBF_HIP(c, hipGetLastError());
@@ -680,6 +681,7 @@ SortBufs sort_of(pbf_ctx* c, const int* scene_off, int nscenes) {
   sb.tmp = c->tmp;
   sb.perm = c->perm;
   sb.scan_part = c->scan_part;
+  sb.ticket = c->ticket;
   sb.bpart = c->bpart;
   sb.xc = c->xc;
   sb.oog_rcnt = c->oog_rcnt;
@@ -1298,7 +1300,8 @@ int pbf_create(const pbf_params* p, pbf_ctx** out) {
       hipEventCreateWithFlags(&c->counters_ev, hipEventDisableTiming) != hipSuccess ||
       hipStreamCreateWithFlags(&c->cap_stream, hipStreamNonBlocking) != hipSuccess ||
       hipMalloc(&c->total_cells, sizeof(int)) != hipSuccess ||
-      hipMalloc(&c->scan_part, sizeof(int) * (kScanDevBlocks + 1)) != hipSuccess ||
+      hipMalloc(&c->scan_part, sizeof(int) * 2 * kScanDevBlocks) != hipSuccess ||
+      hipMalloc(&c->ticket, sizeof(int)) != hipSuccess || hipMemset(c->ticket, 0, sizeof(int)) != hipSuccess ||
       hipMalloc(&c->pairing, sizeof(unsigned long long) * kPairingSlots) != hipSuccess) {
     pbf_destroy(c);
     return PBF_ERR_HIP;
@@ -1323,7 +1326,7 @@ int pbf_destroy(pbf_ctx* c) {
   if (!c) return PBF_ERR_INVALID;
   (void)hipDeviceSynchronize();
   dfree(c->scene_minmax); dfree(c->win); dfree(c->total_cells); dfree(c->scan_part);
-  dfree(c->pairing);
+  dfree(c->pairing); dfree(c->ticket);
   dfree(c->cell_cnt); dfree(c->cell_start);
   dfree(c->key); dfree(c->slot); dfree(c->tmp); dfree(c->perm); dfree(c->inv);
   dfree(c->sid); dfree(c->ssid); dfree(c->bpart); dfree(c->nbr_cnt); dfree(c->cnt_orig);

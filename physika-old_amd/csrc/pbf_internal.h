@@ -185,7 +185,7 @@ struct SortBufs {
   int nscenes;
   int* sid;               // scene of each input particle (in the input's order)
   int* ssid;              // scene of each sorted particle
-  int* scene_minmax;      // 6 per scene: min i,j,k then max i,j,k of in-grid cells
+  int* scene_minmax;      // kBoxInts per scene: min i,j,k then max i,j,k of in-grid cells, out-of-grid particles
   SceneWin* win;          // per scene
   int* total_cells;       // device scalar: sum over scenes of ncell + 1
   long long cell_cap;     // allocated compact cells
@@ -195,7 +195,8 @@ struct SortBufs {
   int* slot;              // its arrival slot in the cell
   int* tmp;               // input indices scattered into cell order
   int* perm;              // original index of each sorted particle
-  int* scan_part;         // partial sums of the device-length scan
+  int* scan_part;         // partial sums of the two device-length scans
+  int* ticket;            // zero between launches
   int* bpart;             // per block of the bounds pass: scene and cell box (bounds_part_ints)
   float* xc;              // sorted x^n as three planes (x, y, z), plane stride xc_stride
   int xc_stride;
@@ -229,6 +230,7 @@ constexpr int kXnPad = 64;
 constexpr int kListPad = 2 * 64 * 8;
 // Blocks of the device-length scan.
 constexpr int kScanDevBlocks = 128;
+constexpr int kBoxInts = 7;
 
 size_t scan_scratch_ints(long long n);
 size_t bounds_part_ints(long long n);

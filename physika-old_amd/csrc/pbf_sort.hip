@@ -111,13 +111,25 @@ __device__ __forceinline__ void dev_chunk(int n, int& lo, int& hi) {
   hi = min(n, lo + per * kScanPerBlock);
 }
 
-// Length min(*n_ptr, n_max), n_max without n_ptr; gate (may be null): the scan runs only when
-// *gate != 0.
-__global__ __launch_bounds__(1024) void k_scan_dev_reduce(const int* in, const int* n_ptr, int n_max, int* part,
-                                                          const unsigned long long* gate) {
+// One scan of a launch: length min(*n_ptr, n_max), n_max without n_ptr; gate
+// (may be null): the scan runs only when *gate != 0. Row y of the grid runs
+// scan y.
+struct ScanJob {
+  int* in;
+  int* out;
+  const int* n_ptr;
+  int n_max;
+  int* part;
+  const unsigned long long* gate;
+};
+
+__global__ __launch_bounds__(1024) void k_scan_dev_reduce(ScanJob j0, ScanJob j1) {
   __shared__ int wsum[16];
-  if (gate && *gate == 0) return;
-  const int n = n_ptr ? min(*n_ptr, n_max) : n_max;
+  const ScanJob& job = blockIdx.y == 0 ? j0 : j1;
+  if (job.gate && *job.gate == 0) return;
+  const int* in = job.in;
+  int* part = job.part;
+  const int n = job.n_ptr ? min(*job.n_ptr, job.n_max) : job.n_max;
   int lo, hi;
   dev_chunk(n, lo, hi);
   int acc = 0;
@@ -136,10 +148,13 @@ __global__ __launch_bounds__(1024) void k_scan_dev_reduce(const int* in, const i
 // and the last block writes the grand total. The counts are zeroed once read,
 // so the next sort starts from zero counts without a clearing pass (the array
 // is zeroed when allocated).
-__global__ __launch_bounds__(1024) void k_scan_dev_down(int* in, int* out, const int* n_ptr, int n_max,
-                                                        const int* part, const unsigned long long* gate) {
-  if (gate && *gate == 0) return;
-  const int n = n_ptr ? min(*n_ptr, n_max) : n_max;
+__global__ __launch_bounds__(1024) void k_scan_dev_down(ScanJob j0, ScanJob j1) {
+  const ScanJob& job = blockIdx.y == 0 ? j0 : j1;
+  if (job.gate && *job.gate == 0) return;
+  int* in = job.in;
+  int* out = job.out;
+  const int* part = job.part;
+  const int n = job.n_ptr ? min(*job.n_ptr, job.n_max) : job.n_max;
   int lo, hi;
   dev_chunk(n, lo, hi);
   int before;
@@ -174,20 +189,20 @@ __global__ __launch_bounds__(1024) void k_scan_dev_down(int* in, int* out, const
 // ---------------------------------------------------------------------------
 // Scene windows
 
-// Empty boxes (min INT_MAX, max INT_MIN). Run once when the boxes are
-// allocated; k_scene_windows empties each box again once it has read it.
+// A scene's box: min i j k, max i j k of its in-grid particles' cells, its
+// out-of-grid particles (kBoxInts ints per scene). Empty boxes hold INT_MAX,
+// INT_MIN and 0: set once when the boxes are allocated; the windows empty each
+// box again once it is read.
+__host__ __device__ constexpr int empty_box(int a) { return a < 3 ? INT_MAX : (a < 6 ? INT_MIN : 0); }
+
 __global__ void k_scene_reset(int* minmax, int nscenes) {
   const int t = blockIdx.x * blockDim.x + threadIdx.x;
-  if (t < 6 * nscenes) minmax[t] = (t % 6) < 3 ? INT_MAX : INT_MIN;
+  if (t < kBoxInts * nscenes) minmax[t] = empty_box(t % kBoxInts);
 }
 
 void launch_scene_reset(int* minmax, int nscenes, hipStream_t st) {
-  if (nscenes > 0) k_scene_reset<<<(6 * nscenes + kBlock - 1) / kBlock, kBlock, 0, st>>>(minmax, nscenes);
+  if (nscenes > 0) k_scene_reset<<<(kBoxInts * nscenes + kBlock - 1) / kBlock, kBlock, 0, st>>>(minmax, nscenes);
 }
-
-// Particle range of scene s (off null: the one scene of a call, all n).
-__device__ __forceinline__ int scene_begin(const int* __restrict__ off, int s) { return off ? off[s] : 0; }
-__device__ __forceinline__ int scene_end(const int* __restrict__ off, int s, int n) { return off ? min(off[s + 1], n) : n; }
 
 __device__ __forceinline__ int scene_of(const int* __restrict__ off, int nscenes, int i) {
   int lo = 0, hi = nscenes;  // off[lo] <= i < off[hi]
@@ -225,6 +240,171 @@ __device__ __forceinline__ bool grid_cell(const GridDev& g, float3 p, int& ci, i
   return !nonfinite && in_grid(g, ci, cj, ck);
 }
 
+// The scene of particle i by one wave, 64 offsets at a time (every lane active).
+__device__ __forceinline__ int scene_of_wave(const int* __restrict__ off, int nscenes, int i) {
+  int lo = 0, hi = nscenes;  // off[lo] <= i < off[hi]
+  while (hi - lo > 1) {
+    const int step = (hi - lo + 63) >> 6;
+    const int at = lo + (int)(threadIdx.x & 63) * step;
+    const bool below = at < hi && (at == lo || off[at] <= i);
+    const int last = 63 - __clzll(__ballot(below));  // the offsets never decrease
+    lo += last * step;
+    hi = min(hi, lo + step);
+  }
+  return lo;
+}
+
+// A word that another workgroup of the same kernel reads after the ticket below
+// (written through to memory, read past the caches that other XCDs' writes do
+// not reach).
+__device__ __forceinline__ void share_store(int* p, int v) {
+  __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ int share_load(const int* p) {
+  return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// What the bounds pass leaves for the windows.
+struct WindowOut {
+  int* minmax;  // the scenes' boxes
+  int nscenes;
+  SceneWin* win;
+  int* total_cells;
+  const int* bpart;
+  int nbounds;
+  unsigned long long* counters;
+  int* cell_cnt;
+};
+
+// Windows and compact cell bases of all scenes, by one workgroup of kWaves
+// waves; each scene's box is emptied again for the next sort, and each
+// out-of-grid bucket gets its count. With one scene the workgroup also reduces
+// the bounds blocks' boxes (read as bload reads them). It also sets the search's
+// counters: the out-of-grid and non-finite totals of the bounds pass, the cell
+// total, and zero for the counters the neighbor pass accumulates.
+template <int kWaves, class BLoad>
+__device__ __forceinline__ void scene_windows(const WindowOut& o, BLoad&& bload) {
+  __shared__ int box[kWaves][8];
+  __shared__ int wsum[kWaves], base;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const bool one = o.nscenes == 1;
+  int r[6] = {INT_MAX, INT_MAX, INT_MAX, INT_MIN, INT_MIN, INT_MIN};
+  int oog = 0, nonfinite = 0;
+#pragma unroll 4
+  for (int b = tid; b < o.nbounds; b += 64 * kWaves) {
+    const int* e = o.bpart + 8 * (size_t)b;
+    const unsigned v = (unsigned)bload(e + 7);
+    oog += v & 0xffffu;
+    nonfinite += v >> 16;
+    if (one) {
+#pragma unroll
+      for (int a = 0; a < 3; ++a) {
+        r[a] = min(r[a], bload(e + 1 + a));
+        r[3 + a] = max(r[3 + a], bload(e + 4 + a));
+      }
+    }
+  }
+  // every lane of the workgroup is active
+#pragma unroll
+  for (int a = 0; a < 3; ++a) {
+    r[a] = wave_min_full(r[a]);
+    r[3 + a] = wave_max_full(r[3 + a]);
+  }
+  oog = wave_sum_full(oog);
+  nonfinite = wave_sum_full(nonfinite);
+  if (lane == 0) {
+#pragma unroll
+    for (int a = 0; a < 6; ++a) box[wave][a] = r[a];
+    box[wave][6] = oog;
+    box[wave][7] = nonfinite;
+  }
+  if (tid == 0) base = 0;
+  __syncthreads();
+#pragma unroll
+  for (int w = 0; w < kWaves; ++w) {
+    if (w == 0) oog = nonfinite = 0;
+#pragma unroll
+    for (int a = 0; a < 3; ++a) {
+      r[a] = min(r[a], box[w][a]);
+      r[3 + a] = max(r[3 + a], box[w][3 + a]);
+    }
+    oog += box[w][6];
+    nonfinite += box[w][7];
+  }
+  for (int s0 = 0; s0 < o.nscenes; s0 += 64 * kWaves) {
+    const int s = s0 + tid;
+    SceneWin w{};
+    int cells = 0, out = 0;
+    if (s < o.nscenes) {
+      int m[7];
+      if (one) {
+#pragma unroll
+        for (int a = 0; a < 6; ++a) m[a] = r[a];
+        m[6] = oog;
+      } else {
+        int* p = o.minmax + kBoxInts * (size_t)s;
+#pragma unroll
+        for (int a = 0; a < 7; ++a) {
+          m[a] = bload(p + a);
+          p[a] = empty_box(a);
+        }
+      }
+      if (m[3] >= m[0]) {
+#pragma unroll
+        for (int a = 0; a < 3; ++a) {
+          w.lo[a] = m[a];
+          w.dim[a] = m[a + 3] - m[a] + 1;
+        }
+      }
+      w.ncell = w.dim[0] * w.dim[1] * w.dim[2];
+      cells = w.ncell + 1;  // + out-of-grid bucket
+      out = m[6];
+    }
+    const int incl = wave_inclusive_scan(cells);
+    if (lane == 63) wsum[wave] = incl;
+    __syncthreads();
+    int before = base, all = 0;
+#pragma unroll
+    for (int k = 0; k < kWaves; ++k) {
+      before += k < wave ? wsum[k] : 0;
+      all += wsum[k];
+    }
+    if (s < o.nscenes) {
+      w.cell_base = before + incl - cells;
+      o.win[s] = w;
+      if (out > 0) o.cell_cnt[w.cell_base + w.ncell] = out;
+    }
+    __syncthreads();
+    if (tid == 0) base += all;
+    __syncthreads();
+  }
+  if (tid == 0) {
+    *o.total_cells = base;
+    o.counters[C_CELLS] = (unsigned long long)base;
+    o.counters[C_OOG] = (unsigned long long)oog;
+    o.counters[C_NONFINITE] = (unsigned long long)nonfinite;
+    o.counters[C_MASK_WORDS] = 0;
+    o.counters[C_FALLBACK] = 0;
+  }
+}
+
+// Whether this workgroup is the last of the launch to get here (each of them
+// calls this once, with all its threads): the words that every workgroup's
+// thread 0 wrote before with share_store are then there for share_load.
+__device__ __forceinline__ bool last_block(int* ticket) {
+  __shared__ int mine;
+  if (threadIdx.x == 0) {
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_waitcnt(0);  // the stores have reached memory
+    asm volatile("" ::: "memory");
+    mine = __hip_atomic_fetch_add(ticket, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  }
+  __syncthreads();
+  const bool last = mine == (int)gridDim.x - 1;
+  if (last && threadIdx.x == 0) *ticket = 0;  // for the next launch
+  return last;
+}
+
 // Scene of every particle and the cell bounding box of each scene's in-grid
 // particles. Each block covers kBoundsSpan particles (kBoundsPer per thread,
 // coalesced). A block whose particles all belong to one scene writes its
@@ -233,19 +413,38 @@ __device__ __forceinline__ bool grid_cell(const GridDev& g, float3 p, int& ci, i
 // scenes mark bpart -1 and update the scenes' boxes with atomics (per wave,
 // per lane where a wave straddles). Same-address atomics from every block
 // would serialize in L2, so the single-scene blocks are reduced per scene by
-// k_scene_reduce (by k_scene_windows for one scene).
+// k_scene_reduce (for one scene by scene_windows: with kWindows the last block
+// to end makes the window, otherwise k_scene_windows).
+//
+// A particle's scene: the block's first and last particle are looked up once
+// each, 64 offsets at a time; threads search between the two only where they
+// differ. A binary search per particle, six dependent loads deep, took 22 us for
+// 40,009 particles in 8 scenes and 40 us for 1.3M in 64.
 constexpr int kBoundsBlock = 256, kBoundsPer = 4, kBoundsSpan = kBoundsBlock * kBoundsPer;
 
 size_t bounds_part_ints(long long n) { return 8 * (size_t)((n + kBoundsSpan - 1) / kBoundsSpan + 1); }
 
-template <bool kCellOrder>
+template <bool kCellOrder, bool kWindows>
 __global__ __launch_bounds__(kBoundsBlock) void k_scene_bounds(SortIn in, int n, GridDev g,
                                                                const int* __restrict__ off, int nscenes,
                                                                int* __restrict__ sid, int* __restrict__ minmax,
-                                                               int* __restrict__ bpart, int* __restrict__ oog_flag) {
+                                                               int* __restrict__ bpart, int* __restrict__ oog_flag,
+                                                               WindowOut windows, int* __restrict__ ticket) {
   __shared__ int red[kBoundsBlock / 64][7];
+  __shared__ int ends[2];
   const int base = blockIdx.x * kBoundsSpan;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  int s_first = 0, s_last = 0;
+  if (nscenes > 1) {
+    if (wave < 2) {
+      const int s = scene_of_wave(off, nscenes, wave == 0 ? base : min(n, base + kBoundsSpan) - 1);
+      if (lane == 0) ends[wave] = s;
+    }
+    __syncthreads();
+    s_first = ends[0];
+    s_last = ends[1];
+  }
+  const bool one_scene = s_first == s_last;  // block-uniform
   int sq[kBoundsPer], cq[kBoundsPer][3];
   bool inq[kBoundsPer];
   int lo[3] = {INT_MAX, INT_MAX, INT_MAX}, hi[3] = {INT_MIN, INT_MIN, INT_MIN};
@@ -256,7 +455,7 @@ __global__ __launch_bounds__(kBoundsBlock) void k_scene_bounds(SortIn in, int n,
     int sc = -1, c[3] = {0, 0, 0};
     bool nonfinite = false, inside = false;
     if (i < n) {
-      sc = scene_of(off, nscenes, i);
+      sc = one_scene ? s_first : s_first + scene_of(off + s_first, s_last - s_first + 1, i);
       sid[i] = sc;
       inside = grid_cell(g, in_pos<kCellOrder>(in, i), c[0], c[1], c[2], nonfinite);
       counts += (inside ? 0 : 1) + (nonfinite ? 1 << 16 : 0);
@@ -286,9 +485,6 @@ __global__ __launch_bounds__(kBoundsBlock) void k_scene_bounds(SortIn in, int n,
     red[wave][6] = counts;
   }
   __syncthreads();
-  // one scene when the block's first and last particles share it (uniform)
-  const int last = min(n, base + kBoundsSpan) - 1;
-  const bool one_scene = scene_of(off, nscenes, base) == scene_of(off, nscenes, last);
   if (threadIdx.x == 0) {
     int r[6] = {INT_MAX, INT_MAX, INT_MAX, INT_MIN, INT_MIN, INT_MIN};
     int tot = 0;
@@ -298,13 +494,63 @@ __global__ __launch_bounds__(kBoundsBlock) void k_scene_bounds(SortIn in, int n,
       tot += red[w][6];
     }
     int* bp = bpart + 8 * (size_t)blockIdx.x;
-    bp[0] = one_scene ? scene_of(off, nscenes, base) : -1;
-    for (int a = 0; a < 6; ++a) bp[1 + a] = r[a];
-    bp[7] = tot;
+    if (kWindows) {
+      for (int a = 0; a < 6; ++a) share_store(bp + 1 + a, r[a]);
+      share_store(bp + 7, tot);
+    } else {
+      bp[0] = one_scene ? s_first : -1;
+      for (int a = 0; a < 6; ++a) bp[1 + a] = r[a];
+      bp[7] = tot;
+    }
+  }
+  if (kWindows) {
+    if (last_block(ticket)) scene_windows<kBoundsBlock / 64>(windows, [](const int* p) { return share_load(p); });
+    return;
   }
   if (one_scene) return;  // block-uniform
-  // a block that straddles scenes: per particle slot q, per wave where the
-  // wave's particles share a scene, else per lane
+  // a block that straddles scenes: a few scenes one after the other, one set of
+  // atomics each (an atomic per wave and slot took 20 us where the scenes'
+  // boundaries meet); many scenes per particle slot q, per wave where the wave's
+  // particles share a scene, else per lane
+  if (s_last - s_first < 8) {
+    for (int s = s_first; s <= s_last; ++s) {
+      int m[7] = {INT_MAX, INT_MAX, INT_MAX, INT_MIN, INT_MIN, INT_MIN, 0};
+#pragma unroll
+      for (int q = 0; q < kBoundsPer; ++q) {
+        if (sq[q] != s) continue;
+#pragma unroll
+        for (int a = 0; a < 3; ++a) {
+          m[a] = min(m[a], inq[q] ? cq[q][a] : INT_MAX);
+          m[3 + a] = max(m[3 + a], inq[q] ? cq[q][a] : INT_MIN);
+        }
+        m[6] += inq[q] ? 0 : 1;
+      }
+#pragma unroll
+      for (int a = 0; a < 7; ++a) m[a] = a < 3 ? wave_min_full(m[a]) : (a < 6 ? wave_max_full(m[a]) : wave_sum_full(m[a]));
+      __syncthreads();  // red is free
+      if (lane == 0) {
+#pragma unroll
+        for (int a = 0; a < 7; ++a) red[wave][a] = m[a];
+      }
+      __syncthreads();
+      if (threadIdx.x < 7) {
+        const int a = threadIdx.x;
+        int v = red[0][a];
+        for (int w = 1; w < kBoundsBlock / 64; ++w)
+          v = a < 3 ? min(v, red[w][a]) : (a < 6 ? max(v, red[w][a]) : v + red[w][a]);
+        int* box = minmax + kBoxInts * (size_t)s + a;
+        if (v != empty_box(a)) {
+          if (a < 3)
+            atomicMin(box, v);
+          else if (a < 6)
+            atomicMax(box, v);
+          else
+            atomicAdd(box, v);
+        }
+      }
+    }
+    return;
+  }
 #pragma unroll
   for (int q = 0; q < kBoundsPer; ++q) {
     const int i = base + q * kBoundsBlock + (int)threadIdx.x;
@@ -316,15 +562,23 @@ __global__ __launch_bounds__(kBoundsBlock) void k_scene_bounds(SortIn in, int n,
         m[a] = wave_min_full(inq[q] ? cq[q][a] : INT_MAX);
         m[3 + a] = wave_max_full(inq[q] ? cq[q][a] : INT_MIN);
       }
-      if (lane == 0 && s0 >= 0 && m[3] >= m[0]) {
-        int* box = minmax + 6 * s0;
-        for (int a = 0; a < 3; ++a) atomicMin(box + a, m[a]);
-        for (int a = 3; a < 6; ++a) atomicMax(box + a, m[a]);
+      const int out = __popcll(__ballot(valid && !inq[q]));
+      if (lane == 0 && s0 >= 0) {
+        int* box = minmax + kBoxInts * (size_t)s0;
+        if (m[3] >= m[0]) {
+          for (int a = 0; a < 3; ++a) atomicMin(box + a, m[a]);
+          for (int a = 3; a < 6; ++a) atomicMax(box + a, m[a]);
+        }
+        if (out) atomicAdd(box + 6, out);
       }
-    } else if (inq[q]) {
-      int* box = minmax + 6 * sq[q];
-      for (int a = 0; a < 3; ++a) atomicMin(box + a, cq[q][a]);
-      for (int a = 0; a < 3; ++a) atomicMax(box + 3 + a, cq[q][a]);
+    } else if (valid) {
+      int* box = minmax + kBoxInts * (size_t)sq[q];
+      if (inq[q]) {
+        for (int a = 0; a < 3; ++a) atomicMin(box + a, cq[q][a]);
+        for (int a = 0; a < 3; ++a) atomicMax(box + 3 + a, cq[q][a]);
+      } else {
+        atomicAdd(box + 6, 1);
+      }
     }
   }
 }
@@ -334,7 +588,7 @@ __global__ __launch_bounds__(kBoundsBlock) void k_scene_bounds(SortIn in, int n,
 // read as two 16-byte loads, four entries per thread in flight.
 constexpr int kReduceBlock = 1024;
 
-__device__ __forceinline__ void merge_box(int r[6], const int* __restrict__ bpart, int b, int s) {
+__device__ __forceinline__ void merge_box(int r[7], const int* __restrict__ bpart, int b, int s) {
   const int4 u = reinterpret_cast<const int4*>(bpart)[2 * (size_t)b];
   const int4 w = reinterpret_cast<const int4*>(bpart)[2 * (size_t)b + 1];
   if (u.x != s) return;
@@ -344,16 +598,17 @@ __device__ __forceinline__ void merge_box(int r[6], const int* __restrict__ bpar
   r[3] = max(r[3], w.x);
   r[4] = max(r[4], w.y);
   r[5] = max(r[5], w.z);
+  r[6] += w.w & 0xffff;
 }
 
 __global__ __launch_bounds__(kReduceBlock) void k_scene_reduce(const int* __restrict__ off, int nscenes,
                                                                const int* __restrict__ bpart,
                                                                int* __restrict__ minmax) {
-  __shared__ int red[kReduceBlock / 64][6];
+  __shared__ int red[kReduceBlock / 64][7];
   const int s = blockIdx.x;
   const int b0 = off[s] / kBoundsSpan;
   const int b1 = off[s + 1] > off[s] ? (off[s + 1] - 1) / kBoundsSpan + 1 : b0;
-  int r[6] = {INT_MAX, INT_MAX, INT_MAX, INT_MIN, INT_MIN, INT_MIN};
+  int r[7] = {INT_MAX, INT_MAX, INT_MAX, INT_MIN, INT_MIN, INT_MIN, 0};
   int b = b0 + (int)threadIdx.x;
   for (; b + 3 * kReduceBlock < b1; b += 4 * kReduceBlock) {
 #pragma unroll
@@ -363,139 +618,38 @@ __global__ __launch_bounds__(kReduceBlock) void k_scene_reduce(const int* __rest
   // every lane of the block is active
   for (int a = 0; a < 3; ++a) r[a] = wave_min_full(r[a]);
   for (int a = 3; a < 6; ++a) r[a] = wave_max_full(r[a]);
+  r[6] = wave_sum_full(r[6]);
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   if (lane == 0)
-    for (int a = 0; a < 6; ++a) red[wave][a] = r[a];
+    for (int a = 0; a < 7; ++a) red[wave][a] = r[a];
   __syncthreads();
   if (threadIdx.x == 0) {
     for (int w = 1; w < kReduceBlock / 64; ++w) {
       for (int a = 0; a < 3; ++a) r[a] = min(r[a], red[w][a]);
       for (int a = 3; a < 6; ++a) r[a] = max(r[a], red[w][a]);
+      r[6] += red[w][6];
     }
-    if (r[3] >= r[0]) {
-      int* m = minmax + 6 * s;
-      atomicMin(m + 0, r[0]);
-      atomicMin(m + 1, r[1]);
-      atomicMin(m + 2, r[2]);
-      atomicMax(m + 3, r[3]);
-      atomicMax(m + 4, r[4]);
-      atomicMax(m + 5, r[5]);
-    }
+    // the only block that writes this scene's box now
+    int* m = minmax + kBoxInts * (size_t)s;
+    for (int a = 0; a < 3; ++a) m[a] = min(m[a], r[a]);
+    for (int a = 3; a < 6; ++a) m[a] = max(m[a], r[a]);
+    m[6] += r[6];
   }
 }
 
-// Windows and compact cell bases of all scenes (one block); each scene's box
-// is emptied again for the next sort. With one scene the block also reduces
-// the bounds blocks' boxes (k_scene_reduce is not launched). The block also
-// sets the search's counters: the out-of-grid and non-finite totals of the
-// bounds pass, the cell total, and zero for the counters the neighbor pass
-// accumulates.
-__global__ __launch_bounds__(1024) void k_scene_windows(int* __restrict__ minmax, int nscenes,
-                                                        SceneWin* __restrict__ win, int* __restrict__ total_cells,
-                                                        const int* __restrict__ bpart, int nbounds,
-                                                        unsigned long long* __restrict__ counters) {
-  __shared__ unsigned long long red[2][16];
-  __shared__ int box[16][6];
-  unsigned long long oog = 0, nonfinite = 0;
-  const bool one = nscenes == 1;
-  int r[6] = {INT_MAX, INT_MAX, INT_MAX, INT_MIN, INT_MIN, INT_MIN};
-#pragma unroll 4
-  for (int b = threadIdx.x; b < nbounds; b += blockDim.x) {
-    const unsigned v = (unsigned)bpart[8 * (size_t)b + 7];
-    oog += v & 0xffffu;
-    nonfinite += v >> 16;
-    if (one) merge_box(r, bpart, b, 0);
-  }
-  if (one) {  // every lane of the block is active
-    for (int a = 0; a < 3; ++a) r[a] = wave_min_full(r[a]);
-    for (int a = 3; a < 6; ++a) r[a] = wave_max_full(r[a]);
-    if ((threadIdx.x & 63) == 0)
-      for (int a = 0; a < 6; ++a) box[threadIdx.x >> 6][a] = r[a];
-    __syncthreads();
-    if (threadIdx.x == 0) {
-      for (int w = 1; w < (int)(blockDim.x >> 6); ++w) {
-        for (int a = 0; a < 3; ++a) r[a] = min(r[a], box[w][a]);
-        for (int a = 3; a < 6; ++a) r[a] = max(r[a], box[w][a]);
-      }
-      for (int a = 0; a < 3; ++a) minmax[a] = min(minmax[a], r[a]);
-      for (int a = 3; a < 6; ++a) minmax[a] = max(minmax[a], r[a]);
-    }
-  }
-#pragma unroll
-  for (int d = 32; d > 0; d >>= 1) {
-    oog += __shfl_xor(oog, d);
-    nonfinite += __shfl_xor(nonfinite, d);
-  }
-  if ((threadIdx.x & 63) == 0) {
-    red[0][threadIdx.x >> 6] = oog;
-    red[1][threadIdx.x >> 6] = nonfinite;
-  }
-  int running = 0;
-  for (int s0 = 0; s0 < nscenes; s0 += 1024) {
-    const int s = s0 + threadIdx.x;
-    SceneWin w{};
-    int cells = 0;
-    if (s < nscenes) {
-      int* m = minmax + 6 * s;
-      if (m[3] >= m[0]) {
-        for (int a = 0; a < 3; ++a) {
-          w.lo[a] = m[a];
-          w.dim[a] = m[a + 3] - m[a] + 1;
-        }
-        w.ncell = w.dim[0] * w.dim[1] * w.dim[2];
-      } else {
-        for (int a = 0; a < 3; ++a) {
-          w.lo[a] = 0;
-          w.dim[a] = 0;
-        }
-        w.ncell = 0;
-      }
-      cells = w.ncell + 1;  // + out-of-grid bucket
-      for (int a = 0; a < 6; ++a) m[a] = a < 3 ? INT_MAX : INT_MIN;
-    }
-    int total;
-    const int e = block_scan4(cells, 0, 0, 0, total);
-    if (s < nscenes) {
-      w.cell_base = running + e;
-      win[s] = w;
-    }
-    running += total;
-  }
-  if (threadIdx.x == 0) {
-    *total_cells = running;
-    unsigned long long o = 0, f = 0;
-    for (int w = 0; w < (int)(blockDim.x >> 6); ++w) {
-      o += red[0][w];
-      f += red[1][w];
-    }
-    counters[C_CELLS] = (unsigned long long)running;
-    counters[C_OOG] = o;
-    counters[C_NONFINITE] = f;
-    counters[C_MASK_WORDS] = 0;
-    counters[C_FALLBACK] = 0;
-  }
+__global__ __launch_bounds__(1024) void k_scene_windows(WindowOut o) {
+  scene_windows<16>(o, [](const int* p) { return *p; });
 }
 
 // K_CalculateParticleNumber (GridHash.cu:78-87): key = compact cell or the
-// scene's out-of-grid bucket; slot = arrival order inside a cell, and inside a
-// bucket the rank of the particle's original index among the scene's
-// out-of-grid particles (oog_pre, the scan of the bounds pass's flags), so a
-// bucket is in original-index order at any size without atomics. Block 0 sets
-// each bucket's count.
+// scene's out-of-grid bucket (whose count the windows set); slot = arrival order
+// inside a cell, -1 in a bucket.
 template <bool kCellOrder>
 __global__ __launch_bounds__(kBlock) void k_bin(SortIn in, int n, GridDev g,
                                                 const int* __restrict__ sid, const SceneWin* __restrict__ win,
                                                 int* __restrict__ key, int* __restrict__ slot,
-                                                int* __restrict__ cell_cnt, const int* __restrict__ scene_off,
-                                                int nscenes, const int* __restrict__ oog_pre,
-                                                const unsigned long long* __restrict__ counters) {
+                                                int* __restrict__ cell_cnt) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (blockIdx.x == 0 && counters[C_OOG] != 0) {
-    for (int s = threadIdx.x; s < nscenes; s += blockDim.x) {
-      const SceneWin w = win[s];
-      cell_cnt[w.cell_base + w.ncell] = oog_pre[scene_end(scene_off, s, n)] - oog_pre[min(scene_begin(scene_off, s), n)];
-    }
-  }
   if (i >= n) return;
   int ci, cj, ck;
   bool nonfinite;
@@ -526,19 +680,26 @@ __global__ __launch_bounds__(kBlock) void k_bin(SortIn in, int n, GridDev g,
   } else if (inside) {
     sl = atomicAdd(&cell_cnt[k], 1);
   }
-  if (!inside) sl = oog_pre[kCellOrder ? in.id[i] : i] - oog_pre[min(scene_begin(scene_off, sid[i]), n)];
-  slot[i] = sl;
+  slot[i] = inside ? sl : -1;
 }
 
-// K_ConstructHashTable (GridHash.cu:187-198): ids into their cell's slots.
-// Input in cell order: tid receives the original index beside each input index.
+// K_ConstructHashTable (GridHash.cu:187-198): ids into their cell's slots. An
+// out-of-grid particle's place in its bucket is the rank of its original index
+// among the scene's out-of-grid particles (oog_pre, the scan of the bounds
+// pass's flags), so a bucket is in original-index order at any size without
+// atomics. Input in cell order: tid receives the original index beside each
+// input index.
 template <bool kCellOrder>
 __global__ __launch_bounds__(kBlock) void k_scatter(const int* __restrict__ key, const int* __restrict__ slot,
                                                     const int* __restrict__ cell_start, int* __restrict__ tmp,
-                                                    const int* __restrict__ id, int* __restrict__ tid, int n) {
+                                                    const int* __restrict__ id, int* __restrict__ tid, int n,
+                                                    const int* __restrict__ sid, const int* __restrict__ scene_off,
+                                                    const int* __restrict__ oog_pre) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= n) return;
-  const int p = cell_start[key[i]] + slot[i];
+  int sl = slot[i];
+  if (sl < 0) sl = oog_pre[kCellOrder ? id[i] : i] - oog_pre[scene_off ? min(scene_off[sid[i]], n) : 0];
+  const int p = cell_start[key[i]] + sl;
   tmp[p] = i;
   if (kCellOrder) tid[p] = id[i];
 }
@@ -815,29 +976,38 @@ void sort_one(const SortBufs& sb, const GridDev& g, const SortIn& in, int n, flo
   k_cell_starts<<<128, kBlock, 0, st>>>(sb.win, sb.key, n, sb.cell_start);
 }
 
+// Bounds blocks of a launch whose last one makes the window: their tickets are
+// same-address atomics, about 9 ns each (256 blocks: 262,144 particles).
+constexpr int kTicketBlocks = 256;
+
 template <bool kCellOrder>
 void sort_in(const SortBufs& sb, const GridDev& g, const SortIn& in, int n, float4* xn, float4* x0, float4* vs,
              const PhysConst* integrate, unsigned long long* counters, hipStream_t st) {
   const int nb = (n + kBlock - 1) / kBlock;
   const int nbounds = (n + kBoundsSpan - 1) / kBoundsSpan;
-  k_scene_bounds<kCellOrder><<<nbounds, kBoundsBlock, 0, st>>>(in, n, g, sb.scene_off, sb.nscenes, sb.sid,
-                                                               sb.scene_minmax, sb.bpart, sb.oog_flag);
-  if (sb.nscenes > 1)
-    k_scene_reduce<<<sb.nscenes, kReduceBlock, 0, st>>>(sb.scene_off, sb.nscenes, sb.bpart, sb.scene_minmax);
-  k_scene_windows<<<1, 1024, 0, st>>>(sb.scene_minmax, sb.nscenes, sb.win, sb.total_cells, sb.bpart, nbounds,
-                                      counters);
-  // out-of-grid ranks by original index (only when the bounds pass found any;
-  // the last scene offset is n)
-  const unsigned long long* any_oog = counters + C_OOG;
-  const int* n_dev = sb.scene_off ? sb.scene_off + sb.nscenes : nullptr;
-  k_scan_dev_reduce<<<kScanDevBlocks, 1024, 0, st>>>(sb.oog_flag, n_dev, n, sb.scan_part, any_oog);
-  k_scan_dev_down<<<kScanDevBlocks, 1024, 0, st>>>(sb.oog_flag, sb.oog_pre, n_dev, n, sb.scan_part, any_oog);
-  k_bin<kCellOrder><<<nb, kBlock, 0, st>>>(in, n, g, sb.sid, sb.win, sb.key, sb.slot, sb.cell_cnt, sb.scene_off,
-                                           sb.nscenes, sb.oog_pre, counters);
-  k_scan_dev_reduce<<<kScanDevBlocks, 1024, 0, st>>>(sb.cell_cnt, sb.total_cells, INT_MAX, sb.scan_part, nullptr);
-  k_scan_dev_down<<<kScanDevBlocks, 1024, 0, st>>>(sb.cell_cnt, sb.cell_start, sb.total_cells, INT_MAX,
-                                                   sb.scan_part, nullptr);
-  k_scatter<kCellOrder><<<nb, kBlock, 0, st>>>(sb.key, sb.slot, sb.cell_start, sb.tmp, in.id, sb.tid, n);
+  const WindowOut windows{sb.scene_minmax, sb.nscenes, sb.win, sb.total_cells, sb.bpart, nbounds, counters, sb.cell_cnt};
+  if (sb.nscenes == 1 && nbounds <= kTicketBlocks) {
+    k_scene_bounds<kCellOrder, true><<<nbounds, kBoundsBlock, 0, st>>>(in, n, g, sb.scene_off, 1, sb.sid,
+                                                                       sb.scene_minmax, sb.bpart, sb.oog_flag,
+                                                                       windows, sb.ticket);
+  } else {
+    k_scene_bounds<kCellOrder, false><<<nbounds, kBoundsBlock, 0, st>>>(in, n, g, sb.scene_off, sb.nscenes, sb.sid,
+                                                                        sb.scene_minmax, sb.bpart, sb.oog_flag,
+                                                                        windows, nullptr);
+    if (sb.nscenes > 1)
+      k_scene_reduce<<<sb.nscenes, kReduceBlock, 0, st>>>(sb.scene_off, sb.nscenes, sb.bpart, sb.scene_minmax);
+    k_scene_windows<<<1, 1024, 0, st>>>(windows);
+  }
+  k_bin<kCellOrder><<<nb, kBlock, 0, st>>>(in, n, g, sb.sid, sb.win, sb.key, sb.slot, sb.cell_cnt);
+  // the cell counts, and the out-of-grid ranks by original index (only when the
+  // bounds pass found any; the last scene offset is n)
+  const ScanJob cells{sb.cell_cnt, sb.cell_start, sb.total_cells, INT_MAX, sb.scan_part, nullptr};
+  const ScanJob flags{sb.oog_flag, sb.oog_pre, sb.scene_off ? sb.scene_off + sb.nscenes : nullptr, n,
+                      sb.scan_part + kScanDevBlocks, counters + C_OOG};
+  k_scan_dev_reduce<<<dim3(kScanDevBlocks, 2), 1024, 0, st>>>(cells, flags);
+  k_scan_dev_down<<<dim3(kScanDevBlocks, 2), 1024, 0, st>>>(cells, flags);
+  k_scatter<kCellOrder><<<nb, kBlock, 0, st>>>(sb.key, sb.slot, sb.cell_start, sb.tmp, in.id, sb.tid, n, sb.sid,
+                                               sb.scene_off, sb.oog_pre);
   PhysConst pc{};
   if (integrate) pc = *integrate;
   k_reorder<kCellOrder><<<nb, kBlock, 0, st>>>(sb.key, sb.cell_start, sb.tmp, sb.tid, sb.sid, in, n, sb.perm,
