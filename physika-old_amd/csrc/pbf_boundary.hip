@@ -360,9 +360,9 @@ __global__ __launch_bounds__(kBlock) void k_csr_viscosity(const float4* __restri
   float tw = 0.0f, dx = 0.0f, dy = 0.0f, dz = 0.0f;
   csr_each(
       nb, row, [&](int j) { return VisPair{xa[j], v_in[j]}; },
-      [&](int, int, const VisPair& q, bool on) {
+      [&](int, int, const VisPair& q) {
         const PairGeom g = pair_geom(xi, q.x, vc.inv_h);
-        if (on && g.r > vc.eps) {
+        if (g.r > vc.eps) {
           const float w = vc.cw * g.t;
           tw += w;
           dx += w * q.v.x;
@@ -370,7 +370,7 @@ __global__ __launch_bounds__(kBlock) void k_csr_viscosity(const float4* __restri
           dz += w * q.v.z;
         }
       },
-      [] {});
+      [] {}, [] {});
   tw = row_sum(tw);
   dx = row_sum(dx);
   dy = row_sum(dy);

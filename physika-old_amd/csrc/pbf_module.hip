@@ -68,11 +68,8 @@ __global__ __launch_bounds__(kBlock) void k_csr_density(const float* __restrict_
   float acc = 0.f, t[kRowUnroll];
   csr_each(
       nb, row, [&](int j) { return load3(x, j); },
-      [&](int u, int, float4 xj, bool on) {
-        const PairGeom p = pair_geom(xi, xj, pc.inv_h);
-        t[u] = on ? p.t : 0.0f;
-      },
-      [&] { acc = row_cubes(acc, t); });
+      [&](int u, int, float4 xj) { t[u] = pair_geom(xi, xj, pc.inv_h).t; },
+      [&] { row_clear(t); }, [&] { acc = row_cubes(acc, t); });
   if (row.lane == 0) rho[row.i] = acc * pc.cW;
 }
 
@@ -157,11 +154,11 @@ __global__ __launch_bounds__(kBlock) void k_csr_lambda(float4* xa, float4* xb, i
     float acc = 0.f, sgx = 0.f, sgy = 0.f, sgz = 0.f, sgg = 0.f, t[kRowUnroll];
     csr_each(
         nb, row, [&](int j) { return MassPos{xs[j], kMass ? minv[j] : 1.0f}; },
-        [&](int u, int j, const MassPos& q, bool on) {
+        [&](int u, int j, const MassPos& q) {
           const PairGeom p = pair_geom(xi, q.x, pc.inv_h);
-          t[u] = on ? p.t : 0.0f;
-          const float t2 = t[u] * t[u];
-          const float gq = on && p.r > pc.pair_eps ? t2 * p.rinv : 0.0f;
+          t[u] = p.t;
+          const float t2 = p.t * p.t;
+          const float gq = p.r > pc.pair_eps ? t2 * p.rinv : 0.0f;
           const float gx = gq * p.dx, gy = gq * p.dy, gz = gq * p.dz;
           sgx += gx;
           sgy += gy;
@@ -170,11 +167,11 @@ __global__ __launch_bounds__(kBlock) void k_csr_lambda(float4* xa, float4* xb, i
           sgg += kMass ? gg * q.m : gg;
           if (kFirst) {
             const unsigned long long r = pairing_r(j);
-            sum_r += on ? r : 0ull;
-            sum_s += on ? pairing_s(r) : 0ull;
+            sum_r += r;
+            sum_s += pairing_s(r);
           }
         },
-        [&] { acc = row_cubes(acc, t); });
+        [&] { row_clear(t); }, [&] { acc = row_cubes(acc, t); });
     acc *= pc.cW;
     sgx = row_sum(sgx);
     sgy = row_sum(sgy);
@@ -234,15 +231,15 @@ __global__ __launch_bounds__(kBlock) void k_csr_displacement(float4* xa, float4*
   if (paired) {
     csr_each(
         nb, row, [&](int j) { return xs[j]; },
-        [&](int, int, float4 xj, bool on) {
+        [&](int, int, float4 xj) {
           const PairGeom p = pair_geom(xi, xj, pc.inv_h);
-          const bool use = on && p.r > pc.pair_eps;
+          const bool use = p.r > pc.pair_eps;
           const float c = scale * (xi.w + xj.w) * (p.t * p.t) * p.rinv;
           ax += use ? c * p.dx : 0.0f;
           ay += use ? c * p.dy : 0.0f;
           az += use ? c * p.dz : 0.0f;
         },
-        [] {});
+        [] {}, [] {});
     const float k = 2.0f * mi;
     ax = row_sum(ax);
     ay = row_sum(ay);
@@ -257,9 +254,9 @@ __global__ __launch_bounds__(kBlock) void k_csr_displacement(float4* xa, float4*
   }
   csr_each(
       nb, row, [&](int j) { return MassPos{xs[j], kMass ? minv[j] : 1.0f}; },
-      [&](int, int j, const MassPos& q, bool on) {
+      [&](int, int j, const MassPos& q) {
         const PairGeom p = pair_geom(xi, q.x, pc.inv_h);
-        if (!on || !(p.r > pc.pair_eps)) return;
+        if (!(p.r > pc.pair_eps)) return;
         const float c = scale * (xi.w + q.x.w) * (p.t * p.t) * p.rinv;
         const float px = c * p.dx, py = c * p.dy, pz = c * p.dz;
         ax += px * mi;
@@ -270,7 +267,7 @@ __global__ __launch_bounds__(kBlock) void k_csr_displacement(float4* xa, float4*
         atomicAdd(d + 1, -py * q.m);
         atomicAdd(d + 2, -pz * q.m);
       },
-      [] {});
+      [] {}, [] {});
   ax = row_sum(ax);
   ay = row_sum(ay);
   az = row_sum(az);
