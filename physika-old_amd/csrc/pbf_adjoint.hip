@@ -92,7 +92,7 @@ __global__ __launch_bounds__(kBlock) void k_adj_lambda(NbrView nv, const float4*
                                                        float4* __restrict__ q1, float4* __restrict__ q2,
                                                        PhysConst pc) {
 #pragma clang fp contract(off)
-  const int s = xcd_block(blockIdx.x, gridDim.x) * blockDim.x + threadIdx.x;
+  const int s = particle_block(nv) * blockDim.x + threadIdx.x;
   if (s >= nv.n) return;
   const float4 ps = P[s], as = f[s];
   float acc[2] = {0.0f, 0.0f};
@@ -110,7 +110,7 @@ __global__ __launch_bounds__(kBlock) void k_adj_lambda2(NbrView nv, const float4
                                                         float4* __restrict__ q1, float4* __restrict__ q2,
                                                         PhysConst pc) {
 #pragma clang fp contract(off)
-  const int g = xcd_block(blockIdx.x, gridDim.x) * blockDim.x + threadIdx.x;
+  const int g = particle_block(nv) * blockDim.x + threadIdx.x;
   const int s = g >> 1, h = g & 1;
   if (s >= nv.n) return;  // both lanes of the pair
   const float4 ps = P[s], as = f[s];
@@ -195,7 +195,7 @@ __global__ __launch_bounds__(kBlock) void k_adj_pos(NbrView nv, const float4* __
                                                     float4* __restrict__ e_out, float4* __restrict__ f_out,
                                                     PhysConst pc) {
 #pragma clang fp contract(off)
-  const int s = xcd_block(blockIdx.x, gridDim.x) * blockDim.x + threadIdx.x;
+  const int s = particle_block(nv) * blockDim.x + threadIdx.x;
   if (s >= nv.n) return;
   const float4 ps = P[s], q1s = q1[s], q2s = q2[s];
   AdjSums b[2];
@@ -213,7 +213,7 @@ __global__ __launch_bounds__(kBlock) void k_adj_pos2(NbrView nv, const float4* _
                                                      float4* __restrict__ e_out, float4* __restrict__ f_out,
                                                      PhysConst pc) {
 #pragma clang fp contract(off)
-  const int g = xcd_block(blockIdx.x, gridDim.x) * blockDim.x + threadIdx.x;
+  const int g = particle_block(nv) * blockDim.x + threadIdx.x;
   const int s = g >> 1, h = g & 1;
   if (s >= nv.n) return;  // both lanes of the pair
   const float4 ps = P[s], q1s = q1[s], q2s = q2[s];

@@ -311,7 +311,7 @@ __global__ __launch_bounds__(kBlock) void k_viscosity(NbrView nv, const float4* 
                                                       const float4* __restrict__ v_in, float4* __restrict__ v_next,
                                                       VisConst vc, const int* __restrict__ perm,
                                                       float* __restrict__ x_out, float* __restrict__ v_out) {
-  const int g = xcd_block(blockIdx.x, gridDim.x) * blockDim.x + threadIdx.x;
+  const int g = particle_block(nv) * blockDim.x + threadIdx.x;
   const int s = kPair ? g >> 1 : g, h = kPair ? g & 1 : 0;
   if (s >= nv.n) return;
   const float4 xi = xs[s];

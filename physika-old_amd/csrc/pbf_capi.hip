@@ -167,7 +167,7 @@ struct pbf_ctx {
   } sg;
   long long graph_replays = 0, graph_captures = 0;
 
-  unsigned long long* counters = nullptr;     // device, C_COUNT
+  unsigned long long* counters = nullptr;     // device, kDeviceCounters
   unsigned long long* h_counters = nullptr;   // pinned, mapped host copy, written by k_wave_stats
   unsigned long long* h_counters_dev = nullptr;  // its device address
   hipEvent_t counters_ev = nullptr;
@@ -1113,7 +1113,7 @@ int ensure_tape(pbf_ctx* c, int m) {
     PBF_HIP(c, hipMalloc(&t.mask, sizeof(uint32_t) * std::max<size_t>(c->slot_mask, 1)));
     PBF_HIP(c, hipMalloc(&t.cell_start, sizeof(int) * ((size_t)c->cell_cap + 2)));
     PBF_HIP(c, hipMalloc(&t.win, sizeof(SceneWin) * (size_t)std::max(c->scene_cap, 1)));
-    PBF_HIP(c, hipMalloc(&t.counters, sizeof(unsigned long long) * C_COUNT));
+    PBF_HIP(c, hipMalloc(&t.counters, sizeof(unsigned long long) * kDeviceCounters));
     PBF_HIP(c, hipMalloc(&t.it, sizeof(float4) * cap * (size_t)std::max(2 * K - 1, 1)));
   }
   if (r.adj_n < c->cap_n) {
@@ -1294,7 +1294,7 @@ int pbf_create(const pbf_params* p, pbf_ctx** out) {
     return st;
   }
   if (hipGetDevice(&c->device) != hipSuccess ||
-      hipMalloc(&c->counters, sizeof(unsigned long long) * C_COUNT) != hipSuccess ||
+      hipMalloc(&c->counters, sizeof(unsigned long long) * kDeviceCounters) != hipSuccess ||
       hipHostMalloc(&c->h_counters, sizeof(unsigned long long) * C_COUNT, hipHostMallocMapped) != hipSuccess ||
       hipHostGetDevicePointer((void**)&c->h_counters_dev, c->h_counters, 0) != hipSuccess ||
       hipEventCreateWithFlags(&c->counters_ev, hipEventDisableTiming) != hipSuccess ||
@@ -1307,7 +1307,7 @@ int pbf_create(const pbf_params* p, pbf_ctx** out) {
     return PBF_ERR_HIP;
   }
   std::memset(c->h_counters, 0, sizeof(unsigned long long) * C_COUNT);
-  (void)hipMemset(c->counters, 0, sizeof(unsigned long long) * C_COUNT);
+  (void)hipMemset(c->counters, 0, sizeof(unsigned long long) * kDeviceCounters);
   {
     const hipError_t e = scratch_address(c->device, &c->noalloc_scratch);
     if (e != hipSuccess)
@@ -1615,7 +1615,7 @@ int pbf_rollout_backward(pbf_ctx* c, float* d_xbar, float* d_vbar, void* stream)
         launch_copy_cells(c->cell_start, t.cell_start, c->total_cells, c->cell_cap, st);
         if (hipMemcpyAsync(t.win, c->win, sizeof(SceneWin) * (size_t)r.nscenes, hipMemcpyDeviceToDevice, st) !=
                 hipSuccess ||
-            hipMemcpyAsync(t.counters, c->counters, sizeof(unsigned long long) * C_COUNT, hipMemcpyDeviceToDevice,
+            hipMemcpyAsync(t.counters, c->counters, sizeof(unsigned long long) * kDeviceCounters, hipMemcpyDeviceToDevice,
                            st) != hipSuccess)
           s = fail(c, PBF_ERR_HIP, "tape copy failed");
       }
@@ -1756,7 +1756,7 @@ int pbf_rollout_backward_f64(pbf_ctx* c, double* d_xbar, double* d_vbar, void* s
         launch_copy_cells(c->cell_start, t.cell_start, c->total_cells, c->cell_cap, st);
         if (hipMemcpyAsync(t.win, c->win, sizeof(SceneWin) * (size_t)r.nscenes, hipMemcpyDeviceToDevice, st) !=
                 hipSuccess ||
-            hipMemcpyAsync(t.counters, c->counters, sizeof(unsigned long long) * C_COUNT, hipMemcpyDeviceToDevice,
+            hipMemcpyAsync(t.counters, c->counters, sizeof(unsigned long long) * kDeviceCounters, hipMemcpyDeviceToDevice,
                            st) != hipSuccess)
           s = fail(c, PBF_ERR_HIP, "tape copy failed");
       }

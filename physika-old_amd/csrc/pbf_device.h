@@ -78,6 +78,25 @@ __device__ __forceinline__ int xcd_block(int b, int nb) {
   return x * per + min(x, rem) + idx;
 }
 
+// The same for the passes over the neighbor lists, whose work is the lists' (see kXcdChunk).
+__device__ __forceinline__ int particle_block(const NbrView& nv) {
+  const int b = blockIdx.x, nb = gridDim.x;
+  if (nv.n >= kUnevenMin) {
+    unsigned long long all = 0, most = 0;
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+      const unsigned long long e = nv.counters[C_EIGHTH + k];
+      all += e;
+      most = max(most, e);
+    }
+    if (8000 * most > kUneven * all) {
+      const int g = kXcdChunk / (int)blockDim.x, x = b & 7, idx = b >> 3;  // g blocks to a chunk
+      return b < nb / (8 * g) * (8 * g) ? (idx / g * 8 + x) * g + idx % g : b;
+    }
+  }
+  return xcd_block(b, nb);
+}
+
 __device__ __forceinline__ int wave_max(int v) {
 #pragma unroll
   for (int d = 32; d > 0; d >>= 1) v = max(v, __shfl_xor(v, d));

@@ -86,8 +86,22 @@ struct Csr {
 
 enum Counter {
   C_PAIRS = 0, C_OOG, C_NONFINITE, C_MASK_WORDS, C_FALLBACK, C_LIST_SLOTS, C_CELLS, C_CANDIDATES, C_LIST_NEED,
-  C_STAGED, C_COUNT
+  C_STAGED, C_COUNT,
+  C_EIGHTH = 16  // on the device only: the pairs of each eighth of the waves (searches of kUnevenMin and more)
 };
+constexpr int kDeviceCounters = C_EIGHTH + 8;
+static_assert(C_COUNT <= C_EIGHTH, "the eighths follow the counters");
+
+// The passes hand each XCD one contiguous eighth of the particles, or, where
+// the neighbor pairs are spread unevenly over the eighths, every eighth chunk of
+// kXcdChunk particles: an XCD that has the dense regions otherwise works on while
+// the others are done. The neighbor pass counts the eighths' pairs; the line is
+// the fullest one at kUneven/1000 of the mean. 1M particles in Gaussian blobs: a
+// frame 8.93 -> 7.16 ms (chunks of 1,024 and 4,096: 7.21 and 7.47); an even
+// lattice of 1M would lose 2% of its four steps to the chunks' shared borders, and
+// loses 0.4% (3.706 -> 3.722 ms) to reading the counts. Below kUnevenMin an
+// eighth is less than one round of the XCD's workgroups.
+constexpr int kXcdChunk = 2048, kUnevenMin = 1 << 18, kUneven = 1250;
 
 // Runs are visited in the order q = 0..8 of run_of(q): first the three rows of
 // the particle's own z-plane (dk = 0), which hold most of its neighbors, then

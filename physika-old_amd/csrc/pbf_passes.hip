@@ -329,6 +329,9 @@ __global__ __launch_bounds__(64) void k_neighbors(NbrView nv, NbrOut out, unsign
     out.list_jbase[wave] = wjlo;
     out.list_mode[wave] = (staged ? kListStaged : mode) | (nfull << 2);
     out.wave_stat[wave] = make_int4(tot, tcand, need, staged ? 1 : 0);
+    // the passes' block order: one wave of each eight counts for its eighth
+    if (nv.n >= kUnevenMin && (blockIdx.x >> 3 & 7) == 0)
+      atomicAdd(&counters[C_EIGHTH + (blockIdx.x & 7)], (unsigned long long)tot);
     if (staged) {
       int* st = out.stage + kStageInts * wave;
       st[0] = sa[0];
@@ -785,7 +788,7 @@ __global__ __launch_bounds__(B) void k_density_lambda(NbrView nv, float4* __rest
                                                       float* __restrict__ rho_out, const int* __restrict__ perm,
                                                       float4* __restrict__ aux) {
   __shared__ float4 stage_buf[B / 64][kStageRecords];
-  const int s = xcd_block(blockIdx.x, gridDim.x) * blockDim.x + threadIdx.x;
+  const int s = particle_block(nv) * blockDim.x + threadIdx.x;
   density_lambda_at(nv, s, xs, pc, rho_out, perm, aux, stage_buf[threadIdx.x >> 6]);
 }
 
@@ -796,7 +799,7 @@ __global__ __launch_bounds__(B) void k_density_lambda2(NbrView nv, float4* __res
                                                        float* __restrict__ rho_out, const int* __restrict__ perm,
                                                        float4* __restrict__ aux) {
   __shared__ float4 stage_buf[B / 64][kStageRecords];
-  const int g = xcd_block(blockIdx.x, gridDim.x) * blockDim.x + threadIdx.x;
+  const int g = particle_block(nv) * blockDim.x + threadIdx.x;
   density_lambda_at2(nv, g >> 1, g & 1, xs, pc, rho_out, perm, aux, stage_buf[threadIdx.x >> 6]);
 }
 
@@ -1063,7 +1066,7 @@ __global__ __launch_bounds__(B) void k_displacement(NbrView nv, const float4* __
                                                     float* __restrict__ v_out, float4* __restrict__ v_sorted,
                                                     int* __restrict__ id_out) {
   __shared__ float4 stage_buf[B / 64][kStageRecords];
-  const int s = xcd_block(blockIdx.x, gridDim.x) * blockDim.x + threadIdx.x;
+  const int s = particle_block(nv) * blockDim.x + threadIdx.x;
   displacement_at(nv, s, xs, xd, pc, last, x0, vs, perm, x_out, v_out, v_sorted, id_out,
                   stage_buf[threadIdx.x >> 6]);
 }
@@ -1076,7 +1079,7 @@ __global__ __launch_bounds__(B) void k_displacement2(NbrView nv, const float4* _
                                                      float* __restrict__ v_out, float4* __restrict__ v_sorted,
                                                      int* __restrict__ id_out) {
   __shared__ float4 stage_buf[B / 64][kStageRecords];
-  const int g = xcd_block(blockIdx.x, gridDim.x) * blockDim.x + threadIdx.x;
+  const int g = particle_block(nv) * blockDim.x + threadIdx.x;
   displacement_at2(nv, g >> 1, g & 1, xs, xd, pc, last, x0, vs, perm, x_out, v_out, v_sorted, id_out,
                    stage_buf[threadIdx.x >> 6]);
 }

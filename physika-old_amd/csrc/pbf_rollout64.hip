@@ -161,7 +161,7 @@ __global__ __launch_bounds__(kBlock) void k64_density_lambda(NbrView nv, double4
                                                              double4* __restrict__ aux, double* __restrict__ rho_out,
                                                              const int* __restrict__ perm) {
 #pragma clang fp contract(off)
-  const int g = xcd_block(blockIdx.x, gridDim.x) * blockDim.x + threadIdx.x;
+  const int g = particle_block(nv) * blockDim.x + threadIdx.x;
   const int s = kPair ? g >> 1 : g, h = kPair ? g & 1 : 0;
   if (s >= nv.n) return;
   const double4 ps = P[s];
@@ -201,7 +201,7 @@ __global__ __launch_bounds__(kBlock) void k64_displacement(NbrView nv, const dou
                                                            const int* __restrict__ perm, double* __restrict__ x_out,
                                                            double* __restrict__ v_out) {
 #pragma clang fp contract(off)
-  const int g = xcd_block(blockIdx.x, gridDim.x) * blockDim.x + threadIdx.x;
+  const int g = particle_block(nv) * blockDim.x + threadIdx.x;
   const int s = kPair ? g >> 1 : g, h = kPair ? g & 1 : 0;
   if (s >= nv.n) return;
   const double4 ps = P[s];
@@ -269,7 +269,7 @@ __global__ __launch_bounds__(kBlock) void k64_adj_lambda(NbrView nv, const doubl
                                                          const double4* __restrict__ f, double4* __restrict__ q1,
                                                          double4* __restrict__ q2, PhysConst64 pc) {
 #pragma clang fp contract(off)
-  const int g = xcd_block(blockIdx.x, gridDim.x) * blockDim.x + threadIdx.x;
+  const int g = particle_block(nv) * blockDim.x + threadIdx.x;
   const int s = kPair ? g >> 1 : g, h = kPair ? g & 1 : 0;
   if (s >= nv.n) return;
   const double4 ps = P[s], as = f[s];
@@ -303,7 +303,7 @@ __global__ __launch_bounds__(kBlock) void k64_adj_pos(NbrView nv, const double4*
                                                       const double4* __restrict__ c, double4* __restrict__ e_out,
                                                       double4* __restrict__ f_out, PhysConst64 pc) {
 #pragma clang fp contract(off)
-  const int g = xcd_block(blockIdx.x, gridDim.x) * blockDim.x + threadIdx.x;
+  const int g = particle_block(nv) * blockDim.x + threadIdx.x;
   const int s = kPair ? g >> 1 : g, h = kPair ? g & 1 : 0;
   if (s >= nv.n) return;
   const double4 ps = P[s], q1s = q1[s], q2s = q2[s];

@@ -385,6 +385,7 @@ __device__ __forceinline__ void scene_windows(const WindowOut& o, BLoad&& bload)
     o.counters[C_NONFINITE] = (unsigned long long)nonfinite;
     o.counters[C_MASK_WORDS] = 0;
     o.counters[C_FALLBACK] = 0;
+    for (int k = 0; k < 8; ++k) o.counters[C_EIGHTH + k] = 0;
   }
 }
 
