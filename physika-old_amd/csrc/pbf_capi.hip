@@ -174,7 +174,10 @@ struct pbf_ctx {
   bool counters_pending = false;
 
   int last_n = -1;  // particle count of the last neighbor search (-1: none)
-  long long csr_total = -1;  // its list elements once cnt_orig holds their row starts (-1: not yet)
+  // its list elements once cnt_orig holds their row starts (-1: not yet), and
+  // C_CALLS then: a replay of a captured call searches without the host
+  long long csr_total = -1;
+  unsigned long long csr_calls = 0;
 
   int pass_block = kBlock;  // threads per workgroup of the PBD passes (pbf_tuning)
   bool pass_persistent = false;  // persistent launches of the PBD passes (pbf_tuning)
@@ -821,7 +824,11 @@ int export_csr(pbf_ctx* c, int n, int* d_index, int* d_elems, long long cap, lon
     *total = 0;
     return PBF_OK;
   }
-  const bool counted = c->csr_total >= 0;
+  bool counted = c->csr_total >= 0;
+  if (counted) {
+    PBF_HIP(c, hipStreamSynchronize(st));
+    counted = c->csr_calls == c->h_counters[C_CALLS];
+  }
   if (!counted) {
     launch_invert(c->perm, c->inv, n, st);
     launch_csr_count(c->nbr_cnt, c->inv, n, c->cnt_orig, st);
@@ -835,6 +842,7 @@ int export_csr(pbf_ctx* c, int n, int* d_index, int* d_elems, long long cap, lon
     PBF_HIP(c, hipMemcpyAsync(&tot, c->cnt_orig + n, sizeof(int), hipMemcpyDeviceToHost, st));
     PBF_HIP(c, hipStreamSynchronize(st));
     c->csr_total = tot;
+    c->csr_calls = c->h_counters[C_CALLS];
   }
   *total = c->csr_total;
   if (d_elems == nullptr) return PBF_OK;

@@ -86,7 +86,7 @@ struct Csr {
 
 enum Counter {
   C_PAIRS = 0, C_OOG, C_NONFINITE, C_MASK_WORDS, C_FALLBACK, C_LIST_SLOTS, C_CELLS, C_CANDIDATES, C_LIST_NEED,
-  C_STAGED, C_COUNT,
+  C_STAGED, C_CALLS, C_COUNT,
   C_EIGHTH = 16  // on the device only: the pairs of each eighth of the waves (searches of kUnevenMin and more)
 };
 constexpr int kDeviceCounters = C_EIGHTH + 8;

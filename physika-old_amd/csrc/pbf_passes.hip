@@ -651,6 +651,7 @@ __global__ __launch_bounds__(1024) void k_wave_stats(const int4* __restrict__ ws
     counters[C_CANDIDATES] = cand;
     counters[C_LIST_NEED] = (unsigned long long)need;
     counters[C_STAGED] = (unsigned long long)staged;
+    counters[C_CALLS] += 1;
     counters[C_LIST_SLOTS] = 64ull * (unsigned long long)nwaves * (unsigned long long)need;
 #pragma unroll
     for (int k = 0; k < C_COUNT; ++k) host[k] = counters[k];

@@ -67,3 +67,33 @@ def test_several_lanes_equal_one(fluid, scene, name, reserve):
                     + [(st["neighbor_pairs"], st["candidates"], st["out_of_grid"])])
     for a, b in zip(*outs):
         np.testing.assert_array_equal(a, b)
+
+
+@pytest.mark.parametrize("n", [1000, 40000])
+def test_lists_after_a_replayed_step(fluid, scene, n):
+    """step_neighbors exports the search of a step that a replayed graph ran
+    after an earlier export (the row starts are kept between the exports)."""
+    say(f"lists of a replayed step, {n} particles")
+    side = int(np.ceil(n ** (1 / 3)))
+    far, near = (scene.jittered_lattice((side,) * 3, (0.2, 0.3, 0.2), d, 0.1, seed=2, count=n)
+                 for d in (0.007, 0.005))
+    ctx = fluid.Context("cuda:0")
+    x, v = dev(near), dev(np.zeros_like(near))
+    ctx.step(x, v)  # reservations for the longer lists
+    torch.cuda.synchronize()
+    ctx.stats()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, capture_error_mode="relaxed"):
+        ctx.step(x, v)
+    for start in (far, near, far):
+        x.copy_(dev(start))
+        v.zero_()
+        graph.replay()
+        got = ctx.step_neighbors(n)
+        one = fluid.Context("cuda:0")
+        xd, vd = dev(start), dev(np.zeros_like(start))
+        one.step(xd, vd)
+        want = one.step_neighbors(n)
+        torch.cuda.synchronize()
+        for a, b in ((x, xd), (got.index, want.index), (got.elements, want.elements)):
+            np.testing.assert_array_equal(a.cpu().numpy(), b.cpu().numpy())
