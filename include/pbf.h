@@ -273,7 +273,9 @@ int pbf_batch_step(pbf_ctx* ctx, float* d_x, float* d_v, float* d_rho, const int
  * step of it re-run with its PBD iterates kept and its neighbor sets rebuilt,
  * and differentiated by hand-written adjoint kernels with the neighbor sets
  * held fixed (the step is C1 across a set change: W and the kernel gradient
- * vanish with their first derivative at r = h). The rollout stays valid for
+ * vanish with their first derivative at r = h). On a context that has run a
+ * backward of that size, the forward records its last segment in the same
+ * buffers and the next backward does not run it again. The rollout stays valid for
  * repeated backward calls until the next pbf_rollout_forward or a parameter
  * change (PBF_ERR_INVALID). Returns PBF_ERR_UNSUPPORTED when a step had
  * particles outside the grid. pbf_rollout_backward is blocking. */
