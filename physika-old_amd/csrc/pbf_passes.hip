@@ -1311,20 +1311,21 @@ void launch_nbr_fixed(const NbrView& nv, const int* perm, int limit, int* counts
 
 // ---------------------------------------------------------------------------
 // CSR export (NeighborList, Framework/Topology/NeighborList.h:27-66) in
-// original ids: one wave writes the rows of its 64 particles. A chunk of
-// sixteen entries per row is decoded by the row's lane (coalesced list loads),
-// turned through LDS and written by four lanes per row with 16-byte stores (4-byte
-// aligned), so that a store instruction fills sixteen runs of 64 bytes instead
-// of one word in each of 64 rows. 845 -> 249 us at 1,048,576 particles (75.6M
-// elements, 302 MB written).
-constexpr int kFillChunk = 16, kFillStride = kFillChunk + 4;  // 16-byte aligned rows
+// original ids: one wave writes the rows of its 64 particles. A chunk of 32
+// entries per row is decoded by the row's lane (coalesced list loads), turned
+// through LDS and written by half a wave per row, so that a store instruction
+// fills two runs of 128 bytes instead of one word in each of 64 rows. The address
+// unit is 89% busy: with a quarter of it gathering the ids and about half storing.
+// 845 -> 213 us at 1,048,576 particles (75.6M elements, 302 MB written); four
+// lanes per row with 16-byte stores to 4-byte aligned places took 249 (the unit
+// takes such a store apart), 64 entries 266 (fewer waves fit, emptier last chunks),
+// and stores that pass the L2 by 305.
+constexpr int kFillChunk = 32, kFillStride = kFillChunk + 1;  // rows in different banks
 
 __global__ __launch_bounds__(64) void k_csr_fill(NbrView nv, const int* __restrict__ perm,
                                                  const int* __restrict__ offsets, int* __restrict__ elems,
                                                  long long cap) {
-  typedef int i4u __attribute__((ext_vector_type(4), aligned(4)));
-  typedef int i4 __attribute__((ext_vector_type(4)));
-  __shared__ __attribute__((aligned(16))) int tile[64 * kFillStride];
+  __shared__ int tile[64 * kFillStride];
   __shared__ int2 dst[64];  // per row: the chunk's first element, its length
   const int wave = xcd_block(blockIdx.x, gridDim.x), lane = threadIdx.x;
   const bool active = (wave << 6) + lane < nv.n;
@@ -1339,38 +1340,32 @@ __global__ __launch_bounds__(64) void k_csr_fill(NbrView nv, const int* __restri
   }
   ListRow lr;
   lr.load(nv, wl, s, fits ? nv.nbr_cnt[s] : 0);
+  constexpr int kParts = kFillChunk / 8;  // list chunks at a time
   const int nchunk = wave_max(lr.chunks());
-  for (int c = 0; c < nchunk; c += 2) {  // two list chunks of every row
-    const int start = lr.before(c), mid = lr.before(c + 1) - start, left = lr.before(c + 2) - start;
-    int j0[8], j1[8];
-    lr.read(c, s, j0);
-    lr.read(c + 1, s, j1);
+  const int g = lane / kFillChunk, u = lane % kFillChunk;
+  for (int c = 0; c < nchunk; c += kParts) {
+    const int start = lr.before(c);
+    int j[kParts][8];
 #pragma unroll
-    for (int u = 0; u < 8; ++u) j0[u] = perm[j0[u]];
+    for (int k = 0; k < kParts; ++k) lr.read(c + k, s, j[k]);
 #pragma unroll
-    for (int u = 0; u < 8; ++u) j1[u] = perm[j1[u]];
+    for (int k = 0; k < kParts; ++k)
+#pragma unroll
+      for (int w = 0; w < 8; ++w) j[k][w] = perm[j[k][w]];
     int* t = tile + kFillStride * lane;
 #pragma unroll
-    for (int u = 0; u < 8; ++u)
-      if (u < mid) t[u] = j0[u];
+    for (int k = 0; k < kParts; ++k) {
+      const int at = lr.before(c + k) - start, left = lr.before(c + k + 1) - start - at;
 #pragma unroll
-    for (int u = 0; u < 8; ++u)
-      if (mid + u < left) t[mid + u] = j1[u];
-    dst[lane] = make_int2(o + start, left);
+      for (int w = 0; w < 8; ++w)
+        if (w < left) t[at + w] = j[k][w];
+    }
+    dst[lane] = make_int2(o + start, lr.before(c + kParts) - start);
     wave_lds_fence();
-#pragma unroll
-    for (int r0 = 0; r0 < 64; r0 += 16) {
-      const int r = r0 + (lane >> 2), u = (lane & 3) << 2;
+#pragma unroll 8
+    for (int r = g; r < 64; r += 64 / kFillChunk) {
       const int2 d = dst[r];
-      const i4 w = *reinterpret_cast<const i4*>(tile + kFillStride * r + u);
-      int* out = elems + (size_t)(unsigned)d.x + u;
-      if (u + 4 <= d.y) {
-        *reinterpret_cast<i4u*>(out) = w;
-      } else {
-        if (u < d.y) out[0] = w[0];
-        if (u + 1 < d.y) out[1] = w[1];
-        if (u + 2 < d.y) out[2] = w[2];
-      }
+      if (u < d.y) elems[(size_t)(unsigned)d.x + u] = tile[kFillStride * r + u];
     }
     wave_lds_fence();
   }
