@@ -73,7 +73,8 @@ struct pbf_ctx {
   long long list_cap = 0;  // 16-bit slots
   long long auto_list_per = 96;  // automatic list reservation, 16-bit slots per particle
   int4* wave_stat = nullptr;     // per wave of the neighbor pass: pairs, candidates, need
-  int stats_waves = 0;           // waves of the last search whose statistics are not yet reduced
+  int stats_n = 0;               // particles of the last search whose statistics are not yet reduced
+  bool even = false;             // the last finished call's search was even (kXcdChunk)
 
   int* scan_scratch = nullptr;
   size_t scan_scratch_n = 0;
@@ -604,6 +605,7 @@ int adapt_reservations(pbf_ctx* c) {
   if (!c->counters_pending) return PBF_OK;
   if (hipEventQuery(c->counters_ev) != hipSuccess) return PBF_OK;
   c->counters_pending = false;
+  c->even = c->h_counters[C_UNEVEN] == 1;
   const long long mw = (long long)c->h_counters[C_MASK_WORDS];
   const long long need = (long long)c->h_counters[C_LIST_NEED];  // slots per particle of the fullest wave
   int st = PBF_OK;
@@ -640,6 +642,7 @@ NbrView view_of(const pbf_ctx* c, int n) {
   nv.counters = c->counters;
   nv.thr2 = c->pc.thr2;
   nv.list_per = list_per_of(c);
+  nv.maybe_uneven = n >= kUnevenMin && !c->even ? 1 : 0;
   nv.n = n;
   nv.pad = n;
   return nv;
@@ -801,7 +804,7 @@ int search(pbf_ctx* c, const SortIn& in, int n, const int* scene_off, int nscene
     o.stage_lists = stages_lists(c, n) ? 1 : 0;
     launch_neighbors(view_of(c, n), o, c->counters, st, t.events());
   }
-  c->stats_waves = (n + 63) / 64;
+  c->stats_n = n;
   PBF_LAUNCHED(c);
   c->last_n = n;
   c->last_slot = -1;
@@ -824,8 +827,8 @@ int record_counters(pbf_ctx* c, hipStream_t st) {
     c->captured = true;
     c->tape_of = 0;
   }
-  launch_wave_stats(c->wave_stat, c->stats_waves, c->counters, c->h_counters_dev, st);
-  c->stats_waves = 0;
+  launch_wave_stats(c->wave_stat, c->stats_n, c->counters, c->h_counters_dev, st);
+  c->stats_n = 0;
   PBF_LAUNCHED(c);
   PBF_HIP(c, hipEventRecord(c->counters_ev, st));
   c->counters_pending = true;

@@ -78,22 +78,29 @@ __device__ __forceinline__ int xcd_block(int b, int nb) {
   return x * per + min(x, rem) + idx;
 }
 
-// The same for the passes over the neighbor lists, whose work is the lists' (see kXcdChunk).
+// Every eighth chunk of kXcdChunk threads for each XCD (the blocks past the last
+// eight chunks in order).
+__device__ __forceinline__ int xcd_chunk_block(int b, int nb) {
+  const int g = kXcdChunk / (int)blockDim.x, x = b & 7, idx = b >> 3;  // g blocks to a chunk
+  return b < nb / (8 * g) * (8 * g) ? (idx / g * 8 + x) * g + idx % g : b;
+}
+
+// Whether a search's pairs are spread unevenly (see kXcdChunk).
+__device__ __forceinline__ bool uneven_pairs(const unsigned long long* counters) {
+  unsigned long long all = 0, most = 0;
+#pragma unroll
+  for (int k = 0; k < 8; ++k) {
+    const unsigned long long e = counters[C_EIGHTH + k];
+    all += e;
+    most = max(most, e);
+  }
+  return 8000 * most > kUneven * all;
+}
+
+// The order of the passes over the neighbor lists, whose work is the lists'.
 __device__ __forceinline__ int particle_block(const NbrView& nv) {
   const int b = blockIdx.x, nb = gridDim.x;
-  if (nv.n >= kUnevenMin) {
-    unsigned long long all = 0, most = 0;
-#pragma unroll
-    for (int k = 0; k < 8; ++k) {
-      const unsigned long long e = nv.counters[C_EIGHTH + k];
-      all += e;
-      most = max(most, e);
-    }
-    if (8000 * most > kUneven * all) {
-      const int g = kXcdChunk / (int)blockDim.x, x = b & 7, idx = b >> 3;  // g blocks to a chunk
-      return b < nb / (8 * g) * (8 * g) ? (idx / g * 8 + x) * g + idx % g : b;
-    }
-  }
+  if (nv.maybe_uneven && uneven_pairs(nv.counters)) return xcd_chunk_block(b, nb);
   return xcd_block(b, nb);
 }
 

@@ -86,7 +86,7 @@ struct Csr {
 
 enum Counter {
   C_PAIRS = 0, C_OOG, C_NONFINITE, C_MASK_WORDS, C_FALLBACK, C_LIST_SLOTS, C_CELLS, C_CANDIDATES, C_LIST_NEED,
-  C_STAGED, C_CALLS, C_COUNT,
+  C_STAGED, C_CALLS, C_UNEVEN, C_COUNT,
   C_EIGHTH = 16  // on the device only: the pairs of each eighth of the waves (searches of kUnevenMin and more)
 };
 constexpr int kDeviceCounters = C_EIGHTH + 8;
@@ -98,9 +98,11 @@ static_assert(C_COUNT <= C_EIGHTH, "the eighths follow the counters");
 // the others are done. The neighbor pass counts the eighths' pairs; the line is
 // the fullest one at kUneven/1000 of the mean. 1M particles in Gaussian blobs: a
 // frame 8.93 -> 7.16 ms (chunks of 1,024 and 4,096: 7.21 and 7.47); an even
-// lattice of 1M would lose 2% of its four steps to the chunks' shared borders, and
-// loses 0.4% (3.706 -> 3.722 ms) to reading the counts. Below kUnevenMin an
-// eighth is less than one round of the XCD's workgroups.
+// lattice of 1M would lose 2% of its four steps to the chunks' shared borders.
+// Reading the counts holds every wave up (0.4%, 3.706 -> 3.722 ms), so the
+// passes leave it out where the last call told that its search was even
+// (C_UNEVEN: 1 even, 2 uneven, 0 too small). Below kUnevenMin an eighth is less
+// than one round of the XCD's workgroups.
 constexpr int kXcdChunk = 2048, kUnevenMin = 1 << 18, kUneven = 1250;
 
 // Runs are visited in the order q = 0..8 of run_of(q): first the three rows of
@@ -163,6 +165,7 @@ struct NbrView {
   const int* oog_rev;          // their sorted indices, kOogRev slots per particle (in no order)
   const unsigned long long* counters;
   float thr2;
+  int maybe_uneven;   // the passes look at the eighths' counts for their block order (kXcdChunk)
   int list_per;       // 16-bit slots per particle of a wave's list region (wave w's list, if any, starts at 64 w list_per)
   int n;
   int pad;            // padding particle of the position buffers (index n)
@@ -263,7 +266,7 @@ void launch_neighbors(const NbrView& nv, const NbrOut& out, unsigned long long* 
 // Sums the per-wave statistics of the last neighbor pass (nwaves waves) into
 // counters[C_PAIRS], [C_CANDIDATES], [C_LIST_SLOTS] and [C_LIST_NEED], and copies
 // all counters to host (mapped host memory).
-void launch_wave_stats(const int4* wave_stat, int nwaves, unsigned long long* counters, unsigned long long* host,
+void launch_wave_stats(const int4* wave_stat, int n, unsigned long long* counters, unsigned long long* host,
                        hipStream_t st);
 // block: threads per workgroup, 64, 128, 256 or 512; persistent: as many
 // blocks as stay resident, each wave walking 64-particle tiles; lanes: 1, or 2

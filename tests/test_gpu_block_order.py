@@ -28,6 +28,13 @@ def scenes(scene, order):
     return [(x, (0.05 * (scene.uniform01(6, 3 * len(x)).reshape(-1, 3) - 0.5)).astype(np.float32)) for x in out]
 
 
+def even_scene():
+    i = np.indices((65,) * 3).reshape(3, -1).T
+    x = (0.2 + 0.0051 * i).astype(np.float32)
+    assert len(x) >= 1 << 18
+    return x
+
+
 def run(fluid, parts, kind):
     """x, v (and rho, or the gradients) of the scenes as one batch; of one scene, alone."""
     off = np.concatenate([[0], np.cumsum([len(x) for x, _ in parts])]).astype(np.int32)
@@ -43,6 +50,10 @@ def run(fluid, parts, kind):
     else:
         rho = torch.zeros(n, dtype=torch.float32, device="cuda:0")
         ctx = fluid.Context("cuda:0", flags=fluid._capi.PBF_FLAG_VISCOSITY if kind == "viscosity" else 0)
+        if kind == "after an even search":  # the context expects another one
+            e = dev(even_scene())
+            ctx.step(e, torch.zeros_like(e))
+            torch.cuda.synchronize()
         if off_d is None:
             ctx.step(x, v, rho, 3)
         else:
@@ -53,7 +64,7 @@ def run(fluid, parts, kind):
 
 
 @pytest.mark.parametrize("order", ["dense first", "dense last"])
-@pytest.mark.parametrize("kind", ["plain", "viscosity", "gradients"])
+@pytest.mark.parametrize("kind", ["plain", "viscosity", "gradients", "after an even search"])
 def test_uneven_batch_equals_its_scenes(fluid, scene, kind, order):
     parts = scenes(scene, order)
     say(f"uneven batch of {sum(len(x) for x, _ in parts)} particles, {kind}, {order}")
