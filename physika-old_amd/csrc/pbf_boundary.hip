@@ -255,6 +255,26 @@ __device__ __forceinline__ void vis_term(VisSums& a, float4 xi, const VisPair& q
   }
 }
 
+// The weights of a lane pair's entries over the iterations of one solve.
+enum VisWeights { kVisNone, kVisWrite, kVisRead };
+constexpr float kVisSkip = -1.0f;  // an entry that adds nothing (r <= eps, or past the lane's count)
+
+// vis_term in two halves: the weight (negative for r <= eps; t >= 0), and its terms.
+__device__ __forceinline__ float vis_weight(float4 xi, float4 xj, const VisConst& vc) {
+#pragma clang fp contract(off)
+  const PairGeom g = pair_geom(xi, xj, vc.inv_h);
+  return g.r > vc.eps ? vc.cw * g.t : kVisSkip;
+}
+__device__ __forceinline__ void vis_add(VisSums& a, float w, float4 v) {
+#pragma clang fp contract(off)
+  if (w >= 0.0f) {
+    a.tw += w;
+    a.dx = fmaf(w, v.x, a.dx);
+    a.dy = fmaf(w, v.y, a.dy);
+    a.dz = fmaf(w, v.z, a.dz);
+  }
+}
+
 // v_new = v_old/(1+b) + (sum w v_j / sum w) b/(1+b) from the total sums t; the
 // last iteration writes positions and velocities back to original order.
 __device__ __forceinline__ void vis_finish(int s, float4 xi, VisSums t, const float4* __restrict__ v_old,
@@ -299,25 +319,124 @@ __device__ __forceinline__ void swap_if(bool c, VisSums& a, VisSums& b) {
   swap_if(c, a.dz, b.dz);
 }
 
+// The entries of parity h of s's list added to t, in order. Positions stay as
+// they are over the iterations, and so do the weights: the first iteration
+// writes them (wt: a float4 for a lane's four entries of a list chunk, a chunk's
+// 128 lanes together) and the others read those 16 bytes instead of gathering
+// four positions. Returns false, with nothing run, when s's wave has no 16-bit
+// or staged list.
+template <VisWeights kW>
+__device__ __forceinline__ bool vis_half(const NbrView& nv, int s, int h, float4 xi, const float4* __restrict__ xs,
+                                         const float4* __restrict__ v_in, float4* __restrict__ wt,
+                                         const VisConst& vc, VisSums& t) {
+  const int wave = __builtin_amdgcn_readfirstlane(s >> 6);
+  ListHead head;
+  head.load(nv, wave, s);
+  const WaveList& wl = head.wl;
+  const int mode = wl.lm & 3;
+  if (wl.lb < 0 || (mode != kListDelta16 && mode != kListStaged)) return false;
+  const int past = s * 16;
+  auto gather = [&](int o) {
+    if constexpr (kW == kVisRead)
+      return record_at(v_in, o);
+    else
+      return VisPair{record_at(xs, o), record_at(v_in, o)};
+  };
+  using T = decltype(gather(0));
+  auto part = [&](int ch, uint4 first, uint4 second, const uint4* L, float4* W, auto&& decode) {
+    const int nc = (ch + 3) >> 2;
+    if (nc == 0) return;
+    Group4 g0, g1;
+    T a0[4], a1[4];
+    float4 w0, w1;
+    uint4 e = first;
+    if (kW == kVisRead) w0 = W[0];
+    g0 = decode(e, 0);
+#pragma unroll
+    for (int u = 0; u < 4; ++u) a0[u] = gather(g0.j[u]);
+    e = second;
+    // chunk c is added while chunk c + 1 is gathered and chunk c + 2 read
+    auto step = [&](int c, const T(&ac)[4], const float4& wc, Group4& gx, T(&ax)[4], float4& wx) {
+      gx = decode(e, c + 1);
+      if (kW == kVisRead) wx = W[(size_t)min(c + 1, nc - 1) << 7];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) ax[u] = gather(gx.j[u]);
+      e = L[(long long)min(c + 2, nc - 1) << 6];
+      asm volatile("" ::: "memory");  // keep the loads above in this step
+      if constexpr (kW == kVisRead) {
+        const float w[4] = {wc.x, wc.y, wc.z, wc.w};
+#pragma unroll
+        for (int u = 0; u < 4; ++u) vis_add(t, w[u], ac[u]);
+      } else {
+        float w[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+          w[u] = 4 * c + u < ch ? vis_weight(xi, ac[u].x, vc) : kVisSkip;
+          vis_add(t, w[u], ac[u].v);
+        }
+        W[(size_t)c << 7] = make_float4(w[0], w[1], w[2], w[3]);
+      }
+    };
+    for (int c = 0; c < nc; c += 2) {
+      step(c, a0, w0, g1, a1, w1);
+      if (c + 1 >= nc) break;
+      step(c + 1, a1, w1, g0, a0, w0);
+    }
+  };
+  float4* W = wt + ((size_t)wave * (size_t)(nv.list_per >> 3) << 7) + (2 * (s & 63) + h);
+  const uint32_t base = (uint32_t)wl.jb << 4, sh = (uint32_t)h << 4;
+  const uint4* L = head.L;
+  if (mode == kListDelta16) {
+    const int ch = (head.cnt - h + 1) >> 1;
+    part(ch, head.c0, head.c1, L, W, [&](uint4 e, int c) { return decode_half<false, 16>(e, sh, base, c, ch, past); });
+    return true;
+  }
+  // as for_each_record_half
+  const int* st = nv.stage + kStageInts * wave;
+  StageMap m;
+  m.load(st);
+  const int ka = st[7], ca = nv.cnt_a[s], cb = head.cnt - ca;
+  const int c1 = (ca - h + 1) >> 1;
+  part(c1, head.c0, head.c1, L, W, [&](uint4 e, int c) { return decode_half_staged<16>(e, sh, m, c, c1, past); });
+  const int hh = h ^ (ca & 1), ch = (cb - hh + 1) >> 1;
+  const uint32_t sh2 = (uint32_t)hh << 4;
+  const uint4* L2 = L + ((long long)(ka >> 3) << 6);
+  if (ch > 0)
+    part(ch, L2[0], L2[ch > 4 ? 64 : 0], L2, W + ((size_t)(ka >> 3) << 7),
+         [&](uint4 e, int c) { return decode_half<false, 16>(e, sh2, base, c, ch, past); });
+  return true;
+}
+
 // One Jacobi iteration (K_ApplyViscosity, ImplicitViscosity.cu:20-62) in
 // sorted order over the step's lists, the sums kept as one partial sum per
 // entry parity in the neighbor order (as the PBD passes). kPair: thread g
 // takes entry parity g & 1 of particle g >> 1 (a lane pair per particle, for
 // small searches; waves with 32-bit lists or none run the list on the even
-// lane); both forms give the same bits.
-template <bool kPair>
+// lane), with the weights kept over the iterations where kW says so; all forms
+// give the same bits. At 100,000 particles 18.0 us an iteration without the
+// weights; with them 22.5 the first and 14.0 the others, where four gathers of
+// twelve bytes and sixteen bytes of weights remain for four entries.
+template <bool kPair, VisWeights kW>
 __global__ __launch_bounds__(kBlock) void k_viscosity(NbrView nv, const float4* __restrict__ xs,
                                                       const float4* __restrict__ v_old,
                                                       const float4* __restrict__ v_in, float4* __restrict__ v_next,
                                                       VisConst vc, const int* __restrict__ perm,
-                                                      float* __restrict__ x_out, float* __restrict__ v_out) {
+                                                      float* __restrict__ x_out, float* __restrict__ v_out,
+                                                      float4* __restrict__ wt) {
   const int g = particle_block(nv) * blockDim.x + threadIdx.x;
   const int s = kPair ? g >> 1 : g, h = kPair ? g & 1 : 0;
   if (s >= nv.n) return;
   const float4 xi = xs[s];
   auto gather = [&](int o) { return VisPair{record_at(xs, o), record_at(v_in, o)}; };
   VisSums t;
-  if (kPair && for_each_record_half<16>(nv, s, h, gather, [&](int, const VisPair& q) { vis_term(t, xi, q, vc); })) {
+  bool done = false;
+  if constexpr (kPair) {
+    if constexpr (kW == kVisNone)
+      done = for_each_record_half<16>(nv, s, h, gather, [&](int, const VisPair& q) { vis_term(t, xi, q, vc); });
+    else
+      done = vis_half<kW>(nv, s, h, xi, xs, v_in, wt, vc, t);
+  }
+  if (done) {
     VisSums o;
     o.tw = __shfl_xor(t.tw, 1);
     o.dx = __shfl_xor(t.dx, 1);
@@ -336,13 +455,20 @@ __global__ __launch_bounds__(kBlock) void k_viscosity(NbrView nv, const float4* 
 }
 
 void launch_viscosity(const NbrView& nv, const float4* xs, const float4* v_old, const float4* v_in, float4* v_next,
-                      const VisConst& vc, const int* perm, float* x_out, float* v_out, hipStream_t st, int lanes) {
-  if (lanes == 2)
-    k_viscosity<true><<<(int)((2ll * nv.n + kBlock - 1) / kBlock), kBlock, 0, st>>>(nv, xs, v_old, v_in, v_next, vc,
-                                                                                    perm, x_out, v_out);
+                      const VisConst& vc, const int* perm, float* x_out, float* v_out, hipStream_t st, int lanes,
+                      float4* wt, bool first) {
+  const int blocks = (int)(((long long)lanes * nv.n + kBlock - 1) / kBlock);
+  auto run = [&](auto* kernel) {
+    kernel<<<blocks, kBlock, 0, st>>>(nv, xs, v_old, v_in, v_next, vc, perm, x_out, v_out, wt);
+  };
+  if (lanes != 2)
+    run(k_viscosity<false, kVisNone>);
+  else if (!wt)
+    run(k_viscosity<true, kVisNone>);
+  else if (first)
+    run(k_viscosity<true, kVisWrite>);
   else
-    k_viscosity<false><<<(nv.n + kBlock - 1) / kBlock, kBlock, 0, st>>>(nv, xs, v_old, v_in, v_next, vc, perm, x_out,
-                                                                        v_out);
+    run(k_viscosity<true, kVisRead>);
 }
 
 // Module path: one iteration over a caller CSR list in original order

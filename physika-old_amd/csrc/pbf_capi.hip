@@ -181,6 +181,9 @@ struct pbf_ctx {
   hipEvent_t counters_ev = nullptr;
   bool counters_pending = false;
 
+  float4* vis_w = nullptr;  // weights of a viscosity solve (vis_weights)
+  size_t vis_cap = 0;
+
   int last_n = -1;  // particle count of the last neighbor search (-1: none)
   // its list elements once cnt_orig holds their row starts (-1: not yet), and
   // C_CALLS then: a replay of a captured call searches without the host
@@ -938,6 +941,37 @@ int pass_lanes_for(const pbf_ctx* c, int n) {
   return (!stages_lists(c, n) || n <= PBF_TWO_LANE_MAX_PARTICLES) ? 2 : 1;
 }
 
+// Room for the weights of a viscosity solve over n particles, or null: a search
+// of more than kVisWeightsMax (100 MB and more, which no cache holds between the
+// iterations), a capture that would have to allocate, or no memory.
+constexpr int kVisWeightsMax = 1 << 18;
+float4* vis_weights(pbf_ctx* c, int n, hipStream_t st) {
+  if (n > kVisWeightsMax) return nullptr;
+  const size_t need = vis_weight_entries(n, list_per_of(c));
+  if (need > c->vis_cap) {
+    if (capturing(st)) return nullptr;
+    dfree(c->vis_w);
+    c->vis_cap = 0;
+    c->gen++;
+    const size_t want = vis_weight_entries(std::min(c->cap_n, kVisWeightsMax), list_per_of(c));
+    if (hipMalloc(&c->vis_w, sizeof(float4) * std::max(want, need)) != hipSuccess) {
+      (void)hipGetLastError();
+      c->vis_w = nullptr;
+      return nullptr;
+    }
+    c->vis_cap = std::max(want, need);
+  }
+  return c->vis_w;
+}
+
+// Buffers for every call over n particles in nscenes scenes.
+int reserve(pbf_ctx* c, int n, int nscenes) {
+  const int s = ensure_particles(c, n, nscenes);
+  if (!s && (c->p.flags & PBF_FLAG_VISCOSITY) && c->p.viscosity_iterations > 1 && pass_lanes_for(c, n) == 2)
+    (void)vis_weights(c, n, nullptr);
+  return s;
+}
+
 // One fused step on a batch of scenes (scene_off: device offsets): the state
 // (x_in, v_in) advances into (x_out, v_out), which may alias the inputs. With
 // a tape (P: K iterate arrays, P[0] = the integrated positions; aux: K arrays)
@@ -1006,11 +1040,12 @@ int step_once(pbf_ctx* c, const float* x_in, const float* v_in, float* x_out, fl
     const float4* v_old = K == 0 ? c->vs : c->vv;
     float4* V[2] = {K == 0 ? c->xa : bufs[K & 1], K == 0 ? c->xb : c->x0};
     const int T = c->p.viscosity_iterations;
+    float4* wt = T > 1 && lanes == 2 ? vis_weights(c, n, st) : nullptr;
     for (int t = 0; t < T; ++t) {
       const bool last = t + 1 == T;
       const float4* vin = t == 0 ? v_old : V[(t - 1) & 1];
       launch_viscosity(nv, xk, v_old, vin, last ? nullptr : V[t & 1], c->vc, c->perm, last ? x_out : nullptr,
-                       last ? v_out : nullptr, st, lanes);
+                       last ? v_out : nullptr, st, lanes, wt, t == 0);
     }
   }
   PBF_LAUNCHED(c);
@@ -1427,6 +1462,7 @@ int pbf_destroy(pbf_ctx* c) {
   dfree(c->key); dfree(c->slot); dfree(c->tmp); dfree(c->perm); dfree(c->inv);
   dfree(c->sid); dfree(c->ssid); dfree(c->bpart); dfree(c->nbr_cnt); dfree(c->cnt_orig);
   dfree(c->tid); dfree(c->pid);
+  dfree(c->vis_w);
   dfree(c->xn); dfree(c->x0); dfree(c->xa); dfree(c->xb); dfree(c->vs); dfree(c->vv); dfree(c->xc);
   dfree(c->mask_base); dfree(c->list_base); dfree(c->list_jbase); dfree(c->list_mode);
   dfree(c->stage); dfree(c->cnt_a); dfree(c->wave_stat); dfree(c->oog_rcnt); dfree(c->oog_rev);
@@ -1482,12 +1518,12 @@ int pbf_get_params(const pbf_ctx* c, pbf_params* out) {
 
 int pbf_reserve(pbf_ctx* c, int n) {
   if (!c || bad_n(n)) return fail(c, PBF_ERR_INVALID, "bad particle count");
-  return ensure_particles(c, n, 1);
+  return reserve(c, n, 1);
 }
 
 int pbf_reserve_batch(pbf_ctx* c, int n, int nscenes) {
   if (!c || bad_n(n) || nscenes < 1) return fail(c, PBF_ERR_INVALID, "bad particle or scene count");
-  return ensure_particles(c, n, nscenes);
+  return reserve(c, n, nscenes);
 }
 
 int pbf_neighbor_query(pbf_ctx* c, const float* d_x, int n, int* d_index, int* d_elems, long long cap,

@@ -338,8 +338,12 @@ void launch_box_sdf(const BoxField& f, const float lo[3], const float hi[3], hip
 void launch_box_constrain(const BoxField& f, const float* x_in, const float* v_in, float* x_out, float* v_out, int n,
                           const int* scene_off, int nscenes, float keep_normal, float damp, hipStream_t st);
 // lanes: 1, or 2 for a lane pair per particle (same results)
+// wt: room for the weights of a lane pair's entries over a solve's iterations
+// (vis_weight_entries float4), or null; first: the solve's first iteration.
 void launch_viscosity(const NbrView& nv, const float4* xs, const float4* v_old, const float4* v_in, float4* v_next,
-                      const VisConst& vc, const int* perm, float* x_out, float* v_out, hipStream_t st, int lanes = 1);
+                      const VisConst& vc, const int* perm, float* x_out, float* v_out, hipStream_t st, int lanes,
+                      float4* wt, bool first);
+inline size_t vis_weight_entries(int n, int list_per) { return (size_t)((n + 63) / 64) * (size_t)(list_per >> 3) * 128; }
 void launch_csr_viscosity(const float4* xa, const Csr& nb, const float4* v_old, const float4* v_in, float4* v_next,
                           float* v_out, const VisConst& vc, hipStream_t st);
 
