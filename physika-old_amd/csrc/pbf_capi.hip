@@ -830,7 +830,8 @@ int record_counters(pbf_ctx* c, hipStream_t st) {
     c->captured = true;
     c->tape_of = 0;
   }
-  launch_wave_stats(c->wave_stat, c->stats_n, c->counters, c->h_counters_dev, st);
+  // a reverse that started from a recorded segment alone searched nothing
+  if (c->stats_n > 0) launch_wave_stats(c->wave_stat, c->stats_n, c->counters, c->h_counters_dev, st);
   c->stats_n = 0;
   PBF_LAUNCHED(c);
   PBF_HIP(c, hipEventRecord(c->counters_ev, st));

@@ -72,10 +72,13 @@ def test_recorded_forward(fluid, scene, double, nsteps, every, between):
         fresh = fluid.Context("cuda:0")
         x, v, token = forward(fresh, x0, double, nsteps, every)
         want = [x, v, *lists(fresh), *reverse(fresh, x, token)]
+        pairs = fresh.stats()["neighbor_pairs"]
         x, v, token = forward(ctx, x0, double, nsteps, every)
         got = [x, v, *lists(ctx)]
         BETWEEN[between](ctx, scene, double)
         got += reverse(ctx, x, token)
+        if between in ("nothing", "lists"):
+            assert ctx.stats()["neighbor_pairs"] == pairs > 0
         again = reverse(ctx, x, token)
         for a, b in zip(got + list(again), want + want[-2:]):
             np.testing.assert_array_equal(a.cpu().numpy(), b.cpu().numpy())
