@@ -822,7 +822,9 @@ int search(pbf_ctx* c, const float* x, const float* v, int n, const int* scene_o
 
 bool capturing(hipStream_t st) {
   hipStreamCaptureStatus s = hipStreamCaptureStatusNone;
-  return hipStreamIsCapturing(st, &s) == hipSuccess && s != hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(st, &s) == hipSuccess) return s != hipStreamCaptureStatusNone;
+  (void)hipGetLastError();
+  return true;  // not known: nothing that a capture would not allow
 }
 
 int record_counters(pbf_ctx* c, hipStream_t st) {
