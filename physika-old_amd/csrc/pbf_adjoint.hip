@@ -259,14 +259,14 @@ void launch_adjoint_step(const NbrView& nv, float4* const* P, float4* const* aux
                          const int* perm, float* xbar, float* vbar, const AdjBufs& ab, hipStream_t st, int lanes) {
   const int n = nv.n;
   const int nb = (n + kBlock - 1) / kBlock;
-  const int nb2 = (int)((2ll * n + kBlock - 1) / kBlock);
+  const int nb2 = (int)((2ll * n + kPairBlock - 1) / kPairBlock);
   k_adj_begin<<<nb, kBlock, 0, st>>>(n, perm, xbar, vbar, pc.dt, ab.e, ab.c, ab.f, ab.vsb, nv.counters, ab.flag);
   float4* e = ab.e;
   float4* e2 = ab.e2;
   for (int k = K - 1; k >= 0; --k) {
     if (lanes == 2) {
-      k_adj_lambda2<<<nb2, kBlock, 0, st>>>(nv, P[k], aux[k], ab.f, ab.q1, ab.q2, pc);
-      k_adj_pos2<<<nb2, kBlock, 0, st>>>(nv, P[k], ab.q1, ab.q2, e, ab.c, e2, ab.f, pc);
+      k_adj_lambda2<<<nb2, kPairBlock, 0, st>>>(nv, P[k], aux[k], ab.f, ab.q1, ab.q2, pc);
+      k_adj_pos2<<<nb2, kPairBlock, 0, st>>>(nv, P[k], ab.q1, ab.q2, e, ab.c, e2, ab.f, pc);
     } else {
       k_adj_lambda<<<nb, kBlock, 0, st>>>(nv, P[k], aux[k], ab.f, ab.q1, ab.q2, pc);
       k_adj_pos<<<nb, kBlock, 0, st>>>(nv, P[k], ab.q1, ab.q2, e, ab.c, e2, ab.f, pc);

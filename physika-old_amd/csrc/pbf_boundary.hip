@@ -457,9 +457,10 @@ __global__ __launch_bounds__(kBlock) void k_viscosity(NbrView nv, const float4* 
 void launch_viscosity(const NbrView& nv, const float4* xs, const float4* v_old, const float4* v_in, float4* v_next,
                       const VisConst& vc, const int* perm, float* x_out, float* v_out, hipStream_t st, int lanes,
                       float4* wt, bool first) {
-  const int blocks = (int)(((long long)lanes * nv.n + kBlock - 1) / kBlock);
+  const int block = lanes == 2 ? kPairBlock : kBlock;
+  const int blocks = (int)(((long long)lanes * nv.n + block - 1) / block);
   auto run = [&](auto* kernel) {
-    kernel<<<blocks, kBlock, 0, st>>>(nv, xs, v_old, v_in, v_next, vc, perm, x_out, v_out, wt);
+    kernel<<<blocks, block, 0, st>>>(nv, xs, v_old, v_in, v_next, vc, perm, x_out, v_out, wt);
   };
   if (lanes != 2)
     run(k_viscosity<false, kVisNone>);

@@ -975,6 +975,12 @@ int reserve(pbf_ctx* c, int n, int nscenes) {
   return s;
 }
 
+// Threads per workgroup of the PBD passes: the context's setting, where the
+// default leaves lane pairs at kPairBlock.
+int pass_block_for(const pbf_ctx* c, int lanes) {
+  return lanes == 2 && c->pass_block == kBlock ? kPairBlock : c->pass_block;
+}
+
 // One fused step on a batch of scenes (scene_off: device offsets): the state
 // (x_in, v_in) advances into (x_out, v_out), which may alias the inputs. With
 // a tape (P: K iterate arrays, P[0] = the integrated positions; aux: K arrays)
@@ -1012,6 +1018,7 @@ int step_once(pbf_ctx* c, const float* x_in, const float* v_in, float* x_out, fl
   if (s) return s;
   NbrView nv = view_of(c, n);
   const int lanes = pass_lanes_for(c, n);
+  const int block = pass_block_for(c, lanes);
   c->last_lanes = lanes;
   float4* bufs[2] = {c->xa, c->xb};
   if (K == 0 && !visc) launch_write_back(c->x0, c->vs, c->perm, n, x_out, v_out, st);
@@ -1022,17 +1029,17 @@ int step_once(pbf_ctx* c, const float* x_in, const float* v_in, float* x_out, fl
     {
       PassTimer t(c, PBF_PASS_DENSITY_LAMBDA, st, true);
       launch_pass_density_lambda(nv, src, c->pc, last ? d_rho : nullptr, c->perm, st, aux ? aux[it] : nullptr,
-                                 c->pass_block, c->pass_persistent, lanes, t.events());
+                                 block, c->pass_persistent, lanes, t.events());
     }
     {
       PassTimer t(c, PBF_PASS_DISPLACEMENT, st, true);
       if (last && to) {
         launch_pass_displacement(nv, src, dst, c->pc, true, c->x0, c->vs, c->perm, nullptr, nullptr, st, c->vv,
-                                 c->pid, c->pass_block, c->pass_persistent, lanes, t.events());
+                                 c->pid, block, c->pass_persistent, lanes, t.events());
         *to = CellState{dst, c->vv, c->pid};
       } else {
         launch_pass_displacement(nv, src, dst, c->pc, last, c->x0, c->vs, c->perm, x_out, v_out, st,
-                                 (last && visc) ? c->vv : nullptr, nullptr, c->pass_block, c->pass_persistent,
+                                 (last && visc) ? c->vv : nullptr, nullptr, block, c->pass_persistent,
                                  lanes, t.events());
       }
     }

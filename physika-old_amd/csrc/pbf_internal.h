@@ -268,6 +268,15 @@ void launch_neighbors(const NbrView& nv, const NbrOut& out, unsigned long long* 
 // all counters to host (mapped host memory).
 void launch_wave_stats(const int4* wave_stat, int n, unsigned long long* counters, unsigned long long* host,
                        hipStream_t st);
+// Threads per workgroup of the kernels that run a lane pair per particle: their
+// searches fill the chip with few rounds of workgroups, and the last round is
+// nearly empty where 256 threads go together. 100,003 particles are 782
+// workgroups of 256 threads, four on some CUs and three on most, or 3,126 of
+// 64, twelve or thirteen. Four frames there (box, viscosity) 1,048 -> 999 us with
+// the PBD passes alone (128 threads 1,010) and 963 with the viscosity; 20 frames at
+// 32,768 2,013 -> 1,986; a frame at 1,728 95.5 -> 93.1; four steps and gradient in
+// double at 8 x 5,000 2.47 -> 2.12 ms. One lane per particle (1M): 64, 128 and 256 alike.
+constexpr int kPairBlock = 64;
 // block: threads per workgroup, 64, 128, 256 or 512; persistent: as many
 // blocks as stay resident, each wave walking 64-particle tiles; lanes: 1, or 2
 // for a lane pair per particle (not persistent). The results depend on none of

@@ -362,7 +362,7 @@ void launch64_round(const double* x, float* xf, int n, hipStream_t st) {
 void launch64_step(const NbrView& nv, const int* perm, const double* x_in, const double* v_in, double* x_out,
                    double* v_out, double* rho, double4* const* P, double4* const* aux, int K, double4* vs,
                    const PhysConst64& pc, const unsigned long long* counters, int* flag, hipStream_t st, int lanes) {
-  const int n = nv.n, nb = blocks_of(n), nbp = (int)((2ll * n + kBlock - 1) / kBlock);
+  const int n = nv.n, nb = blocks_of(n), nbp = (int)((2ll * n + kPairBlock - 1) / kPairBlock);
   k64_begin<<<nb, kBlock, 0, st>>>(n, perm, x_in, v_in, pc, P[0], vs, counters, flag);
   if (K == 0) {
     k64_write<<<nb, kBlock, 0, st>>>(n, perm, P[0], vs, x_out, v_out);
@@ -371,9 +371,9 @@ void launch64_step(const NbrView& nv, const int* perm, const double* x_in, const
   for (int k = 0; k < K; ++k) {
     const bool last = k + 1 == K;
     if (lanes == 2) {
-      k64_density_lambda<true><<<nbp, kBlock, 0, st>>>(nv, P[k], pc, aux ? aux[k] : nullptr, last ? rho : nullptr,
+      k64_density_lambda<true><<<nbp, kPairBlock, 0, st>>>(nv, P[k], pc, aux ? aux[k] : nullptr, last ? rho : nullptr,
                                                        perm);
-      k64_displacement<true><<<nbp, kBlock, 0, st>>>(nv, P[k], last ? nullptr : P[k + 1], pc, last ? 1 : 0, P[0], vs,
+      k64_displacement<true><<<nbp, kPairBlock, 0, st>>>(nv, P[k], last ? nullptr : P[k + 1], pc, last ? 1 : 0, P[0], vs,
                                                      perm, x_out, v_out);
     } else {
       k64_density_lambda<false><<<nb, kBlock, 0, st>>>(nv, P[k], pc, aux ? aux[k] : nullptr, last ? rho : nullptr,
@@ -387,14 +387,14 @@ void launch64_step(const NbrView& nv, const int* perm, const double* x_in, const
 void launch64_adjoint_step(const NbrView& nv, double4* const* P, double4* const* aux, int K, const PhysConst64& pc,
                            const int* perm, double* xbar, double* vbar, const AdjBufs64& ab, hipStream_t st,
                            int lanes) {
-  const int n = nv.n, nb = blocks_of(n), nbp = (int)((2ll * n + kBlock - 1) / kBlock);
+  const int n = nv.n, nb = blocks_of(n), nbp = (int)((2ll * n + kPairBlock - 1) / kPairBlock);
   k64_adj_begin<<<nb, kBlock, 0, st>>>(n, perm, xbar, vbar, pc.dt, ab.e, ab.c, ab.f, ab.vsb);
   double4* e = ab.e;
   double4* e2 = ab.e2;
   for (int k = K - 1; k >= 0; --k) {
     if (lanes == 2) {
-      k64_adj_lambda<true><<<nbp, kBlock, 0, st>>>(nv, P[k], aux[k], ab.f, ab.q1, ab.q2, pc);
-      k64_adj_pos<true><<<nbp, kBlock, 0, st>>>(nv, P[k], ab.q1, ab.q2, e, ab.c, e2, ab.f, pc);
+      k64_adj_lambda<true><<<nbp, kPairBlock, 0, st>>>(nv, P[k], aux[k], ab.f, ab.q1, ab.q2, pc);
+      k64_adj_pos<true><<<nbp, kPairBlock, 0, st>>>(nv, P[k], ab.q1, ab.q2, e, ab.c, e2, ab.f, pc);
     } else {
       k64_adj_lambda<false><<<nb, kBlock, 0, st>>>(nv, P[k], aux[k], ab.f, ab.q1, ab.q2, pc);
       k64_adj_pos<false><<<nb, kBlock, 0, st>>>(nv, P[k], ab.q1, ab.q2, e, ab.c, e2, ab.f, pc);
