@@ -475,12 +475,13 @@ void launch_viscosity(const NbrView& nv, const float4* xs, const float4* v_old, 
 // Module path: one iteration over a caller CSR list in original order
 // (positions xa as float4; v_old, v_in float4; the last iteration writes the
 // caller's packed velocities).
-__global__ __launch_bounds__(kBlock) void k_csr_viscosity(const float4* __restrict__ xa, Csr nb,
+template <int kThreads>
+__global__ __launch_bounds__(kThreads) void k_csr_viscosity(const float4* __restrict__ xa, Csr nb,
                                                           const float4* __restrict__ v_old,
                                                           const float4* __restrict__ v_in,
                                                           float4* __restrict__ v_next, float* __restrict__ v_out,
                                                           VisConst vc) {
-  const CsrRow row = csr_row(nb);
+  const CsrRow row = csr_row<kThreads>(nb);
   if (row.i >= nb.n) return;
   const int i = row.i;
   const float4 xi = xa[i];
@@ -521,7 +522,13 @@ __global__ __launch_bounds__(kBlock) void k_csr_viscosity(const float4* __restri
 
 void launch_csr_viscosity(const float4* xa, const Csr& nb, const float4* v_old, const float4* v_in, float4* v_next,
                           float* v_out, const VisConst& vc, hipStream_t st) {
-  k_csr_viscosity<<<csr_blocks(nb.n), kBlock, 0, st>>>(xa, nb, v_old, v_in, v_next, v_out, vc);
+  // few rows: workgroups of 64 threads (see kPairBlock). Five iterations, us: 33.9 ->
+  // 29.2 at 2,000 rows, 74.7 -> 68.0 at 50,000, 90.4 -> 86.6 at 70,000, but 158.6 ->
+  // 165.5 at 131,072
+  if (nb.n <= 65536)
+    k_csr_viscosity<64><<<csr_blocks(nb.n, 64), 64, 0, st>>>(xa, nb, v_old, v_in, v_next, v_out, vc);
+  else
+    k_csr_viscosity<kBlock><<<csr_blocks(nb.n), kBlock, 0, st>>>(xa, nb, v_old, v_in, v_next, v_out, vc);
 }
 
 }  // namespace pbf

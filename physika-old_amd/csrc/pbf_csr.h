@@ -23,8 +23,9 @@ struct CsrRow {
 
 // The row of this thread in a launch over the rows from `first` on; blocks of
 // neighboring rows run on one XCD.
+template <int kThreads = kBlock>
 __device__ __forceinline__ CsrRow csr_row(const Csr& nb, int first = 0) {
-  const long long g = (long long)xcd_block(blockIdx.x, gridDim.x) * kBlock + threadIdx.x;
+  const long long g = (long long)xcd_block(blockIdx.x, gridDim.x) * kThreads + threadIdx.x;
   const long long i = first + g / kRowLanes;
   return CsrRow{i < nb.n ? (int)i : nb.n, (int)(g % kRowLanes)};
 }
@@ -32,7 +33,9 @@ __device__ __forceinline__ CsrRow csr_row(const Csr& nb, int first = 0) {
 // Blocks of a launch over `rows` rows, at most kRowsPerLaunch (a grid holds
 // fewer than 2^32 threads).
 constexpr int kRowsPerLaunch = 1 << 28;
-inline int csr_blocks(int rows) { return (int)(((long long)rows * kRowLanes + kBlock - 1) / kBlock); }
+inline int csr_blocks(int rows, int block = kBlock) {
+  return (int)(((long long)rows * kRowLanes + block - 1) / block);
+}
 
 typedef int i4u __attribute__((ext_vector_type(4), aligned(4)));
 

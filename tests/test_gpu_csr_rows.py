@@ -192,3 +192,21 @@ def test_limited_rows_and_export(fluid, scene, storage, spacing):
             assert (el[k * i + counts[i]:k * (i + 1)] == -1).all()
     say(f"limited rows and export, {storage}, spacing {spacing}: {n} particles, rows of up to {longest}")
     assert longest > (128 if spacing < 0.005 else 32)
+
+
+def test_viscosity_workgroup_sizes(fluid, scene):
+    """65,536 rows (workgroups of 64 threads) and the same with one isolated
+    particle more (256): the same bits for the rows they share."""
+    say("viscosity over 65,536 and 65,537 rows")
+    x = scene.jittered_lattice((64, 32, 32), (0.2, 0.3, 0.2), 0.005, 0.1, seed=3)
+    n = len(x)
+    v = (0.5 * (scene.uniform01(4, 3 * n).reshape(n, 3) - 0.5)).astype(np.float32)
+    outs = []
+    for extra in (0, 1):
+        xa = np.concatenate([x, np.full((extra, 3), 0.9, np.float32)])
+        va = np.concatenate([v, np.zeros((extra, 3), np.float32)])
+        ctx = fluid.Context("cuda:0")
+        xd, vd = dev(xa), dev(va)
+        ctx.viscosity(xd, vd, ctx.neighbor_query(xd))
+        outs.append(vd.cpu().numpy()[:n].view(np.uint32))
+    np.testing.assert_array_equal(*outs)
