@@ -71,6 +71,9 @@ struct pbf_ctx {
   long long mask_cap = 0;  // words
   uint16_t* list = nullptr;
   long long list_cap = 0;  // 16-bit slots
+  // in place of a list whose allocation failed (list_per is 0 then): kListPad
+  // slots, what a lane pair reads before it knows that its wave has no list
+  uint16_t* list_none = nullptr;
   long long auto_list_per = 96;  // automatic list reservation, 16-bit slots per particle
   int4* wave_stat = nullptr;     // per wave of the neighbor pass: pairs, candidates, need
   int stats_n = 0;               // particles of the last search whose statistics are not yet reduced
@@ -559,6 +562,7 @@ int ensure_particles(pbf_ctx* c, int n, int nscenes) {
   dfree(c->stage); dfree(c->cnt_a); dfree(c->wave_stat); dfree(c->oog_rcnt); dfree(c->oog_rev);
   dfree(c->oog_flag); dfree(c->oog_pre);
   c->cap_n = 0;
+  c->last_n = -1;  // the last search's lists went with the arrays
   const size_t ni = sizeof(int) * (size_t)cap, nf4 = sizeof(float4) * (size_t)cap;
   PBF_HIP(c, hipMalloc(&c->key, ni));
   PBF_HIP(c, hipMalloc(&c->slot, ni));
@@ -595,10 +599,7 @@ int ensure_particles(pbf_ctx* c, int n, int nscenes) {
   c->cap_n = cap;
   st = ensure_mask(c, mask_words_for(c, cap));
   if (st) return st;
-  st = ensure_list(c, list_slots_for(c, cap));
-  if (st) return st;
-  c->last_n = -1;
-  return PBF_OK;
+  return ensure_list(c, list_slots_for(c, cap));
 }
 
 // Grows the mask and list reservations when the last finished call wanted
@@ -639,7 +640,7 @@ NbrView view_of(const pbf_ctx* c, int n) {
   nv.cnt_a = c->cnt_a;
   nv.oog_rcnt = c->oog_rcnt;
   nv.oog_rev = c->oog_rev;
-  nv.list = c->list;
+  nv.list = c->list ? c->list : c->list_none;
   nv.mask_base = c->mask_base;
   nv.mask = c->mask;
   nv.counters = c->counters;
@@ -663,7 +664,7 @@ NbrOut out_of(pbf_ctx* c) {
   NbrOut o;
   o.mask = c->mask;
   o.mask_cap = c->mask_cap;
-  o.list = c->list;
+  o.list = c->list ? c->list : c->list_none;
   o.list_per = list_per_of(c);
   o.mask_base = c->mask_base;
   o.list_base = c->list_base;
@@ -1443,6 +1444,7 @@ int pbf_create(const pbf_params* p, pbf_ctx** out) {
       hipMalloc(&c->total_cells, sizeof(int)) != hipSuccess ||
       hipMalloc(&c->scan_part, sizeof(int) * 2 * kScanDevBlocks) != hipSuccess ||
       hipMalloc(&c->ticket, sizeof(int)) != hipSuccess || hipMemset(c->ticket, 0, sizeof(int)) != hipSuccess ||
+      hipMalloc(&c->list_none, sizeof(uint16_t) * kListPad) != hipSuccess ||
       hipMalloc(&c->pairing, sizeof(unsigned long long) * kPairingSlots) != hipSuccess) {
     pbf_destroy(c);
     return PBF_ERR_HIP;
@@ -1467,7 +1469,7 @@ int pbf_destroy(pbf_ctx* c) {
   if (!c) return PBF_ERR_INVALID;
   (void)hipDeviceSynchronize();
   dfree(c->scene_minmax); dfree(c->win); dfree(c->total_cells); dfree(c->scan_part);
-  dfree(c->pairing); dfree(c->ticket);
+  dfree(c->pairing); dfree(c->ticket); dfree(c->list_none);
   dfree(c->cell_cnt); dfree(c->cell_start);
   dfree(c->key); dfree(c->slot); dfree(c->tmp); dfree(c->perm); dfree(c->inv);
   dfree(c->sid); dfree(c->ssid); dfree(c->bpart); dfree(c->nbr_cnt); dfree(c->cnt_orig);

@@ -1,0 +1,415 @@
+// Host paths of libpbf.so without a GPU: this program defines the HIP runtime
+// calls that the library makes (its definitions come before libamdhip64's).
+// Device memory is host memory, kernels do not run, and every launch and copy is
+// checked: a pointer it hands over has to lie in a live allocation, and the
+// arrays of a neighbor view have to be as long as the kernels read them. A chosen
+// allocation can be made to fail, a stream to say that it is being captured, and
+// the counters of a call to report what the test wants. Run by
+// tests/test_host_paths.py with the name of a scenario; prints one line per
+// violation and exits 1 if there is any.
+#include <cxxabi.h>
+#include <hip/hip_runtime.h>
+
+#include <cstdarg>
+#include <cstdio>
+#include <cstdlib>
+#include <cstring>
+#include <functional>
+#include <map>
+#include <set>
+#include <string>
+#include <vector>
+
+#include "../../physika-old_amd/csrc/pbf_internal.h"
+#include "pbf.h"
+
+namespace {
+
+struct Kernel {
+  std::string name;                 // without template arguments and namespace
+  std::string full;                 // demangled
+  std::vector<std::string> params;  // types
+};
+
+struct Launch {
+  std::string name, full;
+  unsigned block;
+  pbf::NbrView nv;  // where the kernel's first parameter is one
+  bool view;
+};
+
+constexpr long kNever = -1000000;
+
+struct State {
+  std::map<const void*, Kernel> kernels;
+  std::map<const char*, size_t> live;
+  size_t bytes = 0, peak = 0;
+  long mallocs = 0, fail_at = kNever;  // fail_at: the malloc (0-based) that fails
+  size_t fail_over = SIZE_MAX;     // every malloc of more bytes fails
+  long failed = 0;
+  hipError_t last = hipSuccess;
+  int capturing = 0;        // hipStreamIsCapturing: 0 no, 1 yes, 2 an error
+  unsigned long long list_need = 0, calls = 0;
+  std::vector<Launch> launches;
+  std::vector<std::string> ops;  // launches, copies and waits, in order
+  std::map<const void*, long> searched;  // list buffer -> serial of the neighbor pass that last wrote it
+  long searches = 0, exported = -1;      // exported: the search that the last export read
+  dim3 grid, block;
+  size_t shared;
+  hipStream_t stream;
+  int violations = 0;
+};
+
+State& S() {
+  static State* s = new State();
+  return *s;
+}
+
+void violation(const char* fmt, ...) {
+  va_list a;
+  va_start(a, fmt);
+  std::printf("VIOLATION ");
+  std::vprintf(fmt, a);
+  std::printf("\n");
+  va_end(a);
+  ++S().violations;
+}
+
+// Bytes from p to the end of its live allocation (0: in none).
+size_t room(const void* p) {
+  auto it = S().live.upper_bound(static_cast<const char*>(p));
+  if (it == S().live.begin()) return 0;
+  --it;
+  const char* q = static_cast<const char*>(p);
+  return q < it->first + it->second ? (size_t)(it->first + it->second - q) : 0;
+}
+
+void need(const Kernel& k, const char* what, const void* p, size_t bytes) {
+  if (bytes > 0 && room(p) < bytes)
+    violation("%s: %s at %p needs %zu bytes, has %zu", k.name.c_str(), what, p, bytes, room(p));
+}
+
+void check_view(const Kernel& k, const pbf::NbrView& v) {
+  const size_t n = (size_t)v.n, waves = (n + 63) / 64;
+  need(k, "ssid", v.ssid, 4 * n);
+  need(k, "win", v.win, sizeof(pbf::SceneWin));
+  need(k, "cell_start", v.cell_start, 8);
+  need(k, "xn", v.xn, 16 * (n + pbf::kXnPad));
+  need(k, "nbr_cnt", v.nbr_cnt, 4 * n);
+  need(k, "cnt_a", v.cnt_a, 2 * n);
+  need(k, "list_base", v.list_base, 8 * waves);
+  need(k, "list_jbase", v.list_jbase, 4 * waves);
+  need(k, "list_mode", v.list_mode, 4 * waves);
+  need(k, "mask_base", v.mask_base, 8 * waves);
+  need(k, "stage", v.stage, sizeof(int) * pbf::kStageInts * waves);
+  need(k, "counters", v.counters, 8 * pbf::kDeviceCounters);
+  // the lists, and the two chunks that a lane pair reads ahead of the wave's words
+  need(k, "list", v.list, 2 * (64 * waves * (size_t)v.list_per + pbf::kListPad));
+}
+
+void launched(const void* f, dim3 block, void** args) {
+  const Kernel& k = S().kernels[f];
+  Launch l{k.name, k.full, block.x, {}, false};
+  for (size_t i = 0; i < k.params.size(); ++i) {
+    const std::string& t = k.params[i];
+    if (t == "pbf::NbrView") {
+      l.nv = *static_cast<pbf::NbrView*>(args[i]);
+      l.view = true;
+      check_view(k, l.nv);
+    } else if (!t.empty() && t.back() == '*') {
+      const void* p = *static_cast<void**>(args[i]);
+      if (p && room(p) == 0) violation("%s: argument %zu (%s) points at no allocation: %p", k.name.c_str(), i, t.c_str(), p);
+    }
+  }
+  S().launches.push_back(l);
+  S().ops.push_back(k.name);
+  if (S().capturing == 1) return;
+  if (k.name == "k_neighbors" || k.name == "k_neighbors_small") S().searched[l.nv.list] = S().searches++;
+  if (k.name == "k_csr_fill") S().exported = S().searched.count(l.nv.list) ? S().searched[l.nv.list] : -1;
+  if (k.name == "k_wave_stats") {  // the counters of the call
+    auto* host = *static_cast<unsigned long long**>(args[4]);
+    for (int c = 0; c < pbf::C_COUNT; ++c) host[c] = 0;
+    host[pbf::C_LIST_NEED] = S().list_need;
+    host[pbf::C_CALLS] = ++S().calls;
+  }
+}
+
+void copied(const void* dst, const void* src, size_t bytes, hipMemcpyKind kind) {
+  if (kind != hipMemcpyDeviceToHost && room(dst) < bytes) violation("copy of %zu bytes past its target", bytes);
+  if (kind != hipMemcpyHostToDevice && room(src) < bytes) violation("copy of %zu bytes past its source", bytes);
+  std::memmove(dst ? const_cast<void*>(dst) : nullptr, src, bytes);
+}
+
+Kernel parse(const char* mangled) {
+  int status = 0;
+  char* d = abi::__cxa_demangle(mangled, nullptr, nullptr, &status);
+  Kernel k;
+  k.full = status == 0 ? d : mangled;
+  std::free(d);
+  // parameters: the last balanced (...) of the text, split at its commas
+  size_t open = k.full.rfind(')');
+  int depth = 0;
+  for (; open != std::string::npos; --open) {
+    depth += k.full[open] == ')' ? 1 : (k.full[open] == '(' ? -1 : 0);
+    if (depth == 0 || open == 0) break;
+  }
+  std::string head = k.full.substr(0, open), arg;
+  depth = 0;
+  for (size_t i = open + 1; i + 1 < k.full.size(); ++i) {
+    const char c = k.full[i];
+    depth += c == '<' || c == '(' ? 1 : (c == '>' || c == ')' ? -1 : 0);
+    if (c == ',' && depth == 0) {
+      k.params.push_back(arg);
+      arg.clear();
+    } else if (!(c == ' ' && arg.empty())) {
+      arg += c;
+    }
+  }
+  if (!arg.empty()) k.params.push_back(arg);
+  head = head.substr(0, head.find('<'));
+  const size_t at = head.rfind(':');
+  k.name = at == std::string::npos ? head : head.substr(at + 1);
+  if (k.name.rfind("void ", 0) == 0) k.name = k.name.substr(5);
+  return k;
+}
+
+}  // namespace
+
+// -- the HIP runtime --------------------------------------------------------
+extern "C" {
+void** __hipRegisterFatBinary(const void*) {
+  static void* handle = nullptr;
+  return &handle;
+}
+void __hipUnregisterFatBinary(void**) {}
+void __hipRegisterFunction(void**, const void* f, char*, const char* name, unsigned, void*, void*, void*, void*, int*) {
+  S().kernels[f] = parse(name);
+}
+void __hipRegisterVar(void**, void*, char*, char*, int, size_t, int, int) {}
+hipError_t __hipPushCallConfiguration(dim3 g, dim3 b, size_t m, hipStream_t st) {
+  S().grid = g;
+  S().block = b;
+  S().shared = m;
+  S().stream = st;
+  return hipSuccess;
+}
+hipError_t __hipPopCallConfiguration(dim3* g, dim3* b, size_t* m, hipStream_t* st) {
+  *g = S().grid;
+  *b = S().block;
+  *m = S().shared;
+  *st = S().stream;
+  return hipSuccess;
+}
+hipError_t hipLaunchKernel(const void* f, dim3, dim3 b, void** args, size_t, hipStream_t) {
+  launched(f, b, args);
+  return hipSuccess;
+}
+hipError_t hipExtLaunchKernel(const void* f, dim3, dim3 b, void** args, size_t, hipStream_t, hipEvent_t, hipEvent_t,
+                              int) {
+  launched(f, b, args);
+  return hipSuccess;
+}
+hipError_t hipMalloc(void** p, size_t bytes) {
+  *p = nullptr;
+  const long k = S().mallocs++;
+  if (k == S().fail_at || bytes > S().fail_over) {
+    ++S().failed;
+    return S().last = hipErrorOutOfMemory;
+  }
+  *p = std::calloc(bytes ? bytes : 1, 1);
+  S().live[static_cast<char*>(*p)] = bytes;
+  S().bytes += bytes;
+  S().peak = std::max(S().peak, S().bytes);
+  return hipSuccess;
+}
+hipError_t hipFree(void* p) {
+  if (!p) return hipSuccess;
+  auto it = S().live.find(static_cast<char*>(p));
+  if (it == S().live.end()) {
+    violation("free of %p, which is no live allocation", p);
+    return hipErrorInvalidValue;
+  }
+  S().bytes -= it->second;
+  S().live.erase(it);
+  std::free(p);
+  return hipSuccess;
+}
+hipError_t hipHostMalloc(void** p, size_t bytes, unsigned) {
+  *p = std::calloc(bytes, 1);
+  S().live[static_cast<char*>(*p)] = bytes;
+  return hipSuccess;
+}
+hipError_t hipHostFree(void* p) {
+  if (!p) return hipSuccess;
+  S().live.erase(static_cast<char*>(p));
+  std::free(p);
+  return hipSuccess;
+}
+hipError_t hipHostGetDevicePointer(void** d, void* h, unsigned) {
+  *d = h;
+  return hipSuccess;
+}
+hipError_t hipGetSymbolAddress(void** p, const void*) {
+  return hipMalloc(p, 2 * (size_t)PBF_NOALLOC_MAX_PARTICLES * 16 + 4096);
+}
+hipError_t hipMemcpyAsync(void* d, const void* s, size_t bytes, hipMemcpyKind kind, hipStream_t) {
+  copied(d, s, bytes, kind);
+  S().ops.push_back("copy");
+  return hipSuccess;
+}
+hipError_t hipMemcpy(void* d, const void* s, size_t bytes, hipMemcpyKind kind) {
+  return hipMemcpyAsync(d, s, bytes, kind, nullptr);
+}
+hipError_t hipMemset(void* d, int v, size_t bytes) {
+  if (room(d) < bytes) violation("memset of %zu bytes past its target", bytes);
+  else std::memset(d, v, bytes);
+  return hipSuccess;
+}
+hipError_t hipMemsetAsync(void* d, int v, size_t bytes, hipStream_t) { return hipMemset(d, v, bytes); }
+hipError_t hipGetDevice(int* d) {
+  *d = 0;
+  return hipSuccess;
+}
+hipError_t hipGetDevicePropertiesR0600(hipDeviceProp_tR0600* p, int) {
+  std::memset(p, 0, sizeof(*p));
+  std::strcpy(p->gcnArchName, "host");
+  return hipSuccess;
+}
+hipError_t hipDeviceGetAttribute(int* v, hipDeviceAttribute_t, int) {
+  *v = 256;
+  return hipSuccess;
+}
+hipError_t hipOccupancyMaxActiveBlocksPerMultiprocessor(int* v, const void*, int, size_t) {
+  *v = 4;
+  return hipSuccess;
+}
+hipError_t hipDeviceSynchronize() { return hipSuccess; }
+hipError_t hipStreamSynchronize(hipStream_t) {
+  S().ops.push_back("wait");
+  return hipSuccess;
+}
+hipError_t hipStreamCreateWithFlags(hipStream_t* s, unsigned) {
+  *s = nullptr;
+  return hipSuccess;
+}
+hipError_t hipStreamDestroy(hipStream_t) { return hipSuccess; }
+hipError_t hipStreamIsCapturing(hipStream_t, hipStreamCaptureStatus* s) {
+  if (S().capturing == 2) return S().last = hipErrorStreamCaptureImplicit;
+  *s = S().capturing ? hipStreamCaptureStatusActive : hipStreamCaptureStatusNone;
+  return hipSuccess;
+}
+hipError_t hipEventCreateWithFlags(hipEvent_t* e, unsigned) {
+  *e = reinterpret_cast<hipEvent_t>(8);
+  return hipSuccess;
+}
+hipError_t hipEventCreate(hipEvent_t* e) { return hipEventCreateWithFlags(e, 0); }
+hipError_t hipEventDestroy(hipEvent_t) { return hipSuccess; }
+hipError_t hipEventQuery(hipEvent_t) { return hipSuccess; }
+hipError_t hipEventRecord(hipEvent_t, hipStream_t) { return hipSuccess; }
+hipError_t hipEventSynchronize(hipEvent_t) { return hipSuccess; }
+hipError_t hipEventElapsedTime(float* ms, hipEvent_t, hipEvent_t) {
+  *ms = 1.0f;
+  return hipSuccess;
+}
+hipError_t hipGetLastError() {
+  const hipError_t e = S().last;
+  S().last = hipSuccess;
+  return e;
+}
+const char* hipGetErrorString(hipError_t) { return "an error of the test"; }
+}  // extern "C"
+
+namespace {
+
+// -- scenarios --------------------------------------------------------------
+pbf_params small_params() {
+  pbf_params p;
+  pbf_params_default(&p);
+  p.smoothing_length = 0.1f;  // a small grid
+  p.sampling_distance = 0.04f;
+  return p;
+}
+
+template <class T> T* device(size_t n) {
+  void* p = nullptr;
+  const long keep = S().fail_at;
+  const size_t over = S().fail_over;
+  S().fail_at = kNever;
+  S().fail_over = SIZE_MAX;
+  --S().mallocs;
+  (void)hipMalloc(&p, sizeof(T) * n);
+  S().fail_at = keep;
+  S().fail_over = over;
+  return static_cast<T*>(p);
+}
+
+struct Arrays {
+  float *x, *v, *rho;
+  double *dx, *dv;
+  int *index, *elems;
+  explicit Arrays(size_t n)
+      : x(device<float>(3 * n)), v(device<float>(3 * n)), rho(device<float>(n)), dx(device<double>(3 * n)),
+        dv(device<double>(3 * n)), index(device<int>(n)), elems(device<int>(n)) {}
+};
+
+[[maybe_unused]] void expect(bool ok, const char* what) {
+  if (!ok) violation("%s", what);
+}
+
+// Every allocation of a sequence of calls fails once; each call is repeated
+// until it gets through. No launch may see a pointer to nothing.
+void failed_allocations(const std::vector<std::function<int(pbf_ctx*, Arrays&)>>& calls, unsigned flags) {
+  long total = 1;
+  for (long f = -1; f < total; ++f) {
+    Arrays a(3000);
+    pbf_params p = small_params();
+    p.flags = flags;
+    S().list_need = 96;
+    pbf_ctx* c = nullptr;
+    if (pbf_create(&p, &c) != PBF_OK) std::abort();
+    const long start = S().mallocs;
+    S().fail_at = f < 0 ? kNever : start + f;
+    for (size_t k = 0; k < calls.size(); ++k) {
+      int st = PBF_OK;
+      for (int attempt = 0; attempt < 3; ++attempt)
+        if ((st = calls[k](c, a)) == PBF_OK) break;
+      if (st != PBF_OK) violation("call %zu with allocation %ld failing: %s", k, f, pbf_last_error(c));
+    }
+    if (f < 0) total = S().mallocs - start;
+    S().fail_at = kNever;
+    pbf_destroy(c);
+    S().searched.clear();
+  }
+  std::printf("%ld allocations\n", total);
+}
+
+int step(pbf_ctx* c, Arrays& a, int n) { return pbf_step(c, a.x, a.v, a.rho, n, 1, nullptr); }
+
+int dense(pbf_ctx* c, Arrays& a, int n, unsigned long long slots) {  // the next call's lists grow
+  S().list_need = slots;
+  const int st = step(c, a, n);
+  S().list_need = 96;
+  return st;
+}
+
+void list_reservation() {
+  failed_allocations({[](pbf_ctx* c, Arrays& a) { return step(c, a, 500); },
+                      [](pbf_ctx* c, Arrays& a) { return step(c, a, 2000); },
+                      [](pbf_ctx* c, Arrays& a) { return dense(c, a, 2000, 400); },
+                      [](pbf_ctx* c, Arrays& a) { return step(c, a, 2000); }},
+                     0);
+}
+
+const std::map<std::string, void (*)()> kScenarios = {
+    {"list_reservation", list_reservation},
+};
+
+}  // namespace
+
+int main(int argc, char** argv) {
+  auto it = kScenarios.find(argc > 1 ? argv[1] : "");
+  if (it == kScenarios.end()) return std::printf("no such scenario\n"), 2;
+  it->second();
+  std::printf("%s: %zu launches, %d violations\n", argv[1], S().launches.size(), S().violations);
+  return S().violations ? 1 : 0;
+}

@@ -1,0 +1,39 @@
+"""Host paths of libpbf.so that a GPU run reaches only when something fails or
+would fault when it is wrong: tests/cpp/pbf_host_paths.cpp runs the built library
+on a HIP runtime of its own (device memory is host memory, kernels do not run)
+and checks every pointer that a launch or a copy hands over. No GPU needed."""
+import shutil
+import subprocess
+from pathlib import Path
+
+import pytest
+
+ROOT = Path(__file__).resolve().parents[1]
+BUILD = ROOT / "physika-old_amd" / "_build"
+CLANGXX = "/opt/rocm/llvm/bin/clang++"
+
+
+@pytest.fixture(scope="module")
+def host_paths(tmp_path_factory):
+    if not shutil.which(CLANGXX):
+        pytest.skip("clang++ not available")
+    if not (BUILD / "libpbf.so").exists():
+        pytest.skip("libpbf.so not built")
+    exe = tmp_path_factory.mktemp("host_paths") / "pbf_host_paths"
+    subprocess.run([CLANGXX, "-O1", "-std=c++17", "-Wall", "-D__HIP_PLATFORM_AMD__", "-I/opt/rocm/include",
+                    f"-I{ROOT / 'include'}", str(ROOT / "tests" / "cpp" / "pbf_host_paths.cpp"), "-rdynamic",
+                    f"-L{BUILD}", "-lpbf", f"-Wl,-rpath,{BUILD}", "-Wl,-rpath-link,/opt/rocm/lib", "-o", str(exe)],
+                   check=True)
+    return exe
+
+
+def run(exe, scenario):
+    r = subprocess.run([str(exe), scenario], capture_output=True, text=True, timeout=300)
+    assert r.returncode == 0 and "VIOLATION" not in r.stdout, (r.returncode, (r.stdout + r.stderr)[-3000:])
+
+
+def test_failed_list_reservation(host_paths):
+    """Each allocation of a growing context fails once: the calls after it run
+    without lists (bit masks, re-tests), and no kernel is handed a null list,
+    whose first chunks a lane pair reads ahead of the wave's words."""
+    run(host_paths, "list_reservation")
