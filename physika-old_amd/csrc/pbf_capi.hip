@@ -1161,6 +1161,30 @@ bool slots_fit(const pbf_ctx* c) {
          c->slot_K == c->p.iterations;
 }
 
+// The arrays of a slot for the capacities that the slots have; a slot joins
+// the others only when all of them are there.
+int alloc_slot(pbf_ctx* c, pbf_ctx::TapeSlot& t) {
+  const size_t cap = c->slot_n, nwv = cap / 64 + 4;
+  PBF_HIP(c, hipMalloc(&t.perm, sizeof(int) * cap));
+  PBF_HIP(c, hipMalloc(&t.ssid, sizeof(int) * cap));
+  PBF_HIP(c, hipMalloc(&t.nbr_cnt, sizeof(int) * cap));
+  PBF_HIP(c, hipMalloc(&t.xn, sizeof(float4) * (cap + kXnPad)));
+  PBF_HIP(c, hipMalloc(&t.x0, sizeof(float4) * cap));
+  PBF_HIP(c, hipMalloc(&t.list_base, sizeof(long long) * nwv));
+  PBF_HIP(c, hipMalloc(&t.mask_base, sizeof(long long) * nwv));
+  PBF_HIP(c, hipMalloc(&t.list_jbase, sizeof(int) * nwv));
+  PBF_HIP(c, hipMalloc(&t.list_mode, sizeof(int) * nwv));
+  PBF_HIP(c, hipMalloc(&t.stage, sizeof(int) * kStageInts * nwv));
+  PBF_HIP(c, hipMalloc(&t.cnt_a, sizeof(uint16_t) * cap));
+  PBF_HIP(c, hipMalloc(&t.list, sizeof(uint16_t) * (c->slot_list + kListPad)));
+  PBF_HIP(c, hipMalloc(&t.mask, sizeof(uint32_t) * std::max<size_t>(c->slot_mask, 1)));
+  PBF_HIP(c, hipMalloc(&t.cell_start, sizeof(int) * ((size_t)c->slot_cells + 2)));
+  PBF_HIP(c, hipMalloc(&t.win, sizeof(SceneWin) * (size_t)std::max(c->slot_scenes, 1)));
+  PBF_HIP(c, hipMalloc(&t.counters, sizeof(unsigned long long) * kDeviceCounters));
+  PBF_HIP(c, hipMalloc(&t.it, sizeof(float4) * cap * (size_t)std::max(2 * c->slot_K - 1, 1)));
+  return PBF_OK;
+}
+
 // m tape slots and the adjoint arrays for the current capacities and
 // iterations.
 int ensure_tape(pbf_ctx* c, int m) {
@@ -1176,27 +1200,14 @@ int ensure_tape(pbf_ctx* c, int m) {
     c->slot_scenes = c->scene_cap;
     c->slot_K = K;
   }
-  const size_t nwv = cap / 64 + 4;
   while ((int)c->slots.size() < m) {
-    c->slots.emplace_back();
-    auto& t = c->slots.back();
-    PBF_HIP(c, hipMalloc(&t.perm, sizeof(int) * cap));
-    PBF_HIP(c, hipMalloc(&t.ssid, sizeof(int) * cap));
-    PBF_HIP(c, hipMalloc(&t.nbr_cnt, sizeof(int) * cap));
-    PBF_HIP(c, hipMalloc(&t.xn, sizeof(float4) * (cap + kXnPad)));
-    PBF_HIP(c, hipMalloc(&t.x0, sizeof(float4) * cap));
-    PBF_HIP(c, hipMalloc(&t.list_base, sizeof(long long) * nwv));
-    PBF_HIP(c, hipMalloc(&t.mask_base, sizeof(long long) * nwv));
-    PBF_HIP(c, hipMalloc(&t.list_jbase, sizeof(int) * nwv));
-    PBF_HIP(c, hipMalloc(&t.list_mode, sizeof(int) * nwv));
-    PBF_HIP(c, hipMalloc(&t.stage, sizeof(int) * kStageInts * nwv));
-    PBF_HIP(c, hipMalloc(&t.cnt_a, sizeof(uint16_t) * cap));
-    PBF_HIP(c, hipMalloc(&t.list, sizeof(uint16_t) * (c->slot_list + kListPad)));
-    PBF_HIP(c, hipMalloc(&t.mask, sizeof(uint32_t) * std::max<size_t>(c->slot_mask, 1)));
-    PBF_HIP(c, hipMalloc(&t.cell_start, sizeof(int) * ((size_t)c->cell_cap + 2)));
-    PBF_HIP(c, hipMalloc(&t.win, sizeof(SceneWin) * (size_t)std::max(c->scene_cap, 1)));
-    PBF_HIP(c, hipMalloc(&t.counters, sizeof(unsigned long long) * kDeviceCounters));
-    PBF_HIP(c, hipMalloc(&t.it, sizeof(float4) * cap * (size_t)std::max(2 * K - 1, 1)));
+    pbf_ctx::TapeSlot t;
+    const int s = alloc_slot(c, t);
+    if (s) {
+      free_slot(t);
+      return s;
+    }
+    c->slots.push_back(t);
   }
   if (r.adj_n < c->cap_n) {
     dfree(r.adj);

@@ -400,7 +400,36 @@ void list_reservation() {
                      0);
 }
 
+int forward(pbf_ctx* c, Arrays& a, bool f64, int n, int nsteps, int every) {
+  return f64 ? pbf_rollout_forward_f64(c, a.dx, a.dv, nullptr, nullptr, 1, n, nsteps, every, nullptr)
+             : pbf_rollout_forward(c, a.x, a.v, a.rho, nullptr, 1, n, nsteps, every, nullptr);
+}
+
+int backward(pbf_ctx* c, Arrays& a, bool f64) {
+  return f64 ? pbf_rollout_backward_f64(c, a.dx, a.dv, nullptr) : pbf_rollout_backward(c, a.x, a.v, nullptr);
+}
+
+// A reverse that ran out of memory is not tried again: the next forward records
+// into the slots that are there.
+int backward_once(pbf_ctx* c, Arrays& a, bool f64) {
+  const int st = backward(c, a, f64);
+  return st == PBF_ERR_ALLOC ? PBF_OK : st;
+}
+
+void tape_slots() {
+  for (bool f64 : {false, true})
+    for (bool again : {false, true})
+      failed_allocations({[=](pbf_ctx* c, Arrays& a) { return forward(c, a, f64, 1500, 5, 3); },
+                          [=](pbf_ctx* c, Arrays& a) { return again ? backward(c, a, f64) : backward_once(c, a, f64); },
+                          [=](pbf_ctx* c, Arrays& a) { return forward(c, a, f64, 1500, 5, 3); },
+                          [=](pbf_ctx* c, Arrays& a) { return backward(c, a, f64); },
+                          [=](pbf_ctx* c, Arrays& a) { return forward(c, a, !f64, 1500, 3, 3); },
+                          [=](pbf_ctx* c, Arrays& a) { return backward(c, a, !f64); }},
+                         0);
+}
+
 const std::map<std::string, void (*)()> kScenarios = {
+    {"tape_slots", tape_slots},
     {"list_reservation", list_reservation},
 };
 

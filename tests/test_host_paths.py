@@ -37,3 +37,11 @@ def test_failed_list_reservation(host_paths):
     without lists (bit masks, re-tests), and no kernel is handed a null list,
     whose first chunks a lane pair reads ahead of the wave's words."""
     run(host_paths, "list_reservation")
+
+
+def test_failed_tape_slots(host_paths):
+    """Each allocation of a rollout and its reverse fails once, in both
+    precisions: a slot that got only some of its arrays is not used, neither by
+    a reverse that is tried again nor by the next forward, which records into
+    the slots."""
+    run(host_paths, "tape_slots")
