@@ -792,11 +792,15 @@ int drain_marks(pbf_ctx* c) {
   return PBF_OK;
 }
 
+bool capturing(hipStream_t st);
+void adopt_last(pbf_ctx* c);
+
 // NeighborQuery::compute on the positions x for a batch of scenes
 // (GridHash::construct + queryNeighborDynamic), leaving the cell-sorted state
 // and the neighbor lists in the context; with `integrate` the integrator is
 // fused into the reorder.
 int search(pbf_ctx* c, const SortIn& in, int n, const int* scene_off, int nscenes, bool integrate, hipStream_t st) {
+  if (c->last_slot >= 0 && capturing(st)) adopt_last(c);
   {
     PassTimer t(c, PBF_PASS_SORT, st);
     launch_sort(sort_of(c, scene_off, nscenes), c->g, in, n, c->xn, c->x0, c->vs, integrate ? &c->pc : nullptr,
@@ -1240,6 +1244,19 @@ void swap_slot(pbf_ctx* c, pbf_ctx::TapeSlot& t) {
   std::swap(c->mask, t.mask);
 }
 
+// The last search's outputs become the context's own arrays where a slot holds
+// them, before a call is captured: its replays write the context's arrays, and
+// step_neighbors exports the last search until then.
+void adopt_last(pbf_ctx* c) {
+  if (c->last_slot < 0) return;
+  if (slots_fit(c)) {
+    swap_slot(c, c->slots[(size_t)c->last_slot]);
+    c->gen++;
+  }
+  c->last_slot = -1;
+  c->tape_of = 0;
+}
+
 NbrView slot_view(const pbf_ctx* c, const pbf_ctx::TapeSlot& t, int n) {
   NbrView nv = view_of(c, n);
   nv.win = t.win;
@@ -1252,28 +1269,34 @@ NbrView slot_view(const pbf_ctx* c, const pbf_ctx::TapeSlot& t, int n) {
   nv.list_mode = t.list_mode;
   nv.stage = t.stage;
   nv.cnt_a = t.cnt_a;
-  nv.list = t.list;
+  nv.list = t.list ? t.list : c->list_none;
   nv.mask_base = t.mask_base;
   nv.mask = t.mask;
   nv.counters = t.counters;
   return nv;
 }
 
-// Runs step() with the search outputs of slot t in place of the context's, and
-// copies into the slot what the step leaves in the context.
-template <class Step> int taped_step(pbf_ctx* c, pbf_ctx::TapeSlot& t, int nscenes, hipStream_t st, Step&& step) {
+// Runs step() with the search outputs of slot q in place of the context's, and
+// copies into the slot what the step leaves in the context. The slot then holds
+// the last search's lists; a step that failed leaves none.
+template <class Step> int taped_step(pbf_ctx* c, int q, int nscenes, hipStream_t st, Step&& step) {
+  auto& t = c->slots[(size_t)q];
   c->tape_of = 0;
   swap_slot(c, t);
-  int s = step();
+  int s = step(t);
   if (!s) {
     launch_copy_cells(c->cell_start, t.cell_start, c->total_cells, c->cell_cap, st);
     if (hipMemcpyAsync(t.win, c->win, sizeof(SceneWin) * (size_t)nscenes, hipMemcpyDeviceToDevice, st) !=
             hipSuccess ||
         hipMemcpyAsync(t.counters, c->counters, sizeof(unsigned long long) * kDeviceCounters, hipMemcpyDeviceToDevice,
-                       st) != hipSuccess)
+                       st) != hipSuccess) {
+      (void)hipGetLastError();  // not the next call's
       s = fail(c, PBF_ERR_HIP, "tape copy failed");
+    }
   }
   swap_slot(c, t);
+  c->last_slot = s ? -1 : q;
+  if (s) c->last_n = -1;
   return s;
 }
 
@@ -1714,8 +1737,7 @@ int pbf_rollout_forward(pbf_ctx* c, float* d_x, float* d_v, float* d_rho, const 
     }
     float* rho = k + 1 == nsteps ? d_rho : nullptr;
     if (k >= tape) {
-      auto& t = c->slots[(size_t)(k - tape)];
-      s = taped_step(c, t, nscenes, st, [&] {
+      s = taped_step(c, k - tape, nscenes, st, [&](const pbf_ctx::TapeSlot& t) {
         const Iterates it(c, t, c->x0);
         return step_once(c, d_x, d_v, d_x, d_v, rho, n, r.off, nscenes, it.P.data(), it.aux.data(), st);
       });
@@ -1724,7 +1746,6 @@ int pbf_rollout_forward(pbf_ctx* c, float* d_x, float* d_v, float* d_rho, const 
     }
     if (s) return s;
   }
-  if (tape != kTapeNone) c->last_slot = nsteps - 1 - tape;
   s = record_counters(c, st);
   if (s) return s;
   r.n = n;
@@ -1776,8 +1797,7 @@ int pbf_rollout_backward(pbf_ctx* c, float* d_xbar, float* d_vbar, void* stream)
         const float* in = (q & 1) ? sb : sa;
         float* xout = q + 1 == m ? r.out : ((q & 1) ? sa : sb);
         float* vout = q + 1 == m ? r.out + 3 * cap : xout + 3 * (size_t)n;
-        auto& t = c->slots[q];
-        s = taped_step(c, t, r.nscenes, st, [&] {
+        s = taped_step(c, q, r.nscenes, st, [&](const pbf_ctx::TapeSlot& t) {
           const Iterates it(c, t, c->x0);
           return step_once(c, in, in + 3 * (size_t)n, xout, vout, nullptr, n, r.off, r.nscenes, it.P.data(),
                            it.aux.data(), st);
@@ -1848,9 +1868,8 @@ int pbf_rollout_forward_f64(pbf_ctx* c, double* d_x, double* d_v, double* d_rho,
     }
     double* rho = k + 1 == nsteps ? d_rho : nullptr;
     if (k >= tape) {
-      auto& t = c->slots[(size_t)(k - tape)];
-      const Iterates64 it(c, t);
-      s = taped_step(c, t, nscenes, st, [&] {
+      s = taped_step(c, k - tape, nscenes, st, [&](const pbf_ctx::TapeSlot& t) {
+        const Iterates64 it(c, t);
         return step64_once(c, d_x, d_v, d_x, d_v, rho, n, r.off, nscenes, it.P.data(), it.aux.data(), st);
       });
     } else {
@@ -1858,7 +1877,6 @@ int pbf_rollout_forward_f64(pbf_ctx* c, double* d_x, double* d_v, double* d_rho,
     }
     if (s) return s;
   }
-  if (tape != kTapeNone) c->last_slot = nsteps - 1 - tape;
   if ((s = record_counters(c, st))) return s;
   if ((s = read_flag64(c, st, "pbf_rollout_forward_f64"))) return s;
   r.n = n;
@@ -1924,9 +1942,8 @@ int pbf_rollout_backward_f64(pbf_ctx* c, double* d_xbar, double* d_vbar, void* s
         const double* in = (q & 1) ? sb : sa;
         double* xout = q + 1 == m ? r.out : ((q & 1) ? sa : sb);
         double* vout = q + 1 == m ? r.out + 3 * cap : xout + 3 * (size_t)n;
-        auto& t = c->slots[q];
-        const Iterates64 it(c, t);
-        s = taped_step(c, t, r.nscenes, st, [&] {
+        s = taped_step(c, q, r.nscenes, st, [&](const pbf_ctx::TapeSlot& t) {
+          const Iterates64 it(c, t);
           return step64_once(c, in, in + 3 * (size_t)n, xout, vout, nullptr, n, r.off, r.nscenes, it.P.data(),
                              it.aux.data(), st);
         });

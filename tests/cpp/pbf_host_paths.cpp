@@ -46,13 +46,13 @@ struct State {
   size_t bytes = 0, peak = 0;
   long mallocs = 0, fail_at = kNever;  // fail_at: the malloc (0-based) that fails
   size_t fail_over = SIZE_MAX;     // every malloc of more bytes fails
-  long failed = 0;
+  long copy_fail_at = kNever;  // copies left until one fails
   hipError_t last = hipSuccess;
   int capturing = 0;        // hipStreamIsCapturing: 0 no, 1 yes, 2 an error
   unsigned long long list_need = 0, calls = 0;
   std::vector<Launch> launches;
   std::vector<std::string> ops;  // launches, copies and waits, in order
-  std::map<const void*, long> searched;  // list buffer -> serial of the neighbor pass that last wrote it
+  std::map<const void*, long> searched;  // buffer of a search -> serial of the neighbor pass that last wrote it
   long searches = 0, exported = -1;      // exported: the search that the last export read
   dim3 grid, block;
   size_t shared;
@@ -107,6 +107,13 @@ void check_view(const Kernel& k, const pbf::NbrView& v) {
   need(k, "list", v.list, 2 * (64 * waves * (size_t)v.list_per + pbf::kListPad));
 }
 
+// The arrays that a search leaves for the passes and the export.
+std::vector<const void*> outputs(const pbf::NbrView& v) {
+  return {v.list,       v.nbr_cnt,   v.xn,        v.ssid, v.list_base, v.list_jbase,
+          v.list_mode,  v.mask_base, v.mask,      v.cnt_a, v.stage,    v.win,
+          v.cell_start};
+}
+
 void launched(const void* f, dim3 block, void** args) {
   const Kernel& k = S().kernels[f];
   Launch l{k.name, k.full, block.x, {}, false};
@@ -124,8 +131,15 @@ void launched(const void* f, dim3 block, void** args) {
   S().launches.push_back(l);
   S().ops.push_back(k.name);
   if (S().capturing == 1) return;
-  if (k.name == "k_neighbors" || k.name == "k_neighbors_small") S().searched[l.nv.list] = S().searches++;
-  if (k.name == "k_csr_fill") S().exported = S().searched.count(l.nv.list) ? S().searched[l.nv.list] : -1;
+  if (k.name == "k_neighbors" || k.name == "k_neighbors_small") {
+    for (const void* p : outputs(l.nv)) S().searched[p] = S().searches;
+    ++S().searches;
+  }
+  if (k.name == "k_csr_fill") {
+    S().exported = S().searched.count(l.nv.list) ? S().searched[l.nv.list] : -1;
+    for (const void* p : outputs(l.nv))
+      if (!S().searched.count(p) || S().searched[p] != S().exported) violation("k_csr_fill: arrays of different searches");
+  }
   if (k.name == "k_wave_stats") {  // the counters of the call
     auto* host = *static_cast<unsigned long long**>(args[4]);
     for (int c = 0; c < pbf::C_COUNT; ++c) host[c] = 0;
@@ -213,7 +227,6 @@ hipError_t hipMalloc(void** p, size_t bytes) {
   *p = nullptr;
   const long k = S().mallocs++;
   if (k == S().fail_at || bytes > S().fail_over) {
-    ++S().failed;
     return S().last = hipErrorOutOfMemory;
   }
   *p = std::calloc(bytes ? bytes : 1, 1);
@@ -253,6 +266,7 @@ hipError_t hipGetSymbolAddress(void** p, const void*) {
   return hipMalloc(p, 2 * (size_t)PBF_NOALLOC_MAX_PARTICLES * 16 + 4096);
 }
 hipError_t hipMemcpyAsync(void* d, const void* s, size_t bytes, hipMemcpyKind kind, hipStream_t) {
+  if (S().copy_fail_at != kNever && S().copy_fail_at-- == 0) return S().last = hipErrorUnknown;
   copied(d, s, bytes, kind);
   S().ops.push_back("copy");
   return hipSuccess;
@@ -352,7 +366,7 @@ struct Arrays {
         dv(device<double>(3 * n)), index(device<int>(n)), elems(device<int>(n)) {}
 };
 
-[[maybe_unused]] void expect(bool ok, const char* what) {
+void expect(bool ok, const char* what) {
   if (!ok) violation("%s", what);
 }
 
@@ -428,7 +442,75 @@ void tape_slots() {
                          0);
 }
 
+long exported(pbf_ctx* c, Arrays& a) {  // the search that step_neighbors exports
+  long long total = 0;
+  S().exported = -1;
+  if (pbf_step_neighbors(c, a.index, a.elems, 0, &total, nullptr) != PBF_OK) violation("step_neighbors: %s", pbf_last_error(c));
+  return S().exported;
+}
+
+void last_search() {
+  for (bool f64 : {false, true})
+    for (int every : {1, 2, 3, 5, 9}) {
+      Arrays a(3000);
+      pbf_params p = small_params();
+      pbf_ctx* c = nullptr;
+      if (pbf_create(&p, &c) != PBF_OK) std::abort();
+      S().list_need = 96;
+      long last = 0;
+      for (int round = 0; round < 3; ++round) {
+        expect(forward(c, a, f64, 1500, 5, every) == PBF_OK, "forward");
+        last = S().searches - 1;
+        expect(exported(c, a) == last, "lists after a forward");
+        if (round < 2) expect(backward(c, a, f64) == PBF_OK, "reverse");
+      }
+      // a captured call that has not been replayed
+      S().capturing = 1;
+      expect(step(c, a, 1500) == PBF_OK, "captured step");
+      S().capturing = 0;
+      expect(exported(c, a) == last, "lists before the first replay");
+      expect(backward(c, a, f64) == PBF_OK, "reverse");
+      expect(step(c, a, 1500) == PBF_OK, "step");
+      expect(exported(c, a) == S().searches - 1, "lists of the step");
+      pbf_destroy(c);
+      S().searched.clear();
+    }
+}
+
+// A forward or a reverse that fails on its way leaves no lists to export, or
+// whole ones.
+void failed_rollout() {
+  for (bool f64 : {false, true})
+    for (long f = 0; f < 60; ++f) {
+      Arrays a(3000);
+      pbf_params p = small_params();
+      pbf_ctx* c = nullptr;
+      if (pbf_create(&p, &c) != PBF_OK) std::abort();
+      S().list_need = 96;
+      expect(forward(c, a, f64, 1500, 4, 2) == PBF_OK && backward(c, a, f64) == PBF_OK, "rollout");
+      expect(step(c, a, 700) == PBF_OK, "step");
+      for (bool reverse : {false, true}) {
+        S().copy_fail_at = f;
+        const int st = reverse ? backward(c, a, f64) : forward(c, a, f64, 1500, 4, 2);
+        S().copy_fail_at = kNever;
+        expect(S().last == hipSuccess, "an error left for the next call");
+        S().last = hipSuccess;
+        long long total = 0;
+        S().exported = -1;
+        if (pbf_step_neighbors(c, a.index, a.elems, 0, &total, nullptr) == PBF_OK) {
+          expect(!reverse || st != PBF_OK, "lists after a reverse");
+          expect(S().exported == S().searches - 1, "lists after a failed call");
+        }
+        if (!reverse && st != PBF_OK) expect(forward(c, a, f64, 1500, 4, 2) == PBF_OK, "forward again");
+      }
+      pbf_destroy(c);
+      S().searched.clear();
+    }
+}
+
 const std::map<std::string, void (*)()> kScenarios = {
+    {"last_search", last_search},
+    {"failed_rollout", failed_rollout},
     {"tape_slots", tape_slots},
     {"list_reservation", list_reservation},
 };

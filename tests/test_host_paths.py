@@ -45,3 +45,11 @@ def test_failed_tape_slots(host_paths):
     a reverse that is tried again nor by the next forward, which records into
     the slots."""
     run(host_paths, "tape_slots")
+
+
+@pytest.mark.parametrize("scenario", ["last_search", "failed_rollout"])
+def test_lists_of_the_last_search(host_paths, scenario):
+    """step_neighbors exports the last search, whole and from one set of arrays:
+    a recorded forward's last step, also after a call was captured and not yet
+    replayed; and none, or whole ones, after a rollout call that failed midway."""
+    run(host_paths, scenario)
