@@ -772,17 +772,19 @@ __global__ __launch_bounds__(kBlock) void k_reorder(const int* __restrict__ key,
 // The whole sort of a one-scene search of at most kSortOneMax particles in one
 // workgroup: nine launches of 1.5 to 5 us each, most of it launch and memory
 // latency, become one (and one that returns at once unless the window is
-// large). The particles go to LDS buckets of consecutive cells, and a
+// large). The in-grid particles go to LDS buckets of consecutive cells, and a
 // particle's place is its bucket's start plus the number of its bucket's
 // particles before it by (cell, original index): the order of the sort above,
-// for cells and out-of-grid buckets of any size. The starts of the window's
-// cells are found in the sorted keys.
+// for cells of any size. The out-of-grid particles, of which there may be
+// thousands, follow in the order of their original indices, ranked in a bit set.
+// The starts of the window's cells are found in the sorted keys.
 constexpr int kSortOneMax = 4096, kSortOneBlock = 1024, kSortOnePer = kSortOneMax / kSortOneBlock;
 constexpr int kSortBuckets = 8192, kBucketsPer = kSortBuckets / kSortOneBlock;
+constexpr int kSortIdBits = 12, kSortIdWords = kSortOneMax / 32;
+static_assert(1 << kSortIdBits == kSortOneMax, "an index and its cell inside a bucket share a word");
 
-// First position of keys[0..n) whose key is at least c.
-__device__ __forceinline__ int lower_key(const int* keys, int n, int c) {
-  int lo = 0, hi = n;
+// First position of keys[lo..hi) whose key is at least c.
+__device__ __forceinline__ int lower_key(const int* keys, int lo, int hi, int c) {
   while (lo < hi) {
     const int mid = (lo + hi) >> 1;
     if (keys[mid] < c)
@@ -805,11 +807,18 @@ __global__ __launch_bounds__(kSortOneBlock) void k_sort_one(SortIn in, int n, Gr
                                                             int* __restrict__ oog_rcnt) {
 #pragma clang fp contract(off)
   __shared__ int start[kSortBuckets + 1];
-  __shared__ int skey[kSortOneMax], sid[kSortOneMax], src[kSortOneMax];
+  // entries in bucket order: the cell, the cell inside the bucket with the
+  // original index, the input index
+  __shared__ int skey[kSortOneMax], src[kSortOneMax];
+  __shared__ unsigned sord[kSortOneMax];
+  __shared__ unsigned out_bit[kSortIdWords];  // out-of-grid original indices
+  __shared__ int out_pre[kSortIdWords], out_half;
   __shared__ int red[kSortOneBlock / 64][8];
   __shared__ SceneWin sw;
+  __shared__ int nout;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   for (int b = tid; b <= kSortBuckets; b += kSortOneBlock) start[b] = 0;
+  if (tid < kSortIdWords) out_bit[tid] = 0;
   // cells and their box
   int c[kSortOnePer][3];
   bool inside[kSortOnePer];
@@ -867,6 +876,7 @@ __global__ __launch_bounds__(kSortOneBlock) void k_sort_one(SortIn in, int n, Gr
       w.cell_base = 0;
       w.ncell = w.dim[0] * w.dim[1] * w.dim[2];
       sw = w;
+      nout = r[6];
       win[0] = w;
       *total_cells = w.ncell + 1;
       counters[C_CELLS] = (unsigned long long)w.ncell + 1;
@@ -878,15 +888,32 @@ __global__ __launch_bounds__(kSortOneBlock) void k_sort_one(SortIn in, int n, Gr
   }
   __syncthreads();
   const SceneWin w = sw;
-  // buckets of 2^shift consecutive cells (the out-of-grid bucket is cell ncell)
+  const int nin = n - nout;  // in-grid particles
+  // buckets of 2^shift consecutive cells
   const int shift = max(0, 32 - __clz(w.ncell) - 13);
   int key[kSortOnePer], slot[kSortOnePer];
 #pragma unroll
   for (int q = 0; q < kSortOnePer; ++q) {
     key[q] = inside[q] ? window_cell(w, c[q][0], c[q][1], c[q][2]) : w.ncell;
-    slot[q] = tid + q * kSortOneBlock < n ? atomicAdd(&start[key[q] >> shift], 1) : 0;
+    slot[q] = inside[q] ? atomicAdd(&start[key[q] >> shift], 1) : 0;
+  }
+  if (nout > 0) {
+#pragma unroll
+    for (int q = 0; q < kSortOnePer; ++q) {
+      const int i = tid + q * kSortOneBlock;
+      if (i < n && !inside[q]) {
+        const int id = kCellOrder ? in.id[i] : i;
+        atomicOr(&out_bit[id >> 5], 1u << (id & 31));
+      }
+    }
   }
   __syncthreads();
+  if (nout > 0 && tid < kSortIdWords) {
+    const int v = __popc(out_bit[tid]);
+    const int incl = wave_inclusive_scan(v);
+    out_pre[tid] = incl - v;
+    if (tid == 63) out_half = incl;
+  }
   {  // exclusive scan of the bucket counts, kBucketsPer per thread
     int v[kBucketsPer], sum = 0;
 #pragma unroll
@@ -901,34 +928,11 @@ __global__ __launch_bounds__(kSortOneBlock) void k_sort_one(SortIn in, int n, Gr
       start[tid * kBucketsPer + k] = e;
       e += v[k];
     }
-    if (tid == 0) start[kSortBuckets] = n;
+    if (tid == 0) start[kSortBuckets] = nin;
   }
   __syncthreads();
-#pragma unroll
-  for (int q = 0; q < kSortOnePer; ++q) {
-    const int i = tid + q * kSortOneBlock;
-    if (i < n) {
-      const int p = start[key[q] >> shift] + slot[q];
-      skey[p] = key[q];
-      sid[p] = kCellOrder ? in.id[i] : i;
-      src[p] = i;
-    }
-  }
-  __syncthreads();
-  // the place of each entry, then its arrays
-#pragma unroll
-  for (int q = 0; q < kSortOnePer; ++q) {
-    const int t = tid + q * kSortOneBlock;
-    if (t >= n) continue;
-    const int k = skey[t], id = sid[t], b = k >> shift;
-    const int a = start[b], e = start[b + 1];
-    int rank = 0;
-    for (int u = a; u < e; ++u) {
-      const int ku = skey[u];
-      rank += ku < k || (ku == k && sid[u] < id);
-    }
-    const int s = a + rank;
-    const int i = src[t];
+  // input i with original index id and cell k to its sorted place s
+  auto put = [&](int s, int i, int id, int k) {
     perm[s] = id;
     ssid[s] = 0;
     oog_rcnt[s] = 0;
@@ -948,6 +952,36 @@ __global__ __launch_bounds__(kSortOneBlock) void k_sort_one(SortIn in, int n, Gr
     } else {
       x0[s] = make_float4(p.x, p.y, p.z, 0.0f);
     }
+  };
+#pragma unroll
+  for (int q = 0; q < kSortOnePer; ++q) {
+    const int i = tid + q * kSortOneBlock;
+    if (i >= n) continue;
+    const int id = kCellOrder ? in.id[i] : i;
+    if (inside[q]) {
+      const int p = start[key[q] >> shift] + slot[q];
+      skey[p] = key[q];
+      sord[p] = (unsigned)(key[q] & ((1 << shift) - 1)) << kSortIdBits | (unsigned)id;
+      src[p] = i;
+    } else {
+      const int at = id >> 5;
+      put(nin + out_pre[at] + (at >= 64 ? out_half : 0) + __popc(out_bit[at] & ((1u << (id & 31)) - 1u)), i, id,
+          w.ncell);
+    }
+  }
+  __syncthreads();
+  // the place of each in-grid entry
+#pragma unroll
+  for (int q = 0; q < kSortOnePer; ++q) {
+    const int t = tid + q * kSortOneBlock;
+    if (t >= nin) continue;
+    const int k = skey[t], b = k >> shift;
+    const unsigned o = sord[t];
+    const int a = start[b], e = start[b + 1];
+    int rank = 0;
+#pragma unroll 4
+    for (int u = a; u < e; ++u) rank += sord[u] < o ? 1 : 0;
+    put(a + rank, src[t], (int)(o & (kSortOneMax - 1)), k);
   }
   if (tid == 0) x0[n] = make_float4(kPadCoord, kPadCoord, kPadCoord, 0.0f);  // the padding particle
   if (w.ncell >= kSortBuckets) return;  // k_cell_starts
@@ -963,7 +997,7 @@ __global__ __launch_bounds__(kBlock) void k_cell_starts(const SceneWin* __restri
   if (ncell < kSortBuckets) return;
   const int stride = gridDim.x * blockDim.x;
   for (int c = blockIdx.x * blockDim.x + threadIdx.x; c <= ncell + 1; c += stride)
-    cell_start[c] = c <= ncell ? lower_key(keys, n, c) : n;
+    cell_start[c] = c <= ncell ? lower_key(keys, 0, n, c) : n;
 }
 
 template <bool kCellOrder>
