@@ -990,14 +990,39 @@ __global__ __launch_bounds__(kSortOneBlock) void k_sort_one(SortIn in, int n, Gr
 }
 
 // Starts of the cells of a window too large for k_sort_one's buckets, from the
-// sorted keys.
-__global__ __launch_bounds__(kBlock) void k_cell_starts(const SceneWin* __restrict__ win, const int* __restrict__ keys,
-                                                        int n, int* __restrict__ cell_start) {
+// sorted keys in LDS. The window is as large as the particles are spread (a stray
+// one is enough), up to the whole grid: a workgroup narrows the keys down to its
+// contiguous range of cells first, so that most cells, which are empty, cost
+// their share of a 16-byte store.
+constexpr int kStartsBlock = 256, kStartsBlocks = 512;
+
+__global__ __launch_bounds__(kStartsBlock) void k_cell_starts(const SceneWin* __restrict__ win,
+                                                              const int* __restrict__ keys, int n,
+                                                              int* __restrict__ cell_start) {
   const int ncell = win[0].ncell;
   if (ncell < kSortBuckets) return;
-  const int stride = gridDim.x * blockDim.x;
-  for (int c = blockIdx.x * blockDim.x + threadIdx.x; c <= ncell + 1; c += stride)
-    cell_start[c] = c <= ncell ? lower_key(keys, 0, n, c) : n;
+  __shared__ int key[kSortOneMax];
+  for (int t = threadIdx.x; t < n; t += kStartsBlock) key[t] = keys[t];
+  __syncthreads();
+  const int cells = ncell + 2;  // one past the out-of-grid bucket: n
+  const int per = (cells + kStartsBlocks * 4 - 1) / (kStartsBlocks * 4) * 4;
+  const int c0 = blockIdx.x * per, c1 = min(c0 + per, cells);
+  if (c0 >= c1) return;
+  const int lo = lower_key(key, 0, n, c0), hi = lower_key(key, lo, n, c1);
+  for (int c = c0 + 4 * (int)threadIdx.x; c < c1; c += 4 * kStartsBlock) {
+    int4 s;
+    s.x = lower_key(key, lo, hi, c);
+    s.w = lower_key(key, s.x, hi, c + 3);
+    s.y = lower_key(key, s.x, s.w, c + 1);
+    s.z = lower_key(key, s.y, s.w, c + 2);
+    if (c + 4 <= c1) {
+      *reinterpret_cast<int4*>(cell_start + c) = s;
+    } else {
+      cell_start[c] = s.x;
+      if (c + 1 < c1) cell_start[c + 1] = s.y;
+      if (c + 2 < c1) cell_start[c + 2] = s.z;
+    }
+  }
 }
 
 template <bool kCellOrder>
@@ -1008,7 +1033,7 @@ void sort_one(const SortBufs& sb, const GridDev& g, const SortIn& in, int n, flo
   k_sort_one<kCellOrder><<<1, kSortOneBlock, 0, st>>>(in, n, g, sb.win, sb.total_cells, counters, sb.cell_start,
                                                       sb.key, sb.perm, sb.ssid, xn, x0, vs, pc, integrate ? 1 : 0,
                                                       sb.xc, sb.xc_stride, sb.oog_rcnt);
-  k_cell_starts<<<128, kBlock, 0, st>>>(sb.win, sb.key, n, sb.cell_start);
+  k_cell_starts<<<kStartsBlocks, kStartsBlock, 0, st>>>(sb.win, sb.key, n, sb.cell_start);
 }
 
 // Bounds blocks of a launch whose last one makes the window: their tickets are

@@ -1,9 +1,10 @@
 """The sort of a small scene in one workgroup where its particles are not a compact
-block: thousands of them outside the grid. A batch of the scene and an empty one
-takes the general sort; both give the same bits over two steps (caller's order
-and cell order) and the same lists, and the small scene's step takes no more
-than three times that of a block of as many particles, which has far more
-pairs (an order of the out-of-grid particles by comparison took 20 times it)."""
+block: thousands of them outside the grid, or all over the scene box. A batch of
+the scene and an empty one takes the general sort; both give the same bits over
+two steps (caller's order and cell order) and the same lists. A step takes no more
+than three times (outside the grid) or twice (scattered) the time of a block of as
+many particles, which has far more pairs; comparing the out-of-grid particles with
+each other took 20 times it, a search of the keys for every cell four times."""
 import numpy as np
 import pytest
 
@@ -95,3 +96,26 @@ def test_out_of_grid_particles_are_not_compared(fluid, scene):
     base, out = step_time(fluid, block(scene, 4096)), step_time(fluid, inputs(scene, "all out 4096"))
     say(f"a step of 4,096 particles: in a block {base:.0f} us, out of the grid {out:.0f} us")
     assert out < 3 * base
+
+
+@pytest.mark.parametrize("n, h", [(1, 0.0125), (1000, 0.006), (4096, 0.0125), (4096, 0.006), (4096, 0.0041)])
+def test_scattered_scene(fluid, scene, n, h):
+    """A window of up to 28 million cells, most of them empty, whose starts come from
+    the sorted keys."""
+    x = scene.uniform01(4, 3 * n).reshape(-1, 3).astype(np.float32)
+    lists = []
+    for batch in (False, True):
+        ctx = fluid.Context("cuda:0", smoothing_length=h, stage_min_particles=-1)
+        xd, vd = dev(x), torch.zeros((n, 3), dtype=torch.float32, device="cuda:0")
+        if batch:
+            ctx.batch_step(xd, vd, torch.tensor([0, n, n], dtype=torch.int32, device="cuda:0"))
+        else:
+            ctx.step(xd, vd)
+        nl = ctx.step_neighbors(n)
+        lists.append([t.cpu().numpy() for t in (xd, vd, nl.index, nl.elements)])
+    for a, b in zip(*lists):
+        np.testing.assert_array_equal(a, b)
+    if h >= 0.006:
+        base, wide = step_time(fluid, block(scene, n), h), step_time(fluid, x, h)
+        say(f"a step of {n} particles, h {h}: in a block {base:.0f} us, scattered {wide:.0f} us")
+        assert wide < 2 * base
