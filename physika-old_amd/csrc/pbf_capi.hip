@@ -361,7 +361,8 @@ PhysConst64 derive64(const pbf_params* p) {
   pc.lam_rest = p->lambda_rest;
   pc.lam_eps = p->lambda_eps;
   pc.corr = p->corr_scale;
-  pc.pair_eps = p->pair_eps;
+  pc.pair_eps = p->pair_eps == 0.0f ? kSelfR : p->pair_eps;
+  pc.far_eps = std::max(pc.pair_eps, kSelfR);
   pc.dt = p->dt;
   for (int a = 0; a < 3; ++a) pc.g[a] = p->gravity[a];
   return pc;

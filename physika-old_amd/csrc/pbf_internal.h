@@ -319,9 +319,14 @@ void launch_adjoint_step(const NbrView& nv, float4* const* P, float4* const* aux
 
 // Double-precision step and adjoint (reverse mode against FP64 references):
 // the constants of PhysConst in double, computed from the parameters
-// promoted to double.
+// promoted to double. r^2 of a particle paired with itself (or with one in the
+// same place) counts as kSelfR2, and kSelfR lies between its square root and
+// every other distance; pair_eps 0 becomes kSelfR, so that r > pair_eps leaves
+// such pairs out there too.
+constexpr double kSelfR2 = 1e-290, kSelfR = 2e-145;
 struct PhysConst64 {
   double h, inv_h, cW, cG, lam_rest, lam_eps, corr, pair_eps, dt;
+  double far_eps;  // pair_eps, at least kSelfR: 1/r of two particles in one place counts as 0
   double g[3];
 };
 struct AdjBufs64 {

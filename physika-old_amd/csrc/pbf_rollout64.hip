@@ -35,8 +35,8 @@ __device__ __forceinline__ PairGeom64 pair_geom64(const double4& a, const double
   p.dx = a.x - b.x;
   p.dy = a.y - b.y;
   p.dz = a.z - b.z;
-  // r2 >= 1e-60 keeps the reciprocal finite (a particle paired with itself)
-  const double r2 = fma(p.dz, p.dz, fma(p.dy, p.dy, fma(p.dx, p.dx, 1e-60)));
+  // kSelfR2 keeps the reciprocal finite for a particle paired with itself
+  const double r2 = fma(p.dz, p.dz, fma(p.dy, p.dy, fma(p.dx, p.dx, kSelfR2)));
   // 1/sqrt(r2) from the hardware's estimate (relative error below 2^-23) by one
   // step of y (1 + e/2 + 3 e^2/8), e = 1 - r2 y^2, whose error is 5 e^3/16:
   // below an ulp, in 6 operations where a square root and a division take
@@ -315,7 +315,7 @@ __global__ __launch_bounds__(kBlock) void k64_adj_pos(NbrView nv, const double4*
           [&](auto& a, const D4x3& q) {
             // the terms of adj_pos_term (pbf_adjoint.hip)
             const PairGeom64 r = pair_geom64(ps, q.a, pc.inv_h);
-            const bool far = r.r > pc.pair_eps;
+            const bool far = r.r > pc.far_eps;
             const double v = r.t * r.t * r.rinv;
             const double u = far ? v : 0.0;
             const double cg = pc.cG * u;
