@@ -856,8 +856,13 @@ int export_csr(pbf_ctx* c, int n, int* d_index, int* d_elems, long long cap, lon
     *total = 0;
     return PBF_OK;
   }
+  // the caller's row starts are there when this returns, counted now or before
+  auto starts = [&] {
+    return hipMemcpyAsync(d_index, c->cnt_orig, sizeof(int) * (size_t)n, hipMemcpyDeviceToDevice, st);
+  };
   bool counted = c->csr_total >= 0;
   if (counted) {
+    PBF_HIP(c, starts());
     PBF_HIP(c, hipStreamSynchronize(st));
     counted = c->csr_calls == c->h_counters[C_CALLS];
   }
@@ -867,9 +872,7 @@ int export_csr(pbf_ctx* c, int n, int* d_index, int* d_elems, long long cap, lon
     // cnt_orig holds cap_n > n entries: the scan writes n + 1 in place
     scan_exclusive(c->cnt_orig, c->cnt_orig, n, c->scan_scratch, st);
     PBF_LAUNCHED(c);
-  }
-  PBF_HIP(c, hipMemcpyAsync(d_index, c->cnt_orig, sizeof(int) * (size_t)n, hipMemcpyDeviceToDevice, st));
-  if (!counted) {
+    PBF_HIP(c, starts());
     int tot = 0;
     PBF_HIP(c, hipMemcpyAsync(&tot, c->cnt_orig + n, sizeof(int), hipMemcpyDeviceToHost, st));
     PBF_HIP(c, hipStreamSynchronize(st));

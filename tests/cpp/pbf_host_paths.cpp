@@ -508,7 +508,30 @@ void failed_rollout() {
     }
 }
 
+// The row starts are in the caller's array when the call returns: nothing is copied
+// after its last wait, counted by this call or by one before.
+void blocking_export() {
+  Arrays a(3000);
+  pbf_params p = small_params();
+  pbf_ctx* c = nullptr;
+  if (pbf_create(&p, &c) != PBF_OK) std::abort();
+  expect(step(c, a, 1500) == PBF_OK, "step");
+  for (int call = 0; call < 3; ++call) {
+    long long total = 0;
+    S().ops.clear();
+    expect(pbf_step_neighbors(c, a.index, call < 2 ? nullptr : a.elems, 0, &total, nullptr) == PBF_OK, "export");
+    bool copied = false, open = false;
+    for (const std::string& op : S().ops) {
+      copied |= op == "copy";
+      open = op == "copy" || (open && op != "wait");
+    }
+    expect(copied && !open, "a copy after the last wait");
+  }
+  pbf_destroy(c);
+}
+
 const std::map<std::string, void (*)()> kScenarios = {
+    {"blocking_export", blocking_export},
     {"last_search", last_search},
     {"failed_rollout", failed_rollout},
     {"tape_slots", tape_slots},

@@ -53,3 +53,9 @@ def test_lists_of_the_last_search(host_paths, scenario):
     a recorded forward's last step, also after a call was captured and not yet
     replayed; and none, or whole ones, after a rollout call that failed midway."""
     run(host_paths, scenario)
+
+
+def test_row_starts_are_there_when_the_export_returns(host_paths):
+    """A second export of one search takes the row starts counted by the first;
+    the caller's copy of them is waited for all the same."""
+    run(host_paths, "blocking_export")
