@@ -186,6 +186,7 @@ struct pbf_ctx {
 
   float4* vis_w = nullptr;  // weights of a viscosity solve (vis_weights)
   size_t vis_cap = 0;
+  bool vis_refused = false;  // an allocation of them failed
 
   int last_n = -1;  // particle count of the last neighbor search (-1: none)
   // its list elements once cnt_orig holds their row starts (-1: not yet), and
@@ -954,33 +955,48 @@ int pass_lanes_for(const pbf_ctx* c, int n) {
 }
 
 // Room for the weights of a viscosity solve over n particles, or null: a search
-// of more than kVisWeightsMax (100 MB and more, which no cache holds between the
-// iterations), a capture that would have to allocate, or no memory.
+// of more than kVisWeightsMax, weights of more than kVisWeightsBytes, a capture
+// that would have to allocate, or no memory (asked for again only after
+// pbf_reserve or pbf_set_params). The weights are read back from the
+// 256 MB of cache in front of the memory, and past that they cost more than the
+// gathers that they save. One step, with and without: 65,536 particles, 80 MB 424
+// and 448 us, 130 MB 637 and 683, 223 MB 1,121 and 1,121; 131,072, 159 MB 836 and
+// 883, 260 MB 1,530 and 1,454; 262,144, 101 MB 460 and 485, 168 MB 795 and 826,
+// 319 MB 1,636 and 1,525.
 constexpr int kVisWeightsMax = 1 << 18;
+constexpr size_t kVisWeightsBytes = 192u << 20;
 float4* vis_weights(pbf_ctx* c, int n, hipStream_t st) {
-  if (n > kVisWeightsMax) return nullptr;
+  constexpr size_t limit = kVisWeightsBytes / sizeof(float4);
   const size_t need = vis_weight_entries(n, list_per_of(c));
+  if (n > kVisWeightsMax || need > limit) return nullptr;
   if (need > c->vis_cap) {
-    if (capturing(st)) return nullptr;
+    if (c->vis_refused || capturing(st)) return nullptr;
     dfree(c->vis_w);
     c->vis_cap = 0;
     c->gen++;
-    const size_t want = vis_weight_entries(std::min(c->cap_n, kVisWeightsMax), list_per_of(c));
-    if (hipMalloc(&c->vis_w, sizeof(float4) * std::max(want, need)) != hipSuccess) {
+    const size_t want = std::min(vis_weight_entries(std::min(c->cap_n, kVisWeightsMax), list_per_of(c)), limit);
+    const size_t get = std::max(want, need);
+    if (hipMalloc(&c->vis_w, sizeof(float4) * get) != hipSuccess) {
       (void)hipGetLastError();
       c->vis_w = nullptr;
+      c->vis_refused = true;
       return nullptr;
     }
-    c->vis_cap = std::max(want, need);
+    c->vis_cap = get;
   }
   return c->vis_w;
+}
+
+void reserve_vis(pbf_ctx* c, int n) {
+  c->vis_refused = false;
+  if ((c->p.flags & PBF_FLAG_VISCOSITY) && c->p.viscosity_iterations > 1 && pass_lanes_for(c, n) == 2)
+    (void)vis_weights(c, n, nullptr);
 }
 
 // Buffers for every call over n particles in nscenes scenes.
 int reserve(pbf_ctx* c, int n, int nscenes) {
   const int s = ensure_particles(c, n, nscenes);
-  if (!s && (c->p.flags & PBF_FLAG_VISCOSITY) && c->p.viscosity_iterations > 1 && pass_lanes_for(c, n) == 2)
-    (void)vis_weights(c, n, nullptr);
+  if (!s) reserve_vis(c, n);
   return s;
 }
 
@@ -1554,10 +1570,10 @@ int pbf_set_params(pbf_ctx* c, const pbf_params* p) {
   c->last_n = -1;
   if (c->cap_n > 0) {
     st = ensure_mask(c, mask_words_for(c, c->cap_n));
-    if (st) return st;
-    return ensure_list(c, list_slots_for(c, c->cap_n));
+    if (!st) st = ensure_list(c, list_slots_for(c, c->cap_n));
+    if (!st) reserve_vis(c, c->cap_n - 1);
   }
-  return PBF_OK;
+  return st;
 }
 
 int pbf_get_params(const pbf_ctx* c, pbf_params* out) {

@@ -530,7 +530,71 @@ void blocking_export() {
   pbf_destroy(c);
 }
 
+// The weights that a viscosity solve keeps: bounded in bytes, reserved with the
+// other buffers, and not asked for again in every step once there is no room.
+void viscosity_weights() {
+  constexpr size_t limit = 192u << 20;
+  auto kept = [] {  // whether the last step kept them
+    for (auto l = S().launches.rbegin(); l != S().launches.rend(); ++l)
+      if (l->name == "k_viscosity") return l->full.find("VisWeights)2") != std::string::npos;
+    return false;
+  };
+  Arrays a(300000);
+  pbf_params p = small_params();
+  p.flags = PBF_FLAG_VISCOSITY;
+  for (int slots : {96, 200, 400, 800, 1600})
+    for (int n : {2000, 30000, 65536, 190000}) {
+      p.list_slots = slots;
+      pbf_ctx* c = nullptr;
+      if (pbf_create(&p, &c) != PBF_OK) std::abort();
+      expect(pbf_reserve(c, 190000) == PBF_OK, "reserve");
+      pbf_params none = p;
+      none.flags = 0;
+      size_t without = S().bytes;
+      {  // the context without weights
+        pbf_ctx* d = nullptr;
+        const size_t before = S().bytes;
+        if (pbf_create(&none, &d) != PBF_OK || pbf_reserve(d, 190000) != PBF_OK) std::abort();
+        without = S().bytes - before;
+        pbf_destroy(d);
+      }
+      const size_t all = S().bytes;
+      const long mallocs = S().mallocs;
+      expect(step(c, a, n) == PBF_OK && step(c, a, n) == PBF_OK, "step");
+      const size_t bytes = (size_t)((n + 63) / 64) * (slots / 8) * 128 * 16;
+      expect(kept() == (bytes <= limit), "weights kept up to the limit");
+      if (slots == 96) expect(S().mallocs == mallocs, "weights reserved");
+      pbf_destroy(c);
+      expect(all - S().bytes <= without + limit, "weights within the limit");
+    }
+  // viscosity switched on after the reservation
+  p.list_slots = 0;
+  p.flags = 0;
+  pbf_ctx* c = nullptr;
+  if (pbf_create(&p, &c) != PBF_OK || pbf_reserve(c, 30000) != PBF_OK) std::abort();
+  p.flags = PBF_FLAG_VISCOSITY;
+  expect(pbf_set_params(c, &p) == PBF_OK, "set_params");
+  long mallocs = S().mallocs;
+  S().list_need = 96;
+  expect(step(c, a, 20000) == PBF_OK && kept(), "step");
+  expect(S().mallocs == mallocs, "weights reserved with the parameters");
+  pbf_destroy(c);
+  // no room for them
+  p.flags = 0;
+  if (pbf_create(&p, &c) != PBF_OK || pbf_reserve(c, 30000) != PBF_OK) std::abort();
+  p.flags = PBF_FLAG_VISCOSITY;
+  S().fail_over = 1000;
+  expect(pbf_set_params(c, &p) == PBF_OK, "set_params");
+  mallocs = S().mallocs;
+  for (int k = 0; k < 3; ++k) expect(step(c, a, 20000) == PBF_OK && !kept(), "step without weights");
+  expect(S().mallocs == mallocs, "no allocation tried in a step");
+  S().fail_over = SIZE_MAX;
+  expect(pbf_reserve(c, 30000) == PBF_OK && step(c, a, 20000) == PBF_OK && kept(), "room again");
+  pbf_destroy(c);
+}
+
 const std::map<std::string, void (*)()> kScenarios = {
+    {"viscosity_weights", viscosity_weights},
     {"blocking_export", blocking_export},
     {"last_search", last_search},
     {"failed_rollout", failed_rollout},

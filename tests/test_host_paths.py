@@ -59,3 +59,10 @@ def test_row_starts_are_there_when_the_export_returns(host_paths):
     """A second export of one search takes the row starts counted by the first;
     the caller's copy of them is waited for all the same."""
     run(host_paths, "blocking_export")
+
+
+def test_viscosity_weights(host_paths):
+    """The weights kept over a viscosity solve: up to 192 MiB and no more, reserved by
+    pbf_reserve and pbf_set_params, and not asked for in every step once an
+    allocation has failed."""
+    run(host_paths, "viscosity_weights")
