@@ -352,8 +352,9 @@ int pbf_get_profile(pbf_ctx* ctx, pbf_profile* out);
  * of them changes a result: every setting gives bit-identical outputs. */
 typedef struct pbf_tuning {
   int pass_block;          /* threads per workgroup of the density/lambda and
-                              displacement passes: 64, 128, 256 (default; with a
-                              lane pair per particle they then run 64) or 512 */
+                              displacement passes: 64, 128, 256 (default) or
+                              512. While every field has its default, a lane
+                              pair per particle runs in workgroups of 64 */
   int stage_min_particles; /* as pbf_params.stage_min_particles: searches over at
                               least this many particles stage their neighbor
                               lists in LDS; < 0 never */

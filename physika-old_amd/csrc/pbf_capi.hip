@@ -195,6 +195,7 @@ struct pbf_ctx {
   unsigned long long csr_calls = 0;
 
   int pass_block = kBlock;  // threads per workgroup of the PBD passes (pbf_tuning)
+  bool auto_block = true;   // not chosen by the caller: lane pairs run kPairBlock
   bool pass_persistent = false;  // persistent launches of the PBD passes (pbf_tuning)
   int pass_lanes = 0;            // lanes per particle in the PBD passes, 0 automatic (pbf_tuning)
   int last_lanes = 0;            // lanes per particle of the last step's PBD passes
@@ -1000,10 +1001,10 @@ int reserve(pbf_ctx* c, int n, int nscenes) {
   return s;
 }
 
-// Threads per workgroup of the PBD passes: the context's setting, where the
-// default leaves lane pairs at kPairBlock.
+// Threads per workgroup of the PBD passes: the caller's setting, or by default
+// kPairBlock for lane pairs.
 int pass_block_for(const pbf_ctx* c, int lanes) {
-  return lanes == 2 && c->pass_block == kBlock ? kPairBlock : c->pass_block;
+  return lanes == 2 && c->auto_block ? kPairBlock : c->pass_block;
 }
 
 // One fused step on a batch of scenes (scene_off: device offsets): the state
@@ -2123,6 +2124,8 @@ int pbf_set_tuning(pbf_ctx* c, const pbf_tuning* t) {
   if (t->pass_block != c->pass_block || t->stage_min_particles != c->p.stage_min_particles ||
       (t->persistent != 0) != c->pass_persistent || t->pass_lanes != c->pass_lanes) {
     c->pass_block = t->pass_block;
+    c->auto_block =
+        t->pass_block == kBlock && t->stage_min_particles == 0 && t->persistent == 0 && t->pass_lanes == 0;
     c->p.stage_min_particles = t->stage_min_particles;
     c->pass_persistent = t->persistent != 0;
     c->pass_lanes = t->pass_lanes;

@@ -593,7 +593,56 @@ void viscosity_weights() {
   pbf_destroy(c);
 }
 
+// Threads per workgroup of the PBD passes: 64 for lane pairs by default, what the
+// caller sets otherwise; settings read and set again change nothing, and the
+// autotuner's default (its choice here: all settings take the same time) is the
+// context's.
+void pass_blocks() {
+  Arrays a(300000);
+  pbf_params p = small_params();
+  auto block = [&](pbf_ctx* c, int n) {
+    S().launches.clear();
+    expect(step(c, a, n) == PBF_OK, "step");
+    unsigned b = 0;
+    for (const Launch& l : S().launches)
+      if (l.name == "k_density_lambda2" || l.name == "k_displacement2" || l.name == "k_density_lambda" ||
+          l.name == "k_displacement") {
+        if (b && b != l.block) violation("two block sizes");
+        b = l.block;
+      }
+    return (int)b;
+  };
+  for (int smin : {0, -1}) {
+    p.stage_min_particles = smin;
+    pbf_ctx* c = nullptr;
+    if (pbf_create(&p, &c) != PBF_OK) std::abort();
+    expect(block(c, 2000) == 64, "the default, lane pairs");
+    if (smin == 0) expect(block(c, 280000) == 256, "the default, one lane");
+    pbf_tuning t;
+    expect(pbf_get_tuning(c, &t) == PBF_OK && t.pass_block == 256 && pbf_set_tuning(c, &t) == PBF_OK, "round trip");
+    expect(block(c, 2000) == 64, "the default set again");
+    for (int lanes : {0, 2, 1})
+      for (int stage : {-1, 1})
+        for (int b : {64, 128, 256, 512}) {
+          t = pbf_tuning{b, stage, 0, lanes};
+          expect(pbf_set_tuning(c, &t) == PBF_OK && block(c, 2000) == b, "a block that the caller set");
+        }
+    t = pbf_tuning{256, 0, 0, 0};
+    expect(pbf_set_tuning(c, &t) == PBF_OK && block(c, 2000) == 64, "back to the defaults");
+    pbf_tune_report r;
+    S().launches.clear();
+    expect(pbf_autotune(c, a.x, a.v, nullptr, 1, 2000, 1, nullptr, &r, nullptr) == PBF_OK, "autotune");
+    expect(r.best.pass_block == 256 && r.best.stage_min_particles == 0, "its choice");
+    bool pair256 = false;
+    for (const Launch& l : S().launches) pair256 |= l.name == "k_density_lambda2" && l.block == 256;
+    expect(pair256, "it times lane pairs in workgroups of 256");
+    expect(block(c, 2000) == 64, "its default is the context's");
+    pbf_destroy(c);
+  }
+}
+
 const std::map<std::string, void (*)()> kScenarios = {
+    {"pass_blocks", pass_blocks},
     {"viscosity_weights", viscosity_weights},
     {"blocking_export", blocking_export},
     {"last_search", last_search},

@@ -66,3 +66,9 @@ def test_viscosity_weights(host_paths):
     pbf_reserve and pbf_set_params, and not asked for in every step once an
     allocation has failed."""
     run(host_paths, "viscosity_weights")
+
+
+def test_pass_block_that_the_caller_sets(host_paths):
+    """pbf_tuning.pass_block is what the PBD passes run, lane pairs included; only the
+    default settings leave it to the library (64 for lane pairs)."""
+    run(host_paths, "pass_blocks")
