@@ -330,7 +330,7 @@ __device__ __forceinline__ bool vis_half(const NbrView& nv, int s, int h, float4
                                          const float4* __restrict__ v_in, float4* __restrict__ wt,
                                          const VisConst& vc, VisSums& t) {
   const int wave = __builtin_amdgcn_readfirstlane(s >> 6);
-  ListHead head;
+  ListHead<> head;
   head.load(nv, wave, s);
   const WaveList& wl = head.wl;
   const int mode = wl.lm & 3;
@@ -415,9 +415,11 @@ __device__ __forceinline__ bool vis_half(const NbrView& nv, int s, int h, float4
 // lane), with the weights kept over the iterations where kW says so; all forms
 // give the same bits. At 100,000 particles 18.0 us an iteration without the
 // weights; with them 22.5 the first and 14.0 the others, where four gathers of
-// twelve bytes and sixteen bytes of weights remain for four entries.
+// twelve bytes and sixteen bytes of weights remain for four entries. A lane pair
+// without weights is held to the registers of five waves per SIMD: with four, 195,000
+// particles with rows of 440 neighbors are two rounds (a step 2,024 us, 1,975 with five).
 template <bool kPair, VisWeights kW>
-__global__ __launch_bounds__(kBlock) void k_viscosity(NbrView nv, const float4* __restrict__ xs,
+__global__ __launch_bounds__(kBlock, kPair && kW == kVisNone ? 5 : 1) void k_viscosity(NbrView nv, const float4* __restrict__ xs,
                                                       const float4* __restrict__ v_old,
                                                       const float4* __restrict__ v_in, float4* __restrict__ v_next,
                                                       VisConst vc, const int* __restrict__ perm,

@@ -1002,9 +1002,9 @@ int reserve(pbf_ctx* c, int n, int nscenes) {
 }
 
 // Threads per workgroup of the PBD passes: the caller's setting, or by default
-// kPairBlock for lane pairs.
+// kPairBlock for lane pairs, unless their lists are long.
 int pass_block_for(const pbf_ctx* c, int lanes) {
-  return lanes == 2 && c->auto_block ? kPairBlock : c->pass_block;
+  return lanes == 2 && c->auto_block && list_per_of(c) <= kLongLists ? kPairBlock : c->pass_block;
 }
 
 // One fused step on a batch of scenes (scene_off: device offsets): the state

@@ -277,6 +277,13 @@ void launch_wave_stats(const int4* wave_stat, int n, unsigned long long* counter
 // 32,768 2,013 -> 1,986; a frame at 1,728 95.5 -> 93.1; four steps and gradient in
 // double at 8 x 5,000 2.47 -> 2.12 ms. One lane per particle (1M): 64, 128 and 256 alike.
 constexpr int kPairBlock = 64;
+// With lists of more than kLongLists reserved slots the PBD passes' lane pairs keep
+// 256 threads: many rounds of gathers even the last round out, and four list
+// waves together share more of their neighbors. Rows of 440 neighbors (496
+// slots), one step, 64 and 256 threads: 65,536 particles 448 and 432 us, 131,072
+// 983 and 953, 262,143 1,770 and 1,650, but 100,003 890 and 908; rows of 270 (304
+// slots) 305 and 298, 614 and 606, 1,010 and 998, but 540 and 575.
+constexpr int kLongLists = 384;
 // block: threads per workgroup, 64, 128, 256 or 512; persistent: as many
 // blocks as stay resident, each wave walking 64-particle tiles; lanes: 1, or 2
 // for a lane pair per particle (not persistent). The results depend on none of

@@ -396,17 +396,21 @@ __device__ __forceinline__ WaveList wave_list(const NbrView& nv, int wave) {
 // the first two chunks of its list (where the wave's list lies if it has one: at
 // the start of the wave's region; the allocation is padded by two chunks of a
 // wave) and the wave's words. Were the words read first, a search of few waves
-// would wait once more on memory.
-struct ListHead {
+// would wait once more on memory. kTwo false: chunk 1 is left to the traversal,
+// which saves the registers of a wave in flight.
+template <bool kTwo = true> struct ListHead {
   WaveList wl;
   const uint4* L;  // the wave's region at this particle's lane
   int cnt;
   uint4 c0, c1;    // chunks 0 and 1
+  __device__ __forceinline__ uint4 second(int count) const {  // chunk 1 of a lane's count entries
+    return kTwo ? c1 : L[count > 4 ? 64 : 0];
+  }
   __device__ __forceinline__ void load(const NbrView& nv, int wave, int s) {
     L = reinterpret_cast<const uint4*>(nv.list + (long long)wave * 64 * nv.list_per) + (s & 63);
     cnt = nv.nbr_cnt[s];
     c0 = L[0];
-    c1 = L[64];
+    if (kTwo) c1 = L[64];
     wl = wave_list(nv, wave);
     asm volatile("" ::: "memory");  // issue the loads here
   }
@@ -603,11 +607,11 @@ __device__ __forceinline__ void for_each_neighbor_staged(const NbrView& nv, int 
 // own stage region (both waves of a list copy its stage). Returns false, with
 // nothing run, when s's wave has no 16-bit or staged list; the caller then
 // runs the list on one lane of the pair.
-template <bool kW, class Body>
+template <bool kW, bool kTwo, class Body>
 __device__ __forceinline__ bool for_each_neighbor_half(const NbrView& nv, int s, int h, const float4* __restrict__ xs,
                                                        float4* buf, Body&& body) {
   const int wave = __builtin_amdgcn_readfirstlane(s >> 6);
-  ListHead head;
+  ListHead<kTwo> head;
   head.load(nv, wave, s);
   const WaveList& wl = head.wl;
   const int mode = wl.lm & 3;
@@ -626,7 +630,7 @@ __device__ __forceinline__ bool for_each_neighbor_half(const NbrView& nv, int s,
     const uint32_t sh = (uint32_t)h << 4;
     if (ch > 0)
       list_loop_from<true, uint4>(
-        ch, nfull, head.c0, head.c1, [&](int c) { return L[(long long)c << 6]; },
+        ch, nfull, head.c0, head.second(ch), [&](int c) { return L[(long long)c << 6]; },
         [&](uint4 e, int c, auto full) {
           return decode_half<decltype(full)::value, 16>(e, sh, jb16, c, ch, past);
         },
@@ -695,7 +699,7 @@ template <int kRec, class GatherFn, class Body>
 __device__ __forceinline__ bool for_each_record_half(const NbrView& nv, int s, int h, GatherFn&& gather,
                                                      Body&& body) {
   const int wave = __builtin_amdgcn_readfirstlane(s >> 6);
-  ListHead head;
+  ListHead<> head;
   head.load(nv, wave, s);
   const WaveList& wl = head.wl;
   const int mode = wl.lm & 3;

@@ -764,9 +764,12 @@ __device__ __forceinline__ void density_lambda_at(const NbrView& nv, int s, floa
   density_lambda_finish(s, xs, pc, rho_out, perm, aux, t);
 }
 
+constexpr int kPairWaves = 5, kSimds = 4 * 256;  // see pair_waves
+
 // Pass A with a lane pair per particle (lane h = 0 the even entries, 1 the
 // odd ones; stage: the hardware wave's LDS region). Same results as
 // density_lambda_at, bit for bit.
+template <bool kTwo>
 __device__ __forceinline__ void density_lambda_at2(const NbrView& nv, int s, int h, float4* __restrict__ xs,
                                                    const PhysConst& pc, float* __restrict__ rho_out,
                                                    const int* __restrict__ perm, float4* __restrict__ aux,
@@ -774,7 +777,7 @@ __device__ __forceinline__ void density_lambda_at2(const NbrView& nv, int s, int
   if (s >= nv.n) return;  // both lanes of the pair
   const float4 xi = xs[s];
   DensitySums a;
-  if (for_each_neighbor_half<false>(nv, s, h, xs, stage, [&](float4 xj) { density_term(a, xi, xj, pc); })) {
+  if (for_each_neighbor_half<false, kTwo>(nv, s, h, xs, stage, [&](float4 xj) { density_term(a, xi, xj, pc); })) {
     const DensitySums o = partner_sums(a);
     if (h == 0) density_lambda_finish(s, xs, pc, rho_out, perm, aux, add_parities(a, o));
     return;
@@ -799,13 +802,13 @@ __global__ __launch_bounds__(B) void k_density_lambda(NbrView nv, float4* __rest
 
 // Lane-pair form: thread g of the grid takes entry parity g & 1 of particle
 // g >> 1, so a wave holds 32 particles of one 64-particle list wave.
-template <int B>
-__global__ __launch_bounds__(B) void k_density_lambda2(NbrView nv, float4* __restrict__ xs, PhysConst pc,
+template <int B, int W>
+__global__ __launch_bounds__(B, W == kPairWaves ? 1 : W) void k_density_lambda2(NbrView nv, float4* __restrict__ xs, PhysConst pc,
                                                        float* __restrict__ rho_out, const int* __restrict__ perm,
                                                        float4* __restrict__ aux) {
   __shared__ float4 stage_buf[B / 64][kStageRecords];
   const int g = particle_block(nv) * blockDim.x + threadIdx.x;
-  density_lambda_at2(nv, g >> 1, g & 1, xs, pc, rho_out, perm, aux, stage_buf[threadIdx.x >> 6]);
+  density_lambda_at2<W == kPairWaves>(nv, g >> 1, g & 1, xs, pc, rho_out, perm, aux, stage_buf[threadIdx.x >> 6]);
 }
 
 // Persistent form: as many blocks as stay resident; each wave walks the
@@ -860,11 +863,22 @@ void launch_timed(K kernel, int grid, int block, hipStream_t st, const KernelEve
     kernel<<<grid, block, 0, st>>>(args...);
 }
 
+// Waves per SIMD that a lane-pair launch over n particles keeps: kPairWaves, which
+// leaves the registers to read two list chunks ahead, or one more where that
+// saves a round of waves. One wave more costs 1% at most sizes (100,003 particles
+// 511 -> 520 us for three steps), a round of waves more 4% (195,000: 740 -> 770).
+int pair_waves(int n) {
+  const long long waves = (2ll * n + 63) / 64;
+  auto rounds = [&](int w) { return (waves + w * kSimds - 1) / (w * kSimds); };
+  return rounds(kPairWaves + 1) < rounds(kPairWaves) ? kPairWaves + 1 : kPairWaves;
+}
+
 template <int B>
 void density_lambda_as(const NbrView& nv, float4* xs, const PhysConst& pc, float* rho_out, const int* perm,
                        hipStream_t st, float4* aux, bool persistent, int lanes, const KernelEvents* ev) {
   if (lanes == 2) {
-    launch_timed(k_density_lambda2<B>, (int)((2ll * nv.n + B - 1) / B), B, st, ev, nv, xs, pc, rho_out, perm, aux);
+    launch_timed(pair_waves(nv.n) == kPairWaves ? k_density_lambda2<B, kPairWaves> : k_density_lambda2<B, kPairWaves + 1>,
+                 (int)((2ll * nv.n + B - 1) / B), B, st, ev, nv, xs, pc, rho_out, perm, aux);
   } else if (persistent) {
     static const int resident = resident_blocks(k_density_lambda_p<B>, B);  // one device type per process
     launch_timed(k_density_lambda_p<B>, persistent_grid(resident, B, nv.n), B, st, ev, nv, xs, pc, rho_out, perm,
@@ -1036,6 +1050,7 @@ __device__ __forceinline__ void displacement_at(const NbrView& nv, int s, const 
 }
 
 // Pass B with a lane pair per particle, as density_lambda_at2.
+template <bool kTwo>
 __device__ __forceinline__ void displacement_at2(const NbrView& nv, int s, int h, const float4* __restrict__ xs,
                                                  float4* __restrict__ xd, const PhysConst& pc, int last,
                                                  const float4* __restrict__ x0, const float4* __restrict__ vs,
@@ -1047,7 +1062,7 @@ __device__ __forceinline__ void displacement_at2(const NbrView& nv, int s, int h
   const float4 xi = xs[s];
   const bool any_oog = nv.counters[C_OOG] != 0;
   DispSums a;
-  if (for_each_neighbor_half<true>(nv, s, h, xs, stage, [&](float4 xj) { disp_term(a, xi, xj, pc); })) {
+  if (for_each_neighbor_half<true, kTwo>(nv, s, h, xs, stage, [&](float4 xj) { disp_term(a, xi, xj, pc); })) {
     const DispSums o = partner_sums(a);
     if (h == 0)
       displacement_finish(nv, s, xs, xd, pc, last, x0, vs, perm, x_out, v_out, v_sorted, id_out, xi,
@@ -1076,8 +1091,8 @@ __global__ __launch_bounds__(B) void k_displacement(NbrView nv, const float4* __
                   stage_buf[threadIdx.x >> 6]);
 }
 
-template <int B>
-__global__ __launch_bounds__(B) void k_displacement2(NbrView nv, const float4* __restrict__ xs,
+template <int B, int W>
+__global__ __launch_bounds__(B, W == kPairWaves ? 1 : W) void k_displacement2(NbrView nv, const float4* __restrict__ xs,
                                                      float4* __restrict__ xd, PhysConst pc, int last,
                                                      const float4* __restrict__ x0, const float4* __restrict__ vs,
                                                      const int* __restrict__ perm, float* __restrict__ x_out,
@@ -1085,7 +1100,7 @@ __global__ __launch_bounds__(B) void k_displacement2(NbrView nv, const float4* _
                                                      int* __restrict__ id_out) {
   __shared__ float4 stage_buf[B / 64][kStageRecords];
   const int g = particle_block(nv) * blockDim.x + threadIdx.x;
-  displacement_at2(nv, g >> 1, g & 1, xs, xd, pc, last, x0, vs, perm, x_out, v_out, v_sorted, id_out,
+  displacement_at2<W == kPairWaves>(nv, g >> 1, g & 1, xs, xd, pc, last, x0, vs, perm, x_out, v_out, v_sorted, id_out,
                    stage_buf[threadIdx.x >> 6]);
 }
 
@@ -1112,8 +1127,9 @@ void displacement_as(const NbrView& nv, const float4* xs, float4* xd, const Phys
                      float4* v_sorted, int* id_out, bool persistent, int lanes, const KernelEvents* ev) {
   const int l = last ? 1 : 0;
   if (lanes == 2) {
-    launch_timed(k_displacement2<B>, (int)((2ll * nv.n + B - 1) / B), B, st, ev, nv, xs, xd, pc, l, x0, vs, perm,
-                 x_out, v_out, v_sorted, id_out);
+    launch_timed(pair_waves(nv.n) == kPairWaves ? k_displacement2<B, kPairWaves> : k_displacement2<B, kPairWaves + 1>,
+                 (int)((2ll * nv.n + B - 1) / B), B, st, ev, nv, xs, xd, pc, l, x0, vs, perm, x_out, v_out, v_sorted,
+                 id_out);
   } else if (persistent) {
     static const int resident = resident_blocks(k_displacement_p<B>, B);  // one device type per process
     launch_timed(k_displacement_p<B>, persistent_grid(resident, B, nv.n), B, st, ev, nv, xs, xd, pc, l, x0, vs,

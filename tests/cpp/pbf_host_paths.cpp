@@ -627,7 +627,13 @@ void pass_blocks() {
           t = pbf_tuning{b, stage, 0, lanes};
           expect(pbf_set_tuning(c, &t) == PBF_OK && block(c, 2000) == b, "a block that the caller set");
         }
-    t = pbf_tuning{256, 0, 0, 0};
+    pbf_params q = p;
+    q.list_slots = 400;
+    expect(pbf_set_tuning(c, &(t = pbf_tuning{256, 0, 0, 0})) == PBF_OK, "the defaults");
+    pbf_ctx* wide = nullptr;
+    if (pbf_create(&q, &wide) != PBF_OK) std::abort();
+    expect(block(wide, 2000) == 256, "the default, lane pairs with long lists");
+    pbf_destroy(wide);
     expect(pbf_set_tuning(c, &t) == PBF_OK && block(c, 2000) == 64, "back to the defaults");
     pbf_tune_report r;
     S().launches.clear();
