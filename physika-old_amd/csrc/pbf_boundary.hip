@@ -477,13 +477,13 @@ void launch_viscosity(const NbrView& nv, const float4* xs, const float4* v_old, 
 // Module path: one iteration over a caller CSR list in original order
 // (positions xa as float4; v_old, v_in float4; the last iteration writes the
 // caller's packed velocities).
-template <int kThreads>
+template <int kThreads, int kL>
 __global__ __launch_bounds__(kThreads) void k_csr_viscosity(const float4* __restrict__ xa, Csr nb,
                                                           const float4* __restrict__ v_old,
                                                           const float4* __restrict__ v_in,
                                                           float4* __restrict__ v_next, float* __restrict__ v_out,
                                                           VisConst vc) {
-  const CsrRow row = csr_row<kThreads>(nb);
+  const CsrRow<kL> row = csr_row<kL, kThreads>(nb);
   if (row.i >= nb.n) return;
   const int i = row.i;
   const float4 xi = xa[i];
@@ -501,10 +501,10 @@ __global__ __launch_bounds__(kThreads) void k_csr_viscosity(const float4* __rest
         }
       },
       [] {}, [] {});
-  tw = row_sum(tw);
-  dx = row_sum(dx);
-  dy = row_sum(dy);
-  dz = row_sum(dz);
+  tw = row_sum<kL>(tw);
+  dx = row_sum<kL>(dx);
+  dy = row_sum<kL>(dy);
+  dz = row_sum<kL>(dz);
   if (row.lane != 0) return;
   const float b = tw < vc.eps ? 0.0f : vc.b;
   tw = tw < vc.eps ? 1.0f : tw;
@@ -527,10 +527,15 @@ void launch_csr_viscosity(const float4* xa, const Csr& nb, const float4* v_old, 
   // few rows: workgroups of 64 threads (see kPairBlock). Five iterations, us: 33.9 ->
   // 29.2 at 2,000 rows, 74.7 -> 68.0 at 50,000, 90.4 -> 86.6 at 70,000, but 158.6 ->
   // 165.5 at 131,072
-  if (nb.n <= 65536)
-    k_csr_viscosity<64><<<csr_blocks(nb.n, 64), 64, 0, st>>>(xa, nb, v_old, v_in, v_next, v_out, vc);
+  auto run = [&](auto* kernel, int lanes, int block) {
+    kernel<<<csr_blocks(nb.n, lanes, block), block, 0, st>>>(xa, nb, v_old, v_in, v_next, v_out, vc);
+  };
+  if (row_lanes(nb) == 1)
+    run(k_csr_viscosity<kBlock, 1>, 1, kBlock);
+  else if (nb.n <= 65536)
+    run(k_csr_viscosity<64, kRowLanes>, kRowLanes, 64);
   else
-    k_csr_viscosity<kBlock><<<csr_blocks(nb.n), kBlock, 0, st>>>(xa, nb, v_old, v_in, v_next, v_out, vc);
+    run(k_csr_viscosity<kBlock, kRowLanes>, kRowLanes, kBlock);
 }
 
 }  // namespace pbf

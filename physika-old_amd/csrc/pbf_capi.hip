@@ -24,7 +24,7 @@ using namespace pbf;
 // In host code the name is no device address: each device's copy is looked
 // up once (scratch_address) and only that pointer reaches kernels.
 static __device__ __align__(256) unsigned char
-    scratch[2 * (size_t)PBF_NOALLOC_MAX_PARTICLES * sizeof(float4) + kPairingSlots * sizeof(unsigned long long)];
+    scratch[2 * (size_t)PBF_NOALLOC_MAX_PARTICLES * sizeof(float4) + kPairingWords * sizeof(unsigned long long)];
 
 struct pbf_ctx {
   pbf_params p{};
@@ -55,7 +55,7 @@ struct pbf_ctx {
   int *nbr_cnt = nullptr, *cnt_orig = nullptr;
   float4 *xn = nullptr, *x0 = nullptr, *xa = nullptr, *xb = nullptr, *vs = nullptr, *vv = nullptr;
   float* xc = nullptr;  // sorted x^n as three coordinate planes of cap + kXnPad floats
-  unsigned long long* pairing = nullptr;  // kPairingSlots: pairing sums of a caller's list
+  unsigned long long* pairing = nullptr;  // kPairingWords: pairing sums of a caller's list
   // neighbor pass output: per-wave metadata, bit masks (scratch), lists
   long long* mask_base = nullptr;
   long long* list_base = nullptr;
@@ -1500,7 +1500,7 @@ int pbf_create(const pbf_params* p, pbf_ctx** out) {
       hipMalloc(&c->scan_part, sizeof(int) * 2 * kScanDevBlocks) != hipSuccess ||
       hipMalloc(&c->ticket, sizeof(int)) != hipSuccess || hipMemset(c->ticket, 0, sizeof(int)) != hipSuccess ||
       hipMalloc(&c->list_none, sizeof(uint16_t) * kListPad) != hipSuccess ||
-      hipMalloc(&c->pairing, sizeof(unsigned long long) * kPairingSlots) != hipSuccess) {
+      hipMalloc(&c->pairing, sizeof(unsigned long long) * kPairingWords) != hipSuccess) {
     pbf_destroy(c);
     return PBF_ERR_HIP;
   }

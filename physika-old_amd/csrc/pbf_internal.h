@@ -373,9 +373,11 @@ void launch_integrate(float* x, float* v, const float* f, int n, const PhysConst
 void launch_csr_density(const float* x, const Csr& nb, float* rho, const PhysConst& pc, hipStream_t st);
 void launch_aos_to_f4(const float* x, float4* xa, int n, hipStream_t st);
 // DensityPBD::constrain, K rounds, over a caller list of any form: xa and xb
-// hold n float4 each, pairing kPairingSlots words (nothing of them is read
-// before it is written).
-constexpr int kPairingSlots = 16;
+// hold n float4 each, pairing kPairingWords words (nothing of them is read
+// before it is written): kPairingSlots sums, each in a line of its own, since the
+// blocks' atomics to one line wait for each other (15,625 blocks, 1,000,000 rows: 78 us
+// of a first pass of 100, 3 of 14 with a line each and one lane per row).
+constexpr int kPairingSlots = 16, kPairingStride = 16, kPairingWords = kPairingSlots * kPairingStride;
 void launch_csr_constrain(float4* xa, float4* xb, unsigned long long* pairing, const Csr& nb, float* x, float* v,
                           float* rho, const PhysConst& pc, int K, const float* minv, hipStream_t st);
 // Fixed-capacity rows (the `limit` nearest of each neighbor set, by distance

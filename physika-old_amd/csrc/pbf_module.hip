@@ -60,23 +60,28 @@ __device__ __forceinline__ void csr_finish(int i, float4 p, float* __restrict__ 
 }
 
 // K_ComputeDensity (SummationDensity.cu:13-36) over a CSR list.
+template <int kL>
 __global__ __launch_bounds__(kBlock) void k_csr_density(const float* __restrict__ x, Csr nb,
                                                         float* __restrict__ rho, PhysConst pc, int first) {
-  const CsrRow row = csr_row(nb, first);
+  const CsrRow<kL> row = csr_row<kL>(nb, first);
   if (row.i >= nb.n) return;
   const float4 xi = load3(x, row.i);
   float acc = 0.f, t[kRowUnroll];
   csr_each(
       nb, row, [&](int j) { return load3(x, j); },
       [&](int u, int, float4 xj) { t[u] = pair_geom(xi, xj, pc.inv_h).t; },
-      [&] { row_clear(t); }, [&] { acc = row_cubes(acc, t); });
+      [&] { row_clear(t); }, [&] { acc = row_cubes<kL>(acc, t); });
   if (row.lane == 0) rho[row.i] = acc * pc.cW;
 }
 
 void launch_csr_density(const float* x, const Csr& nb, float* rho, const PhysConst& pc, hipStream_t st) {
   for (long long first = 0; first < nb.n; first += kRowsPerLaunch) {
     const int rows = (int)std::min<long long>(nb.n - first, kRowsPerLaunch);
-    k_csr_density<<<csr_blocks(rows), kBlock, 0, st>>>(x, nb, rho, pc, (int)first);
+    const int lanes = row_lanes(nb), blocks = csr_blocks(rows, lanes);
+    if (lanes == 1)
+      k_csr_density<1><<<blocks, kBlock, 0, st>>>(x, nb, rho, pc, (int)first);
+    else
+      k_csr_density<kRowLanes><<<blocks, kBlock, 0, st>>>(x, nb, rho, pc, (int)first);
   }
 }
 
@@ -96,7 +101,7 @@ __global__ __launch_bounds__(kBlock) void k_csr_begin(const float* __restrict__ 
                                                       float4* __restrict__ xb, int n,
                                                       unsigned long long* __restrict__ pairing) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < kPairingSlots) pairing[i] = 0ull;
+  if (i < kPairingWords) pairing[i] = 0ull;
   if (i >= n) return;
   xa[i] = load3(x, i);
   xb[i] = make_float4(0.f, 0.f, 0.f, 0.f);
@@ -124,7 +129,7 @@ __device__ __forceinline__ unsigned long long pairing_s(unsigned long long r) {
 __device__ __forceinline__ bool csr_paired(const unsigned long long* __restrict__ pairing) {
   unsigned long long v = 0;
 #pragma unroll
-  for (int k = 0; k < kPairingSlots; ++k) v += pairing[k];
+  for (int k = 0; k < kPairingSlots; ++k) v += pairing[k * kPairingStride];
   return v == 0ull;
 }
 
@@ -135,17 +140,25 @@ __device__ __forceinline__ float4* csr_iterate(float4* xa, float4* xb, bool pair
   return paired && (it & 1) ? xb : xa;
 }
 
+// The displacement sums of particle j of any other list: three floats each, packed.
+// The atomics of neighboring particles fall into fewer lines than with a float4
+// each: five iterations at 262,144 rows of 3 elements 575 -> 522 us, of 72 9,970 ->
+// 8,990.
+__device__ __forceinline__ float* csr_sums(float4* xb, int j) {
+  return reinterpret_cast<float*>(xb) + 3 * (size_t)j;
+}
+
 // Density and K_ComputeLambdas (DensityPBD.cu:46-90) over a CSR list; lambda
 // goes to w of the iterate. With minv (inverse masses) the massInv variant
 // (DensityPBD.cu:93-131): S = sum_j |g|^2 m_j^-1 + |sum g|^2 m_i^-1. The first
 // iteration (kFirst) also adds up the pairing sums of the rows.
-template <bool kFirst, bool kMass>
+template <bool kFirst, bool kMass, int kL>
 __global__ __launch_bounds__(kBlock) void k_csr_lambda(float4* xa, float4* xb, int it, Csr nb,
                                                        float* __restrict__ rho, PhysConst pc,
                                                        const float* __restrict__ minv,
                                                        unsigned long long* __restrict__ pairing) {
   float4* xs = kFirst ? xa : csr_iterate(xa, xb, csr_paired(pairing), it);
-  const CsrRow row = csr_row(nb);
+  const CsrRow<kL> row = csr_row<kL>(nb);
   const bool active = row.i < nb.n;
   unsigned long long sum_r = 0, sum_s = 0;
   if (active) {
@@ -171,12 +184,12 @@ __global__ __launch_bounds__(kBlock) void k_csr_lambda(float4* xa, float4* xb, i
             sum_s += pairing_s(r);
           }
         },
-        [&] { row_clear(t); }, [&] { acc = row_cubes(acc, t); });
+        [&] { row_clear(t); }, [&] { acc = row_cubes<kL>(acc, t); });
     acc *= pc.cW;
-    sgx = row_sum(sgx);
-    sgy = row_sum(sgy);
-    sgz = row_sum(sgz);
-    sgg = row_sum(sgg);
+    sgx = row_sum<kL>(sgx);
+    sgy = row_sum<kL>(sgy);
+    sgz = row_sum<kL>(sgz);
+    sgg = row_sum<kL>(sgg);
     if (row.lane == 0) {
       const float G2 = sgx * sgx + sgy * sgy + sgz * sgz;
       const float S = (pc.cG * pc.cG) * (sgg + (kMass ? G2 * minv[i] : G2));
@@ -197,7 +210,7 @@ __global__ __launch_bounds__(kBlock) void k_csr_lambda(float4* xa, float4* xb, i
     __syncthreads();
     if (threadIdx.x == 0) {
       for (int w = 1; w < kBlock / 64; ++w) v += part[w];
-      atomicAdd(&pairing[blockIdx.x % kPairingSlots], v);
+      atomicAdd(&pairing[blockIdx.x % kPairingSlots * kPairingStride], v);
     }
   }
 }
@@ -209,19 +222,19 @@ __global__ __launch_bounds__(kBlock) void k_csr_lambda(float4* xa, float4* xb, i
 // dp_ji = -dp_ij: row i alone gives 2 sum_j dp_ij, with no atomics and in a
 // fixed order. Any other list takes float atomics on the displacement sums (in
 // xb), as the reference, applied by k_csr_apply. The atomics are what the
-// general form costs: 2,106 us per pass at 262,144 particles (18.9M pairs, about
-// 27 G atomics/s), against 36 us without. With minv the massInv variant
+// general form costs: 1,747 us per pass at 262,144 particles (18.9M pairs, about
+// 32 G atomics/s), against 36 us without. With minv the massInv variant
 // (DensityPBD.cu:182-224): dp_ij m_i^-1 to i, -dp_ij m_j^-1 to j. The last
 // iteration of a paired list also makes the velocity update
 // (DensityPBD.cu:368-378) and writes the caller's arrays.
-template <bool kMass>
+template <bool kMass, int kL>
 __global__ __launch_bounds__(kBlock) void k_csr_displacement(float4* xa, float4* xb, int it, int last, Csr nb,
                                                              PhysConst pc, const float* __restrict__ minv,
                                                              const unsigned long long* __restrict__ pairing,
                                                              float* __restrict__ x, float* __restrict__ v) {
   const bool paired = csr_paired(pairing);
   const float4* xs = csr_iterate(xa, xb, paired, it);
-  const CsrRow row = csr_row(nb);
+  const CsrRow<kL> row = csr_row<kL>(nb);
   if (row.i >= nb.n) return;
   const int i = row.i;
   const float4 xi = xs[i];
@@ -241,9 +254,9 @@ __global__ __launch_bounds__(kBlock) void k_csr_displacement(float4* xa, float4*
         },
         [] {}, [] {});
     const float k = 2.0f * mi;
-    ax = row_sum(ax);
-    ay = row_sum(ay);
-    az = row_sum(az);
+    ax = row_sum<kL>(ax);
+    ay = row_sum<kL>(ay);
+    az = row_sum<kL>(az);
     if (row.lane != 0) return;
     const float nx = fmaf(k, ax, xi.x), ny = fmaf(k, ay, xi.y), nz = fmaf(k, az, xi.z);
     if (last)
@@ -262,17 +275,17 @@ __global__ __launch_bounds__(kBlock) void k_csr_displacement(float4* xa, float4*
         ax += px * mi;
         ay += py * mi;
         az += pz * mi;
-        float* d = reinterpret_cast<float*>(xb + j);
+        float* d = csr_sums(xb, j);
         atomicAdd(d, -px * q.m);
         atomicAdd(d + 1, -py * q.m);
         atomicAdd(d + 2, -pz * q.m);
       },
       [] {}, [] {});
-  ax = row_sum(ax);
-  ay = row_sum(ay);
-  az = row_sum(az);
+  ax = row_sum<kL>(ax);
+  ay = row_sum<kL>(ay);
+  az = row_sum<kL>(az);
   if (row.lane != 0) return;
-  float* d = reinterpret_cast<float*>(xb + i);
+  float* d = csr_sums(xb, i);
   atomicAdd(d, ax);
   atomicAdd(d + 1, ay);
   atomicAdd(d + 2, az);
@@ -288,16 +301,16 @@ __global__ __launch_bounds__(kBlock) void k_csr_apply(float4* __restrict__ xa, f
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= n) return;
   float4 p = xa[i];
-  const float4 d = xb[i];
-  p.x += d.x;
-  p.y += d.y;
-  p.z += d.z;
+  float* d = csr_sums(xb, i);
+  p.x += d[0];
+  p.y += d[1];
+  p.z += d[2];
   if (last) {
     csr_finish(i, p, x, v, dt);
     return;
   }
   xa[i] = p;
-  xb[i] = make_float4(0.f, 0.f, 0.f, 0.f);
+  d[0] = d[1] = d[2] = 0.f;
 }
 
 // x := x + 0 and v := v + 0/dt of a constraint without iterations
@@ -308,18 +321,18 @@ __global__ __launch_bounds__(kBlock) void k_csr_finish(const float4* __restrict_
   if (i < n) csr_finish(i, xa[i], x, v, dt);
 }
 
-template <bool kMass>
+template <bool kMass, int kL>
 void csr_rounds(float4* xa, float4* xb, unsigned long long* pairing, const Csr& nb, float* x, float* v, float* rho,
                 const PhysConst& pc, int K, const float* minv, hipStream_t st) {
-  const int nb1 = (nb.n + kBlock - 1) / kBlock, nbr = csr_blocks(nb.n);
+  const int nb1 = (nb.n + kBlock - 1) / kBlock, nbr = csr_blocks(nb.n, kL);
   for (int it = 0; it < K; ++it) {
     const int last = it + 1 == K;
     float* r = last ? rho : nullptr;
     if (it == 0)
-      k_csr_lambda<true, kMass><<<nbr, kBlock, 0, st>>>(xa, xb, it, nb, r, pc, minv, pairing);
+      k_csr_lambda<true, kMass, kL><<<nbr, kBlock, 0, st>>>(xa, xb, it, nb, r, pc, minv, pairing);
     else
-      k_csr_lambda<false, kMass><<<nbr, kBlock, 0, st>>>(xa, xb, it, nb, r, pc, minv, pairing);
-    k_csr_displacement<kMass><<<nbr, kBlock, 0, st>>>(xa, xb, it, last, nb, pc, minv, pairing, x, v);
+      k_csr_lambda<false, kMass, kL><<<nbr, kBlock, 0, st>>>(xa, xb, it, nb, r, pc, minv, pairing);
+    k_csr_displacement<kMass, kL><<<nbr, kBlock, 0, st>>>(xa, xb, it, last, nb, pc, minv, pairing, x, v);
     k_csr_apply<<<nb1, kBlock, 0, st>>>(xa, xb, nb.n, last, pairing, x, v, pc.dt);
   }
   if (K == 0) k_csr_finish<<<nb1, kBlock, 0, st>>>(xa, x, v, nb.n, pc.dt);
@@ -327,12 +340,13 @@ void csr_rounds(float4* xa, float4* xb, unsigned long long* pairing, const Csr& 
 
 void launch_csr_constrain(float4* xa, float4* xb, unsigned long long* pairing, const Csr& nb, float* x, float* v,
                           float* rho, const PhysConst& pc, int K, const float* minv, hipStream_t st) {
-  const int blocks = (std::max(nb.n, kPairingSlots) + kBlock - 1) / kBlock;
+  const int blocks = (std::max(nb.n, kPairingWords) + kBlock - 1) / kBlock;
   k_csr_begin<<<blocks, kBlock, 0, st>>>(x, xa, xb, nb.n, pairing);
-  if (minv)
-    csr_rounds<true>(xa, xb, pairing, nb, x, v, rho, pc, K, minv, st);
+  auto run = [&](auto* rounds) { rounds(xa, xb, pairing, nb, x, v, rho, pc, K, minv, st); };
+  if (row_lanes(nb) == 1)
+    run(minv ? csr_rounds<true, 1> : csr_rounds<false, 1>);
   else
-    csr_rounds<false>(xa, xb, pairing, nb, x, v, rho, pc, K, nullptr, st);
+    run(minv ? csr_rounds<true, kRowLanes> : csr_rounds<false, kRowLanes>);
 }
 
 }  // namespace pbf
