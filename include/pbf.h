@@ -275,13 +275,19 @@ int pbf_batch_step(pbf_ctx* ctx, float* d_x, float* d_v, float* d_rho, const int
  * held fixed (the step is C1 across a set change: W and the kernel gradient
  * vanish with their first derivative at r = h). On a context that has run a
  * backward of that size, the forward records its last segment in the same
- * buffers and the next backward does not run it again. The rollout stays valid for
+ * buffers and the next backward does not run it again (pbf_rollout_record
+ * switches that off). The rollout stays valid for
  * repeated backward calls until the next pbf_rollout_forward or a parameter
  * change (PBF_ERR_INVALID). Returns PBF_ERR_UNSUPPORTED when a step had
  * particles outside the grid. pbf_rollout_backward is blocking. */
 int pbf_rollout_forward(pbf_ctx* ctx, float* d_x, float* d_v, float* d_rho, const int* d_scene_offsets,
                         int nscenes, int n, int nsteps, int checkpoint_every, void* stream);
 int pbf_rollout_backward(pbf_ctx* ctx, float* d_xbar, float* d_vbar, void* stream);
+/* Whether the forwards of the context record (on != 0, the default), for
+ * callers that know that no backward follows: recording costs a forward 1 to 8%
+ * and saves the backward that segment's steps. The results, and which calls are
+ * valid, are the same either way. */
+int pbf_rollout_record(pbf_ctx* ctx, int on);
 
 /* Reverse mode in double precision: pbf_rollout_forward / _backward with the
  * state (x, v, rho and their adjoints: packed xyz doubles, original order) and

@@ -130,7 +130,13 @@ void backward_call(int64_t handle, Tensor& xb, Tensor& vb, int64_t generation, i
 // x0 and v0 through the library's adjoint kernels (rho_N carries none).
 struct Rollout : public torch::autograd::Function<Rollout> {
   static variable_list forward(AutogradContext* fc, Tensor x0, Tensor v0, int64_t handle, int64_t nsteps,
-                               int64_t every, c10::optional<Tensor> offsets, int64_t stream) {
+                               int64_t every, c10::optional<Tensor> offsets, int64_t stream, bool differentiated) {
+    // without a gradient to come the forward records nothing for the backward
+    struct Recording {
+      pbf_ctx* c;
+      Recording(pbf_ctx* ctx, bool on) : c(ctx) { check(pbf_rollout_record(c, on), c); }
+      ~Recording() { (void)pbf_rollout_record(c, 1); }
+    } recording(ctx_of(handle), differentiated);
     Tensor x = x0.detach().clone().contiguous();
     Tensor v = v0.detach().clone().contiguous();
     Tensor rho = torch::empty({x.size(0)}, x.options());
@@ -150,7 +156,7 @@ struct Rollout : public torch::autograd::Function<Rollout> {
     Tensor vb = gv.defined() ? gv.detach().clone().contiguous() : torch::zeros_like(like);
     backward_call(fc->saved_data["handle"].toInt(), xb, vb, fc->saved_data["generation"].toInt(),
                   fc->saved_data["stream"].toInt());
-    return {xb, vb, Tensor(), Tensor(), Tensor(), Tensor(), Tensor()};
+    return {xb, vb, Tensor(), Tensor(), Tensor(), Tensor(), Tensor(), Tensor()};
   }
 };
 
@@ -161,7 +167,10 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("abi_version", &pbf_abi_version);
   m.def("rollout",
         [](Tensor x0, Tensor v0, int64_t handle, int64_t nsteps, int64_t every, c10::optional<Tensor> offsets,
-           int64_t stream) { return Rollout::apply(x0, v0, handle, nsteps, every, offsets, stream); },
+           int64_t stream) {
+          const bool differentiated = c10::GradMode::is_enabled() && (x0.requires_grad() || v0.requires_grad());
+          return Rollout::apply(x0, v0, handle, nsteps, every, offsets, stream, differentiated);
+        },
         "differentiable nsteps of the fluid step: (x_N, v_N, rho_N)");
   m.def("rollout_forward",
         [](int64_t handle, Tensor x, Tensor v, c10::optional<Tensor> rho, int64_t nsteps, int64_t every,

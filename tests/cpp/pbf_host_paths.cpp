@@ -508,6 +508,38 @@ void failed_rollout() {
     }
 }
 
+// Steps recorded by a forward (or run again by a reverse): where recording is off a
+// forward records none, and the reverse runs its segment again.
+void unrecorded_forward() {
+  auto taped = [] {
+    int k = 0;
+    for (const Launch& l : S().launches) k += l.name == "k_copy_cells";
+    S().launches.clear();
+    return k;
+  };
+  for (bool f64 : {false, true}) {
+    Arrays a(3000);
+    pbf_params p = small_params();
+    pbf_ctx* c = nullptr;
+    if (pbf_create(&p, &c) != PBF_OK) std::abort();
+    S().list_need = 96;
+    taped();
+    // a first rollout, recorded ones, one that is not, a recorded one again
+    const int on[] = {1, 1, 0, 0, 1}, want[] = {0, 2, 0, 0, 2};
+    for (int k = 0; k < 5; ++k) {
+      expect(pbf_rollout_record(c, on[k]) == PBF_OK, "pbf_rollout_record");
+      expect(forward(c, a, f64, 1500, 5, 3) == PBF_OK && taped() == want[k], "steps that the forward records");
+      expect(exported(c, a) == S().searches - 1, "lists of the forward");
+      if (k == 2) continue;  // nothing follows
+      S().launches.clear();
+      expect(backward(c, a, f64) == PBF_OK && taped() == 5 - want[k], "steps that the reverse runs");
+    }
+    expect(pbf_rollout_record(nullptr, 1) == PBF_ERR_INVALID, "null context");
+    pbf_destroy(c);
+    S().searched.clear();
+  }
+}
+
 // The row starts are in the caller's array when the call returns: nothing is copied
 // after its last wait, counted by this call or by one before.
 void blocking_export() {
@@ -651,6 +683,7 @@ const std::map<std::string, void (*)()> kScenarios = {
     {"pass_blocks", pass_blocks},
     {"viscosity_weights", viscosity_weights},
     {"blocking_export", blocking_export},
+    {"unrecorded_forward", unrecorded_forward},
     {"last_search", last_search},
     {"failed_rollout", failed_rollout},
     {"tape_slots", tape_slots},

@@ -72,3 +72,9 @@ def test_pass_block_that_the_caller_sets(host_paths):
     """pbf_tuning.pass_block is what the PBD passes run, lane pairs included; only the
     default settings leave it to the library (64 for lane pairs)."""
     run(host_paths, "pass_blocks")
+
+
+def test_forward_without_a_reverse_records_nothing(host_paths):
+    """With pbf_rollout_record off a forward records no step, whatever reverses ran
+    before; its lists are exported and a reverse still follows it."""
+    run(host_paths, "unrecorded_forward")
