@@ -829,15 +829,18 @@ int search(pbf_ctx* c, const float* x, const float* v, int n, const int* scene_o
   return search(c, SortIn{x, v, nullptr, nullptr, nullptr}, n, scene_off, nscenes, integrate, st);
 }
 
-bool capturing(hipStream_t st) {
+// Whether st is being captured: 1, 0, or -1 where HIP does not say (the null stream
+// while another stream is).
+int capture_state(hipStream_t st) {
   hipStreamCaptureStatus s = hipStreamCaptureStatusNone;
-  if (hipStreamIsCapturing(st, &s) == hipSuccess) return s != hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(st, &s) == hipSuccess) return s != hipStreamCaptureStatusNone ? 1 : 0;
   (void)hipGetLastError();
-  return true;  // not known: nothing that a capture would not allow
+  return -1;
 }
+bool capturing(hipStream_t st) { return capture_state(st) != 0; }  // not known: nothing that a capture would not allow
 
 int record_counters(pbf_ctx* c, hipStream_t st) {
-  if (!c->captured && capturing(st)) {
+  if (!c->captured && capture_state(st) > 0) {
     c->captured = true;
     c->tape_of = 0;
   }

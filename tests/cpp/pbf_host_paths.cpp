@@ -540,6 +540,33 @@ void unrecorded_forward() {
   }
 }
 
+// A call on a stream that HIP says nothing about (the null stream while another one
+// is captured) is not taken for a captured one: the forwards after it record again.
+void unknown_capture() {
+  for (bool f64 : {false, true}) {
+    Arrays a(3000);
+    pbf_params p = small_params();
+    pbf_ctx* c = nullptr;
+    if (pbf_create(&p, &c) != PBF_OK) std::abort();
+    S().list_need = 96;
+    expect(forward(c, a, f64, 1500, 5, 3) == PBF_OK && backward(c, a, f64) == PBF_OK, "rollout");
+    for (int state : {2, 1}) {
+      S().capturing = state;
+      expect(step(c, a, 1500) == PBF_OK, "step");
+      S().capturing = 0;
+      expect(S().last == hipSuccess, "an error left for the next call");
+      S().launches.clear();
+      expect(forward(c, a, f64, 1500, 5, 3) == PBF_OK, "forward");
+      int taped = 0;
+      for (const Launch& l : S().launches) taped += l.name == "k_copy_cells";
+      expect(taped == (state == 2 ? 2 : 0), "steps that the forward records");
+      expect(backward(c, a, f64) == PBF_OK, "reverse");
+    }
+    pbf_destroy(c);
+    S().searched.clear();
+  }
+}
+
 // The row starts are in the caller's array when the call returns: nothing is copied
 // after its last wait, counted by this call or by one before.
 void blocking_export() {
@@ -684,6 +711,7 @@ const std::map<std::string, void (*)()> kScenarios = {
     {"viscosity_weights", viscosity_weights},
     {"blocking_export", blocking_export},
     {"unrecorded_forward", unrecorded_forward},
+    {"unknown_capture", unknown_capture},
     {"last_search", last_search},
     {"failed_rollout", failed_rollout},
     {"tape_slots", tape_slots},

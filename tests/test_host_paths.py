@@ -78,3 +78,9 @@ def test_forward_without_a_reverse_records_nothing(host_paths):
     """With pbf_rollout_record off a forward records no step, whatever reverses ran
     before; its lists are exported and a reverse still follows it."""
     run(host_paths, "unrecorded_forward")
+
+
+def test_unknown_capture_state(host_paths):
+    """Where HIP cannot say whether the call's stream is being captured, the context is
+    not taken for a captured one for good (it would never record again)."""
+    run(host_paths, "unknown_capture")
