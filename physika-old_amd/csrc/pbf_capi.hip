@@ -176,6 +176,7 @@ struct pbf_ctx {
     unsigned long long gen = ~0ull;
     int n = -1, nscenes = -1, iters = -1;
     const int* off = nullptr;
+    bool even = false;  // its passes do not look at the counts (NbrView::maybe_uneven)
   } sg;
   long long graph_replays = 0, graph_captures = 0;
 
@@ -1102,7 +1103,7 @@ int step_once(pbf_ctx* c, const float* x_in, const float* v_in, float* x_out, fl
 int replay_middle_step(pbf_ctx* c, int n, const int* scene_off, int nscenes, CellState& cs, hipStream_t st) {
   auto& g = c->sg;
   if (!g.exec || g.gen != c->gen || g.n != n || g.nscenes != nscenes || g.off != scene_off ||
-      g.iters != c->p.iterations) {
+      g.iters != c->p.iterations || (g.even && !c->even)) {
     if (g.exec) {
       (void)hipGraphExecDestroy(g.exec);
       g.exec = nullptr;
@@ -1133,6 +1134,7 @@ int replay_middle_step(pbf_ctx* c, int n, const int* scene_off, int nscenes, Cel
     g.nscenes = nscenes;
     g.off = scene_off;
     g.iters = c->p.iterations;
+    g.even = n >= kUnevenMin && c->even;
     c->graph_captures++;
   }
   PBF_HIP(c, hipGraphLaunch(g.exec, st));

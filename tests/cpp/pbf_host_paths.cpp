@@ -49,8 +49,9 @@ struct State {
   long copy_fail_at = kNever;  // copies left until one fails
   hipError_t last = hipSuccess;
   int capturing = 0;        // hipStreamIsCapturing: 0 no, 1 yes, 2 an error
-  unsigned long long list_need = 0, calls = 0;
-  std::vector<Launch> launches;
+  unsigned long long list_need = 0, calls = 0, uneven = 0;
+  bool graph = false;  // between hipStreamBeginCapture and hipStreamEndCapture
+  std::vector<Launch> launches, recorded;  // recorded: by the last graph
   std::vector<std::string> ops;  // launches, copies and waits, in order
   std::map<const void*, long> searched;  // buffer of a search -> serial of the neighbor pass that last wrote it
   long searches = 0, exported = -1;      // exported: the search that the last export read
@@ -128,6 +129,10 @@ void launched(const void* f, dim3 block, void** args) {
       if (p && room(p) == 0) violation("%s: argument %zu (%s) points at no allocation: %p", k.name.c_str(), i, t.c_str(), p);
     }
   }
+  if (S().graph) {
+    S().recorded.push_back(l);
+    return;
+  }
   S().launches.push_back(l);
   S().ops.push_back(k.name);
   if (S().capturing == 1) return;
@@ -145,6 +150,7 @@ void launched(const void* f, dim3 block, void** args) {
     for (int c = 0; c < pbf::C_COUNT; ++c) host[c] = 0;
     host[pbf::C_LIST_NEED] = S().list_need;
     host[pbf::C_CALLS] = ++S().calls;
+    host[pbf::C_UNEVEN] = S().uneven;
   }
 }
 
@@ -310,6 +316,28 @@ hipError_t hipStreamDestroy(hipStream_t) { return hipSuccess; }
 hipError_t hipStreamIsCapturing(hipStream_t, hipStreamCaptureStatus* s) {
   if (S().capturing == 2) return S().last = hipErrorStreamCaptureImplicit;
   *s = S().capturing ? hipStreamCaptureStatusActive : hipStreamCaptureStatusNone;
+  return hipSuccess;
+}
+hipError_t hipStreamBeginCapture(hipStream_t, hipStreamCaptureMode) {
+  S().graph = true;
+  S().recorded.clear();
+  return hipSuccess;
+}
+hipError_t hipStreamEndCapture(hipStream_t, hipGraph_t* g) {
+  S().graph = false;
+  *g = reinterpret_cast<hipGraph_t>(8);
+  return hipSuccess;
+}
+hipError_t hipGraphInstantiate(hipGraphExec_t* x, hipGraph_t, hipGraphNode_t*, char*, size_t) {
+  *x = reinterpret_cast<hipGraphExec_t>(8);
+  S().ops.push_back("instantiate");
+  return hipSuccess;
+}
+hipError_t hipGraphDestroy(hipGraph_t) { return hipSuccess; }
+hipError_t hipGraphExecDestroy(hipGraphExec_t) { return hipSuccess; }
+hipError_t hipGraphLaunch(hipGraphExec_t, hipStream_t) {
+  for (const Launch& l : S().recorded) S().launches.push_back(l);
+  S().ops.push_back("replay");
   return hipSuccess;
 }
 hipError_t hipEventCreateWithFlags(hipEvent_t* e, unsigned) {
@@ -567,6 +595,41 @@ void unknown_capture() {
   }
 }
 
+// Frames replayed from a graph that was captured when the scene was even look at the
+// counts again once it is uneven; the graph stays otherwise.
+void replays_of_uneven_scenes() {
+  Arrays a(300000);
+  pbf_params p = small_params();
+  pbf_ctx* c = nullptr;
+  if (pbf_create(&p, &c) != PBF_OK) std::abort();
+  S().list_need = 96;
+  auto frames = [&](unsigned long long uneven_after) {  // how many passes look at the counts
+    S().launches.clear();
+    S().ops.clear();
+    S().uneven = uneven_after;
+    expect(pbf_step(c, a.x, a.v, a.rho, 280000, 4, nullptr) == PBF_OK, "frames");
+    int look = 0, passes = 0;
+    for (const Launch& l : S().launches)
+      if (l.name == "k_density_lambda") ++passes, look += l.nv.maybe_uneven;
+    expect(passes == 20, "passes of four frames");
+    return look;
+  };
+  auto captures = [&] {
+    int k = 0;
+    for (const std::string& op : S().ops) k += op == "instantiate";
+    return k;
+  };
+  expect(step(c, a, 280000) == PBF_OK, "a frame");  // says that the scene is even
+  S().uneven = 1;
+  expect(step(c, a, 280000) == PBF_OK, "a frame");
+  expect(frames(1) == 0 && captures() == 1, "an even scene");
+  expect(frames(2) == 0 && captures() == 0, "the scene turns uneven during the call");
+  expect(frames(2) == 20 && captures() == 1, "an uneven scene");
+  expect(frames(1) == 20 && captures() == 0, "it turns even again");
+  expect(frames(1) == 10 && captures() == 0, "the graph's frames still look, the others do not");
+  pbf_destroy(c);
+}
+
 // The row starts are in the caller's array when the call returns: nothing is copied
 // after its last wait, counted by this call or by one before.
 void blocking_export() {
@@ -712,6 +775,7 @@ const std::map<std::string, void (*)()> kScenarios = {
     {"blocking_export", blocking_export},
     {"unrecorded_forward", unrecorded_forward},
     {"unknown_capture", unknown_capture},
+    {"replays_of_uneven_scenes", replays_of_uneven_scenes},
     {"last_search", last_search},
     {"failed_rollout", failed_rollout},
     {"tape_slots", tape_slots},

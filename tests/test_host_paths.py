@@ -84,3 +84,9 @@ def test_unknown_capture_state(host_paths):
     """Where HIP cannot say whether the call's stream is being captured, the context is
     not taken for a captured one for good (it would never record again)."""
     run(host_paths, "unknown_capture")
+
+
+def test_replayed_frames_of_a_scene_that_turns_uneven(host_paths):
+    """A graph captured while the scene was even is captured again once it is uneven:
+    its frames then choose the block order by the counts, as the others do."""
+    run(host_paths, "replays_of_uneven_scenes")
