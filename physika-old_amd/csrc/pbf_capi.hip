@@ -78,6 +78,8 @@ struct pbf_ctx {
   int4* wave_stat = nullptr;     // per wave of the neighbor pass: pairs, candidates, need
   int stats_n = 0;               // particles of the last search whose statistics are not yet reduced
   bool even = false;             // the last finished call's search was even (kXcdChunk)
+  int counted_n = 0;             // particles of the last call's last search
+  float mean_row = 0.0f;         // neighbors per particle in the last finished call (0: none yet)
 
   int* scan_scratch = nullptr;
   size_t scan_scratch_n = 0;
@@ -615,6 +617,7 @@ int adapt_reservations(pbf_ctx* c) {
   if (hipEventQuery(c->counters_ev) != hipSuccess) return PBF_OK;
   c->counters_pending = false;
   c->even = c->h_counters[C_UNEVEN] == 1;
+  if (c->counted_n > 0) c->mean_row = (float)c->h_counters[C_PAIRS] / (float)c->counted_n;
   const long long mw = (long long)c->h_counters[C_MASK_WORDS];
   const long long need = (long long)c->h_counters[C_LIST_NEED];  // slots per particle of the fullest wave
   int st = PBF_OK;
@@ -663,6 +666,19 @@ NbrView view_of(const pbf_ctx* c, int n) {
 // spacings (4 a run; 32,768 particles 13.4 -> 11.9 us, 65,536 14.3 -> 19.8 us).
 int small_search_max(const pbf_ctx* c) {
   return c->p.smoothing_length >= 2.25f * c->p.sampling_distance ? 65536 : 32768;
+}
+
+// Whether a limited query's rows are inserted by one lane each: rows of a few
+// neighbors (as the last finished call's, or a fluid's at rest), which leave most of eight
+// lanes idle, and few places in a search that fills the chip anyway. One lane and
+// eight, us: rows of 7, limit 20, 50,000 particles 85 and 95, 400,000 143 and 185, 1,000,000
+// 243 and 330; rows of 14, 400,000 particles, limit 4 168 and 202, 20 209 and 205; rows of
+// 81, 1,000,000 particles, limit 4 617 and 639, 8 770 and 753; 50,000 particles, limit 2
+// 120 and 120, 4 127 and 122.
+bool fixed_inserts(const pbf_ctx* c, int n, int limit) {
+  const float spacings = c->p.smoothing_length / c->p.sampling_distance;
+  const float row = c->mean_row > 0.0f ? c->mean_row : 4.19f * spacings * spacings * spacings;
+  return row < 12.0f || (n >= 65536 && limit <= 4);
 }
 
 NbrOut out_of(pbf_ctx* c) {
@@ -847,6 +863,7 @@ int record_counters(pbf_ctx* c, hipStream_t st) {
   }
   // a reverse that started from a recorded segment alone searched nothing
   if (c->stats_n > 0) launch_wave_stats(c->wave_stat, c->stats_n, c->counters, c->h_counters_dev, st);
+  if (c->stats_n > 0) c->counted_n = c->stats_n;
   c->stats_n = 0;
   PBF_LAUNCHED(c);
   PBF_HIP(c, hipEventRecord(c->counters_ev, st));
@@ -2013,7 +2030,7 @@ int pbf_neighbor_query_fixed(pbf_ctx* c, const float* d_x, int n, int limit, int
   if (s) return s;
   s = search(c, d_x, nullptr, n, nullptr, 1, false, st);
   if (s) return s;
-  launch_nbr_fixed(view_of(c, n), c->perm, limit, d_counts, d_elems, st);
+  launch_nbr_fixed(view_of(c, n), c->perm, limit, fixed_inserts(c, n, limit), d_counts, d_elems, st);
   PBF_LAUNCHED(c);
   return record_counters(c, st);
 }

@@ -381,9 +381,10 @@ constexpr int kPairingSlots = 16, kPairingStride = 16, kPairingWords = kPairingS
 void launch_csr_constrain(float4* xa, float4* xb, unsigned long long* pairing, const Csr& nb, float* x, float* v,
                           float* rho, const PhysConst& pc, int K, const float* minv, hipStream_t st);
 // Fixed-capacity rows (the `limit` nearest of each neighbor set, by distance
-// then id) in original ids; limit <= kFixedMax.
+// then id) in original ids; limit <= kFixedMax; insert: a lane per particle.
 constexpr int kFixedMax = 32;
-void launch_nbr_fixed(const NbrView& nv, const int* perm, int limit, int* counts, int* elems, hipStream_t st);
+void launch_nbr_fixed(const NbrView& nv, const int* perm, int limit, bool insert, int* counts, int* elems,
+                      hipStream_t st);
 
 // Records msg as the context's last error and returns status (host code of
 // the library's other translation units).

@@ -1217,20 +1217,68 @@ struct ListRow {
 // (glm's dot, then sqrtf). Rows sorted by (distance, id), in original ids:
 // counts[i], elems[limit*i + k].
 //
-// Eight lanes share a particle. The (distance, id) keys of its neighbors go to
-// LDS, each lane counts for every eighth key how many are smaller, and a key
-// with fewer than `limit` below it belongs at that place: the same few
-// instructions per pair of keys on every lane, where an insertion into a
-// sorted row takes a serial, divergent loop per neighbor. A row of more than
-// kFixedKeys neighbors runs in rounds, the `limit` smallest keys of one round
-// in front of the next round's. 168 -> 39 us for 50,021 particles, limit 20.
+// k_nbr_fixed: eight lanes share a particle and put the (distance, id) keys of its
+// neighbors into LDS. Many places are ranked: each lane counts for every eighth key how
+// many are smaller, and a key with fewer than `limit` below it belongs at that place:
+// the same few instructions per pair of keys on every lane, where an insertion into a
+// sorted row takes a serial, divergent loop per neighbor. That is quadratic in the
+// row; few places, kFixedExtract of them to the longest row's keys, are extracted
+// instead, the smallest key above the last one each time (twelve places of 81 keys
+// take either way the same). When the room is used up only the `limit` smallest stay,
+// and later keys enter only below the largest of them. Particles, neighbors, limit:
+// one lane inserting, ranks alone, now, in us: 50,021 x 81, 20: 286, 131, 131; 300,000
+// x 81, 8: 387, 332, 294; 600,000 in blobs (up to 500), 8: 1,351, 1,970, 1,016; 32:
+// 3,116, 2,171, 1,681. k_nbr_fixed_insert: one lane per particle inserts, where
+// fixed_inserts (pbf_capi.hip) says so.
 constexpr int kFixedLanes = 8, kFixedRows = 64 / kFixedLanes;
 constexpr int kFixedKeys = 128;
-constexpr int kFixedPer = 5;  // keys that a lane ranks in one walk over the row
+constexpr int kFixedPer = 5;      // keys that a lane ranks in one walk over the row
+constexpr int kFixedExtract = 7;  // keys per place from which the places are extracted
+
+typedef unsigned long long FixedKey;  // (distance bits, id)
+__device__ __forceinline__ FixedKey fixed_key(float4 xi, float4 xj, int id) {
+#pragma clang fp contract(off)
+  const float dx = xi.x - xj.x, dy = xi.y - xj.y, dz = xi.z - xj.z;
+  const float d = sqrtf((dx * dx + dy * dy) + dz * dz);
+  return ((FixedKey)__float_as_uint(d) << 32) | (unsigned)id;
+}
+
+// The row of particle s by one lane: each neighbor is inserted into the sorted row K
+// (kStride keys apart).
+template <int kStride>
+__device__ __forceinline__ void fixed_insert(const NbrView& nv, int s, FixedKey* K, const int* __restrict__ perm,
+                                             int limit, int* __restrict__ counts, int* __restrict__ elems) {
+  const float4 xi = nv.xn[s];
+  int cnt = 0;
+  for_each_neighbor(
+      nv, s, [&](int j) { return nv.xn[j]; },
+      [&](int j, float4 xj) {
+        const FixedKey key = fixed_key(xi, xj, perm[j]);
+        int k;
+        if (cnt < limit) {
+          k = cnt++;
+        } else {
+          k = limit - 1;
+          if (key >= K[kStride * k]) return;
+        }
+        for (; k > 0 && key < K[kStride * (k - 1)]; --k) K[kStride * k] = K[kStride * (k - 1)];
+        K[kStride * k] = key;
+      });
+  const size_t i = (size_t)perm[s];
+  counts[i] = cnt;
+  for (int k = 0; k < cnt; ++k) elems[(size_t)limit * i + k] = (int)(unsigned)K[kStride * k];
+}
+
+__global__ __launch_bounds__(64) void k_nbr_fixed_insert(NbrView nv, const int* __restrict__ perm, int limit,
+                                                         int* __restrict__ counts, int* __restrict__ elems) {
+  __shared__ FixedKey keys[kFixedMax][64];
+  const int s = xcd_block(blockIdx.x, gridDim.x) * 64 + threadIdx.x;
+  if (s < nv.n) fixed_insert<64>(nv, s, &keys[0][threadIdx.x], perm, limit, counts, elems);
+}
 
 __global__ __launch_bounds__(64) void k_nbr_fixed(NbrView nv, const int* __restrict__ perm, int limit,
                                                   int* __restrict__ counts, int* __restrict__ elems) {
-  typedef unsigned long long u64;
+  typedef FixedKey u64;
   // one key more than a row holds: the eight rows' reads of one key each fall
   // into different banks
   __shared__ u64 keys[kFixedRows][kFixedKeys + 1];
@@ -1243,33 +1291,9 @@ __global__ __launch_bounds__(64) void k_nbr_fixed(NbrView nv, const int* __restr
   const WaveList wl = wave_list(nv, __builtin_amdgcn_readfirstlane(s >> 6));
   const float4 xi = nv.xn[s];
   const size_t i = (size_t)perm[s];
-  u64* K = keys[row];
-  auto key_of = [&](int j, float4 xj) {
-#pragma clang fp contract(off)
-    const float dx = xi.x - xj.x, dy = xi.y - xj.y, dz = xi.z - xj.z;
-    const float d = sqrtf((dx * dx + dy * dy) + dz * dz);
-    return ((u64)__float_as_uint(d) << 32) | (unsigned)perm[j];
-  };
-  if (wl.lb < 0) {
-    // no list (reservation full): one lane inserts into the sorted row
-    if (!active || q != 0) return;
-    int cnt = 0;
-    for_each_neighbor(
-        nv, s, [&](int j) { return nv.xn[j]; },
-        [&](int j, float4 xj) {
-          const u64 key = key_of(j, xj);
-          int k;
-          if (cnt < limit) {
-            k = cnt++;
-          } else {
-            k = limit - 1;
-            if (key >= K[k]) return;
-          }
-          for (; k > 0 && key < K[k - 1]; --k) K[k] = K[k - 1];
-          K[k] = key;
-        });
-    counts[i] = cnt;
-    for (int k = 0; k < cnt; ++k) elems[(size_t)limit * i + k] = (int)(unsigned)K[k];
+  u64* const K = keys[row];
+  if (wl.lb < 0) {  // no list (reservation full)
+    if (active && q == 0) fixed_insert<1>(nv, s, K, perm, limit, counts, elems);
     return;
   }
   ListRow lr;
@@ -1295,38 +1319,95 @@ __global__ __launch_bounds__(64) void k_nbr_fixed(NbrView nv, const int* __restr
         if (r[u] < limit) out(r[u], own[u]);
     }
   };
+  // the same, place by place: the smallest of the keys above the last one, of each
+  // lane's and then of the row's (keys differ: they hold the ids)
+  auto extract = [&](int n, auto&& out) {
+    const int places = min(n, limit);
+    u64 last = 0;
+    for (int r = 0; r < places; ++r) {
+      u64 m = ~0ull;
+      for (int k = q; k < n; k += kFixedLanes) {
+        const u64 kt = K[k];
+        m = (r == 0 || kt > last) && kt < m ? kt : m;
+      }
+#pragma unroll
+      for (int d = 1; d < kFixedLanes; d <<= 1) {
+        const u64 o = __shfl_xor(m, d);
+        m = o < m ? o : m;
+      }
+      last = m;
+      if (q == 0) out(r, m);
+    }
+  };
+  auto smallest = [&](int n, auto&& out) {  // by every lane of the wave
+    if (kFixedExtract * limit <= wave_max(n))
+      extract(n, out);
+    else
+      rank(n, out);
+  };
   const int nchunk = lr.chunks();
-  int kept = 0, c = 0, n = 0;
-  for (;;) {
-    const int c1 = min(c + ((kFixedKeys - kept) >> 3), nchunk), d0 = lr.before(c);
-    for (int cc = c + q; cc < c1; cc += kFixedLanes) {
+  u64 worst = ~0ull;  // once `limit` keys are kept: a key from here on has no place
+  bool kept = false;
+  int c = 0, n = 0;
+  while (__any(c < nchunk)) {
+    if (__any(n > kFixedKeys - 8)) {  // no room for a chunk: only the smallest stay
+      kept = true;
+      smallest(n, [&](int r, u64 k) { best[row][r] = k; });
+      wave_lds_fence();
+      n = min(n, limit);
+      for (int k = q; k < n; k += kFixedLanes) K[k] = best[row][k];
+      if (n == limit) worst = best[row][limit - 1];
+      wave_lds_fence();
+    }
+    const int c1 = min(c + min((kFixedKeys - n) >> 3, kFixedLanes), nchunk);
+    const int cc = c + q, left = cc < c1 ? lr.before(cc + 1) - lr.before(cc) : 0;
+    u64 key[8];
+    if (left > 0) {
       int j[8];
       lr.read(cc, s, j);
-      const int at = kept + lr.before(cc) - d0, left = lr.before(cc + 1) - lr.before(cc);
       float4 xj[8];
 #pragma unroll
       for (int u = 0; u < 8; ++u) xj[u] = nv.xn[j[u]];
 #pragma unroll
-      for (int u = 0; u < 8; ++u)
-        if (u < left) K[at + u] = key_of(j[u], xj[u]);
+      for (int u = 0; u < 8; ++u) key[u] = fixed_key(xi, xj[u], perm[j[u]]);
     }
-    n = kept + lr.before(c1) - d0;
-    c = c1;
-    wave_lds_fence();
-    if (!__any(c < nchunk)) break;
-    rank(n, [&](int r, u64 k) { best[row][r] = k; });
-    wave_lds_fence();
-    kept = min(n, limit);
-    for (int k = q; k < kept; k += kFixedLanes) K[k] = best[row][k];
+    if (!kept) {
+      const int at = n + lr.before(cc) - lr.before(c);
+#pragma unroll
+      for (int u = 0; u < 8; ++u)
+        if (u < left) K[at + u] = key[u];
+      n += lr.before(max(c, c1)) - lr.before(c);
+    } else {
+      // the keys that may have a place, the lanes' one after the other
+      unsigned take = 0;
+#pragma unroll
+      for (int u = 0; u < 8; ++u) take |= (u < left && key[u] < worst ? 1u : 0u) << u;
+      const int mine = __popc(take);
+      int upto = mine;
+#pragma unroll
+      for (int d = 1; d < kFixedLanes; d <<= 1) {
+        const int o = __shfl_up(upto, d, kFixedLanes);
+        upto += q >= d ? o : 0;
+      }
+      int at = n + upto - mine;
+#pragma unroll
+      for (int u = 0; u < 8; ++u)
+        if (take >> u & 1) K[at++] = key[u];
+      n += __shfl(upto, kFixedLanes - 1, kFixedLanes);
+    }
+    c = max(c, c1);
     wave_lds_fence();
   }
-  if (!active) return;
-  if (q == 0) counts[i] = min(lr.cnt, limit);
-  rank(n, [&](int r, u64 k) { elems[(size_t)limit * i + r] = (int)(unsigned)k; });
+  if (active && q == 0) counts[i] = min(lr.cnt, limit);
+  smallest(n, [&](int r, u64 k) { elems[(size_t)limit * i + r] = (int)(unsigned)k; });  // n is 0 past the last particle
 }
 
-void launch_nbr_fixed(const NbrView& nv, const int* perm, int limit, int* counts, int* elems, hipStream_t st) {
-  k_nbr_fixed<<<(nv.n + kFixedRows - 1) / kFixedRows, 64, 0, st>>>(nv, perm, limit, counts, elems);
+void launch_nbr_fixed(const NbrView& nv, const int* perm, int limit, bool insert, int* counts, int* elems,
+                      hipStream_t st) {
+  if (insert)
+    k_nbr_fixed_insert<<<(nv.n + 63) / 64, 64, 0, st>>>(nv, perm, limit, counts, elems);
+  else
+    k_nbr_fixed<<<(nv.n + kFixedRows - 1) / kFixedRows, 64, 0, st>>>(nv, perm, limit, counts, elems);
 }
 
 // ---------------------------------------------------------------------------
