@@ -375,9 +375,11 @@ void launch_aos_to_f4(const float* x, float4* xa, int n, hipStream_t st);
 // DensityPBD::constrain, K rounds, over a caller list of any form: xa and xb
 // hold n float4 each, pairing kPairingWords words (nothing of them is read
 // before it is written): kPairingSlots sums, each in a line of its own, since the
-// blocks' atomics to one line wait for each other (15,625 blocks, 1,000,000 rows: 78 us
-// of a first pass of 100, 3 of 14 with a line each and one lane per row).
-constexpr int kPairingSlots = 16, kPairingStride = 16, kPairingWords = kPairingSlots * kPairingStride;
+// blocks' atomics to one line wait for each other and every later pass reads all of
+// them. Five iterations with 16 sums in one line, 16, 4 and 1 in a line each, us: 262,144
+// rows of 72 elements 350, 356, 349 and 371; 1,000,000 rows of 7 (both ways, one lane) 341
+// with four lanes, 207, 197 and 229.
+constexpr int kPairingSlots = 4, kPairingStride = 16, kPairingWords = kPairingSlots * kPairingStride;
 void launch_csr_constrain(float4* xa, float4* xb, unsigned long long* pairing, const Csr& nb, float* x, float* v,
                           float* rho, const PhysConst& pc, int K, const float* minv, hipStream_t st);
 // Fixed-capacity rows (the `limit` nearest of each neighbor set, by distance
