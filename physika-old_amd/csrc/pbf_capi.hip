@@ -186,6 +186,7 @@ struct pbf_ctx {
   unsigned long long* h_counters = nullptr;   // pinned, mapped host copy, written by k_wave_stats
   unsigned long long* h_counters_dev = nullptr;  // its device address
   hipEvent_t counters_ev = nullptr;
+  hipEvent_t starts_ev = nullptr;  // export_csr
   bool counters_pending = false;
 
   float4* vis_w = nullptr;  // weights of a viscosity solve (vis_weights)
@@ -885,12 +886,14 @@ int export_csr(pbf_ctx* c, int n, int* d_index, int* d_elems, long long cap, lon
     return hipMemcpyAsync(d_index, c->cnt_orig, sizeof(int) * (size_t)n, hipMemcpyDeviceToDevice, st);
   };
   bool counted = c->csr_total >= 0;
-  if (counted) {
-    PBF_HIP(c, starts());
+  if (counted && c->captured) {  // a replay may have searched
     PBF_HIP(c, hipStreamSynchronize(st));
     counted = c->csr_calls == c->h_counters[C_CALLS];
   }
-  if (!counted) {
+  if (counted) {
+    PBF_HIP(c, starts());
+    PBF_HIP(c, hipEventRecord(c->starts_ev, st));  // waited for below, while the lists are written
+  } else {
     launch_invert(c->perm, c->inv, n, st);
     launch_csr_count(c->nbr_cnt, c->inv, n, c->cnt_orig, st);
     // cnt_orig holds cap_n > n entries: the scan writes n + 1 in place
@@ -904,13 +907,16 @@ int export_csr(pbf_ctx* c, int n, int* d_index, int* d_elems, long long cap, lon
     c->csr_calls = c->h_counters[C_CALLS];
   }
   *total = c->csr_total;
-  if (d_elems == nullptr) return PBF_OK;
-  if (cap < c->csr_total)
-    return fail(c, PBF_ERR_CAPACITY, "neighbor element buffer holds " + std::to_string(cap) + ", need " +
-                                         std::to_string(c->csr_total));
-  launch_csr_fill(view_of(c, n), c->perm, c->cnt_orig, d_elems, cap, st);
-  PBF_LAUNCHED(c);
-  return PBF_OK;
+  int s = PBF_OK;
+  if (d_elems != nullptr && cap < c->csr_total) {
+    s = fail(c, PBF_ERR_CAPACITY, "neighbor element buffer holds " + std::to_string(cap) + ", need " +
+                                      std::to_string(c->csr_total));
+  } else if (d_elems != nullptr) {
+    launch_csr_fill(view_of(c, n), c->perm, c->cnt_orig, d_elems, cap, st);
+    PBF_LAUNCHED(c);
+  }
+  if (counted) PBF_HIP(c, hipEventSynchronize(c->starts_ev));
+  return s;
 }
 
 // A caller's list (index of n row starts, nelems elements) as the kernels
@@ -1521,6 +1527,7 @@ int pbf_create(const pbf_params* p, pbf_ctx** out) {
       hipHostMalloc(&c->h_counters, sizeof(unsigned long long) * C_COUNT, hipHostMallocMapped) != hipSuccess ||
       hipHostGetDevicePointer((void**)&c->h_counters_dev, c->h_counters, 0) != hipSuccess ||
       hipEventCreateWithFlags(&c->counters_ev, hipEventDisableTiming) != hipSuccess ||
+      hipEventCreateWithFlags(&c->starts_ev, hipEventDisableTiming) != hipSuccess ||
       hipStreamCreateWithFlags(&c->cap_stream, hipStreamNonBlocking) != hipSuccess ||
       hipMalloc(&c->total_cells, sizeof(int)) != hipSuccess ||
       hipMalloc(&c->scan_part, sizeof(int) * 2 * kScanDevBlocks) != hipSuccess ||
@@ -1569,6 +1576,7 @@ int pbf_destroy(pbf_ctx* c) {
   dfree(c->counters);
   if (c->h_counters) (void)hipHostFree(c->h_counters);
   if (c->counters_ev) (void)hipEventDestroy(c->counters_ev);
+  if (c->starts_ev) (void)hipEventDestroy(c->starts_ev);
   if (c->sg.exec) (void)hipGraphExecDestroy(c->sg.exec);
   if (c->cap_stream) (void)hipStreamDestroy(c->cap_stream);
   for (auto& m : c->marks) {
