@@ -110,8 +110,9 @@ __global__ __launch_bounds__(kBlock) void k_csr_begin(const float* __restrict__ 
 // Whether every listed pair is listed both ways, with equal multiplicity: the
 // matrix A of the list (A_ij: how often row i lists j) is symmetric exactly
 // when the bilinear form sum_ij (A_ij - A_ji) r_i s_j vanishes for all r, s.
-// Row i adds r_i sum_j s_j - s_i sum_j r_j with r, s two 64-bit SplitMix64
-// values per particle (Freivalds' check of a matrix identity, modulo 2^64): a
+// Row i adds r_i sum_j s_j - s_i sum_j r_j with r a 64-bit SplitMix64 value per
+// particle and s another xorshift-multiply mix of it (Freivalds' check of a matrix
+// identity, modulo 2^64): a
 // symmetric list gives 0, another one does with probability of order 2^-60.
 // Only integers are added, so the sum depends on no order.
 __device__ __forceinline__ unsigned long long pairing_r(int j) {

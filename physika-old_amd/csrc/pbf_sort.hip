@@ -391,7 +391,11 @@ __device__ __forceinline__ void scene_windows(const WindowOut& o, BLoad&& bload)
 
 // Whether this workgroup is the last of the launch to get here (each of them
 // calls this once, with all its threads): the words that every workgroup's
-// thread 0 wrote before with share_store are then there for share_load.
+// thread 0 wrote before with share_store are then there for share_load. The
+// order is this chip's, not the language's: agent-scope stores are written through
+// the L2, the wait holds the ticket back until they are acknowledged, and
+// agent-scope loads pass the caches by. A release on the ticket would also write
+// the rest of the L2 back, which nothing here needs.
 __device__ __forceinline__ bool last_block(int* ticket) {
   __shared__ int mine;
   if (threadIdx.x == 0) {
