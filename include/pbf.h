@@ -360,8 +360,9 @@ typedef struct pbf_tuning {
   int pass_block;          /* threads per workgroup of the density/lambda and
                               displacement passes: 64, 128, 256 (default) or
                               512. While every field has its default, a lane
-                              pair per particle runs in workgroups of 64 where
-                              its list has at most 384 slots */
+                              pair per particle runs in workgroups of 64, unless
+                              lists have more than 384 slots, most of them used,
+                              and the search fills the chip evenly */
   int stage_min_particles; /* as pbf_params.stage_min_particles: searches over at
                               least this many particles stage their neighbor
                               lists in LDS; < 0 never */

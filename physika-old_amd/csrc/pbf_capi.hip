@@ -1030,9 +1030,16 @@ int reserve(pbf_ctx* c, int n, int nscenes) {
 }
 
 // Threads per workgroup of the PBD passes: the caller's setting, or by default
-// kPairBlock for lane pairs, unless their lists are long.
-int pass_block_for(const pbf_ctx* c, int lanes) {
-  return lanes == 2 && c->auto_block && list_per_of(c) <= kLongLists ? kPairBlock : c->pass_block;
+// kPairBlock for lane pairs, unless their lists are long and even (the mean row takes
+// most of the slots) and the workgroups are: many, or at least 19 of 20 places are taken
+// when each SIMD has as many waves as the fullest one.
+int pass_block_for(const pbf_ctx* c, int n, int lanes) {
+  if (lanes != 2 || !c->auto_block) return c->pass_block;
+  const int per = list_per_of(c);
+  const long long waves = (2ll * n + 63) / 64, rounds = (waves + kSimds - 1) / kSimds;
+  const bool shared = per > kLongLists && c->mean_row > 0.6f * (float)per &&
+                      (n >= 131072 || (n >= 65536 && 20 * waves >= 19 * rounds * kSimds));
+  return shared ? c->pass_block : kPairBlock;
 }
 
 // One fused step on a batch of scenes (scene_off: device offsets): the state
@@ -1072,7 +1079,7 @@ int step_once(pbf_ctx* c, const float* x_in, const float* v_in, float* x_out, fl
   if (s) return s;
   NbrView nv = view_of(c, n);
   const int lanes = pass_lanes_for(c, n);
-  const int block = pass_block_for(c, lanes);
+  const int block = pass_block_for(c, n, lanes);
   c->last_lanes = lanes;
   float4* bufs[2] = {c->xa, c->xb};
   if (K == 0 && !visc) launch_write_back(c->x0, c->vs, c->perm, n, x_out, v_out, st);

@@ -277,13 +277,16 @@ void launch_wave_stats(const int4* wave_stat, int n, unsigned long long* counter
 // 32,768 2,013 -> 1,986; a frame at 1,728 95.5 -> 93.1; four steps and gradient in
 // double at 8 x 5,000 2.47 -> 2.12 ms. One lane per particle (1M): 64, 128 and 256 alike.
 constexpr int kPairBlock = 64;
-// With lists of more than kLongLists reserved slots the PBD passes' lane pairs keep
-// 256 threads: many rounds of gathers even the last round out, and four list
-// waves together share more of their neighbors. Rows of 440 neighbors (496
-// slots), one step, 64 and 256 threads: 65,536 particles 448 and 432 us, 131,072
-// 983 and 953, 262,143 1,770 and 1,650, but 100,003 890 and 908; rows of 270 (304
-// slots) 305 and 298, 614 and 606, 1,010 and 998, but 540 and 575.
-constexpr int kLongLists = 384;
+// With lists of more than kLongLists reserved slots, most of them used, the PBD
+// passes' lane pairs keep 256 threads where their waves fill the SIMDs evenly, and from
+// 131,072 particles on (pass_block_for): four list waves together share more of their
+// neighbors, but a last round of such workgroups, or one wave's longer rows, leaves CUs
+// idle. Rows of 340 neighbors (452 slots), one step, 64 and 256 threads, us: 65,536 particles
+// 406 and 393, 131,072 900 and 869, 200,000 1,250 and 1,215, 250,000 1,515 and 1,445, but
+// 50,000 370 and 378, 80,000 673 and 711, 100,000 797 and 826; dense blobs (rows of 253 in
+// 540 slots to 542 in 1,036) of 140,000 1,550 and 1,691, 200,000 4,816 and 4,837, 262,000
+// 9,132 and 9,653.
+constexpr int kLongLists = 384, kSimds = 4 * 256;
 // block: threads per workgroup, 64, 128, 256 or 512; persistent: as many
 // blocks as stay resident, each wave walking 64-particle tiles; lanes: 1, or 2
 // for a lane pair per particle (not persistent). The results depend on none of

@@ -764,7 +764,7 @@ __device__ __forceinline__ void density_lambda_at(const NbrView& nv, int s, floa
   density_lambda_finish(s, xs, pc, rho_out, perm, aux, t);
 }
 
-constexpr int kPairWaves = 5, kSimds = 4 * 256;  // see pair_waves
+constexpr int kPairWaves = 5;  // see pair_waves
 
 // Pass A with a lane pair per particle (lane h = 0 the even entries, 1 the
 // odd ones; stage: the hardware wave's LDS region). Same results as

@@ -49,7 +49,7 @@ struct State {
   long copy_fail_at = kNever;  // copies left until one fails
   hipError_t last = hipSuccess;
   int capturing = 0;        // hipStreamIsCapturing: 0 no, 1 yes, 2 an error
-  unsigned long long list_need = 0, calls = 0, uneven = 0;
+  unsigned long long list_need = 0, calls = 0, uneven = 0, pairs = 0;
   bool graph = false;  // between hipStreamBeginCapture and hipStreamEndCapture
   std::vector<Launch> launches, recorded;  // recorded: by the last graph
   std::vector<std::string> ops;  // launches, copies and waits, in order
@@ -151,6 +151,7 @@ void launched(const void* f, dim3 block, void** args) {
     host[pbf::C_LIST_NEED] = S().list_need;
     host[pbf::C_CALLS] = ++S().calls;
     host[pbf::C_UNEVEN] = S().uneven;
+    host[pbf::C_PAIRS] = S().pairs;
   }
 }
 
@@ -757,7 +758,14 @@ void pass_blocks() {
     expect(pbf_set_tuning(c, &(t = pbf_tuning{256, 0, 0, 0})) == PBF_OK, "the defaults");
     pbf_ctx* wide = nullptr;
     if (pbf_create(&q, &wide) != PBF_OK) std::abort();
-    expect(block(wide, 2000) == 256, "the default, lane pairs with long lists");
+    for (int n : {2000, 65536, 80000, 131000, 200000})
+      for (int row : {300, 200}) {  // of 400 slots
+        S().pairs = (unsigned long long)row * (unsigned)n;
+        (void)block(wide, n);  // says how long the rows are
+        const bool even = row == 300 && (n == 65536 || n >= 131000);
+        expect(block(wide, n) == (even ? 256 : 64), "the default, lane pairs with long lists");
+      }
+    S().pairs = 0;
     pbf_destroy(wide);
     expect(pbf_set_tuning(c, &t) == PBF_OK && block(c, 2000) == 64, "back to the defaults");
     pbf_tune_report r;
